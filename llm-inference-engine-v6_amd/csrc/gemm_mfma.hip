@@ -27,6 +27,8 @@
 // a slab of a tile being whole blocks, and puts it into LDS as rows as before.
 #include "common.h"
 
+#include <type_traits>
+
 namespace llme {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
@@ -65,10 +67,20 @@ template <int MODE> __device__ __forceinline__ float stored_value(float v) {
 constexpr bool is_gated(int mode) {
     return mode == kGatedBF16 || mode == kGatedReluBF16 || mode == kGatedGeluBF16 || mode == kGatedExtraBF16;
 }
+// z sigmoid(a z), a z given: the exponential as 2^(hi + lo) with hi + lo = log2(e) (-a z) in two pieces (the piece that the first
+// product rounds away put back as a factor 1 + ln(2) lo), then one hardware reciprocal. A gated epilogue is bound by this
+// arithmetic: expf and a division are twice the instructions.
+__device__ __forceinline__ float times_sigmoid(float z, float az) {
+    const float x = fminf(-az, 150.f);                  // (2^hi is infinite there and the result zero; lo stays finite)
+    const float hi = x * 1.44269504f;
+    const float lo = __builtin_fmaf(x, 1.44269504f, -hi) + x * 1.92596299e-8f;
+    const float e = __builtin_amdgcn_exp2f(hi);
+    return z * __builtin_amdgcn_rcpf(__builtin_fmaf(e, __builtin_fmaf(lo, 0.693147181f, 1.0f), 1.0f));
+}
 template <int MODE> __device__ __forceinline__ float gate_act(float g) {
     if (MODE == kGatedReluBF16) return fmaxf(g, 0.f);
     if (MODE == kGatedGeluBF16) return 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g)));
-    return g / (1.0f + expf(-g));
+    return times_sigmoid(g, g);
 }
 // What kGatedExtraBF16 does around the activation. bias [N] in the order of w's rows (so in the order of the product's
 // columns): added to gate and up first. limit > 0: gate <- min(gate, limit), up <- clamp(up, -limit, limit) and the
@@ -94,9 +106,9 @@ template <int MODE> __device__ __forceinline__ float gated_value(float g, float 
     if (gx.limit > 0.f) {
         g = fminf(g, gx.limit);
         u = fminf(fmaxf(u, -gx.limit), gx.limit);
-        return g / (1.0f + expf(-gx.alpha * g)) * (u + 1.0f);
+        return times_sigmoid(g, gx.alpha * g) * (u + 1.0f);
     }
-    return g / (1.0f + expf(-g)) * u;
+    return times_sigmoid(g, g) * u;
 }
 // The extras of the launches that an entry point is making (set and cleared inside one call, on the caller's thread).
 static thread_local GateExtra t_gate_extra;
@@ -670,13 +682,19 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(const bf16* __restric
 // LDS is cut into three buffers for A's slabs (64 k each) and four for halves of W's slabs (32 k:
 // one block per 16 rows), so that A is asked for two slabs ahead and W three half slabs: with two
 // buffers of whole slabs the loads, asked for one slab ahead, arrived late (from asking for A's
-// 32 KB to having them takes 1.06 us, W's 1.4 us, a slab's products 1.1 us; 1,060 against 1,111
-// TFLOP/s). The price is a barrier per half slab, at which a half buffer of W changes hands. The
-// loads are counted by hand (nothing else of a turn goes through the vector memory path).
+// 32 KB to having them takes 1.06 us, W's 1.4 us, a slab's products 1.1 us). The price is a barrier
+// per half slab, at which a half buffer of W changes hands. The loads are counted by hand (nothing
+// else of a turn goes through the vector memory path).
 // Half turn h (k = 32 h ..) has its operands in registers when it starts. It waits for half slab
-// h + 1, meets the barrier, asks for W's half slab h + 4 into the buffer of h, which everybody has
-// read, and, if h is odd, for A's slab (h - 1) / 2 + 3 into the buffer of the slab that ends here;
-// then it reads the operands of h + 1 while it multiplies.
+// h + 1, meets the barrier, and, row of tiles by row of tiles, multiplies, reads the operands of h + 1 and
+// asks for W's half slab h + 4 (into the buffer of h, which everybody has read) and half of an A slab: an odd
+// half turn for the first half of slab (h - 1) / 2 + 3 (into the buffer of the slab that ends here), the even
+// one behind it for the second. A half turn of 32 products a wavefront is 1,024 cycles of the matrix pipe: with all
+// of a half turn's loads asked for in one go, A's only in every second, it took 1,480 to 1,570 cycles; dealt out over
+// the rows and over both half turns it takes 1,300 to 1,360 (without loads 1,140; 8,191 x 28,672 x 4,096 went from 1,265 to
+// 1,311 TFLOP/s by this). The chip lowers its clock under this load (1.9 of 2.4 GHz), so fewer stalls win less than
+// their cycles. (Four wavefronts of 128 x 128 read a third less of LDS: 1,360 to 1,390 cycles at 2.05 GHz, and the
+// epilogue with half the wavefronts took more than that won.)
 // Needs: W blocked (N a multiple of 16, K of 32). A slab that hangs over the end of k reads zeros
 // there (the loads of A's second half get an offset behind the descriptor's end).
 constexpr int DK = 64;
@@ -699,18 +717,191 @@ __device__ __forceinline__ void load_b128_to_lds(u32x4 rsrc, unsigned lds_base, 
                  : "s"(lds_base), "v"(voffset), "s"(rsrc), "s"(soffset)
                  : "memory", "m0");
 }
+// The end of the direct kernel. Everything that is stored in bfloat16 becomes it in the registers that the products left it in
+// (a gate and its up, a rotated entry and its partner are columns of one lane), so that the whole tile fits into LDS at once and
+// goes out in pieces of 16 bytes behind one barrier; 32-bit sums go through LDS in two passes, and what they are added to is asked
+// for before a pass is staged. (Measured on a tile of 256 x 256, from the last product to the last store issued: gated 8.6 us
+// when it went through LDS in 32 bits, adding 21 us when a thread asked for its addends piece by piece.)
+template <int WR, int WC, int WMT, int WNT, int MODE>
+__device__ __forceinline__ void direct_epilogue(f32x4 (&acc)[WMT][WNT], unsigned char* lds_raw, void* __restrict__ out, int M, int N,
+                                                int m0, int n0, int wm, int wn, int tid, int r, int q, const QkvTarget& qt,
+                                                const RowPlace& place, const GateExtra& gx) {
+    constexpr int BM = WR * 16 * WMT, BN = WC * 16 * WNT, NT = 64 * WR * WC;
+    if (is_gated(MODE) || is_stored_bf16(MODE) || MODE == kRopeCache) {
+        constexpr int COLS = is_gated(MODE) ? BN / 2 : BN, SH = COLS + 8;        // (rows 16 bytes off the banks' round)
+        static_assert(static_cast<size_t>(BM) * SH * 2 + BM * 8 <= 160 * 1024, "the tile fits into LDS");
+        bf16* stage = reinterpret_cast<bf16*>(lds_raw);
+        int* row_pos = reinterpret_cast<int*>(lds_raw + static_cast<size_t>(BM) * SH * 2);
+        int* row_page = row_pos + BM;
+        if (is_gated(MODE)) {
+            float bg[WNT / 2], bu[WNT / 2];
+#pragma unroll
+            for (int j = 0; j < WNT / 2; ++j) {
+                const int n = n0 + wn + j * 32 + r;
+                const bool biased = MODE == kGatedExtraBF16 && gx.bias != nullptr && n < N;
+                bg[j] = biased ? static_cast<float>(gx.bias[n]) : 0.f;
+                bu[j] = biased ? static_cast<float>(gx.bias[n + 16]) : 0.f;
+            }
+#pragma unroll
+            for (int i = 0; i < WMT; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int row = wm + i * 16 + q * 4 + e;
+                    const float rs = MODE == kGatedExtraBF16 && m0 + row < M ? gate_row_scale(gx, m0 + row) : 1.f;
+#pragma unroll
+                    for (int j = 0; j < WNT / 2; ++j)
+                        stage[row * SH + wn / 2 + j * 16 + r] = static_cast<__bf16>(
+                            gated_value<MODE>(acc[i][2 * j][e] * rs, acc[i][2 * j + 1][e] * rs, gx, bg[j], bu[j]));
+                }
+        } else if (is_stored_bf16(MODE)) {
+#pragma unroll
+            for (int i = 0; i < WMT; ++i)
+#pragma unroll
+                for (int j = 0; j < WNT; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        stage[(wm + i * 16 + q * 4 + e) * SH + wn + j * 16 + r] = static_cast<__bf16>(stored_value<MODE>(acc[i][j][e]));
+        } else {
+            // heads of 64 or 128 columns: whole ones in a wavefront's columns; dims i and i + hd / 2 are columns hd / 32 tiles apart
+            if (tid < BM) {
+                row_pos[tid] = place.pos;
+                row_page[tid] = place.page;
+            }
+            __syncthreads();
+            auto rotate = [&](auto ht) {
+                constexpr int HT = decltype(ht)::value;             // tiles of half a head
+                const int half = 16 * HT;
+#pragma unroll
+                for (int i = 0; i < WMT; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int row = wm + i * 16 + q * 4 + e;
+                        const float* cs = qt.cos_t + static_cast<size_t>(row_pos[row]) * half + r;
+                        const float* sn = qt.sin_t + static_cast<size_t>(row_pos[row]) * half + r;
+                        float c[HT], s[HT];
+#pragma unroll
+                        for (int j = 0; j < HT; ++j) {
+                            c[j] = cs[j * 16];
+                            s[j] = sn[j * 16];
+                        }
+#pragma unroll
+                        for (int h = 0; h < WNT / (2 * HT); ++h) {
+                            const bool rotated = (n0 + wn) / (2 * half) + h < qt.n_q + qt.n_kv;
+#pragma unroll
+                            for (int j = 0; j < HT; ++j) {
+                                const float x = acc[i][h * 2 * HT + j][e], y = acc[i][h * 2 * HT + HT + j][e];
+                                bf16* sp = stage + row * SH + wn + h * 2 * half + j * 16 + r;
+                                sp[0] = static_cast<__bf16>(rotated ? x * c[j] - y * s[j] : x);
+                                sp[half] = static_cast<__bf16>(rotated ? y * c[j] + x * s[j] : y);
+                            }
+                        }
+                    }
+            };
+            if (qt.hd == 64) rotate(std::integral_constant<int, 2>{});
+            else rotate(std::integral_constant<int, 4>{});
+        }
+        __syncthreads();
+        constexpr int PIECES = COLS / 8;                            // of 16 bytes, a row
+        if (MODE != kRopeCache) {
+            const int ld = is_gated(MODE) ? N / 2 : N, c0 = is_gated(MODE) ? n0 / 2 : n0;
+#pragma unroll 4
+            for (int idx = tid; idx < BM * PIECES; idx += NT) {
+                const int row = idx / PIECES, col = (idx % PIECES) * 8;
+                if (m0 + row >= M || c0 + col >= ld) continue;
+                *reinterpret_cast<bf16x8*>(static_cast<bf16*>(out) + static_cast<size_t>(m0 + row) * ld + c0 + col) =
+                    *reinterpret_cast<const bf16x8*>(stage + row * SH + col);
+            }
+            return;
+        }
+        const int hd = qt.hd, rotated = qt.n_q + qt.n_kv;
+        for (int idx = tid; idx < BM * PIECES; idx += NT) {
+            const int row = idx / PIECES, col = (idx % PIECES) * 8;
+            const int m = m0 + row, head = (n0 + col) / hd, d = (n0 + col) % hd;
+            if (m >= M || head >= rotated) continue;
+            const int pos = row_pos[row];
+            bf16* dst = head < qt.n_q
+                ? qt.q_out + (static_cast<size_t>(m) * qt.n_q + head) * hd + d
+                : qt.k_cache + ((static_cast<size_t>(row_page[row]) * qt.n_kv + (head - qt.n_q)) * qt.page + pos % qt.page) * hd + d;
+            *reinterpret_cast<bf16x8*>(dst) = *reinterpret_cast<const bf16x8*>(stage + row * SH + col);
+        }
+        // v: a thread takes one dim of 16 consecutive rows, which lie together in the transposed page where they are 16
+        // consecutive positions of one request that begin at a multiple of 16 (a page belongs to one request)
+        for (int idx = tid; idx < (BM / 16) * BN; idx += NT) {
+            const int row = idx / BN * 16, col = idx % BN;
+            const int n = n0 + col, kvh = n / hd - rotated, d = n % hd, m = m0 + row;
+            if (kvh < 0 || n >= N || m >= M) continue;
+            const int nt = M - m < 16 ? M - m : 16;
+            const bf16* sp = stage + row * SH + col;
+            const int pos0 = row_pos[row];
+            if (nt == 16 && row_page[row] == row_page[row + 15] && pos0 % 16 == 0 && qt.page % 16 == 0 && row_pos[row + 15] == pos0 + 15) {
+                bf16* dst = qt.v_cache + ((static_cast<size_t>(row_page[row]) * qt.n_kv + kvh) * hd + d) * qt.page + pos0 % qt.page;
+                bf16x8 lo, hi;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    lo[j] = sp[j * SH];
+                    hi[j] = sp[(j + 8) * SH];
+                }
+                *reinterpret_cast<bf16x8*>(dst) = lo;
+                *reinterpret_cast<bf16x8*>(dst + 8) = hi;
+            } else {
+                for (int j = 0; j < nt; ++j)
+                    qt.v_cache[((static_cast<size_t>(row_page[row + j]) * qt.n_kv + kvh) * hd + d) * qt.page + row_pos[row + j] % qt.page] = sp[j * SH];
+            }
+        }
+        return;
+    }
+    constexpr int PASSES = 2, HB = BM / PASSES, SS = BN + 4, PIECES = BN / 4, COUNT = HB * PIECES / NT;
+    static_assert(WR % PASSES == 0 && HB * PIECES % NT == 0 && static_cast<size_t>(HB) * SS * 4 <= 160 * 1024, "a pass is whole wavefront rows");
+    float* stage = reinterpret_cast<float*>(lds_raw);
+    float* o = static_cast<float*>(out);
+    float4 had[COUNT];
+    auto ask = [&](int pass) {                                      // (pieces past an edge ask for a place that exists)
+#pragma unroll
+        for (int it = 0; it < COUNT; ++it) {
+            const int idx = tid + it * NT;
+            const int m = m0 + pass * HB + idx / PIECES, n = n0 + (idx % PIECES) * 4;
+            had[it] = *reinterpret_cast<const float4*>(o + (m < M && n < N ? static_cast<size_t>(m) * N + n : 0));
+        }
+    };
+#pragma unroll
+    for (int pass = 0; pass < PASSES; ++pass) {
+        if (MODE == kAddF32) ask(pass);
+        if (pass > 0) __syncthreads();                              // (the pass before has been read)
+        if (wm / HB == pass) {
+#pragma unroll
+            for (int i = 0; i < WMT; ++i)
+#pragma unroll
+                for (int j = 0; j < WNT; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) stage[(wm - pass * HB + i * 16 + q * 4 + e) * SS + wn + j * 16 + r] = acc[i][j][e];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int it = 0; it < COUNT; ++it) {
+            const int idx = tid + it * NT;
+            const int row = idx / PIECES, col = (idx % PIECES) * 4;
+            const int m = m0 + pass * HB + row, n = n0 + col;
+            if (m >= M || n >= N) continue;
+            float4 v = *reinterpret_cast<const float4*>(stage + row * SS + col);
+            if (MODE == kAddF32) {
+                v.x += had[it].x; v.y += had[it].y; v.z += had[it].z; v.w += had[it].w;
+            }
+            *reinterpret_cast<float4*>(o + static_cast<size_t>(m) * N + n) = v;
+        }
+    }
+}
 template <int WR, int WC, int WMT, int WNT, int MODE>
 __global__ __launch_bounds__(64 * WR * WC, 1) void gemm_tile_direct_kernel(
     const bf16* __restrict__ a, const bf16* __restrict__ w, void* __restrict__ out, int M, int N, int K, int tiles_m,
     int tiles_n, int ksplit, QkvTarget qt, Groups, GateExtra gx) {  // (no grouped instances: the argument keeps the launches alike)
     constexpr int BM = WR * 16 * WMT, BN = WC * 16 * WNT, NW = WR * WC;
     constexpr int AC = BM / 8, WB = BN / 16;                    // loads: chunks of a slab of A, blocks of half a slab of W
-    static_assert(AC % NW == 0 && WB % NW == 0, "every wavefront has the same loads");
-    constexpr int LA = AC / NW, LW = WB / NW;
+    static_assert(AC % (2 * NW) == 0 && WB % NW == 0, "every wavefront has the same loads in every half turn");
+    constexpr int LA = AC / NW, LW = WB / NW, HA = LA / 2;
     constexpr int NSA = 3, NHW = 4;
     constexpr int A_STAGE = AC * 1024, W_STAGE = WB * 1024, W_BASE = NSA * A_STAGE;
     static_assert(W_BASE + NHW * W_STAGE <= 160 * 1024, "LDS");
-    static_assert(3 * LW + 2 * LA < 64, "the count of loads in flight has six bits");
+    static_assert(3 * LW + 3 * HA < 64, "the count of loads in flight has six bits");
     extern __shared__ __align__(16) unsigned char lds_raw[];
 
     const int per_split = tiles_m * tiles_n;
@@ -756,20 +947,25 @@ __global__ __launch_bounds__(64 * WR * WC, 1) void gemm_tile_direct_kernel(
 #pragma unroll
     for (int i = 0; i < LW; ++i) w_off[i] = static_cast<unsigned>(wave + NW * i) * (K / 32) * 1024u + lane * 16u;
     // (past the end of the share: the last one again, nobody reads it)
-    auto ask_a = [&](int kt, int stage) {
+    auto ask_a = [&](int kt, int stage, int i) {
         const int last = (h_end - 1) >> 1;
         if (kt > last) kt = last;
         const bool tail = 2 * kt + 1 >= nh_all;                 // the slab is half a slab: k ends in it
-        const unsigned base = lds_origin + stage * A_STAGE + wave * 1024;
-#pragma unroll
-        for (int i = 0; i < LA; ++i) load_b128_to_lds(a_rsrc, base + i * (NW * 1024), tail ? a_tail[i] : a_off[i], kt * (DK * 2));
+        load_b128_to_lds(a_rsrc, lds_origin + stage * A_STAGE + wave * 1024 + i * (NW * 1024), tail ? a_tail[i] : a_off[i], kt * (DK * 2));
     };
-    auto ask_w = [&](int h, int stage) {
+    auto ask_w = [&](int h, int stage, int i) {
         if (h >= h_end) h = h_end - 1;
-        const unsigned base = lds_origin + W_BASE + stage * W_STAGE + wave * 1024;
-#pragma unroll
-        for (int i = 0; i < LW; ++i) load_b128_to_lds(w_rsrc, base + i * (NW * 1024), w_off[i], h * 1024);
+        load_b128_to_lds(w_rsrc, lds_origin + W_BASE + stage * W_STAGE + wave * 1024 + i * (NW * 1024), w_off[i], h * 1024);
     };
+    // Rotating epilogue: where row m0 + tid goes is looked up by thread tid in front of the first slab and behind the last one
+    // that is asked for ahead (the lookups are older than the loads that a turn counts, so the counts hold).
+    RowPlace place;
+    int place_seq = 0;
+    if (MODE == kRopeCache) {
+        const int mrow = m0 + tid < M ? m0 + tid : M - 1;
+        place.pos = qt.positions[mrow];
+        place_seq = qt.seq_idx[mrow];
+    }
 
     f32x4 acc[WMT][WNT];
 #pragma unroll
@@ -781,62 +977,95 @@ __global__ __launch_bounds__(64 * WR * WC, 1) void gemm_tile_direct_kernel(
         // this lane's place in an operand of A: chunk 2 g + r / 8, then [kb][q, or q ^ 1 in odd chunks][r % 8]
         const unsigned a_lane = (wm / 8 + (r >> 3)) * 1024 + (q ^ (r >> 3)) * 128 + (r & 7) * 16;
         const unsigned w_lane = W_BASE + (wn / 16) * 1024 + lane * 16;
-        auto read_frags = [&](int sa, int kk, int sw, bf16x8 (&fa)[WMT], bf16x8 (&fw)[WNT]) {
-            const unsigned char* sA = lds_raw + sa * A_STAGE + a_lane + kk * 512;
-            const unsigned char* sW = lds_raw + sw * W_STAGE + w_lane;
-#pragma unroll
-            for (int i = 0; i < WMT; ++i) fa[i] = *reinterpret_cast<const bf16x8*>(sA + i * 2048);
-#pragma unroll
-            for (int j = 0; j < WNT; ++j) fw[j] = *reinterpret_cast<const bf16x8*>(sW + j * 1024);
+        auto read_a = [&](int stage, int kk, int i) {
+            return *reinterpret_cast<const bf16x8*>(lds_raw + stage * A_STAGE + a_lane + kk * 512 + i * 2048);
         };
-        auto multiply = [&](const bf16x8 (&fa)[WMT], const bf16x8 (&fw)[WNT]) {
+        auto read_w = [&](int stage, int j) { return *reinterpret_cast<const bf16x8*>(lds_raw + stage * W_STAGE + w_lane + j * 1024); };
+        // In front of the loop, what the half turns -5 .. -1 would have asked for, in their order: W's half slab, then half of
+        // an A slab. The waits count on this order: at an even half turn the loads behind W(h + 1) are half an A slab, W(h + 2),
+        // half, W(h + 3), half; at an odd one W(h + 2), half, W(h + 3), half, and A's slab (h + 1) / 2 is older than these.
+        const int kt0 = h_begin >> 1;
+        auto ask_half_a = [&](int kt, int stage, int part) {
+#pragma unroll
+            for (int i = 0; i < HA; ++i) ask_a(kt, stage, part * HA + i);
+        };
+        auto ask_all_w = [&](int h, int stage) {
+#pragma unroll
+            for (int i = 0; i < LW; ++i) ask_w(h, stage, i);
+        };
+        ask_half_a(kt0, 0, 0);
+        ask_all_w(h_begin, 0);
+        ask_half_a(kt0, 0, 1);
+        ask_all_w(h_begin + 1, 1);
+        ask_half_a(kt0 + 1, 1, 0);
+        ask_all_w(h_begin + 2, 2);
+        ask_half_a(kt0 + 1, 1, 1);
+        ask_all_w(h_begin + 3, 3);
+        ask_half_a(kt0 + 2, 2, 0);
+        if (MODE == kRopeCache) place.page = qt.block_table[static_cast<size_t>(place_seq) * qt.max_blocks + place.pos / qt.page];
+        wait_vm<3 * LW + 3 * HA>();
+        lds_barrier();
+        bf16x8 fa[WMT], fw0[WNT], fw1[WNT];
+#pragma unroll
+        for (int i = 0; i < WMT; ++i) fa[i] = read_a(0, 0, i);
+#pragma unroll
+        for (int j = 0; j < WNT; ++j) fw0[j] = read_w(0, j);
+        // The products of half a slab, a row of tiles at a time: behind each row its operand of the next half slab is read
+        // into the same registers, with a share of W's, and a share of the half turn's loads is asked for.
+        auto half_turn = [&](int a_stage, int kk, int w_stage, const bf16x8 (&now)[WNT], bf16x8 (&next)[WNT], auto&& ask) {
+#pragma unroll
+            for (int i = 0; i < WMT; ++i) {
+#pragma unroll
+                for (int j = 0; j < WNT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], now[j], acc[i][j], 0, 0, 0);
+                fa[i] = read_a(a_stage, kk, i);
+#pragma unroll
+                for (int j = 0; j < WNT; ++j)
+                    if (j * WMT / WNT == i) next[j] = read_w(w_stage, j);
+                ask(i);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        int sa = 0, pair = 0;                           // A's buffer of this slab; W's buffers of it are 2 pair and 2 pair + 1
+        int h = h_begin;
+        for (int turns = (h_end - h_begin) >> 1; turns > 0; --turns, h += 2) {
+            wait_vm<2 * LW + 3 * HA>();                 // half slab h + 1 has landed (the later ones may be on their way)
+            lds_barrier();                              // .. everybody's share of it, and everybody has read half slab h
+            const int before = sa == 0 ? NSA - 1 : sa - 1;
+            half_turn(sa, 1, 2 * pair + 1, fw0, fw1, [&](int i) {
+#pragma unroll
+                for (int t = 0; t < LW + HA; ++t)
+                    if (t * WMT / (LW + HA) == i) {
+                        if (t < LW) ask_w(h + 4, 2 * pair, t);
+                        else ask_a((h >> 1) + 2, before, HA + t - LW);
+                    }
+            });
+            wait_vm<2 * LW + 2 * HA>();
+            lds_barrier();
+            const int old_a = sa, old_pair = pair;
+            sa = sa + 1 == NSA ? 0 : sa + 1;
+            pair ^= 1;
+            half_turn(sa, 0, 2 * pair, fw1, fw0, [&](int i) {
+#pragma unroll
+                for (int t = 0; t < LW + HA; ++t)
+                    if (t * WMT / (LW + HA) == i) {
+                        if (t < LW) ask_w(h + 5, 2 * old_pair + 1, t);
+                        else ask_a((h >> 1) + 3, old_a, t - LW);
+                    }
+            });
+        }
+        if (h < h_end) {                                // (a share that ends in half a slab: k ends there)
 #pragma unroll
             for (int i = 0; i < WMT; ++i)
 #pragma unroll
-                for (int j = 0; j < WNT; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fw[j], acc[i][j], 0, 0, 0);
-        };
-        // In front of the loop, what the half turns -5 .. -1 would have asked for, in their order
-        // (W, then A): A(0); W(0); W(1), A(1); W(2); W(3), A(2). The waits count on this order: at an
-        // even half turn h the loads behind W(h + 1) are A, W(h + 2), W(h + 3), A; at an odd one
-        // W(h + 2), A, W(h + 3), and A's slab (h + 1) / 2 is older than W(h + 1).
-        const int kt0 = h_begin >> 1;
-        ask_a(kt0, 0);
-        ask_w(h_begin, 0);
-        ask_w(h_begin + 1, 1);
-        ask_a(kt0 + 1, 1);
-        ask_w(h_begin + 2, 2);
-        ask_w(h_begin + 3, 3);
-        ask_a(kt0 + 2, 2);
-        wait_vm<3 * LW + 2 * LA>();
-        lds_barrier();
-        bf16x8 fa0[WMT], fw0[WNT];
-        read_frags(0, 0, 0, fa0, fw0);
-        int sa = 0, pair = 0;                           // A's buffer of this slab; W's buffers of it are 2 pair and 2 pair + 1
-        for (int h = h_begin; h < h_end; h += 2) {
-            bf16x8 fa1[WMT], fw1[WNT];
-            wait_vm<2 * LW + 2 * LA>();                 // half slab h + 1 has landed (the later ones may be on their way)
-            lds_barrier();                              // .. everybody's share of it, and everybody has read half slab h
-            ask_w(h + 4, 2 * pair);
-            read_frags(sa, 1, 2 * pair + 1, fa1, fw1);
-            multiply(fa0, fw0);
-            deal_between_products<kDsRead, WMT + WNT>();
-            __builtin_amdgcn_sched_barrier(0);
-            wait_vm<2 * LW + LA>();
-            lds_barrier();
-            ask_w(h + 5, 2 * pair + 1);
-            ask_a((h >> 1) + 3, sa);
-            sa = sa + 1 == NSA ? 0 : sa + 1;
-            pair ^= 1;
-            read_frags(sa, 0, 2 * pair, fa0, fw0);
-            if (h + 1 < h_end) multiply(fa1, fw1);      // (a share that ends in half a slab: k ends there)
-            deal_between_products<kDsRead, WMT + WNT>();
-            __builtin_amdgcn_sched_barrier(0);
+                for (int j = 0; j < WNT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fw0[j], acc[i][j], 0, 0, 0);
         }
     }
     wait_vm<0>();                                       // (loads past the end are still on their way into LDS)
     __syncthreads();                                    // the epilogue reuses the slabs' LDS
-    tile_epilogue<WMT, WNT, MODE, 160 * 1024, WR, WC>(acc, lds_raw, out, M, N, m0, n0, wm, wn, tid, r, q, qt, {}, RowPlace{}, gx);
+    if constexpr (MODE == kAtomicF32)
+        tile_epilogue<WMT, WNT, MODE, 160 * 1024, WR, WC>(acc, lds_raw, out, M, N, m0, n0, wm, wn, tid, r, q);
+    else
+        direct_epilogue<WR, WC, WMT, WNT, MODE>(acc, lds_raw, out, M, N, m0, n0, wm, wn, tid, r, q, qt, place, gx);
 }
 
 template <auto KERNEL, int THREADS = 256>
@@ -945,6 +1174,11 @@ static int launch_tile_direct(const bf16* A, const bf16* W, void* out, int M, in
 
 // ----------------------------------------------------------------------------------------
 // skinny kernel: MT row tiles of 16 (M <= 16 MT), NW wavefronts per workgroup splitting k
+static int launch_direct_rope(const bf16* A, const bf16* W, int M, int N, int K, const QkvTarget& qt, hipStream_t stream) {
+    return launch_tile_kernel<gemm_tile_direct_kernel<4, 2, 4, 8, kRopeCache>, 512>(160 * 1024, 256, 256, A, W, nullptr, M, N, K, 1,
+                                                                                    stream, qt);
+}
+
 template <int WMT, int WNT>
 static int launch_tile_rope(const bf16* A, const bf16* W, int M, int N, int K, int blocked, const QkvTarget& qt,
                             hipStream_t stream) {
@@ -1214,7 +1448,7 @@ extern "C" int llme_gemm_bf16(const void* a, const void* w, void* out, int out_d
         if (mode != kAddF32) return kErrBadArgument;
         mode = kAtomicF32;
     }
-    if (auto_shape && blocked && direct != 0 && mode != kAddF32 && mode != kAtomicF32 && tiles_cost > 0.f) {
+    if (auto_shape && blocked && direct != 0 && mode != kAtomicF32 && tiles_cost > 0.f) {
         // Wide outputs that are stored, not added (gate/up, q/k/v of long prompts): tiles of 256 x 256
         // by eight wavefronts, their slabs straight into LDS, load half the bytes per product; one
         // workgroup fills a compute unit. In the units of the estimate above a round of them costs
@@ -1358,7 +1592,11 @@ extern "C" int llme_gemm_bf16_qkv_rope(const void* a, const void* w, int M, int 
                 tile_shape = shapes[c];
             }
         }
+        // Long prompts: 256 x 256 tiles of the direct kernel (rotation in the registers), in the same units.
+        const long wgs = static_cast<long>((M + 255) / 256) * ((N + 255) / 256);
+        if (blocked && (hd == 64 || hd == 128) && static_cast<double>((wgs + cus - 1) / cus) * (11.0 * K + 41000.0) < best) tile_shape = 256256;
     }
+    if (tile_shape == 256256 && blocked && (hd == 64 || hd == 128)) return launch_direct_rope(A, W, M, N, K, qt, stream);
     if (tile_shape == 128) return launch_tile_rope<4, 4>(A, W, M, N, K, blocked, qt, stream);
     if (tile_shape == 64 && hd <= 64) return launch_tile_rope<2, 2>(A, W, M, N, K, blocked, qt, stream);
     if (tile_shape == 128064 && hd <= 64) return launch_tile_rope<4, 2>(A, W, M, N, K, blocked, qt, stream);

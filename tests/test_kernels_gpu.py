@@ -1022,3 +1022,34 @@ def test_gemm_qkv_rope(ops, n_q, n_kv, hd, K, page, new, tile):
             assert (got.float() - want.float()).abs().max() <= 1.6e-2 * want.float().abs().max()
             assert ((got != want).float().mean()) < 2e-3
             assert torch.equal(got == 0, want == 0)            # nothing else was written
+
+
+@pytest.mark.parametrize("n_q,n_kv,hd,K", [(4, 2, 64, 128), (3, 1, 128, 96), (24, 8, 128, 512), (32, 8, 64, 224), (2, 1, 64, 32)])
+@pytest.mark.parametrize("new", [[70, 130, 3, 16, 33], [300], [1, 90, 17], [512]])
+def test_gemm_qkv_rope_in_wide_tiles(ops, n_q, n_kv, hd, K, new):
+    """The rotating epilogue of the 256 x 256 tile kernel against the one of 128 x 128 tiles: portions that start anywhere,
+    groups of 16 rows that span two requests, tiles that hang over the rows and over the heads, k of one half slab, of an odd
+    and of an even number. The sums are added in the same order; a rotation may contract a product and a sum into one rounding,
+    which moves a rounded value by one unit of bfloat16 (2^-8 of it) where it moves it at all."""
+    g, page = _gen(93), 16
+    T, N = sum(new), (n_q + 2 * n_kv) * hd
+    x = torch.randn(T, K, generator=g).to(torch.bfloat16).to(DEV)
+    w = ops.block_weight((0.05 * torch.randn(N, K, generator=g)).to(torch.bfloat16).to(DEV))
+    ctx = [16 * s + 5 * (s % 2) for s in range(len(new))]
+    positions = torch.cat([torch.arange(c, c + n) for c, n in zip(ctx, new)]).to(torch.int32).to(DEV)
+    seq_idx = torch.cat([torch.full((n,), s) for s, n in enumerate(new)]).to(torch.int32).to(DEV)
+    blocks = max((c + n + page - 1) // page for c, n in zip(ctx, new))
+    table = torch.randperm(len(new) * blocks, generator=g).view(len(new), blocks).to(torch.int32).to(DEV)
+    ang = torch.arange(blocks * page, dtype=torch.float64)[:, None] / (10000.0 ** (torch.arange(hd // 2, dtype=torch.float64) * 2 / hd))[None, :]
+    cos, sin = torch.cos(ang).float().to(DEV), torch.sin(ang).float().to(DEV)
+    out = []
+    for tile in (128, 256256):
+        made = (torch.zeros(T, n_q * hd, dtype=torch.bfloat16, device=DEV),
+                torch.zeros(table.numel(), n_kv, page, hd, dtype=torch.bfloat16, device=DEV),
+                torch.zeros(table.numel(), n_kv, hd, page, dtype=torch.bfloat16, device=DEV))
+        ops.gemm_qkv_rope(x, w, cos, sin, positions, seq_idx, table, *made, n_q, n_kv, hd, tile=tile)
+        out.append(made)
+    for want, got in zip(*out):
+        assert torch.equal(got == 0, want == 0)                 # nothing else was written
+        assert bool(((got.float() - want.float()).abs() <= want.float().abs() * 2.0 ** -7).all())
+    assert torch.equal(out[0][2], out[1][2])                    # v is not rotated
