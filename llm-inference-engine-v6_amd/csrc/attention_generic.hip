@@ -24,7 +24,10 @@ namespace llme {
 
 constexpr int kMaxHead = 256;
 
-template <typename TQ, typename TC, int NW>
+// VEC: head and page sizes are multiples of 4: a lane reads its key's row four dims at a time, and its value dim's four keys at
+// a time (the values lie by dim, so four keys are 16 bytes). One by one, a decoded token's 80 keys took 22.4 us, so
+// 12.5; the rows of a 77-token prompt 42 and 21.
+template <typename TQ, typename TC, int NW, bool VEC>
 __global__ __launch_bounds__(NW * 64) void attention_generic_kernel(
     const TQ* __restrict__ q, const TC* __restrict__ k_cache, const TC* __restrict__ v_cache,
     TQ* __restrict__ out, const int* __restrict__ positions, const int* __restrict__ seq_idx,
@@ -50,34 +53,71 @@ __global__ __launch_bounds__(NW * 64) void attention_generic_kernel(
     float m = -INFINITY, l = 0.f;
     float acc[PER_LANE] = {0.f, 0.f, 0.f, 0.f};
 
-    // this wavefront's chunks of 64 keys (no barrier inside: the wavefronts take different numbers of turns)
-    for (int t0 = lo + wave * kWave; t0 < hi; t0 += NW * kWave) {
+    // this wavefront's chunks of 64 keys (no barrier inside: the wavefronts take different numbers of turns); VEC: chunks
+    // begin at multiples of 4, so the first may hold up to three keys in front of the first that is seen
+    const int first = VEC ? lo & ~3 : lo;
+    for (int t0 = first + wave * kWave; t0 < hi; t0 += NW * kWave) {
         const int key = t0 + lane;
+        const bool seen = key >= lo && key < hi;
         float sc = -INFINITY;
-        if (key < hi) {
+        if (seen) {
             const int pg = table[key / page];
             const TC* kr = k_cache + ((static_cast<size_t>(pg) * n_kv + kvh) * page + key % page) * hd;
             float dot = 0.f;
-            for (int d = 0; d < hd; ++d) dot = fmaf(qs[d], to_float(kr[d]), dot);
+            if (VEC) {
+#pragma unroll 4
+                for (int d = 0; d < hd; d += 4) {
+                    float kv[4];
+                    load4<TC>(kr + d, kv);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) dot = fmaf(qs[d + e], kv[e], dot);
+                }
+            } else {
+                for (int d = 0; d < hd; ++d) dot = fmaf(qs[d], to_float(kr[d]), dot);
+            }
             sc = dot * scale;
         }
-        const float m_new = fmaxf(m, wave_max(sc));       // finite: the chunk holds at least key t0
+        const float m_new = fmaxf(m, wave_max(sc));       // finite: the chunk holds a key that is seen
         const float alpha = expf(m - m_new);              // 0 on the first chunk (m = -inf)
-        const float p = (key < hi) ? expf(sc - m_new) : 0.f;
+        const float p = seen ? expf(sc - m_new) : 0.f;
         l = l * alpha + wave_sum(p);
         m = m_new;
 #pragma unroll
         for (int i = 0; i < PER_LANE; ++i) acc[i] *= alpha;
         const int n = (hi - t0 < kWave) ? hi - t0 : kWave;
-        for (int j = 0; j < n; ++j) {
-            const int kj = t0 + j;
-            const int pg = table[kj / page];
-            const TC* vb = v_cache + (static_cast<size_t>(pg) * n_kv + kvh) * hd * page + kj % page;
-            const float pj = __shfl(p, j, kWave);
+        if (VEC) {
+            // (four keys of a dim; keys of the four that are not seen have weight 0 and count as 0 whatever their place holds)
+#pragma unroll 4
+            for (int j = 0; j < n; j += 4) {
+                const int kj = t0 + j;
+                const TC* vb = v_cache + (static_cast<size_t>(table[kj / page]) * n_kv + kvh) * hd * page + kj % page;
+                const bool whole = kj >= lo && kj + 4 <= hi;
+                float pj[4];
 #pragma unroll
-            for (int i = 0; i < PER_LANE; ++i) {
-                const int d = lane + i * kWave;
-                if (d < hd) acc[i] = fmaf(pj, to_float(vb[static_cast<size_t>(d) * page]), acc[i]);
+                for (int e = 0; e < 4; ++e)
+                    pj[e] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, p), j + e));
+#pragma unroll
+                for (int i = 0; i < PER_LANE; ++i) {
+                    const int d = lane + i * kWave;
+                    if (d >= hd) continue;
+                    float vv[4];
+                    load4<TC>(vb + static_cast<size_t>(d) * page, vv);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        acc[i] = fmaf(pj[e], whole || (kj + e >= lo && kj + e < hi) ? vv[e] : 0.f, acc[i]);
+                }
+            }
+        } else {
+            for (int j = 0; j < n; ++j) {
+                const int kj = t0 + j;
+                const int pg = table[kj / page];
+                const TC* vb = v_cache + (static_cast<size_t>(pg) * n_kv + kvh) * hd * page + kj % page;
+                const float pj = __shfl(p, j, kWave);
+#pragma unroll
+                for (int i = 0; i < PER_LANE; ++i) {
+                    const int d = lane + i * kWave;
+                    if (d < hd) acc[i] = fmaf(pj, to_float(vb[static_cast<size_t>(d) * page]), acc[i]);
+                }
             }
         }
     }
@@ -126,18 +166,19 @@ extern "C" int llme_attention_generic(const void* q, int q_dtype, const void* k_
     const dim3 grid(T, n_q);
     // few (token, head) pairs, as in decoding: 16 wavefronts each, so that the chip has work
     const bool few = static_cast<long>(T) * n_q < 4096;
+    const bool vec = hd % 4 == 0 && page % 4 == 0 && reinterpret_cast<uintptr_t>(k_cache) % 16 == 0 &&
+                     reinterpret_cast<uintptr_t>(v_cache) % 16 == 0;
+#define LLME_ATTN_AS(TQ, TC, NW, VEC)                                                                  \
+    hipLaunchKernelGGL((attention_generic_kernel<TQ, TC, NW, VEC>), grid, dim3(NW * 64), 0, stream,    \
+                       static_cast<const TQ*>(q), static_cast<const TC*>(k_cache),                     \
+                       static_cast<const TC*>(v_cache), static_cast<TQ*>(out), positions,              \
+                       seq_idx, block_table, max_blocks, n_q, n_kv, hd, page, scale, window)
 #define LLME_ATTN(TQ, TC)                                                                              \
     do {                                                                                               \
-        if (few)                                                                                       \
-            hipLaunchKernelGGL((attention_generic_kernel<TQ, TC, 16>), grid, dim3(16 * 64), 0, stream, \
-                               static_cast<const TQ*>(q), static_cast<const TC*>(k_cache),             \
-                               static_cast<const TC*>(v_cache), static_cast<TQ*>(out), positions,      \
-                               seq_idx, block_table, max_blocks, n_q, n_kv, hd, page, scale, window);  \
-        else                                                                                           \
-            hipLaunchKernelGGL((attention_generic_kernel<TQ, TC, 1>), grid, dim3(64), 0, stream,       \
-                               static_cast<const TQ*>(q), static_cast<const TC*>(k_cache),             \
-                               static_cast<const TC*>(v_cache), static_cast<TQ*>(out), positions,      \
-                               seq_idx, block_table, max_blocks, n_q, n_kv, hd, page, scale, window);  \
+        if (few && vec) LLME_ATTN_AS(TQ, TC, 16, true);                                                \
+        else if (few) LLME_ATTN_AS(TQ, TC, 16, false);                                                 \
+        else if (vec) LLME_ATTN_AS(TQ, TC, 1, true);                                                   \
+        else LLME_ATTN_AS(TQ, TC, 1, false);                                                           \
     } while (0)
     if (q_dtype == kF32 && cache_dtype == kF32) LLME_ATTN(float, float);
     else if (q_dtype == kBF16 && cache_dtype == kBF16) LLME_ATTN(bf16, bf16);
@@ -145,6 +186,7 @@ extern "C" int llme_attention_generic(const void* q, int q_dtype, const void* k_
     else if (q_dtype == kBF16 && cache_dtype == kF32) LLME_ATTN(bf16, float);
     else return kErrBadArgument;
 #undef LLME_ATTN
+#undef LLME_ATTN_AS
     return launch_status();
 }
 

@@ -6,11 +6,13 @@
 // operand types or shapes that the MFMA kernels refuse. Any M, N, K. W may also come in the
 // MFMA kernels' blocked layout ([N / 16][K / 32] blocks of [4][16][8]; N % 16 == 0, K % 32 == 0).
 //
-// Up to 16 rows (decoding) go to a kernel of their own that streams the weights once (further
-// down). Tiling otherwise: a workgroup of 256 threads makes a 64 x 64 tile of the output, 4 x 4 per
-// thread, stepping through K in slabs of 16 staged in LDS (stored k-major so that
-// the inner loop reads consecutive addresses).
+// Up to 16 rows (decoding) go to a kernel of their own that streams the weights once, and more rows of 32-bit
+// operands to one on the matrix cores' 32-bit instruction (both further down). Tiling otherwise: a workgroup of 256
+// threads makes a 64 x 64 tile of the output, 4 x 4 per thread, stepping through K in slabs of 16 staged in LDS (stored
+// k-major so that the inner loop reads consecutive addresses).
 #include "common.h"
+
+#include <type_traits>
 
 namespace llme {
 
@@ -87,34 +89,25 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(const TA* __restrict_
 constexpr int GV_COLS = 4;
 constexpr int GV_MAX_ROWS = 16;
 
-template <typename T>
-__device__ __forceinline__ void load4(const T* p, float (&v)[4]);
-template <>
-__device__ __forceinline__ void load4<float>(const float* p, float (&v)[4]) {
-    const float4 x = *reinterpret_cast<const float4*>(p);
-    v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
-}
-template <>
-__device__ __forceinline__ void load4<bf16>(const bf16* p, float (&v)[4]) {
-    typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
-    const bf16x4 x = *reinterpret_cast<const bf16x4*>(p);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = static_cast<float>(x[i]);
-}
-
-template <typename TA, typename TW, typename TO, bool ACC, int MR>
+// KS wavefronts of a workgroup share the columns and take every KS-th piece of k; their sums meet in LDS, in one order.
+// (An output of 2,048 columns is 512 wavefronts of whole columns, half of one per scheduler: two rows times the o-proj's and
+// the down-proj's 32-bit weights of the 1B sizes, 16.8 and 67 MB, took 19.6 us on average so, and take 11.9 with k in four;
+// q/k/v, 768 wavefronts, 11.7 and 8.5. At 4,096 wavefronts, gate/up, 134 MB take 28.7 us, the rate of memory, without.)
+template <typename TA, typename TW, typename TO, bool ACC, int MR, int KS>
 __global__ __launch_bounds__(256) void gemv_generic_kernel(const TA* __restrict__ a, const TW* __restrict__ w,
                                                            TO* __restrict__ out, int M, int N, int K) {
+    __shared__ float part[KS > 1 ? KS : 1][MR * GV_COLS];
     const int lane = threadIdx.x & 63;
-    const int wave_id = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int n0 = wave_id * GV_COLS;
-    if (n0 >= N) return;                                  // (whole wavefronts)
+    const int wave = threadIdx.x >> 6, share = wave % KS;
+    const int n0 = (blockIdx.x * (4 / KS) + wave / KS) * GV_COLS;
+    if (n0 >= N) return;                                  // (whole wavefronts; with KS of 4 the whole workgroup)
     float acc[MR][GV_COLS];
 #pragma unroll
     for (int m = 0; m < MR; ++m)
 #pragma unroll
         for (int c = 0; c < GV_COLS; ++c) acc[m][c] = 0.f;
-    for (int k = lane * 4; k < K; k += 64 * 4) {
+#pragma unroll 2
+    for (int k = (share * 64 + lane) * 4; k < K; k += KS * 64 * 4) {
         float wv[GV_COLS][4];
 #pragma unroll
         for (int c = 0; c < GV_COLS; ++c) {
@@ -136,34 +129,202 @@ __global__ __launch_bounds__(256) void gemv_generic_kernel(const TA* __restrict_
 #pragma unroll
         for (int c = 0; c < GV_COLS; ++c) {
             const float s = wave_sum(acc[m][c]);
-            if (lane == 0 && m < M && n0 + c < N) {
+            if (KS > 1) {
+                if (lane == 0) part[share][m * GV_COLS + c] = s;
+            } else if (lane == 0 && m < M && n0 + c < N) {
                 TO* o = out + static_cast<size_t>(m) * N + n0 + c;
                 *o = from_float<TO>(ACC ? to_float(*o) + s : s);
             }
         }
+    if (KS == 1) return;
+    __syncthreads();
+    const int m = threadIdx.x / GV_COLS, c = threadIdx.x % GV_COLS;
+    if (m >= MR || m >= M || n0 + c >= N) return;
+    float s = part[0][threadIdx.x];
+#pragma unroll
+    for (int i = 1; i < KS; ++i) s += part[i][threadIdx.x];
+    TO* o = out + static_cast<size_t>(m) * N + n0 + c;
+    *o = from_float<TO>(ACC ? to_float(*o) + s : s);
 }
 
 template <typename TA, typename TW, typename TO>
 static int launch_gemv_generic(const void* a, const void* w, void* out, int M, int N, int K, int accumulate,
                                hipStream_t stream) {
     const int waves = (N + GV_COLS - 1) / GV_COLS;
-    const dim3 grid((waves + 3) / 4);
-#define LLME_GEMV(ACC, MR)                                                                          \
-    hipLaunchKernelGGL((gemv_generic_kernel<TA, TW, TO, ACC, MR>), grid, dim3(256), 0, stream,     \
+    // (k in four where whole columns are less than two wavefronts for each of a compute unit's four schedulers)
+    const bool split = waves < 8 * compute_units() && K >= 1024;
+    const dim3 grid(split ? waves : (waves + 3) / 4);
+#define LLME_GEMV_KS(ACC, MR, KS)                                                                   \
+    hipLaunchKernelGGL((gemv_generic_kernel<TA, TW, TO, ACC, MR, KS>), grid, dim3(256), 0, stream, \
                        static_cast<const TA*>(a), static_cast<const TW*>(w), static_cast<TO*>(out), M, N, K)
+#define LLME_GEMV(ACC, MR)                                                                          \
+    do {                                                                                            \
+        if (split) LLME_GEMV_KS(ACC, MR, 4);                                                        \
+        else LLME_GEMV_KS(ACC, MR, 1);                                                              \
+    } while (0)
     // (rows in steps: the partial sums live in registers, 4 per row)
-    if (accumulate) {
-        if (M <= 1) LLME_GEMV(true, 1);
-        else if (M <= 4) LLME_GEMV(true, 4);
-        else if (M <= 8) LLME_GEMV(true, 8);
-        else LLME_GEMV(true, 16);
-    } else {
-        if (M <= 1) LLME_GEMV(false, 1);
-        else if (M <= 4) LLME_GEMV(false, 4);
-        else if (M <= 8) LLME_GEMV(false, 8);
-        else LLME_GEMV(false, 16);
-    }
+#define LLME_GEMV_ROWS(ACC)                                                                         \
+    do {                                                                                            \
+        if (M <= 1) LLME_GEMV(ACC, 1);                                                              \
+        else if (M <= 2) LLME_GEMV(ACC, 2);                                                         \
+        else if (M <= 4) LLME_GEMV(ACC, 4);                                                         \
+        else if (M <= 8) LLME_GEMV(ACC, 8);                                                         \
+        else LLME_GEMV(ACC, 16);                                                                    \
+    } while (0)
+    if (accumulate) LLME_GEMV_ROWS(true);
+    else LLME_GEMV_ROWS(false);
+#undef LLME_GEMV_ROWS
 #undef LLME_GEMV
+#undef LLME_GEMV_KS
+    return launch_status();
+}
+
+// 32-bit operands, more than 16 rows: v_mfma_f32_16x16x4_f32, whose products and sums are 32-bit like the vector unit's, at
+// twice its rate (64 multiply-adds a cycle and scheduler: 157 TFLOP/s). At that rate the operands need no LDS: a lane loads
+// 8 consecutive k of a row (two loads of 16 bytes; the four lanes of a row take 128 bytes together), and step s of eight
+// multiplies element s of every lane, which is k = 8 q + s for lane group q in both operands. A wavefront makes
+// 16 WMT x 16 WNT of the output; KW wavefronts share an output and take every KW-th 32 of k, their sums meeting in LDS in one
+// order (the same bits in every run). D blocks of 32 k are in flight per wavefront.
+// Measured at 149 rows, the 1B sizes (before: the 64 x 64 tile kernel above on 96 to 768 workgroups, one load at a time):
+// o-proj and down-proj 587 -> 69 us on average, q/k/v 236 -> 32, gate/up 398 -> 159 (67 TFLOP/s of its 10.7 GFLOP with
+// 32 x 64 tiles). The error against 64 bits is half the former's (2.4e-6 of the logits, 4.7e-6): more and shorter sums.
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+
+template <int WMT, int WNT, int WR, int WC, int KW, int D, bool ACC>
+__global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__ a, const float* __restrict__ w,
+                                                       float* __restrict__ out, int M, int N, int K, int tiles_m) {
+    static_assert(WR * WC * KW == 4, "four wavefronts");
+    constexpr int BM = 16 * WMT * WR, BN = 16 * WNT * WC;
+    __shared__ f32x4 part[KW > 1 ? KW * WMT * WNT * 64 : 1];
+    int pid = blockIdx.x;                               // (a die gets consecutive tiles: they share a tile's rows of W)
+    if (gridDim.x % 8 == 0) pid = (pid % 8) * (gridDim.x / 8) + pid / 8;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, q = lane >> 4;
+    const int kw = wave % KW, wr = wave / KW / WC, wc = wave / KW % WC;
+    const int m0 = (pid % tiles_m) * BM + wr * 16 * WMT, n0 = (pid / tiles_m) * BN + wc * 16 * WNT;
+    const float *ap[WMT], *wp[WNT];                     // (rows past an edge: the last one again, not stored)
+#pragma unroll
+    for (int i = 0; i < WMT; ++i) ap[i] = a + static_cast<size_t>(m0 + i * 16 + r < M ? m0 + i * 16 + r : M - 1) * K + q * 8;
+#pragma unroll
+    for (int j = 0; j < WNT; ++j) wp[j] = w + static_cast<size_t>(n0 + j * 16 + r < N ? n0 + j * 16 + r : N - 1) * K + q * 8;
+    f32x4 acc[WMT][WNT];
+#pragma unroll
+    for (int i = 0; i < WMT; ++i)
+#pragma unroll
+        for (int j = 0; j < WNT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    struct Block {
+        f32x4 a[WMT][2], w[WNT][2];
+    };
+    const int whole = K / 32;                           // blocks of 32 k
+    auto load = [&](int b) {
+        Block x;
+        const int k = (b < whole ? b : whole - 1) * 32; // (past the end: the last one again, not multiplied)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+#pragma unroll
+            for (int i = 0; i < WMT; ++i) x.a[i][u] = *reinterpret_cast<const f32x4*>(ap[i] + k + u * 4);
+#pragma unroll
+            for (int j = 0; j < WNT; ++j) x.w[j][u] = *reinterpret_cast<const f32x4*>(wp[j] + k + u * 4);
+        }
+        return x;
+    };
+    auto multiply = [&](const Block& x) {
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+#pragma unroll
+            for (int i = 0; i < WMT; ++i)
+#pragma unroll
+                for (int j = 0; j < WNT; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.a[i][s / 4][s % 4], x.w[j][s / 4][s % 4], acc[i][j], 0, 0, 0);
+    };
+    if (kw < whole) {
+        const int mine = (whole - kw + KW - 1) / KW;    // this wavefront's blocks
+        Block x[D];
+#pragma unroll
+        for (int d = 0; d < D; ++d) x[d] = load(kw + d * KW);
+        int at = 0;
+        for (; at + D <= mine; at += D) {
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                multiply(x[d]);
+                x[d] = load(kw + (at + D + d) * KW);
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < D - 1; ++d)
+            if (at + d < mine) multiply(x[d]);
+    }
+    if (K % 32 != 0 && kw == whole % KW) {              // what is left of k (a multiple of 4): zeros behind its end
+        Block x;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const bool in = whole * 32 + q * 8 + u * 4 < K;
+#pragma unroll
+            for (int i = 0; i < WMT; ++i)
+                x.a[i][u] = in ? *reinterpret_cast<const f32x4*>(ap[i] + whole * 32 + u * 4) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < WNT; ++j)
+                x.w[j][u] = in ? *reinterpret_cast<const f32x4*>(wp[j] + whole * 32 + u * 4) : f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        multiply(x);
+    }
+    // column r, rows 4 q + e of every tile of 16 x 16
+    auto store = [&](int i, int j, const f32x4& v) {
+        const int n = n0 + j * 16 + r;
+        if (n >= N) return;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int m = m0 + i * 16 + q * 4 + e;
+            if (m >= M) continue;
+            float* o = out + static_cast<size_t>(m) * N + n;
+            *o = ACC ? *o + v[e] : v[e];
+        }
+    };
+    if (KW == 1) {
+#pragma unroll
+        for (int i = 0; i < WMT; ++i)
+#pragma unroll
+            for (int j = 0; j < WNT; ++j) store(i, j, acc[i][j]);
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < WMT; ++i)
+#pragma unroll
+        for (int j = 0; j < WNT; ++j) part[(kw * WMT * WNT + i * WNT + j) * 64 + lane] = acc[i][j];
+    __syncthreads();
+    for (int t = kw; t < WMT * WNT; t += KW) {          // (a wavefront adds up and stores every KW-th tile)
+        f32x4 v = part[t * 64 + lane];
+#pragma unroll
+        for (int s = 1; s < KW; ++s) v += part[(s * WMT * WNT + t) * 64 + lane];
+        store(t / WNT, t % WNT, v);
+    }
+}
+
+template <bool ACC>
+static int launch_gemm_f32(const float* a, const float* w, float* out, int M, int N, int K, hipStream_t stream) {
+    // The tile whose rounds of workgroups over the compute units take the least time: a round is the products of one of a
+    // workgroup's wavefronts, over how well its loads are used (a 32 x 32 tile loads twice what a 64 x 64 one does per product).
+    const int cus = compute_units();
+    struct Shape { int bm, bn, products; float eff; };
+    constexpr Shape shapes[4] = {{128, 128, 64, 1.0f}, {64, 64, 16, 0.95f}, {32, 64, 8, 0.9f}, {32, 32, 4, 0.8f}};
+    int best = 0;
+    float least = 0.f;
+    for (int c = 0; c < 4; ++c) {
+        const long tiles = static_cast<long>((M + shapes[c].bm - 1) / shapes[c].bm) * ((N + shapes[c].bn - 1) / shapes[c].bn);
+        const float cost = static_cast<float>((tiles + cus - 1) / cus) * shapes[c].products / shapes[c].eff;
+        if (c == 0 || cost < least) {
+            least = cost;
+            best = c;
+        }
+    }
+    const int tiles_m = (M + shapes[best].bm - 1) / shapes[best].bm, tiles_n = (N + shapes[best].bn - 1) / shapes[best].bn;
+    const dim3 grid(tiles_m * tiles_n), block(256);
+    switch (best) {
+        case 0: hipLaunchKernelGGL((gemm_f32_kernel<4, 4, 2, 2, 1, 2, ACC>), grid, block, 0, stream, a, w, out, M, N, K, tiles_m); break;
+        case 1: hipLaunchKernelGGL((gemm_f32_kernel<4, 4, 1, 1, 4, 2, ACC>), grid, block, 0, stream, a, w, out, M, N, K, tiles_m); break;
+        case 2: hipLaunchKernelGGL((gemm_f32_kernel<2, 4, 1, 1, 4, 3, ACC>), grid, block, 0, stream, a, w, out, M, N, K, tiles_m); break;
+        default: hipLaunchKernelGGL((gemm_f32_kernel<2, 2, 1, 1, 4, 4, ACC>), grid, block, 0, stream, a, w, out, M, N, K, tiles_m); break;
+    }
     return launch_status();
 }
 
@@ -173,6 +334,13 @@ static int launch_generic(const void* a, const void* w, void* out, int M, int N,
     if (M <= GV_MAX_ROWS && !blocked && K % 4 == 0 && reinterpret_cast<uintptr_t>(a) % 16 == 0 &&
         reinterpret_cast<uintptr_t>(w) % 16 == 0)
         return launch_gemv_generic<TA, TW, TO>(a, w, out, M, N, K, accumulate, stream);
+    if constexpr (std::is_same_v<TA, float> && std::is_same_v<TW, float> && std::is_same_v<TO, float>) {
+        if (!blocked && K % 4 == 0 && reinterpret_cast<uintptr_t>(a) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0) {
+            const float *fa = static_cast<const float*>(a), *fw = static_cast<const float*>(w);
+            return accumulate ? launch_gemm_f32<true>(fa, fw, static_cast<float*>(out), M, N, K, stream)
+                              : launch_gemm_f32<false>(fa, fw, static_cast<float*>(out), M, N, K, stream);
+        }
+    }
     const dim3 grid((N + GB - 1) / GB, (M + GB - 1) / GB);
     if (accumulate)
         hipLaunchKernelGGL((gemm_generic_kernel<TA, TW, TO, true>), grid, dim3(256), 0, stream,

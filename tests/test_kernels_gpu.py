@@ -1053,3 +1053,43 @@ def test_gemm_qkv_rope_in_wide_tiles(ops, n_q, n_kv, hd, K, new):
         assert torch.equal(got == 0, want == 0)                 # nothing else was written
         assert bool(((got.float() - want.float()).abs() <= want.float().abs() * 2.0 ** -7).all())
     assert torch.equal(out[0][2], out[1][2])                    # v is not rotated
+
+
+@pytest.mark.parametrize("M,N,K", [(17, 16, 4), (31, 33, 28), (33, 65, 32), (64, 64, 36), (149, 2048, 260), (149, 331, 1020),
+                                   (300, 1030, 132), (1025, 1500, 64), (2, 2048, 1028), (1, 70, 4096), (9, 515, 1024), (16, 8200, 96)])
+def test_gemm_in_32_bits(ops, M, N, K):
+    """32-bit products on the matrix cores (more than 16 rows: each of the four tiles, rows, columns and k past the last tile,
+    k of less than a block) and of few rows with k in four, stored and added: against 64 bits within sqrt(K) roundings of the
+    largest terms (each sum has K of them), and the same bits in every run."""
+    a = torch.randn(M, K, generator=_gen(3))
+    w = torch.randn(N, K, generator=_gen(4))
+    ad, wd = a.to(DEV), w.to(DEV)
+    ref = plain_linear(a.double(), w.double())
+    out, again = torch.full((M, N), 7.0, device=DEV), torch.full((M, N), 5.0, device=DEV)
+    ops.gemm_generic(ad, wd, out)
+    ops.gemm_generic(ad, wd, again)
+    assert torch.equal(out, again)
+    assert (out.cpu().double() - ref).abs().max() < 2.0 ** -23 * K ** 0.5 * 32
+    assert _rel(out.cpu().double(), ref) < 2e-6
+    base = torch.randn(M, N, generator=_gen(5))
+    out2 = base.clone().to(DEV)
+    ops.gemm_generic(ad, wd, out2, accumulate=True)
+    assert torch.equal(out2, base.to(DEV) + out)
+
+
+@pytest.mark.parametrize("page,window", [(4, 0), (16, 0), (16, 5), (16, 70), (8, 131)])
+def test_attention_generic_four_keys_at_a_time(ops, page, window):
+    """What lies in a page behind a request's last key, or in front of its window, is not read into the sum: places that hold no
+    number leave every row as it is. Lengths around multiples of 4 and of 64."""
+    lens, n_q, n_kv, hd = [1, 3, 63, 66, 133], 2, 1, 20
+    s = _paged_setup(ops, lens, n_q, n_kv, hd, page, torch.float32, seed=6, rotate=False)
+    last = (torch.tensor(lens).cumsum(0) - 1).tolist()
+    for r, n in enumerate(lens):                            # (behind the last key of every request)
+        if n % page:
+            pg = int(s["table"][r, n // page])
+            s["k_cache"][pg, :, n % page:] = float("nan")
+            s["v_cache"][pg, :, :, n % page:] = float("nan")
+    out = torch.empty_like(s["q"])
+    ops.attention_generic(s["q"], s["k_cache"], s["v_cache"], out, s["positions"], s["seq_idx"], s["table"], n_q, n_kv, hd, 0.3, window)
+    ref = torch.cat([plain_attention(q * (0.3 * math.sqrt(hd)), k, v, window).reshape(-1, n_q * hd) for q, k, v in s["plain"]])
+    assert _rel(out.cpu().double()[last], ref[last]) < 3e-6 and _rel(out.cpu().double(), ref) < 3e-6
