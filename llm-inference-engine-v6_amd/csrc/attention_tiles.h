@@ -362,21 +362,34 @@ __host__ __device__ constexpr int decode_lds_floats(int hd) { return DEC_WAVES *
 // hd], full rotation, head size 64 or 128), and the workgroup does what the rotation kernel would have
 // done for its request and kv head: it rotates its query heads into operand registers, rotates the new key,
 // writes key and value into the request's page, and sets what it has read of the row to zero (the buffer
-// is one that a product cut over k adds into). Only with a single split: every value of the row is then
-// read by one workgroup. The cache is non-const here: the new key and value go into it.
+// is one that a product cut over k adds into). The cache is non-const here: the new key and value go into it.
+// With several splits of the keys every one of them rotates the query heads for itself, the one that holds the
+// last key writes the new key and value, and the one that is done last joins the parts in the splits' order (so the
+// result does not depend on which it is), and clears the query heads, which by then all have read, and its counter.
+// Splits in front of a window or behind the last key are no parts: they leave at once and are not waited for.
 struct RawQkv {
     float* qkv = nullptr;            // [rows, (n_q + 2 n_kv) hd]
     const float* cos_t = nullptr;    // [max_pos, hd / 2]
     const float* sin_t = nullptr;
     bf16* k_cache = nullptr;
     bf16* v_cache = nullptr;
+    int* done = nullptr;             // [rows, n_kv], zero: parts that are done (several splits only)
 };
+
+// Parts that another workgroup of the same launch joins are written through to where all dies see them and read from there,
+// value by value. (A fence for the whole device instead writes back and throws away a die's L2: with two splits of 64
+// requests such fences took 240 us a layer.)
+template <bool SHARED> __device__ __forceinline__ void put_part(float* p, float v) {
+    if (SHARED) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else *p = v;
+}
+__device__ __forceinline__ float get_part(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
 // (k_cache and v_cache carry no promise that nothing else points at them: RAW writes into them)
 template <int HD, bool STREAM, bool RAW = false>
 __device__ __forceinline__ void decode_item(
     const bf16* __restrict__ q, const bf16* k_cache, const bf16* v_cache,
-    bf16* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml,
+    bf16* __restrict__ out, float* part_o, float* part_ml,
     const int* __restrict__ q_start, const int* __restrict__ ctx_len, const int* __restrict__ block_table,
     int max_blocks, int n_q, int n_kv, int page, float scale, int window, int split_len, int nsplit, int s,
     int head_tile, int split, float* sh, const RawQkv& raw = RawQkv{}) {
@@ -394,13 +407,16 @@ __device__ __forceinline__ void decode_item(
     const int table_line = block_table[static_cast<size_t>(s) * max_blocks +
                                        (first_block < max_blocks ? first_block : max_blocks - 1)];
     if (row1 - row0 != 1) return;                       // not a decoding request (whole workgroup)
+    const int lo_all = (window > 0 && pos - window + 1 > 0) ? pos - window + 1 : 0;
+    const int first_split = RAW ? (lo_all & ~31) / split_len : 0, last_split = RAW ? pos / split_len : nsplit - 1;
+    if (RAW && (split < first_split || split > last_split)) return;
+    const int parts = RAW ? last_split - first_split + 1 : nsplit;
     asm volatile("" ::"v"(table_line));                 // (the load is wanted for its effect on the cache)
     const int G = n_q / n_kv;
     const int gtiles = (G + 15) / 16;
     const int kvh = head_tile / gtiles, gt = head_tile % gtiles;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g4 = lane >> 4;
 
-    const int lo_all = (window > 0 && pos - window + 1 > 0) ? pos - window + 1 : 0;
     int k_begin = split * split_len, k_end = k_begin + split_len;
     if (k_end > pos + 1) k_end = pos + 1;
     if (k_begin < (lo_all & ~31)) k_begin = lo_all & ~31;
@@ -449,7 +465,7 @@ __device__ __forceinline__ void decode_item(
         // the new key and value of this kv head: the first wavefront's lanes take 8 dims each
         const PagePlace at = page_of(kv, pos);
         const int pg = __builtin_amdgcn_readfirstlane(kv.table[at.block]);
-        if (wave == 0) {
+        if (wave == 0 && split == last_split) {
             float* krow = qkv_row + static_cast<size_t>(n_q + kvh) * HD;
             float* vrow = qkv_row + static_cast<size_t>(n_q + n_kv + kvh) * HD;
             if (lane < HALF / 8) {
@@ -473,7 +489,7 @@ __device__ __forceinline__ void decode_item(
             }
         }
         __syncthreads();                                // the key and the value are in the page; every wavefront has read q
-        if (wave == 0 && row_ok) {
+        if (wave == 0 && row_ok && parts == 1) {
 #pragma unroll
             for (int c = 0; c < DC / 2; ++c) {
                 zero8(qhead + c * 32 + g4 * 8);
@@ -523,16 +539,43 @@ __device__ __forceinline__ void decode_item(
             lsum += f * sh_l[w][row];
         }
         const int h = kvh * G + gt * 16 + row;
-        if (nsplit == 1) {
+        if (parts == 1) {
             out[(static_cast<size_t>(row0) * n_q + h) * HD + d] = static_cast<bf16>(acc / lsum);
         } else {
             const size_t pidx = (static_cast<size_t>(s) * n_q + h) * nsplit + split;
-            part_o[pidx * HD + d] = acc;
+            put_part<RAW>(part_o + pidx * HD + d, acc);
             if (d == 0) {
-                part_ml[pidx * 2] = mx;
-                part_ml[pidx * 2 + 1] = lsum;
+                put_part<RAW>(part_ml + pidx * 2, mx);
+                put_part<RAW>(part_ml + pidx * 2 + 1, lsum);
             }
         }
+    }
+    if constexpr (RAW) {
+        if (parts == 1) return;
+        int* last = reinterpret_cast<int*>(sh);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (the part is where every workgroup sees it)
+        __syncthreads();
+        if (threadIdx.x == 0)
+            *last = __hip_atomic_fetch_add(raw.done + static_cast<size_t>(row0) * n_kv + kvh, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if (*last != parts - 1) return;
+        for (int item = threadIdx.x; item < G * HD; item += DEC_WAVES * 64) {
+            const int h = kvh * G + item / HD, d = item % HD;
+            const size_t base = (static_cast<size_t>(s) * n_q + h) * nsplit + first_split;
+            float mx = kNoMax;
+            for (int i = 0; i < parts; ++i) mx = fmaxf(mx, get_part(part_ml + (base + i) * 2));
+            float acc = 0.f, lsum = 0.f;
+#pragma unroll 4
+            for (int i = 0; i < parts; ++i) {
+                const float mi = get_part(part_ml + (base + i) * 2);
+                const float f = (mi <= kNoMax) ? 0.f : exp2f(mi - mx);
+                acc += f * get_part(part_o + (base + i) * HD + d);
+                lsum += f * get_part(part_ml + (base + i) * 2 + 1);
+            }
+            out[(static_cast<size_t>(row0) * n_q + h) * HD + d] = static_cast<bf16>(acc / lsum);
+            raw.qkv[static_cast<size_t>(row0) * (n_q + 2 * n_kv) * HD + static_cast<size_t>(h) * HD + d] = 0.f;
+        }
+        if (threadIdx.x == 0) raw.done[static_cast<size_t>(row0) * n_kv + kvh] = 0;
     }
 }
 

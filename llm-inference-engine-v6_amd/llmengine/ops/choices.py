@@ -59,6 +59,7 @@ class KernelChoices:
     decode_cut_piece_us: float = 0.5    # and per piece
     decode_cut_join_us: float = 4.6     # a cut costs the join kernel (17 requests and more)
     decode_cut_rope_us: float = 4.8     # and the rotation kernel, where the single split would have rotated itself
+    decode_cut_inside_us: float = 2.0   # what both cost at most where the decode kernel rotates: it then joins its splits itself
     decode_cut_each_us: float = 1.0     # and this per split
     decode_cut_gain: float = 0.05       # and must promise this fraction of the whole keys' time
     # Portions of prompts: work items (a span of rows x a group of heads) the prefill kernel should

@@ -367,6 +367,8 @@ def decode_cut(lens, n_q: int, n_kv: int, head_dim: int, plan_len: int | None = 
     apart_us = 0.0
     if first == 1:
         apart_us = (ch.decode_cut_join_us if S > GEMV_NORM_MAX_ROWS else 0.0) + (ch.decode_cut_rope_us if rotates else 0.0)
+        if rotates:                                        # (the kernel that rotates joins its splits itself)
+            apart_us = min(apart_us, ch.decode_cut_inside_us)
     from ..runtime import native
     n = native.library().llme_decode_cut((ctypes.c_int * S)(*lens), S, tiles, units, head_dim, longest, first, most,
                                          ch.decode_cut_tbs, ch.decode_cut_key_ns, ch.decode_cut_lone_ns,
@@ -503,15 +505,16 @@ def _fast_attention_project(q, k_cache, v_cache, o, step, block_table, n_q, n_kv
 kernels._fast_attention_project = _fast_attention_project
 
 declare("llme_attention_decode_rope_bf16", [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _f, _i,
-                                            _i, _vp])
+                                            _i, _i, _vp, _vp, _vp, _vp])
 
 
 def attention_decode_rope(qkv, cos, sin, k_cache, v_cache, out, step, block_table, n_q: int, n_kv: int, head_dim: int,
-                          scale: float, window: int) -> bool:
+                          scale: float, window: int, done: torch.Tensor | None = None) -> bool:
     """A step of single decoded tokens whose q/k/v rows [S, (n_q + 2 n_kv) head_dim] are still 32-bit and
     unrotated: rotation, the cache write at each request's position, attention over the pages into out
-    [S, n_q head_dim] and the clearing of qkv, in the attention kernel (one workgroup per request and kv
-    head, the keys in a single split). False, and nothing done, where the step or the sizes are not such."""
+    [S, n_q head_dim] and the clearing of qkv, in the attention kernel (one workgroup per request, kv
+    head and split of the keys; several splits need done, S * n_kv zeroed 32-bit values that are left zero). False, and
+    nothing done, where the step or the sizes are not such."""
     T = qkv.shape[0]
     ch = choices_of(step)
     if (not ch.decode_rope or not ch.fast_attention or T != step.num_seqs or head_dim not in (64, 128)
@@ -521,7 +524,8 @@ def attention_decode_rope(qkv, cos, sin, k_cache, v_cache, out, step, block_tabl
             or k_cache.data_ptr() % 16):
         return False
     plan = _step_plan(step, n_q, n_kv, head_dim)
-    if plan["n_decode"] != T or plan["groups"] or plan["nsplit"] != 1:
+    nsplit = plan["nsplit"]
+    if plan["n_decode"] != T or plan["groups"] or (nsplit != 1 and done is None):
         return False
     # (measured, ms a decode step at a context of 2,048, apart / inside: 1B sizes 1.238 / 1.203 at 17 requests,
     # 1.340 / 1.297 at 32, 1.758 / 1.724 at 64; 3B 2.950 / 2.889, 3.350 / 3.288, 4.84 / 4.88; 8B 4.369 / 4.298,
@@ -537,10 +541,17 @@ def attention_decode_rope(qkv, cos, sin, k_cache, v_cache, out, step, block_tabl
     page = k_cache.shape[2]
     require(v_cache, "v_cache", torch.bfloat16, (k_cache.shape[0], n_kv, head_dim, page))
     require(block_table, "block_table", torch.int32, (S, None))
+    part_o = part_ml = None
+    if nsplit > 1:
+        require(done, "done", torch.float32)
+        if done.numel() < S * n_kv:
+            raise kernels.KernelError("attention_decode_rope: a counter per request and kv head")
+        part_o = step.buffer("attn.part_o", (S * n_q * nsplit * head_dim,), torch.float32)
+        part_ml = step.buffer("attn.part_ml", (S * n_q * nsplit * 2,), torch.float32)
     check(entry("llme_attention_decode_rope_bf16")(
         ptr(qkv), ptr(cos), ptr(sin), ptr(k_cache), ptr(v_cache), ptr(out), ptr(step.q_start), ptr(step.ctx_len),
         ptr(block_table), block_table.shape[1], S, n_q, n_kv, head_dim, page, float(scale), int(window),
-        plan["split_len"], stream()), "attention_decode_rope")
+        plan["split_len"], nsplit, ptr(part_o), ptr(part_ml), ptr(done) if nsplit > 1 else None, stream()), "attention_decode_rope")
     return True
 
 

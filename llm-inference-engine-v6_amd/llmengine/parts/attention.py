@@ -142,7 +142,14 @@ class Attention(Mixer):
                     and x.dtype == torch.bfloat16 and self.w_qkv.dtype == torch.bfloat16
                     and (T * (self.q_dim + 2 * self.kv_dim)) % 4 == 0)
             # (the product that adds has a buffer that nothing else writes: what it is left holding is known)
-            qkv = step.buffer("attn.qkv_sum" if adds else "attn.qkv", (T, self.q_dim + 2 * self.kv_dim), torch.float32)
+            width, done = self.q_dim + 2 * self.kv_dim, None
+            inside = adds and not applies and rot == hd and T == step.num_seqs
+            if inside:
+                # (behind the rows: what the attention kernel counts its splits with, zero whenever the rows are)
+                held = step.buffer("attn.qkv_sum", (T * width + (T * n_kv + 3) // 4 * 4,), torch.float32)
+                qkv, done = held[:T * width].view(T, width), held[T * width:]
+            else:
+                held = qkv = step.buffer("attn.qkv_sum" if adds else "attn.qkv", (T, width), torch.float32)
             if adds:
                 # a few dozen rows (decoding at larger batches): q/k/v has too few output tiles for the
                 # chip, so the product is cut over k and adds its parts into a cleared buffer
@@ -150,8 +157,8 @@ class Attention(Mixer):
                 # is cleared for the step's first such layer; the rotation kernel leaves it zero for
                 # the next one (a clearing kernel per layer took 4.6 us). The note of that is the
                 # step's: every step, and every recording of one, clears for itself.
-                if step.extra.get("attn.qkv_sum zero", (0, 0)) != (qkv.data_ptr(), qkv.numel()):
-                    ops.clear(qkv)
+                if step.extra.get("attn.qkv_sum zero", (0, 0)) != (held.data_ptr(), held.numel()):
+                    ops.clear(held)
                 step.extra.pop("attn.qkv_sum zero", None)
                 ops.gemm(x, self.w_qkv, qkv, accumulate=True, fixed_order=step.fixed_order, choices=step.choices)
             else:
@@ -159,18 +166,18 @@ class Attention(Mixer):
             if applies:
                 self.position.apply(qkv[:, :self.q_dim].view(T, n_q, hd),
                                     qkv[:, self.q_dim:self.q_dim + self.kv_dim].view(T, n_kv, hd), step.positions)
-            if adds and not applies and rot == hd and T == step.num_seqs:
+            if inside:
                 # decoded tokens only: the attention kernel rotates, writes the cache and clears the rows itself
                 o = step.buffer("attn.o", (T, self.q_dim), act)
                 if ops.mfma.attention_decode_rope(qkv, cos, sin, k_cache, v_cache, o, step, block_table, n_q, n_kv, hd,
-                                                  self.scale, self.window):
-                    step.extra["attn.qkv_sum zero"] = (qkv.data_ptr(), qkv.numel())
+                                                  self.scale, self.window, done):
+                    step.extra["attn.qkv_sum zero"] = (held.data_ptr(), held.numel())
                     ops.gemm(o, self.w_o, out, accumulate, fixed_order=step.fixed_order, choices=step.choices)
                     return
             ops.rope_kv_write(qkv, cos, sin, step.positions, step.seq_idx, block_table, q, k_cache, v_cache,
                               n_q, n_kv, hd, rot, write_cache=True, zero_input=adds)
             if adds:
-                step.extra["attn.qkv_sum zero"] = (qkv.data_ptr(), qkv.numel())
+                step.extra["attn.qkv_sum zero"] = (held.data_ptr(), held.numel())
         else:
             # A layer that reads another layer's cache projects queries only.
             q32 = step.buffer("attn.q32", (T, self.q_dim), torch.float32)

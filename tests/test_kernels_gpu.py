@@ -1093,3 +1093,49 @@ def test_attention_generic_four_keys_at_a_time(ops, page, window):
     ops.attention_generic(s["q"], s["k_cache"], s["v_cache"], out, s["positions"], s["seq_idx"], s["table"], n_q, n_kv, hd, 0.3, window)
     ref = torch.cat([plain_attention(q * (0.3 * math.sqrt(hd)), k, v, window).reshape(-1, n_q * hd) for q, k, v in s["plain"]])
     assert _rel(out.cpu().double()[last], ref[last]) < 3e-6 and _rel(out.cpu().double(), ref) < 3e-6
+
+
+@pytest.mark.parametrize("n_q,n_kv,hd,split_len,window", [(4, 2, 64, 64, 0), (32, 8, 64, 160, 0), (24, 8, 128, 96, 0), (3, 1, 128, 32, 0),
+                                                          (4, 2, 64, 64, 70), (8, 1, 128, 128, 33)])
+def test_attention_decode_rope_joins_its_splits(ops, n_q, n_kv, hd, split_len, window):
+    """The decode kernel that rotates, with its keys in several splits: requests of one key, of a split's length and one more,
+    of all splits; a window that leaves out the first ones. Against the same plan through the rotation kernel, the decode kernel
+    and the join kernel, whose weights are normed before the sum and not after: two roundings of bfloat16 apart at most (2^-7 of
+    a value, 2^-9 of the largest where terms cancel). The rows and the counters are left zero, and a second launch on the same
+    numbers gives the same bits whichever split is done last."""
+    import types
+    page, lens = 16, [1, split_len, split_len + 1, 3 * split_len - 1, 17, 2 * split_len, 5 * split_len - 3] * 3
+    S, nsplit, width, scale = len(lens), 5, (n_q + 2 * n_kv) * hd, 0.11
+    g = _gen(72)
+    nblk = (max(lens) + page - 1) // page
+    table = torch.randperm(S * nblk, generator=g).view(S, nblk).to(torch.int32).to(DEV)
+    ang = torch.arange(max(lens) + 1, dtype=torch.float64)[:, None] / (10000.0 ** (torch.arange(hd // 2, dtype=torch.float64) * 2 / hd))[None, :]
+    cos, sin = torch.cos(ang).float().to(DEV), torch.sin(ang).float().to(DEV)
+    k0 = torch.randn(S * nblk, n_kv, page, hd, generator=g).to(torch.bfloat16).to(DEV)
+    v0 = torch.randn(S * nblk, n_kv, hd, page, generator=g).to(torch.bfloat16).to(DEV)
+    qkv = torch.randn(S, width, generator=g).to(DEV)
+    i32 = dict(dtype=torch.int32, device=DEV)
+    q_start, ctx = torch.arange(S + 1, **i32), torch.tensor([n - 1 for n in lens], **i32)
+    plan = {"n_decode": S, "groups": 0, "split_len": split_len, "nsplit": nsplit, "prefill_splits": 1, "prefill_run": 1, "tuning": 0}
+
+    def scratch(*shape):
+        return torch.full(shape, float("nan"), device=DEV)
+    k1, v1, q = k0.clone(), v0.clone(), torch.empty(S, n_q * hd, dtype=torch.bfloat16, device=DEV)
+    ops.rope_kv_write(qkv.clone(), cos, sin, ctx, torch.arange(S, **i32), table, q, k1, v1, n_q, n_kv, hd, hd)
+    apart = torch.zeros(S, n_q * hd, dtype=torch.bfloat16, device=DEV)
+    ops.mfma.attention_bf16(q, k1, v1, apart, q_start, ctx, table, n_q, n_kv, hd, scale, window, plan,
+                            scratch(S * n_q * nsplit * hd), scratch(S * n_q * nsplit * 2))
+    step = types.SimpleNamespace(num_seqs=S, new_lens=[1] * S, ctx_lens=[n - 1 for n in lens], plan_len=None, q_start=q_start,
+                                 ctx_len=ctx, extra={("attention_plan", n_q, n_kv, hd): plan},
+                                 buffer=lambda name, shape, dtype: scratch(*shape))
+    done, outs = torch.zeros(S * n_kv, device=DEV), []
+    for _ in range(2):
+        k2, v2, raw = k0.clone(), v0.clone(), qkv.clone()
+        out = torch.zeros(S, n_q * hd, dtype=torch.bfloat16, device=DEV)
+        assert ops.mfma.attention_decode_rope(raw, cos, sin, k2, v2, out, step, table, n_q, n_kv, hd, scale, window, done)
+        assert not raw.any() and not done.view(torch.int32).any()
+        assert torch.equal(k1, k2) and torch.equal(v1, v2)
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1])
+    want = apart.float()
+    assert bool(((outs[0].float() - want).abs() <= want.abs() * 2.0 ** -7 + want.abs().max() * 2.0 ** -9).all())
