@@ -36,6 +36,7 @@
 // Limits (the caller checks them and otherwise uses the plain-precision kernel): head size a
 // multiple of 16 up to 128; page size a multiple of 16.
 #include <mutex>
+#include <type_traits>
 
 #include "attention_tiles.h"
 #include "llmengine_noalloc.h"
@@ -44,15 +45,20 @@ namespace llme {
 
 // ------------------------------------------------------------------------------------------
 // decode: one token per request; the work of a workgroup is decode_item (attention_tiles.h).
+// Heads of 128 go through LDS (attend_range_staged).
+constexpr bool staged_decode(int hd, bool stream) { return stream && hd == 128; }
 template <int HD, bool STREAM>
 __global__ __launch_bounds__(DEC_WAVES * 64) void attention_decode_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k_cache, const bf16* __restrict__ v_cache,
     bf16* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml,
     const int* __restrict__ q_start, const int* __restrict__ ctx_len, const int* __restrict__ block_table,
     int max_blocks, int n_q, int n_kv, int page, float scale, int window, int split_len, int nsplit) {
-    __shared__ float sh[decode_lds_floats(HD)];
-    decode_item<HD, STREAM>(q, k_cache, v_cache, out, part_o, part_ml, q_start, ctx_len, block_table, max_blocks, n_q,
-                            n_kv, page, scale, window, split_len, nsplit, blockIdx.y, blockIdx.x, blockIdx.z, sh);
+    constexpr bool STAGED = staged_decode(HD, STREAM);
+    __shared__ float own[STAGED ? 1 : decode_lds_floats(HD)];
+    extern __shared__ __align__(16) float staged[];
+    decode_item<HD, STREAM, false, STAGED>(q, k_cache, v_cache, out, part_o, part_ml, q_start, ctx_len, block_table, max_blocks, n_q,
+                                           n_kv, page, scale, window, split_len, nsplit, blockIdx.y, blockIdx.x, blockIdx.z,
+                                           STAGED ? staged : own);
 }
 
 // The same for a step whose q/k/v rows are still as the projection left them (RAW in attention_tiles.h):
@@ -63,11 +69,13 @@ __global__ __launch_bounds__(DEC_WAVES * 64) void attention_decode_raw_kernel(
     bf16* __restrict__ out, const int* __restrict__ q_start, const int* __restrict__ ctx_len,
     const int* __restrict__ block_table, int max_blocks, int n_q, int n_kv, int page, float scale, int window,
     int split_len, int nsplit, float* part_o, float* part_ml, int* done) {
-    __shared__ float sh[decode_lds_floats(HD)];
+    constexpr bool STAGED = staged_decode(HD, true);
+    __shared__ float own[STAGED ? 1 : decode_lds_floats(HD)];
+    extern __shared__ __align__(16) float staged[];
     const RawQkv raw{qkv, cos_t, sin_t, k_cache, v_cache, done};
-    decode_item<HD, true, true>(nullptr, k_cache, v_cache, out, part_o, part_ml, q_start, ctx_len, block_table,
+    decode_item<HD, true, true, STAGED>(nullptr, k_cache, v_cache, out, part_o, part_ml, q_start, ctx_len, block_table,
                                 max_blocks, n_q, n_kv, page, scale, window, split_len, nsplit, blockIdx.y, blockIdx.x,
-                                blockIdx.z, sh, raw);
+                                blockIdx.z, STAGED ? staged : own, raw);
 }
 
 // Joins the splits of one (row, head): one wavefront, lanes over the splits for the statistics,
@@ -270,6 +278,19 @@ __global__ __launch_bounds__(256) void attention_prefill_kernel(
     }
 }
 
+// Launches a decode kernel with the LDS that its blocks are staged through, if they are, having told the kernel of it once.
+template <auto KERNEL, typename... ARGS>
+static int launch_staged(int hd, dim3 grid, hipStream_t stream, ARGS... args) {
+    static bool told = false;                           // per kernel
+    const int lds = staged_decode(hd, true) ? decode_staged_bytes(hd) : 0;
+    if (!told && lds) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(KERNEL), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (e != hipSuccess) return static_cast<int>(e);
+        told = true;
+    }
+    hipLaunchKernelGGL(KERNEL, grid, dim3(DEC_WAVES * 64), lds, stream, args...);
+    return launch_status();
+}
 // What a caller may override of the launch choices, for tests and measurements, packed into
 // the entry points' `tuning` argument (0: every choice is the entry point's):
 //   bits 0-7   rows per work item of the prefill kernel without LDS: 16, 32 or 64 (0: by head size)
@@ -310,11 +331,12 @@ static int launch_for_head(const bf16* q, const bf16* kc, const bf16* vc, bf16* 
     const bool together = n_decode > 0 && prefill_groups > 0 && shared_rows > 0 && decode_reads_once(tuning);
     if (n_decode > 0 && !together) {
         const dim3 grid(head_tiles, n_seq, nsplit);
-        if (decode_reads_once(tuning))
-            hipLaunchKernelGGL((attention_decode_kernel<HD, true>), grid, dim3(DEC_WAVES * 64), 0, stream, q, kc, vc, out,
-                               part_o, part_ml, q_start, ctx_len, table, max_blocks, n_q, n_kv, page, scale, window,
-                               split_len, nsplit);
-        else
+        if (decode_reads_once(tuning)) {
+            const int status = launch_staged<&attention_decode_kernel<HD, true>>(HD, grid, stream, q, kc, vc, out, part_o, part_ml, q_start,
+                                                                                ctx_len, table, max_blocks, n_q, n_kv, page, scale, window,
+                                                                                split_len, nsplit);
+            if (status != 0) return status;
+        } else
             hipLaunchKernelGGL((attention_decode_kernel<HD, false>), grid, dim3(DEC_WAVES * 64), 0, stream, q, kc, vc, out,
                                part_o, part_ml, q_start, ctx_len, table, max_blocks, n_q, n_kv, page, scale, window,
                                split_len, nsplit);
@@ -470,17 +492,14 @@ extern "C" int llme_attention_decode_rope_bf16(float* qkv, const float* cos_t, c
         reinterpret_cast<uintptr_t>(sin_t) % 16 != 0 || reinterpret_cast<uintptr_t>(k_cache) % 16 != 0)
         return kErrUnsupported;
     const dim3 grid(n_kv, n_seq, nsplit);
-    if (hd == 64)
-        hipLaunchKernelGGL(attention_decode_raw_kernel<64>, grid, dim3(DEC_WAVES * 64), 0, stream, qkv, cos_t, sin_t,
-                           static_cast<bf16*>(k_cache), static_cast<bf16*>(v_cache), static_cast<bf16*>(out), q_start,
-                           ctx_len, block_table, max_blocks, n_q, n_kv, page, scale, window, split_len, nsplit, part_o,
-                           part_ml, done);
-    else
-        hipLaunchKernelGGL(attention_decode_raw_kernel<128>, grid, dim3(DEC_WAVES * 64), 0, stream, qkv, cos_t, sin_t,
-                           static_cast<bf16*>(k_cache), static_cast<bf16*>(v_cache), static_cast<bf16*>(out), q_start,
-                           ctx_len, block_table, max_blocks, n_q, n_kv, page, scale, window, split_len, nsplit, part_o,
-                           part_ml, done);
-    return launch_status();
+    auto launch = [&](auto kernel) {
+        return launch_staged<decltype(kernel)::value>(hd, grid, stream, qkv, cos_t, sin_t, static_cast<bf16*>(k_cache),
+                                                      static_cast<bf16*>(v_cache), static_cast<bf16*>(out), q_start, ctx_len,
+                                                      block_table, max_blocks, n_q, n_kv, page, scale, window, split_len, nsplit,
+                                                      part_o, part_ml, done);
+    };
+    if (hd == 64) return launch(std::integral_constant<decltype(&attention_decode_raw_kernel<64>), &attention_decode_raw_kernel<64>>{});
+    return launch(std::integral_constant<decltype(&attention_decode_raw_kernel<128>), &attention_decode_raw_kernel<128>>{});
 }
 
 // ------------------------------------------------------------------------------------------

@@ -337,6 +337,138 @@ __device__ __forceinline__ void attend_range(const PagedKV& kv, int first, int s
         attend_edge_block<HD, QT>(kv, t0, key_lo, key_end, qf, row_pos, row_lo, tile_free, scale_log2, m, l, o);
 }
 
+// ------------------------------------------------------------------------------------------
+// The same walk for one row tile of a decoding request with the blocks staged through LDS: a wavefront asks for whole halves of
+// 16 keys in pieces of 1 KB (16 bytes a lane, consecutive where they lie so) that go straight into LDS, two blocks ahead of the
+// products, in buffers of its own (no barrier: it counts its own loads). Loads into operand registers are asked for only when
+// the registers are free, one block ahead at most, and fetch 64-byte halves of lines: a workgroup alone on a compute unit drew
+// 32 GB/s that way, however many wavefronts it had, where consecutive loads draw 60.
+// In LDS a half of K is [16 keys][HD] with the 16-byte pieces of key r in the order j ^ (r % 8), so that the eight keys that a
+// read takes together lie in different banks; a half of V is [HD][16 keys]. Halves without a key in [key_lo, key_end) are
+// read from the range's last half instead (they are masked), so every page that is looked up exists.
+// Heads of 128 only. Measured, us through registers / staged, 2,048 keys: 8 workgroups 32.2 / 27.1, 192 43.9 / 37.1, 512 92.9 /
+// 87.7; 192 of 4,096 keys 81.2 / 67.8, of 256 11.0 / 9.3. With heads of 64 a block is 8 KB, which comes in less time than a
+// wavefront's products and weights take (1.1 us): 8 workgroups 13.8 / 18.6, 256 25.3 / 31.1 (eight wavefronts 25.1), 512 48.1 /
+// 45.4, and a decode step of 8 requests at 4,096 of the 1B sizes 0.864 / 0.879 ms with eight, of 64 at 1,800 1.654 / 1.662.
+__device__ __forceinline__ void load_1kb_to_lds_once(const void* base, unsigned bytes, unsigned lds_base, unsigned voffset, unsigned soffset) {
+    typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
+    const unsigned long long p = reinterpret_cast<unsigned long long>(base);
+    const u32x4 rsrc{static_cast<unsigned>(p), static_cast<unsigned>(p >> 32) & 0xFFFFu, bytes, 0x00020000u};
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
+                 :
+                 : "s"(lds_base), "v"(voffset), "s"(rsrc), "s"(soffset)
+                 : "memory", "m0");
+}
+// Waits until at most N of the wavefront's vector memory operations are on their way, for the compiler's loads from LDS too.
+template <int N> __device__ __forceinline__ void wait_loads() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+__device__ __forceinline__ void wait_lds_reads() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
+template <int HD> constexpr int staged_wave_bytes() { return 2 * 2 * 32 * HD * 2; }        // two blocks of K and of V
+
+template <int HD>
+__device__ __forceinline__ void attend_range_staged(const PagedKV& kv, int first, int stride, int key_lo, int key_end,
+                                                    const bf16x8 (&qf)[1][(HD + 31) / 32], const int (&row_pos)[1],
+                                                    const int (&row_lo)[1], float scale_log2, float (&m)[1], float (&l)[1],
+                                                    f32x4 (&o)[1][HD / 16], unsigned char* lds) {
+    static_assert(HD == 64 || HD == 128, "rows of 8 or 16 pieces");
+    constexpr int DC = HD / 32, DT = HD / 16, HALF = 16 * HD * 2, PER = HALF / 1024, L = 2 * PER;   // L: loads of a block's K, or V
+    const int lane = threadIdx.x & 63, r = lane & 15, g4 = lane >> 4;
+    if (first >= key_end) return;
+    const int blocks = (key_end - first + stride - 1) / stride;
+    const int last_half = (key_end - 1) & ~15;
+    // The page ids of 32 blocks, a half's in a lane: looked up one by one, in the loop, each was a trip to memory that the waits
+    // for LDS waited for as well.
+    auto look_up = [&](int b) {
+        int h0 = first + (b + (lane >> 1)) * stride + (lane & 1) * 16;
+        if (h0 > last_half || h0 + 15 < key_lo) h0 = last_half;
+        return kv.table[page_of(kv, h0).block];
+    };
+    int ids = look_up(0);
+    const unsigned lds_k = static_cast<unsigned>(reinterpret_cast<size_t>((__attribute__((address_space(3))) unsigned char*)lds));
+    const unsigned lds_v = lds_k + 2 * 2 * HALF;
+    // a lane's piece in K: row lane / (HD / 8) of the 1 KB, the piece that belongs into its slot (rows go on by 8 or 4 a piece)
+    unsigned koff[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int row = lane / (HD / 8) + (HD == 128 ? 4 * u : 0), slot = lane % (HD / 8);
+        koff[u] = static_cast<unsigned>(lane / (HD / 8)) * (HD * 2) + static_cast<unsigned>(slot ^ (row & 7)) * 16;
+    }
+    const unsigned voff = static_cast<unsigned>(lane >> 1) * (kv.page * 2) + (lane & 1) * 16;
+    struct Half {
+        int pg, off;
+    };
+    auto place = [&](int b, int hf) {
+        int h0 = first + b * stride + hf * 16;
+        if (h0 > last_half || h0 + 15 < key_lo) h0 = last_half;
+        return Half{__builtin_amdgcn_readlane(ids, (b & 31) * 2 + hf), __builtin_amdgcn_readfirstlane(page_of(kv, h0).offset)};
+    };
+    auto ask_k = [&](int b) {
+        const int stage = b & 1;
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf) {
+            const Half p = place(b, hf);
+            const bf16* base = kv.k + static_cast<size_t>(p.pg) * kv.page_stride + kv.head_off + static_cast<size_t>(p.off) * HD;
+#pragma unroll
+            for (int i = 0; i < PER; ++i)
+                load_1kb_to_lds_once(base, HALF, lds_k + (stage * 2 + hf) * HALF + i * 1024, koff[i & 1], i * 1024);
+        }
+    };
+    auto ask_v = [&](int b) {
+        const int stage = b & 1;
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf) {
+            const Half p = place(b, hf);
+            const bf16* base = kv.v + static_cast<size_t>(p.pg) * kv.page_stride + kv.head_off + p.off;
+#pragma unroll
+            for (int i = 0; i < PER; ++i)
+                load_1kb_to_lds_once(base, static_cast<unsigned>(HD - 1) * kv.page * 2 + 32, lds_v + (stage * 2 + hf) * HALF + i * 1024, voff,
+                                     i * 32 * kv.page * 2);
+        }
+    };
+    ask_k(0);
+    ask_v(0);
+    if (blocks > 1) {
+        ask_k(1);
+        ask_v(1);
+    }
+    const int tile_free[1] = {-1};                          // (few blocks, heads may be missing: always checked)
+    for (int b = 0; b < blocks; ++b) {
+        const int stage = b & 1, t0 = first + b * stride;
+        const bool one = b + 1 < blocks, two = b + 2 < blocks;
+        if (two && ((b + 2) & 31) == 0) ids = look_up(b + 2);
+        if (one) wait_loads<3 * L>();                       // K is there; V and the next block may be on their way
+        else wait_loads<L>();
+        KFrag<HD> kf;
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+            for (int c = 0; c < DC; ++c)
+                kf.kf[hf][c] = *reinterpret_cast<const bf16x8*>(lds + (stage * 2 + hf) * HALF + r * (HD * 2) + ((c * 4 + g4) ^ (r & 7)) * 16);
+        wait_lds_reads();
+        if (two) ask_k(b + 2);
+        f32x4 s[1][2];
+        block_scores<HD, 1>(kf, qf, s);
+        bf16x8 pf[1];
+        block_weights<HD, 1>(s, t0, row_pos, row_lo, tile_free, scale_log2, m, l, o, pf);
+        if (two) wait_loads<3 * L>();
+        else if (one) wait_loads<2 * L>();
+        else wait_loads<0>();
+        VFrag<HD> vf;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+            const unsigned char* at = lds + 2 * 2 * HALF + stage * 2 * HALF + (dt * 16 + r) * 32 + g4 * 8;
+            const bf16x4 lo4 = *reinterpret_cast<const bf16x4*>(at), hi4 = *reinterpret_cast<const bf16x4*>(at + HALF);
+            vf.vf[dt] = __builtin_shufflevector(lo4, hi4, 0, 1, 2, 3, 4, 5, 6, 7);
+        }
+        wait_lds_reads();
+        if (two) ask_v(b + 2);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) o[0][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf[0], vf.vf[dt], o[0][dt], 0, 0, 0);
+    }
+}
+
 // Loads the query fragments of one 16-row tile: lane holds row r, dims c * 32 + 8 g4 ..
 template <int HD>
 __device__ __forceinline__ void load_q(const bf16* qrow, bool ok, bf16x8 (&qf)[(HD + 31) / 32]) {
@@ -386,7 +518,9 @@ template <bool SHARED> __device__ __forceinline__ void put_part(float* p, float 
 __device__ __forceinline__ float get_part(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
 // (k_cache and v_cache carry no promise that nothing else points at them: RAW writes into them)
-template <int HD, bool STREAM, bool RAW = false>
+// STAGED: the keys go through LDS (attend_range_staged; head size 64 or 128); `sh` then has decode_staged_bytes(HD) bytes.
+__host__ __device__ constexpr int decode_staged_bytes(int hd) { return DEC_WAVES * 2 * 2 * 32 * hd * 2; }
+template <int HD, bool STREAM, bool RAW = false, bool STAGED = false>
 __device__ __forceinline__ void decode_item(
     const bf16* __restrict__ q, const bf16* k_cache, const bf16* v_cache,
     bf16* __restrict__ out, float* part_o, float* part_ml,
@@ -488,6 +622,7 @@ __device__ __forceinline__ void decode_item(
                 zero8(vrow + d0);
             }
         }
+        if (STAGED) wait_loads<0>();                    // (the stores too)
         __syncthreads();                                // the key and the value are in the page; every wavefront has read q
         if (wave == 0 && row_ok && parts == 1) {
 #pragma unroll
@@ -508,8 +643,14 @@ __device__ __forceinline__ void decode_item(
     for (int dt = 0; dt < DT; ++dt) o[0][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     const int first = k_begin + __builtin_amdgcn_readfirstlane(wave) * 32;
-    attend_range<HD, 1, STREAM>(kv, first, DEC_WAVES * 32, lo_all, k_end, qf, row_pos, row_lo, tile_free,
-                              scale * kLog2e, m, l, o);
+    if constexpr (STAGED) {
+        static_assert(!STAGED || DEC_WAVES * staged_wave_bytes<HD>() >= decode_lds_floats(HD) * 4, "the join fits into the buffers");
+        attend_range_staged<HD>(kv, first, DEC_WAVES * 32, lo_all, k_end, qf, row_pos, row_lo, scale * kLog2e, m, l, o,
+                                reinterpret_cast<unsigned char*>(sh) + __builtin_amdgcn_readfirstlane(wave) * staged_wave_bytes<HD>());
+        __syncthreads();                                // (the join reuses the buffers)
+    } else {
+        attend_range<HD, 1, STREAM>(kv, first, DEC_WAVES * 32, lo_all, k_end, qf, row_pos, row_lo, tile_free, scale * kLog2e, m, l, o);
+    }
 
     float lt = l[0];
     lt += __shfl_xor(lt, 16, 64);
