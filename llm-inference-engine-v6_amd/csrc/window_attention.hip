@@ -298,20 +298,24 @@ enum FinishMode : int { kFinishPlain = 0, kFinishGate = 1, kFinishDifference = 2
 // mixer's last step. gate [T, ld_gate] 32-bit, one entry per output entry (kFinishGate) or one per head
 // (kFinishHeadGate). kFinishDifference: o = a_1 - lambda a_2 over the head's two maps, o / sqrt(mean(o^2) + eps).
 // sinks [heads] (32-bit, or null; one map a head): the joined sum also holds e^(sink - maximum). All times out_scale.
-template <typename TO, int MODE>
+// PER_LANE: a lane's entries of a head, 1, 2 or 4. A decoding step has a wavefront for every head and little else: what it
+// waits for is trips to memory, so the values of as many runs as the registers hold are asked for at once (32 for heads of
+// 64, 16 for two maps of 128), the first together with the runs' maxima, and both of these are read once. Two requests behind
+// 1,500 tokens, us, with 8 at a time behind two readings of the maxima / so: 32 heads of 64 8.9 / 5.6, gated 9.4 / 6.4, the
+// difference of 16 heads' maps over 128 13.4 / 12.3.
+template <typename TO, int MODE, int PER_LANE>
 __global__ __launch_bounds__(256) void window_attention_finish_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                                                       int runs, int T, int heads, int maps, int dv,
                                                                       const float* __restrict__ gate, int ld_gate, float lambda,
                                                                       float eps, float out_scale, const float* __restrict__ sinks,
                                                                       TO* __restrict__ out, int ld_out) {
-    constexpr int PER_LANE = kMaxHeadEntries / kWave;
     const int lane = threadIdx.x & 63;
     const size_t item = static_cast<size_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
     if (item >= static_cast<size_t>(T) * heads) return;
     const int t = static_cast<int>(item / heads), head = static_cast<int>(item % heads);
     const int nq = heads * maps;
     constexpr int MAPS = MODE == kFinishDifference ? 2 : 1;
-    constexpr int CHUNK = 8;                // runs whose values are asked for together
+    constexpr int CHUNK = 64 / (PER_LANE * MAPS) > 32 ? 32 : 64 / (PER_LANE * MAPS);    // runs whose values are asked for together
     const size_t stride = static_cast<size_t>(T) * nq;
     const size_t at0 = static_cast<size_t>(t) * nq + head * MAPS;
     float a[MAPS][PER_LANE], l[MAPS];
@@ -322,13 +326,39 @@ __global__ __launch_bounds__(256) void window_attention_finish_kernel(const floa
         for (int i = 0; i < PER_LANE; ++i) a[mp][i] = 0.f;
     }
     // lane r holds run r's maximum and sum (64 runs at a time); the runs' values are then added in the order of the
-    // runs, eight runs of every map of the head asked for before the first is used
-    float mx[MAPS];
+    // runs, CHUNK runs of every map of the head asked for before the first is used
+    float v[CHUNK][MAPS][PER_LANE];
+    auto ask = [&](int r0, int n) {         // runs r0 .. r0 + CHUNK - 1, the first n of which exist
+#pragma unroll
+        for (int j = 0; j < CHUNK; ++j)
+#pragma unroll
+            for (int mp = 0; mp < MAPS; ++mp)
+#pragma unroll
+                for (int i = 0; i < PER_LANE; ++i) {
+                    const int d = lane + i * kWave;
+                    v[j][mp][i] = (j < n && d < dv) ? part_o[((r0 + j) * stride + at0 + mp) * dv + d] : 0.f;
+                }
+    };
+    if (runs > 1) ask(0, runs);
+    float gates[PER_LANE] = {};
+    if (MODE == kFinishGate)
+#pragma unroll
+        for (int i = 0; i < PER_LANE; ++i) gates[i] = lane + i * kWave < dv ? gate[static_cast<size_t>(t) * ld_gate + head * dv + lane + i * kWave] : 0.f;
+    float mx[MAPS], m_own[MAPS], l_own[MAPS];               // (the first 64 runs': a lane's own)
 #pragma unroll
     for (int mp = 0; mp < MAPS; ++mp) {
-        float v = -INFINITY;
-        for (int r = lane; r < (runs == 1 ? 0 : runs); r += kWave) v = fmaxf(v, part_ml[(r * stride + at0 + mp) * 2]);
-        mx[mp] = wave_max(v);
+        m_own[mp] = -INFINITY;
+        l_own[mp] = 0.f;
+        if (runs > 1 && lane < runs) {
+            m_own[mp] = part_ml[(lane * stride + at0 + mp) * 2];
+            l_own[mp] = part_ml[(lane * stride + at0 + mp) * 2 + 1];
+        }
+    }
+#pragma unroll
+    for (int mp = 0; mp < MAPS; ++mp) {
+        float top = m_own[mp];
+        for (int r = lane + kWave; r < runs; r += kWave) top = fmaxf(top, part_ml[(r * stride + at0 + mp) * 2]);
+        mx[mp] = wave_max(top);
     }
     if (runs == 1) {                         // (prompts: one run, nothing to join)
 #pragma unroll
@@ -348,23 +378,14 @@ __global__ __launch_bounds__(256) void window_attention_finish_kernel(const floa
         for (int mp = 0; mp < MAPS; ++mp) {
             fr[mp] = lr[mp] = 0.f;
             if (r < runs) {
-                const float mr = part_ml[(r * stride + at0 + mp) * 2];
+                const float mr = r0 == 0 ? m_own[mp] : part_ml[(r * stride + at0 + mp) * 2];
                 fr[mp] = mr == -INFINITY ? 0.f : expf(mr - mx[mp]);            // (a run in which the row saw no key)
-                lr[mp] = part_ml[(r * stride + at0 + mp) * 2 + 1];
+                lr[mp] = r0 == 0 ? l_own[mp] : part_ml[(r * stride + at0 + mp) * 2 + 1];
             }
         }
         const int n = runs - r0 < kWave ? runs - r0 : kWave;
         for (int j0 = 0; j0 < n; j0 += CHUNK) {
-            float v[CHUNK][MAPS][PER_LANE];
-#pragma unroll
-            for (int j = 0; j < CHUNK; ++j)
-#pragma unroll
-                for (int mp = 0; mp < MAPS; ++mp)
-#pragma unroll
-                    for (int i = 0; i < PER_LANE; ++i) {
-                        const int d = lane + i * kWave;
-                        v[j][mp][i] = (j0 + j < n && d < dv) ? part_o[((r0 + j0 + j) * stride + at0 + mp) * dv + d] : 0.f;
-                    }
+            if (r0 + j0 > 0) ask(r0 + j0, n - j0);
 #pragma unroll
             for (int j = 0; j < CHUNK; ++j)
 #pragma unroll
@@ -412,8 +433,7 @@ __global__ __launch_bounds__(256) void window_attention_finish_kernel(const floa
         if (d >= dv) continue;
         float v = o[i] * f;
         if (MODE == kFinishGate) {
-            const float g = gate[static_cast<size_t>(t) * ld_gate + head * dv + d];
-            v *= 1.0f / (1.0f + expf(-g));
+            v *= 1.0f / (1.0f + expf(-gates[i]));
         }
         out[static_cast<size_t>(t) * ld_out + head * dv + d] = from_float<TO>(v);
     }
@@ -514,9 +534,15 @@ extern "C" int llme_window_attention_finish(const float* part_o, const float* pa
     if ((mode == kFinishGate || mode == kFinishHeadGate) && gate == nullptr) return kErrBadArgument;
     if (sinks != nullptr && maps != 1) return kErrBadArgument;
     const dim3 grid(static_cast<unsigned>((static_cast<size_t>(T) * heads + 3) / 4));
-#define LLME_FIN(TO, MODE)                                                                                            \
-    hipLaunchKernelGGL((window_attention_finish_kernel<TO, MODE>), grid, dim3(256), 0, stream, part_o, part_ml, runs, T, heads, \
-                       maps, dv, gate, ld_gate, lambda, eps, out_scale, sinks, static_cast<TO*>(out), ld_out)
+#define LLME_FIN_AS(TO, MODE, PER)                                                                                          \
+    hipLaunchKernelGGL((window_attention_finish_kernel<TO, MODE, PER>), grid, dim3(256), 0, stream, part_o, part_ml, runs, T, \
+                       heads, maps, dv, gate, ld_gate, lambda, eps, out_scale, sinks, static_cast<TO*>(out), ld_out)
+#define LLME_FIN(TO, MODE)                                       \
+    do {                                                         \
+        if (dv <= kWave) LLME_FIN_AS(TO, MODE, 1);               \
+        else if (dv <= 2 * kWave) LLME_FIN_AS(TO, MODE, 2);      \
+        else LLME_FIN_AS(TO, MODE, 4);                           \
+    } while (0)
 #define LLME_FIN_T(TO)                                                     \
     do {                                                                   \
         if (mode == kFinishPlain) LLME_FIN(TO, kFinishPlain);              \
@@ -530,6 +556,7 @@ extern "C" int llme_window_attention_finish(const float* part_o, const float* pa
     else return kErrBadArgument;
 #undef LLME_FIN_T
 #undef LLME_FIN
+#undef LLME_FIN_AS
     return launch_status();
 }
 
