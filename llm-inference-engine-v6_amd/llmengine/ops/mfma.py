@@ -570,12 +570,17 @@ def qkv_sum_max_rows(decoded_only: bool, head_dim: int, choices: KernelChoices |
     single decoded tokens keeps that way further: with heads of 64 (choices.qkv_sum_rows_decoding) the
     attention kernel then rotates and writes the cache itself (attention_decode_rope); with heads of 128
     (choices.qkv_sum_rows_decoding_128) the rotation kernel does, and the product's tiles of 96 or 128 rows
-    with the rotation in their epilogue are the slower way until then."""
+    with the rotation in their epilogue are the slower way until then. A step that holds prompt rows is launched
+    kernel by kernel, which takes the host longer than a layer of heads of 64 takes the chip (82 against 64 us at the
+    1B sizes, 45 rows): its product rotates and writes the cache in its epilogue, a launch a layer fewer
+    (45 rows 1.339 / 1.179 ms; layers with heads of 128 are the chip's time, and keep the sum)."""
     ch = choices or DEFAULT
     if decoded_only and head_dim == 64 and ch.decode_rope:
         return max(QKV_SUM_MAX_ROWS, ch.qkv_sum_rows_decoding)
     if decoded_only and head_dim == 128:
         return max(QKV_SUM_MAX_ROWS, ch.qkv_sum_rows_decoding_128)
+    if not decoded_only and head_dim <= 64:
+        return GEMV_NORM_MAX_ROWS
     return QKV_SUM_MAX_ROWS
 
 
