@@ -1449,13 +1449,14 @@ extern "C" int llme_gemm_bf16(const void* a, const void* w, void* out, int out_d
         mode = kAtomicF32;
     }
     if (auto_shape && blocked && direct != 0 && mode != kAtomicF32 && tiles_cost > 0.f) {
-        // Wide outputs that are stored, not added (gate/up, q/k/v of long prompts): tiles of 256 x 256
-        // by eight wavefronts, their slabs straight into LDS, load half the bytes per product; one
-        // workgroup fills a compute unit. In the units of the estimate above a round of them costs
-        // 65,536 / 1.15 (measured: 1.07 to 1.16 times the 128 x 128 tiles' speed where whole rounds cover
-        // the output; 8B gate/up at 448 rows, one round against 3.5 of 128 x 128: 105 against 129 us).
+        // Large outputs: tiles of 256 x 256 by eight wavefronts, their slabs straight into LDS, load half the bytes per
+        // product; one workgroup fills a compute unit. In the units of the estimate above a round of them costs 65,536 / 1.36:
+        // one round beats three of 128 x 128 tiles and two beat six, two do not beat five. (Measured, us, 128 x 128 / 256 x 256:
+        // gate/up of the 1B sizes at 700 rows 55 / 47, 1,300 rows 99 / 94, 500 rows 40 / 47; of the 8B sizes at 300 rows 98 / 90,
+        // 600 rows 158 / 166; down-proj, added: 8B sizes at 3,000 rows 341 / 287, 2,048 rows 234 / 283; 1B sizes at 6,000
+        // rows 197 / 170, 4,096 rows 135 / 167.)
         const long rounds = (static_cast<long>((M + 255) / 256) * ((N + 255) / 256) + cus - 1) / cus;
-        if (static_cast<float>(rounds) * 65536.f / 1.15f < tiles_cost)
+        if (static_cast<float>(rounds) * 65536.f / 1.36f < tiles_cost)
             return launch_tile_direct<4, 2, 4, 8>(A, W, out, M, N, K, mode, ksplit, stream);
     }
     if (blocked && direct == 1 && tile_shape == 256256)
