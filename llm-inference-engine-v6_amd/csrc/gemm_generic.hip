@@ -186,8 +186,8 @@ static int launch_gemv_generic(const void* a, const void* w, void* out, int M, i
 // 16 WMT x 16 WNT of the output; KW wavefronts share an output and take every KW-th 32 of k, their sums meeting in LDS in one
 // order (the same bits in every run). D blocks of 32 k are in flight per wavefront.
 // Measured at 149 rows, the 1B sizes (before: the 64 x 64 tile kernel above on 96 to 768 workgroups, one load at a time):
-// o-proj and down-proj 587 -> 69 us on average, q/k/v 236 -> 32, gate/up 398 -> 159 (67 TFLOP/s of its 10.7 GFLOP with
-// 32 x 64 tiles). The error against 64 bits is half the former's (2.4e-6 of the logits, 4.7e-6): more and shorter sums.
+// o-proj and down-proj 587 -> 69 us on average, q/k/v 236 -> 32, gate/up 398 -> 140 (71 TFLOP/s of its 10.0 GFLOP with
+// 64 x 64 tiles; 159 with 32 x 64). The error against 64 bits is half the former's (2.4e-6 of the logits, 4.7e-6): more and shorter sums.
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 template <int WMT, int WNT, int WR, int WC, int KW, int D, bool ACC>
@@ -304,9 +304,12 @@ template <bool ACC>
 static int launch_gemm_f32(const float* a, const float* w, float* out, int M, int N, int K, hipStream_t stream) {
     // The tile whose rounds of workgroups over the compute units take the least time: a round is the products of one of a
     // workgroup's wavefronts, over how well its loads are used (a 32 x 32 tile loads twice what a 64 x 64 one does per product).
+    // Measured, outputs of 2,048 to 16,384 columns, 17 to 900 rows: with 1, 0.95, 0.9 and 0.8 the rule took smaller tiles in 25 of
+    // 128 sizes, and 64 x 64 or 128 x 128 are up to 1.36 times as fast there (200 rows x 3,072 of k 2,048: 60 -> 45 us; 149 x
+    // 16,384: 148 -> 133; 200 x 16,384: 206 -> 167) and never more than 4% slower (65 x 16,384: 87 -> 91).
     const int cus = compute_units();
     struct Shape { int bm, bn, products; float eff; };
-    constexpr Shape shapes[4] = {{128, 128, 64, 1.0f}, {64, 64, 16, 0.95f}, {32, 64, 8, 0.9f}, {32, 32, 4, 0.8f}};
+    constexpr Shape shapes[4] = {{128, 128, 64, 1.0f}, {64, 64, 16, 1.0f}, {32, 64, 8, 0.75f}, {32, 32, 4, 0.65f}};
     int best = 0;
     float least = 0.f;
     for (int c = 0; c < 4; ++c) {
