@@ -67,20 +67,10 @@ template <int MODE> __device__ __forceinline__ float stored_value(float v) {
 constexpr bool is_gated(int mode) {
     return mode == kGatedBF16 || mode == kGatedReluBF16 || mode == kGatedGeluBF16 || mode == kGatedExtraBF16;
 }
-// z sigmoid(a z), a z given: the exponential as 2^(hi + lo) with hi + lo = log2(e) (-a z) in two pieces (the piece that the first
-// product rounds away put back as a factor 1 + ln(2) lo), then one hardware reciprocal. A gated epilogue is bound by this
-// arithmetic: expf and a division are twice the instructions.
-__device__ __forceinline__ float times_sigmoid(float z, float az) {
-    const float x = fminf(-az, 150.f);                  // (2^hi is infinite there and the result zero; lo stays finite)
-    const float hi = x * 1.44269504f;
-    const float lo = __builtin_fmaf(x, 1.44269504f, -hi) + x * 1.92596299e-8f;
-    const float e = __builtin_amdgcn_exp2f(hi);
-    return z * __builtin_amdgcn_rcpf(__builtin_fmaf(e, __builtin_fmaf(lo, 0.693147181f, 1.0f), 1.0f));
-}
 template <int MODE> __device__ __forceinline__ float gate_act(float g) {
     if (MODE == kGatedReluBF16) return fmaxf(g, 0.f);
     if (MODE == kGatedGeluBF16) return 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g)));
-    return times_sigmoid(g, g);
+    return g / (1.0f + expf(-g));
 }
 // What kGatedExtraBF16 does around the activation. bias [N] in the order of w's rows (so in the order of the product's
 // columns): added to gate and up first. limit > 0: gate <- min(gate, limit), up <- clamp(up, -limit, limit) and the
@@ -106,9 +96,9 @@ template <int MODE> __device__ __forceinline__ float gated_value(float g, float 
     if (gx.limit > 0.f) {
         g = fminf(g, gx.limit);
         u = fminf(fmaxf(u, -gx.limit), gx.limit);
-        return times_sigmoid(g, gx.alpha * g) * (u + 1.0f);
+        return g / (1.0f + expf(-gx.alpha * g)) * (u + 1.0f);
     }
-    return times_sigmoid(g, g) * u;
+    return g / (1.0f + expf(-g)) * u;
 }
 // The extras of the launches that an entry point is making (set and cleared inside one call, on the caller's thread).
 static thread_local GateExtra t_gate_extra;

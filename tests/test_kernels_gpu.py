@@ -1139,3 +1139,33 @@ def test_attention_decode_rope_joins_its_splits(ops, n_q, n_kv, hd, split_len, w
     assert torch.equal(outs[0], outs[1])
     want = apart.float()
     assert bool(((outs[0].float() - want).abs() <= want.abs() * 2.0 ** -7 + want.abs().max() * 2.0 ** -9).all())
+
+
+@pytest.mark.parametrize("T,tile,direct", [(5, 0, -1), (40, 64, 0), (70, 96064, 0), (70, 128064, 0), (70, 96128, 0), (130, 128, 0), (300, 256256, 1)])
+def test_gated_product_of_gates_over_the_whole_range(ops, T, tile, direct):
+    """silu(gate) * up for gates from zero to infinity, whichever kernel has the rows: a gate that is large is its own SiLU. Against
+    the formula in 64 bits within a rounding of bfloat16 (2^-8), and 3e-37 where e^-gate leaves the 32-bit range (at -88.7, where
+    the value is 2.6e-37)."""
+    gates = [0.0, 1e-3, -1e-3, 1.0, -1.0, 20.0, -20.0, 87.0, -87.0, 88.0, -88.0, -90.0, -150.0, 1e38, -1e38, 2.3e38, 2.5e38, 3e38, -3e38, math.inf]
+    g = torch.tensor((gates * 2)[:32], dtype=torch.float64).to(torch.bfloat16)
+    K, FF = 64, 32
+    w = torch.zeros(2 * FF, K, dtype=torch.bfloat16)
+    w.view(FF // 16, 2, 16, K)[:, 0, :, 0] = g.view(FF // 16, 16)
+    w.view(FF // 16, 2, 16, K)[:, 1, :, 1] = 0.5
+    x = torch.zeros(T, K, dtype=torch.bfloat16)
+    x[:, :2] = 1.0
+    out = torch.zeros(T, FF, dtype=torch.bfloat16, device=DEV)
+    weight = ops.block_weight(w.to(DEV))
+    if tile:
+        ops.gemm_bf16(x.to(DEV), weight, out, gated=True, tile=tile, direct=direct)
+    else:
+        ops.gemm_gated(x.to(DEV), weight, out, 16, None)
+    want = (g.double() / (1 + torch.exp(-g.double())) * 0.5).expand(T, FF)
+    got = out.cpu().double()
+    whole = torch.isfinite(want)
+    assert torch.equal(got[~whole], want[~whole])
+    assert bool(((got - want)[whole].abs() <= want[whole].abs() * 2.0 ** -8 + 3e-37).all())
+    if T >= 17:                                             # the epilogue with extras, without any
+        extra = torch.zeros_like(out)
+        assert ops.gemm_gated_extra(x.to(DEV), weight, extra, 16)
+        assert torch.equal(extra, out)
