@@ -186,6 +186,11 @@ struct AddendsAhead {
     }
 };
 
+// A rotated pair (a, b) -> (a c - b s, b c + a s) with the product that is rounded first named: left to the compiler, which of the
+// two it is differs from kernel to kernel, and with it the last bit of a row by the tile that made it.
+__device__ __forceinline__ float rotated_first(float a, float b, float c, float s) { return __builtin_fmaf(a, c, -(b * s)); }
+__device__ __forceinline__ float rotated_second(float a, float b, float c, float s) { return __builtin_fmaf(b, c, a * s); }
+
 // Where row m0 + tid of the tile goes (rotating epilogue): its position and the page that holds it,
 // looked up by thread tid while the products run (see the kernel).
 struct RowPlace {
@@ -257,9 +262,8 @@ __device__ __forceinline__ void tile_epilogue(f32x4 (&acc)[WMT][WNT], unsigned c
                 bf16x8 lo, hi;
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
-                    const float a = sp[j], b = sp[half + j], c = cs[j], sv = sn[j];
-                    lo[j] = static_cast<__bf16>(a * c - b * sv);
-                    hi[j] = static_cast<__bf16>(b * c + a * sv);
+                    lo[j] = static_cast<__bf16>(rotated_first(sp[j], sp[half + j], cs[j], sn[j]));
+                    hi[j] = static_cast<__bf16>(rotated_second(sp[j], sp[half + j], cs[j], sn[j]));
                 }
                 bf16* dst;
                 if (head < qt.n_q) {
@@ -781,8 +785,8 @@ __device__ __forceinline__ void direct_epilogue(f32x4 (&acc)[WMT][WNT], unsigned
                             for (int j = 0; j < HT; ++j) {
                                 const float x = acc[i][h * 2 * HT + j][e], y = acc[i][h * 2 * HT + HT + j][e];
                                 bf16* sp = stage + row * SH + wn + h * 2 * half + j * 16 + r;
-                                sp[0] = static_cast<__bf16>(rotated ? x * c[j] - y * s[j] : x);
-                                sp[half] = static_cast<__bf16>(rotated ? y * c[j] + x * s[j] : y);
+                                sp[0] = static_cast<__bf16>(rotated ? rotated_first(x, y, c[j], s[j]) : x);
+                                sp[half] = static_cast<__bf16>(rotated ? rotated_second(x, y, c[j], s[j]) : y);
                             }
                         }
                     }

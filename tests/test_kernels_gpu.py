@@ -1029,8 +1029,7 @@ def test_gemm_qkv_rope(ops, n_q, n_kv, hd, K, page, new, tile):
 def test_gemm_qkv_rope_in_wide_tiles(ops, n_q, n_kv, hd, K, new):
     """The rotating epilogue of the 256 x 256 tile kernel against the one of 128 x 128 tiles: portions that start anywhere,
     groups of 16 rows that span two requests, tiles that hang over the rows and over the heads, k of one half slab, of an odd
-    and of an even number. The sums are added in the same order; a rotation may contract a product and a sum into one rounding,
-    which moves a rounded value by one unit of bfloat16 (2^-8 of it) where it moves it at all."""
+    and of an even number. The sums are added in the same order and rotated with the same roundings: the same bits."""
     g, page = _gen(93), 16
     T, N = sum(new), (n_q + 2 * n_kv) * hd
     x = torch.randn(T, K, generator=g).to(torch.bfloat16).to(DEV)
@@ -1050,9 +1049,7 @@ def test_gemm_qkv_rope_in_wide_tiles(ops, n_q, n_kv, hd, K, new):
         ops.gemm_qkv_rope(x, w, cos, sin, positions, seq_idx, table, *made, n_q, n_kv, hd, tile=tile)
         out.append(made)
     for want, got in zip(*out):
-        assert torch.equal(got == 0, want == 0)                 # nothing else was written
-        assert bool(((got.float() - want.float()).abs() <= want.float().abs() * 2.0 ** -7).all())
-    assert torch.equal(out[0][2], out[1][2])                    # v is not rotated
+        assert torch.equal(got, want)                           # (and nothing else was written)
 
 
 @pytest.mark.parametrize("M,N,K", [(17, 16, 4), (31, 33, 28), (33, 65, 32), (64, 64, 36), (149, 2048, 260), (149, 331, 1020),
@@ -1169,3 +1166,26 @@ def test_gated_product_of_gates_over_the_whole_range(ops, T, tile, direct):
         extra = torch.zeros_like(out)
         assert ops.gemm_gated_extra(x.to(DEV), weight, extra, 16)
         assert torch.equal(extra, out)
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("K", [96, 512, 2048])
+def test_gemm_qkv_rope_gives_the_same_bits_in_every_tile(ops, hd, K):
+    """Whichever tile a step's rows are given, the rotated rows are the same bits: the tiles add the products in the same order and
+    rotate with the same two roundings."""
+    g, page, n_q, n_kv, T = _gen(94), 16, 8, 2, 530
+    x = torch.randn(T, K, generator=g).to(torch.bfloat16).to(DEV)
+    w = ops.block_weight((0.05 * torch.randn((n_q + 2 * n_kv) * hd, K, generator=g)).to(torch.bfloat16).to(DEV))
+    ang = torch.arange(T, dtype=torch.float64)[:, None] / (10000.0 ** (torch.arange(hd // 2, dtype=torch.float64) * 2 / hd))[None, :]
+    cos, sin = torch.cos(ang).float().to(DEV), torch.sin(ang).float().to(DEV)
+    blocks = (T + page - 1) // page
+    positions, seq_idx = torch.arange(T, dtype=torch.int32, device=DEV), torch.zeros(T, dtype=torch.int32, device=DEV)
+    table = torch.randperm(blocks, generator=g).view(1, blocks).to(torch.int32).to(DEV)
+    made = []
+    for tile in (128, 96128, 256256) + ((64, 96064, 128064) if hd == 64 else ()):
+        made.append((torch.zeros(T, n_q * hd, dtype=torch.bfloat16, device=DEV),
+                     torch.zeros(blocks, n_kv, page, hd, dtype=torch.bfloat16, device=DEV),
+                     torch.zeros(blocks, n_kv, hd, page, dtype=torch.bfloat16, device=DEV)))
+        ops.gemm_qkv_rope(x, w, cos, sin, positions, seq_idx, table, *made[-1], n_q, n_kv, hd, tile=tile)
+        for want, got in zip(made[0], made[-1]):
+            assert torch.equal(want, got), tile
