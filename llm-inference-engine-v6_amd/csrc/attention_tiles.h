@@ -345,13 +345,15 @@ __device__ __forceinline__ void attend_range(const PagedKV& kv, int first, int s
 // 32 GB/s that way, however many wavefronts it had, where consecutive loads draw 60.
 // In LDS a half of K is [16 keys][HD] with the 16-byte pieces of key r in the order j ^ (r % 8), so that the eight keys that a
 // read takes together lie in different banks; a half of V is [HD][16 keys]. Halves without a key in [key_lo, key_end) are
-// read from the range's last half instead (they are masked), so every page that is looked up exists.
+// read from the range's last half instead (they are masked), so every page that is looked up exists. What a half holds outside
+// [key_lo, key_end) may be anything that an earlier request left in the page: such a key's score is replaced, and its values
+// become zeros in the blocks at the range's edges (a weight of zero alone would let an infinity or NaN through).
 // Heads of 128 only. Measured, us through registers / staged, 2,048 keys: 8 workgroups 32.2 / 27.1, 192 43.9 / 37.1, 512 92.9 /
 // 87.7; 192 of 4,096 keys 81.2 / 67.8, of 256 11.0 / 9.3. With heads of 64 a block is 8 KB, which comes in less time than a
 // wavefront's products and weights take (1.1 us): 8 workgroups 13.8 / 18.6, 256 25.3 / 31.1 (eight wavefronts 25.1), 512 48.1 /
 // 45.4, and a decode step of 8 requests at 4,096 of the 1B sizes 0.864 / 0.879 ms with eight, of 64 at 1,800 1.654 / 1.662.
+typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
 __device__ __forceinline__ void load_1kb_to_lds_once(const void* base, unsigned bytes, unsigned lds_base, unsigned voffset, unsigned soffset) {
-    typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
     const unsigned long long p = reinterpret_cast<unsigned long long>(base);
     const u32x4 rsrc{static_cast<unsigned>(p), static_cast<unsigned>(p >> 32) & 0xFFFFu, bytes, 0x00020000u};
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
@@ -464,6 +466,16 @@ __device__ __forceinline__ void attend_range_staged(const PagedKV& kv, int first
         }
         wait_lds_reads();
         if (two) ask_v(b + 2);
+        if (t0 < key_lo || t0 + 32 > key_end) {             // (the same for the whole wavefront)
+            u32x4 seen;                                     // two values a word
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                const int t = t0 + (w / 2) * 16 + g4 * 4 + (w % 2) * 2;
+                seen[w] = (t >= key_lo && t < key_end ? 0xFFFFu : 0u) | (t + 1 >= key_lo && t + 1 < key_end ? 0xFFFF0000u : 0u);
+            }
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) vf.vf[dt] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, vf.vf[dt]) & seen);
+        }
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) o[0][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf[0], vf.vf[dt], o[0][dt], 0, 0, 0);
     }

@@ -1189,3 +1189,50 @@ def test_gemm_qkv_rope_gives_the_same_bits_in_every_tile(ops, hd, K):
         ops.gemm_qkv_rope(x, w, cos, sin, positions, seq_idx, table, *made[-1], n_q, n_kv, hd, tile=tile)
         for want, got in zip(made[0], made[-1]):
             assert torch.equal(want, got), tile
+
+
+@pytest.mark.parametrize("n_q,n_kv,nsplit,page,window", [(4, 1, 1, 16, 0), (6, 2, 1, 32, 0), (4, 1, 2, 16, 0), (16, 1, 1, 16, 4100),
+                                                         (4, 1, 1, 16, 77), (6, 2, 3, 16, 131)])
+@pytest.mark.parametrize("rotates", [False, True], ids=["plain", "rotating"])
+def test_attention_decode_with_heads_of_128_reads_only_what_is_seen(ops, n_q, n_kv, nsplit, page, window, rotates):
+    """The decode kernel whose keys go through LDS: requests of one key to some thousand (a wavefront looks up the pages of 32 of
+    its blocks, 4,096 keys of a workgroup, at a time: lengths around that and around twice that), behind windows that begin
+    anywhere in a block. Places of a page that a row does not see (behind its last key, in front of its window) hold NaN and
+    infinities here, as an earlier request may have left them: the row is what the keys that it sees give."""
+    import types
+    hd, lens = 128, [1, 2, 16, 17, 31, 33, 127, 129, 3969, 4096, 4099, 4230, 8192, 8301]
+    S, scale, g = len(lens), 0.09, _gen(95)
+    nblk = (max(lens) + page - 1) // page
+    table = torch.randperm(S * nblk, generator=g).view(S, nblk).to(torch.int32)
+    k = torch.randn(S, nblk * page, n_kv, hd, generator=g).to(torch.bfloat16)
+    v = torch.randn(S, nblk * page, n_kv, hd, generator=g).to(torch.bfloat16)
+    q = torch.randn(S, n_q, hd, generator=g).to(torch.bfloat16)
+    qkv = torch.cat([q.float().view(S, -1), torch.stack([k[s, n - 1] for s, n in enumerate(lens)]).float().view(S, -1),
+                     torch.stack([v[s, n - 1] for s, n in enumerate(lens)]).float().view(S, -1)], dim=1).to(DEV)
+    rows = []
+    for s, n in enumerate(lens):
+        lo = max(0, n - window) if window else 0
+        rows.append(_plain_attention_last_row(q[s:s + 1].double() * (scale * math.sqrt(hd)), k[s, lo:n].double(), v[s, lo:n].double()).reshape(1, -1))
+        for bad, held in ((float("nan"), k), (float("inf"), v)):
+            held[s, :lo], held[s, n:] = bad, bad
+    k_cache, v_cache = torch.empty(S * nblk, n_kv, page, hd, dtype=torch.bfloat16), torch.empty(S * nblk, n_kv, hd, page, dtype=torch.bfloat16)
+    k_cache[table.view(-1).long()] = k.view(S * nblk, page, n_kv, hd).transpose(1, 2)
+    v_cache[table.view(-1).long()] = v.view(S * nblk, page, n_kv, hd).permute(0, 2, 3, 1)
+    k_cache, v_cache, table = k_cache.to(DEV), v_cache.to(DEV), table.to(DEV)
+    i32 = dict(dtype=torch.int32, device=DEV)
+    q_start, ctx = torch.arange(S + 1, **i32), torch.tensor([n - 1 for n in lens], **i32)
+    split_len = ((max(lens) + nsplit - 1) // nsplit + 31) // 32 * 32
+    plan = {"n_decode": S, "groups": 0, "split_len": split_len, "nsplit": nsplit, "prefill_splits": 1, "prefill_run": 1, "tuning": 0}
+    scratch = lambda *shape: torch.full(shape, float("nan"), device=DEV)
+    out = torch.zeros(S, n_q * hd, dtype=torch.bfloat16, device=DEV)
+    if rotates:                                             # (by no angle: cos 1, sin 0)
+        one, none = torch.ones(max(lens), hd // 2, device=DEV), torch.zeros(max(lens), hd // 2, device=DEV)
+        step = types.SimpleNamespace(num_seqs=S, new_lens=[1] * S, ctx_lens=[n - 1 for n in lens], plan_len=None, q_start=q_start,
+                                     ctx_len=ctx, extra={("attention_plan", n_q, n_kv, hd): plan},
+                                     buffer=lambda name, shape, dtype: scratch(*shape))
+        assert ops.mfma.attention_decode_rope(qkv, one, none, k_cache, v_cache, out, step, table, n_q, n_kv, hd, scale, window,
+                                              torch.zeros(S * n_kv, device=DEV))
+    else:
+        ops.mfma.attention_bf16(q.view(S, -1).to(DEV), k_cache, v_cache, out, q_start, ctx, table, n_q, n_kv, hd, scale, window, plan,
+                                scratch(S * n_q * nsplit * hd), scratch(S * n_q * nsplit * 2))
+    assert _rel(out.cpu().double(), torch.cat(rows)) < 8e-3
