@@ -278,15 +278,14 @@ __global__ __launch_bounds__(256) void attention_prefill_kernel(
     }
 }
 
-// Launches a decode kernel with the LDS that its blocks are staged through, if they are, having told the kernel of it once.
+// Launches a decode kernel with the LDS that its blocks are staged through, if they are.
 template <auto KERNEL, typename... ARGS>
 static int launch_staged(int hd, dim3 grid, hipStream_t stream, ARGS... args) {
-    static bool told = false;                           // per kernel
+    static OncePerDevice told;                          // per kernel
     const int lds = staged_decode(hd, true) ? decode_staged_bytes(hd) : 0;
-    if (!told && lds) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(KERNEL), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        if (e != hipSuccess) return static_cast<int>(e);
-        told = true;
+    if (lds > 0) {
+        const int status = allow_lds(told, reinterpret_cast<const void*>(KERNEL), lds);
+        if (status != 0) return status;
     }
     hipLaunchKernelGGL(KERNEL, grid, dim3(DEC_WAVES * 64), lds, stream, args...);
     return launch_status();

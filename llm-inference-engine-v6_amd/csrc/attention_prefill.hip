@@ -457,13 +457,9 @@ static int launch_shared(const bf16* q, const bf16* kc, const bf16* vc, bf16* ou
                          float* part_ml, const DecodeBeside& beside, hipStream_t stream) {
     constexpr int LDS = StageLayout<HD>::BYTES;
     auto kernel = attention_prefill_shared_kernel<HD, QT, HPW, KW, SPLIT>;
-    static bool attr_set = false;                      // per instantiation
-    if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
-        if (e != hipSuccess) return static_cast<int>(e);
-        attr_set = true;
-    }
+    static OncePerDevice told;                         // per instantiation
+    const int status = allow_lds(told, reinterpret_cast<const void*>(kernel), LDS);
+    if (status != 0) return status;
     static int resident = 0;                           // workgroups the chip holds at a time
     if (resident == 0) {
         int dev = 0, cus = 0, per_cu = 0;

@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "once_per_device.h"
+
 namespace llme {
 
 constexpr int kWave = 64;
@@ -101,6 +103,15 @@ inline int compute_units() {
         cus = 256;
     cached = cus;
     return cus;
+}
+
+// Tells a kernel how much LDS its launches ask for, before the first one on the current device. `told`: a static of the place that
+// launches it, one per kernel.
+inline int allow_lds(OncePerDevice& told, const void* kernel, int bytes) {
+    int device = -1;
+    const hipError_t e = hipGetDevice(&device);
+    if (e != hipSuccess) return static_cast<int>(e);
+    return told(device, bytes, [&] { return static_cast<int>(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes)); });
 }
 
 // Every entry point returns hipGetLastError() after its launches: 0 on success.

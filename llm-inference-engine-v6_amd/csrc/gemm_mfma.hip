@@ -1065,13 +1065,9 @@ __global__ __launch_bounds__(64 * WR * WC, 1) void gemm_tile_direct_kernel(
 template <auto KERNEL, int THREADS = 256>
 static int launch_tile_kernel(int LDS, int BM, int BN, const bf16* A, const bf16* W, void* out, int M, int N, int K,
                               int ksplit, hipStream_t stream, const QkvTarget& qt = QkvTarget{}) {
-    static bool attr_set = false;                      // per kernel
-    if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(KERNEL),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
-        if (e != hipSuccess) return static_cast<int>(e);
-        attr_set = true;
-    }
+    static OncePerDevice told;                         // per kernel
+    const int status = allow_lds(told, reinterpret_cast<const void*>(KERNEL), LDS);
+    if (status != 0) return status;
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
     hipLaunchKernelGGL(KERNEL, dim3(tiles_m * tiles_n * ksplit), dim3(THREADS), LDS, stream, A, W, out, M, N, K, tiles_m,
                        tiles_n, ksplit, qt, Groups{}, t_gate_extra);
@@ -1084,19 +1080,16 @@ static int launch_grouped_mode(const bf16* A, const bf16* W, void* out, int M, i
                                hipStream_t stream) {
     constexpr int LDS = tile_lds_bytes<WMT, WNT>(), BN = 32 * WNT;
     const int tiles_n = (N + BN - 1) / BN;
-    auto go = [&](auto kernel) -> int {
-        static bool attr_set = false;
-        if (!attr_set) {
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
-            if (e != hipSuccess) return static_cast<int>(e);
-            attr_set = true;
-        }
+    static OncePerDevice told[2];                      // (the two kernels have one type)
+    auto go = [&](auto kernel, int which) -> int {
+        const int status = allow_lds(told[which], reinterpret_cast<const void*>(kernel), LDS);
+        if (status != 0) return status;
         hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n), dim3(256), LDS, stream, A, W, out, M, N, K, tiles_m, tiles_n, 1,
                            QkvTarget{}, gr, t_gate_extra);
         return launch_status();
     };
-    if (K % TK != 0) return go(&gemm_tile_kernel<WMT, WNT, MODE, false, false, true>);
-    return go(&gemm_tile_kernel<WMT, WNT, MODE, true, false, true>);
+    if (K % TK != 0) return go(&gemm_tile_kernel<WMT, WNT, MODE, false, false, true>, 0);
+    return go(&gemm_tile_kernel<WMT, WNT, MODE, true, false, true>, 1);
 }
 template <int WMT, int WNT>
 static int launch_grouped(const bf16* A, const bf16* W, void* out, int M, int N, int K, int mode, int tiles_m, const Groups& gr,

@@ -387,13 +387,9 @@ static int launch_gemv_norm_held(const float* h, const int* rows, const void* no
     const size_t lds = static_cast<size_t>(16) * (K + 8) * 2 + static_cast<size_t>(NW) * (EPI == kGated ? 2 : 1) * 64 * 16 + 64;
     if (lds > 160 * 1024) return kErrUnsupported;
     auto kernel = gemv_norm_kernel<NW, TPR, EPI, TNW, PU>;
-    static size_t granted = 0;                          // per instantiation
-    if (lds > granted) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-        if (e != hipSuccess) return static_cast<int>(e);
-        granted = lds;
-    }
+    static OncePerDevice told;                          // per instantiation
+    const int status = allow_lds(told, reinterpret_cast<const void*>(kernel), static_cast<int>(lds));
+    if (status != 0) return status;
     const int tiles = (N + 15) / 16;
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(NW * 64), lds, stream, h, rows, static_cast<const TNW*>(norm_w), eps,
                        w, out, M, N, K, tiles, blocked, rope);

@@ -339,13 +339,9 @@ template <int DC, int RC>
 static int launch_latent(const LatentArgs& a, int max_new, int n_seq, hipStream_t stream) {
     const int D = a.R + a.r;
     const int lds = (32 * lat_k_stride(D) + a.R * kVtStride) * 2;
-    static int attr_lds = 0;
-    if (lds > attr_lds) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&latent_attention_mfma_kernel<DC, RC>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        if (e != hipSuccess) return static_cast<int>(e);
-        attr_lds = lds;
-    }
+    static OncePerDevice told;
+    const int status = allow_lds(told, reinterpret_cast<const void*>(&latent_attention_mfma_kernel<DC, RC>), lds);
+    if (status != 0) return status;
     const dim3 grid((static_cast<long>(max_new) * a.n + 63) / 64, n_seq, a.nsplit);
     hipLaunchKernelGGL((latent_attention_mfma_kernel<DC, RC>), grid, dim3(256), lds, stream, a);
     return launch_status();

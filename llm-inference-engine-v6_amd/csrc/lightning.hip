@@ -772,13 +772,9 @@ extern "C" int llme_lightning_chunked(const float* p, int ld, int q_col, int k_c
     const dim3 read_grid(n_seq * n_chunks * 2, heads);
 #define LLME_READ_DS(NW, NCT, DS)                                                                                                       \
     do {                                                                                                                                \
-        static bool attr_set = false;                                                                                                   \
-        if (!attr_set) {                                                                                                                \
-            const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(&lightning_chunk_read_kernel<NW, NCT, DS>),        \
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024);                         \
-            if (err != hipSuccess) return static_cast<int>(err);                                                                        \
-            attr_set = true;                                                                                                            \
-        }                                                                                                                               \
+        static OncePerDevice told;                                                                                                      \
+        const int status = allow_lds(told, reinterpret_cast<const void*>(&lightning_chunk_read_kernel<NW, NCT, DS>), 150 * 1024);       \
+        if (status != 0) return status;                                                                                                 \
         hipLaunchKernelGGL((lightning_chunk_read_kernel<NW, NCT, DS>), read_grid, dim3(NW * 64), lds, stream, in, q_start, n_chunks, ck, o); \
     } while (0)
 #define LLME_READ(NW, NCT)                             \

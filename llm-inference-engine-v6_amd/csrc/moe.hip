@@ -424,13 +424,9 @@ extern "C" int llme_moe_decide(const void* x, const void* w, int T, int K, int r
 #define LLME_DECIDE(TILES)                                                                                                              \
     do {                                                                                                                                \
         constexpr int LDS = 16 * TILES * 64 * 16;                                                                                       \
-        static bool attr_set = false;                                                                                                   \
-        if (!attr_set) {                                                                                                                \
-            const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(&moe_decide_kernel<TILES>),                        \
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, LDS);                                \
-            if (err != hipSuccess) return static_cast<int>(err);                                                                        \
-            attr_set = true;                                                                                                            \
-        }                                                                                                                               \
+        static OncePerDevice told;                                                                                                      \
+        const int status = allow_lds(told, reinterpret_cast<const void*>(&moe_decide_kernel<TILES>), LDS);                              \
+        if (status != 0) return status;                                                                                                 \
         hipLaunchKernelGGL((moe_decide_kernel<TILES>), dim3(1), dim3(1024), LDS, stream, static_cast<const bf16*>(x),                   \
                            static_cast<const bf16*>(w), T, K, rows, E, top, scale, renorm, sigmoid, logits, ld, wts, tile, cap, place_pair, \
                            pair_place, tile_expert, n_tiles);                                                                           \

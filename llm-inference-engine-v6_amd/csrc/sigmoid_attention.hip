@@ -433,12 +433,10 @@ static int launch_sigmoid_attention_mfma(const void* q, const void* k_cache, con
                                          int run_len, int runs, int tiles, hipStream_t stream) {
     const size_t lds = sizeof(float) * (static_cast<size_t>(H) * 512 + static_cast<size_t>(H) * H + H);
     auto kernel = sigmoid_attention_mfma_kernel<DIM32, VT>;
-    static size_t allowed = 0;
-    if (lds > 64 * 1024 && lds > allowed) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                 static_cast<int>(lds));
-        if (e != hipSuccess) return static_cast<int>(e);
-        allowed = lds;
+    static OncePerDevice told;
+    if (lds > 64 * 1024) {
+        const int status = allow_lds(told, reinterpret_cast<const void*>(kernel), static_cast<int>(lds));
+        if (status != 0) return status;
     }
     kernel<<<dim3(tiles, runs), (H / 4) * 64, lds, stream>>>(
         static_cast<const bf16*>(q), static_cast<const bf16*>(k_cache), static_cast<const bf16*>(v_cache), mix_t, bias, positions,
