@@ -9,6 +9,7 @@ new model code.
 """
 from __future__ import annotations
 
+import math
 from dataclasses import dataclass
 
 import torch
@@ -74,6 +75,13 @@ class DecoderModel(Part):
             out[n["pass_input"]] = self.pass_input
         out.update(self.shared)
         return out
+
+    def load_params(self, get, placement):
+        size = torch.empty((), dtype=placement.compute_dtype).element_size()
+        for layer in self.layers:
+            mixer = getattr(layer, "mixer", None)
+            if mixer is not None:
+                mixer.layer_bytes = size * sum(math.prod(spec.shape) for spec in layer.named_specs().values() if None not in spec.shape)
 
     def aliases(self):
         # A tied head is the embedding table under a second name (src/weights.cpp:244-267): a

@@ -35,6 +35,16 @@ class KernelChoices:
     # 2.151 / 2.053 / 2.057, 112: 2.432 / 2.403 / 2.340, 128: 2.564 / 2.556 / 2.498; 8B sizes 65: 2.313 / 2.223 / 2.218,
     # 96: 2.568 / 2.466 / 2.467, 112: 2.879 / 2.864 / 2.806, 128: 3.014 / 3.030 / 2.984.
     qkv_sum_rows_decoding_128: int = 128
+    # Steps of 17 to 64 rows that hold prompt rows, heads of up to 64: the most bytes that a layer reads with which the host's
+    # launches set the time, so that a launch less (rotation and cache write in the q/k/v product's epilogue) wins. Measured
+    # over 8 layers with heads of 64 on a host that takes 75 to 83 us for a layer's launches, ms a step with the cut sum and the rotation
+    # kernel / with the rotating product, 17, 45 and 64 rows: widths 512 to 2,048 (1B sizes: 122 MB) 0.66 / 0.60 at all three; 2,560
+    # with 157 MB 0.67 / 0.60, 0.70 / 0.63, 0.70 / 0.63; with 189 MB 0.70 / 0.63, 0.70 / 0.67, 0.70 / 0.72; 3,072 with 195 MB
+    # 0.71 / 0.64, 0.70 / 0.65, 0.70 / 0.68; with 270 MB 0.68 / 0.68, 0.71 / 0.76, 0.78 / 0.82; 4,096 with 428 MB 0.79 / 0.88,
+    # 0.89 / 0.97, 0.98 / 1.03. (Layers with heads of 128 have always kept the sum.) A step that also decodes takes the host some
+    # 20 us a layer longer, so keys and values count a third: 32 prompt rows beside 16 requests at the 1B sizes, 4 MB of keys and
+    # values 0.83 / 0.74, 98 MB 0.85 / 0.77, 197 MB 0.85 / 0.79, where the chip begins to set the time.
+    launch_bound_layer_bytes: int = 170_000_000
     # prompt attention: work items of half the rows where a step has few items
     prefill_half_rows: bool = True
     # Workgroups (of four wavefronts) the decode kernel should have at most when it cuts the keys: one

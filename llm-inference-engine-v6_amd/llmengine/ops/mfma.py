@@ -565,21 +565,24 @@ GEMV_NORM_MAX_ROWS = 16
 QKV_SUM_MAX_ROWS = 64
 
 
-def qkv_sum_max_rows(decoded_only: bool, head_dim: int, choices: KernelChoices | None = None) -> int:
+def qkv_sum_max_rows(decoded_only: bool, head_dim: int, choices: KernelChoices | None = None,
+                     rotating_layer_bytes: int | None = None) -> int:
     """The most rows of a step whose q/k/v product is cut over k and added into a cleared buffer. A step of
     single decoded tokens keeps that way further: with heads of 64 (choices.qkv_sum_rows_decoding) the
     attention kernel then rotates and writes the cache itself (attention_decode_rope); with heads of 128
     (choices.qkv_sum_rows_decoding_128) the rotation kernel does, and the product's tiles of 96 or 128 rows
-    with the rotation in their epilogue are the slower way until then. A step that holds prompt rows is launched
-    kernel by kernel, which takes the host longer than a layer of heads of 64 takes the chip (82 against 64 us at the
-    1B sizes, 45 rows): its product rotates and writes the cache in its epilogue, a launch a layer fewer
-    (45 rows 1.339 / 1.179 ms; layers with heads of 128 are the chip's time, and keep the sum)."""
+    with the rotation in their epilogue are the slower way until then.
+    rotating_layer_bytes: of a step that holds prompt rows and whose product can rotate and write the cache in
+    its epilogue, the bytes that the layer reads (None: any other step). Such steps are launched kernel by kernel,
+    and with heads of up to 64 and up to choices.launch_bound_layer_bytes the chip is through with a layer before
+    the host has launched the next: a launch less is then worth more than the few microseconds that the rotating
+    product takes longer on the chip."""
     ch = choices or DEFAULT
     if decoded_only and head_dim == 64 and ch.decode_rope:
         return max(QKV_SUM_MAX_ROWS, ch.qkv_sum_rows_decoding)
     if decoded_only and head_dim == 128:
         return max(QKV_SUM_MAX_ROWS, ch.qkv_sum_rows_decoding_128)
-    if not decoded_only and head_dim <= 64:
+    if rotating_layer_bytes is not None and head_dim <= 64 and rotating_layer_bytes <= ch.launch_bound_layer_bytes:
         return GEMV_NORM_MAX_ROWS
     return QKV_SUM_MAX_ROWS
 

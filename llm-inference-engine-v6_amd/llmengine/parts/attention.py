@@ -104,6 +104,16 @@ class Attention(Mixer):
         return (rms is not None and step.act_dtype == torch.bfloat16
                 and ops.gemv_norm_supported(h, rms[0], self.w_qkv, h.shape[0], gated=False, choices=step.choices))
 
+    def _bytes_read(self, step) -> int | None:
+        """What a step of few rows reads in this layer: its weights, and the requests' keys and values, which count a third
+        (see KernelChoices.launch_bound_layer_bytes)."""
+        if self.layer_bytes is None:
+            return None
+        tokens = step.extra.get("attn.tokens held")
+        if tokens is None:
+            tokens = step.extra["attn.tokens held"] = sum(step.ctx_lens) + step.num_tokens
+        return self.layer_bytes + tokens * 2 * self.kv_dim * 2 // 3
+
     def forward(self, x, step, cache, out, accumulate, write_cache=True, pre_norm=None):
         """pre_norm: the norm in front of this mixer when `fuses_norm` said yes; x is then the
         un-normed 32-bit stream and the projection applies pre_norm.fused_rms() itself."""
@@ -120,7 +130,10 @@ class Attention(Mixer):
         act = step.act_dtype
         q = step.buffer("attn.q", (T, self.q_dim), act)
         rms = pre_norm.fused_rms() if pre_norm is not None else None
-        sum_rows = ops.mfma.qkv_sum_max_rows(T == step.num_seqs and rot == hd and not applies, hd, step.choices)
+        rotates = (write_cache and rms is None and cos is not None
+                   and ops.gemm_qkv_rope_supported(x, self.w_qkv, k_cache, hd, rot, step.choices))
+        sum_rows = ops.mfma.qkv_sum_max_rows(T == step.num_seqs and rot == hd and not applies, hd, step.choices,
+                                             self._bytes_read(step) if rotates and T > step.num_seqs else None)
 
         def project(weight, dst):
             if rms is not None:
@@ -132,8 +145,7 @@ class Attention(Mixer):
             # decoding: norm, projection, rotation and the cache write are one kernel
             ops.gemv_norm_rope(x, rms[0], rms[1], self.w_qkv_paired, step.positions, step.seq_idx,
                                block_table, cos, sin, q, k_cache, v_cache, n_q, n_kv, hd)
-        elif (write_cache and rms is None and T > sum_rows and cos is not None
-              and ops.gemm_qkv_rope_supported(x, self.w_qkv, k_cache, hd, rot, step.choices)):
+        elif rotates and T > sum_rows:
             # many rows (prompts): rotation and the cache write are the projection's epilogue
             ops.gemm_qkv_rope(x, self.w_qkv, cos, sin, step.positions, step.seq_idx, block_table, q, k_cache, v_cache,
                               n_q, n_kv, hd)

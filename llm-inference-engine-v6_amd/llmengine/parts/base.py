@@ -246,6 +246,10 @@ class PositionEncoding(Part):
 
 
 class Mixer(Part):
+    # the bytes of the weights of the layer that the mixer stands in, as the model computes with them (set when a model is
+    # loaded; None: not known): how long a step of few rows keeps the chip busy with a layer
+    layer_bytes: int | None = None
+
     def cache_spec(self) -> CacheSpec | None:
         return None
 
