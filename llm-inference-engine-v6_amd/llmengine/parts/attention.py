@@ -153,15 +153,15 @@ class Attention(Mixer):
             adds = (rms is None and ops.mfma.GEMV_NORM_MAX_ROWS < T <= sum_rows
                     and x.dtype == torch.bfloat16 and self.w_qkv.dtype == torch.bfloat16
                     and (T * (self.q_dim + 2 * self.kv_dim)) % 4 == 0)
-            # (the product that adds has a buffer that nothing else writes: what it is left holding is known)
-            width, done = self.q_dim + 2 * self.kv_dim, None
-            inside = adds and not applies and rot == hd and T == step.num_seqs
-            if inside:
-                # (behind the rows: what the attention kernel counts its splits with, zero whenever the rows are)
-                held = step.buffer("attn.qkv_sum", (T * width + (T * n_kv + 3) // 4 * 4,), torch.float32)
+            # (the product that adds has a buffer that nothing else writes: what it is left holding is known; behind the
+            # rows: what the attention kernel counts its splits with, zero whenever the rows are. Every layer of a step
+            # asks for the same, whether its attention kernel counts or not, so that what one leaves zero is zero for the next)
+            width, counters = self.q_dim + 2 * self.kv_dim, (T * n_kv + 3) // 4 * 4
+            if adds:
+                held = step.buffer("attn.qkv_sum", (T * width + counters,), torch.float32)
                 qkv, done = held[:T * width].view(T, width), held[T * width:]
             else:
-                held = qkv = step.buffer("attn.qkv_sum" if adds else "attn.qkv", (T, width), torch.float32)
+                qkv = step.buffer("attn.qkv", (T, width), torch.float32)
             if adds:
                 # a few dozen rows (decoding at larger batches): q/k/v has too few output tiles for the
                 # chip, so the product is cut over k and adds its parts into a cleared buffer
@@ -178,7 +178,7 @@ class Attention(Mixer):
             if applies:
                 self.position.apply(qkv[:, :self.q_dim].view(T, n_q, hd),
                                     qkv[:, self.q_dim:self.q_dim + self.kv_dim].view(T, n_kv, hd), step.positions)
-            if inside:
+            if adds and not applies and rot == hd and T == step.num_seqs:
                 # decoded tokens only: the attention kernel rotates, writes the cache and clears the rows itself
                 o = step.buffer("attn.o", (T, self.q_dim), act)
                 if ops.mfma.attention_decode_rope(qkv, cos, sin, k_cache, v_cache, o, step, block_table, n_q, n_kv, hd,

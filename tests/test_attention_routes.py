@@ -47,8 +47,8 @@ def _step(new_lens, ctx_lens, choices=None):
                                  buffer=buffer, extra={}, choices=choices, fixed_order=False)
 
 
-def _run(monkeypatch, attn, step):
-    calls = []
+def _run(monkeypatch, attn, step, calls=None):
+    calls = [] if calls is None else calls
     for name in ("gemm", "gemm_qkv_rope", "rope_kv_write", "clear", "attention_project"):
         monkeypatch.setattr(ops, name, lambda *a, _name=name, **k: calls.append(_name + (" add" if k.get("accumulate") else "")))
     monkeypatch.setattr(ops.mfma, "attention_decode_rope", lambda *a, **k: calls.append("attention_decode_rope") or True)
@@ -98,6 +98,16 @@ def test_choices_decide(monkeypatch):
 def test_more_rows_and_decoding_as_before(monkeypatch):
     assert _route(monkeypatch, _attention(64, Tables(64), 428), _step([65], [0])) == "epilogue"
     assert "attention_decode_rope" in _run(monkeypatch, _attention(64, Tables(64)), _step([1] * 20, [100] * 20))
+
+
+@pytest.mark.parametrize("lens", [([1] * 20, [100] * 20), ([1] * 33, [7] * 33)])
+def test_layers_with_and_without_rotation_share_the_cleared_sum(monkeypatch, lens):
+    """What one layer's kernels leave zero is zero for the next, whichever of them it is: a step clears once."""
+    step, calls = _step(*lens), []
+    for position in (Tables(64), None, Tables(64), Tables(32), Tables(64)):
+        _run(monkeypatch, _attention(64, position), step, calls)
+    assert calls.count("gemm add") == 5 and calls.count("attention_decode_rope") == 3 and calls.count("rope_kv_write") == 2
+    assert calls.count("clear") == 1 and calls[0] == "clear"
 
 
 def test_a_model_tells_its_mixers_what_a_layer_weighs():
