@@ -26,7 +26,8 @@ constexpr int kMaxHead = 256;
 
 // VEC: head and page sizes are multiples of 4: a lane reads its key's row four dims at a time, and its value dim's four keys at
 // a time (the values lie by dim, so four keys are 16 bytes). One by one, a decoded token's 80 keys took 22.4 us, so
-// 12.5; the rows of a 77-token prompt 42 and 21.
+// 12.5; the rows of a 77-token prompt 42 and 21. The sums are those of the other variant, in its order: the bits depend on the
+// page size in neither.
 template <typename TQ, typename TC, int NW, bool VEC>
 __global__ __launch_bounds__(NW * 64) void attention_generic_kernel(
     const TQ* __restrict__ q, const TC* __restrict__ k_cache, const TC* __restrict__ v_cache,
@@ -53,14 +54,11 @@ __global__ __launch_bounds__(NW * 64) void attention_generic_kernel(
     float m = -INFINITY, l = 0.f;
     float acc[PER_LANE] = {0.f, 0.f, 0.f, 0.f};
 
-    // this wavefront's chunks of 64 keys (no barrier inside: the wavefronts take different numbers of turns); VEC: chunks
-    // begin at multiples of 4, so the first may hold up to three keys in front of the first that is seen
-    const int first = VEC ? lo & ~3 : lo;
-    for (int t0 = first + wave * kWave; t0 < hi; t0 += NW * kWave) {
+    // this wavefront's chunks of 64 keys (no barrier inside: the wavefronts take different numbers of turns)
+    for (int t0 = lo + wave * kWave; t0 < hi; t0 += NW * kWave) {
         const int key = t0 + lane;
-        const bool seen = key >= lo && key < hi;
         float sc = -INFINITY;
-        if (seen) {
+        if (key < hi) {
             const int pg = table[key / page];
             const TC* kr = k_cache + ((static_cast<size_t>(pg) * n_kv + kvh) * page + key % page) * hd;
             float dot = 0.f;
@@ -77,25 +75,29 @@ __global__ __launch_bounds__(NW * 64) void attention_generic_kernel(
             }
             sc = dot * scale;
         }
-        const float m_new = fmaxf(m, wave_max(sc));       // finite: the chunk holds a key that is seen
+        const float m_new = fmaxf(m, wave_max(sc));       // finite: the chunk holds at least key t0
         const float alpha = expf(m - m_new);              // 0 on the first chunk (m = -inf)
-        const float p = seen ? expf(sc - m_new) : 0.f;
+        const float p = (key < hi) ? expf(sc - m_new) : 0.f;
         l = l * alpha + wave_sum(p);
         m = m_new;
 #pragma unroll
         for (int i = 0; i < PER_LANE; ++i) acc[i] *= alpha;
         const int n = (hi - t0 < kWave) ? hi - t0 : kWave;
         if (VEC) {
-            // (four keys of a dim; keys of the four that are not seen have weight 0 and count as 0 whatever their place holds)
+            // (four keys of a dim, groups that begin at a multiple of 4, so behind a window's edge up to three keys in front of
+            // the chunk's first; keys of a group that are not the chunk's have weight 0 and count as 0 whatever their place holds)
 #pragma unroll 4
-            for (int j = 0; j < n; j += 4) {
+            for (int j = -(t0 & 3); j < n; j += 4) {
                 const int kj = t0 + j;
                 const TC* vb = v_cache + (static_cast<size_t>(table[kj / page]) * n_kv + kvh) * hd * page + kj % page;
-                const bool whole = kj >= lo && kj + 4 <= hi;
                 float pj[4];
+                bool in[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    pj[e] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, p), j + e));
+                for (int e = 0; e < 4; ++e) {
+                    in[e] = j + e >= 0 && j + e < n;
+                    const float pe = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, p), (j + e) & 63));
+                    pj[e] = in[e] ? pe : 0.f;
+                }
 #pragma unroll
                 for (int i = 0; i < PER_LANE; ++i) {
                     const int d = lane + i * kWave;
@@ -104,7 +106,7 @@ __global__ __launch_bounds__(NW * 64) void attention_generic_kernel(
                     load4<TC>(vb + static_cast<size_t>(d) * page, vv);
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        acc[i] = fmaf(pj[e], whole || (kj + e >= lo && kj + e < hi) ? vv[e] : 0.f, acc[i]);
+                        acc[i] = fmaf(pj[e], in[e] ? vv[e] : 0.f, acc[i]);
                 }
             }
         } else {

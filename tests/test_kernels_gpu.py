@@ -1236,3 +1236,16 @@ def test_attention_decode_with_heads_of_128_reads_only_what_is_seen(ops, n_q, n_
         ops.mfma.attention_bf16(q.view(S, -1).to(DEV), k_cache, v_cache, out, q_start, ctx, table, n_q, n_kv, hd, scale, window, plan,
                                 scratch(S * n_q * nsplit * hd), scratch(S * n_q * nsplit * 2))
     assert _rel(out.cpu().double(), torch.cat(rows)) < 8e-3
+
+
+@pytest.mark.parametrize("window", [1, 5, 70, 131])
+def test_attention_generic_gives_the_same_bits_for_every_page_size(ops, window):
+    """The 32-bit sums walk the keys in an order that the paging does not touch, under a window too and also for pages that do not
+    hold whole groups of four keys."""
+    lens, n_q, n_kv, hd = [1, 3, 63, 66, 133, 270], 2, 1, 20
+    outs = []
+    for page in (16, 4, 64, 6, 5, 7):
+        s = _paged_setup(ops, lens, n_q, n_kv, hd, page, torch.float32, seed=6, rotate=False)
+        outs.append(torch.empty_like(s["q"]))
+        ops.attention_generic(s["q"], s["k_cache"], s["v_cache"], outs[-1], s["positions"], s["seq_idx"], s["table"], n_q, n_kv, hd, 0.3, window)
+        assert torch.equal(outs[0], outs[-1]), page
