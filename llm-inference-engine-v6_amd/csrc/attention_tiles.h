@@ -367,14 +367,14 @@ template <int N> __device__ __forceinline__ void wait_loads() {
 }
 __device__ __forceinline__ void wait_lds_reads() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
-template <int HD> constexpr int staged_wave_bytes() { return 2 * 2 * 32 * HD * 2; }        // two blocks of K and of V
+__host__ __device__ constexpr int staged_wave_bytes(int hd) { return 2 * 2 * 32 * hd * 2; }        // two blocks of K and of V
 
 template <int HD>
 __device__ __forceinline__ void attend_range_staged(const PagedKV& kv, int first, int stride, int key_lo, int key_end,
                                                     const bf16x8 (&qf)[1][(HD + 31) / 32], const int (&row_pos)[1],
                                                     const int (&row_lo)[1], float scale_log2, float (&m)[1], float (&l)[1],
                                                     f32x4 (&o)[1][HD / 16], unsigned char* lds) {
-    static_assert(HD == 64 || HD == 128, "rows of 8 or 16 pieces");
+    static_assert(HD == 128, "rows of 16 pieces");
     constexpr int DC = HD / 32, DT = HD / 16, HALF = 16 * HD * 2, PER = HALF / 1024, L = 2 * PER;   // L: loads of a block's K, or V
     const int lane = threadIdx.x & 63, r = lane & 15, g4 = lane >> 4;
     if (first >= key_end) return;
@@ -390,12 +390,12 @@ __device__ __forceinline__ void attend_range_staged(const PagedKV& kv, int first
     int ids = look_up(0);
     const unsigned lds_k = static_cast<unsigned>(reinterpret_cast<size_t>((__attribute__((address_space(3))) unsigned char*)lds));
     const unsigned lds_v = lds_k + 2 * 2 * HALF;
-    // a lane's piece in K: row lane / (HD / 8) of the 1 KB, the piece that belongs into its slot (rows go on by 8 or 4 a piece)
+    // a lane's piece in K: row lane / 16 of the 1 KB, the piece that belongs into its slot (1 KB further on are 4 rows)
     unsigned koff[2];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-        const int row = lane / (HD / 8) + (HD == 128 ? 4 * u : 0), slot = lane % (HD / 8);
-        koff[u] = static_cast<unsigned>(lane / (HD / 8)) * (HD * 2) + static_cast<unsigned>(slot ^ (row & 7)) * 16;
+        const int row = lane / 16 + 4 * u, slot = lane % 16;
+        koff[u] = static_cast<unsigned>(lane / 16) * (HD * 2) + static_cast<unsigned>(slot ^ (row & 7)) * 16;
     }
     const unsigned voff = static_cast<unsigned>(lane >> 1) * (kv.page * 2) + (lane & 1) * 16;
     struct Half {
@@ -530,8 +530,8 @@ template <bool SHARED> __device__ __forceinline__ void put_part(float* p, float 
 __device__ __forceinline__ float get_part(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
 // (k_cache and v_cache carry no promise that nothing else points at them: RAW writes into them)
-// STAGED: the keys go through LDS (attend_range_staged; head size 64 or 128); `sh` then has decode_staged_bytes(HD) bytes.
-__host__ __device__ constexpr int decode_staged_bytes(int hd) { return DEC_WAVES * 2 * 2 * 32 * hd * 2; }
+// STAGED: the keys go through LDS (attend_range_staged; head size 128); `sh` then has decode_staged_bytes(HD) bytes.
+__host__ __device__ constexpr int decode_staged_bytes(int hd) { return DEC_WAVES * staged_wave_bytes(hd); }
 template <int HD, bool STREAM, bool RAW = false, bool STAGED = false>
 __device__ __forceinline__ void decode_item(
     const bf16* __restrict__ q, const bf16* k_cache, const bf16* v_cache,
@@ -656,9 +656,9 @@ __device__ __forceinline__ void decode_item(
 
     const int first = k_begin + __builtin_amdgcn_readfirstlane(wave) * 32;
     if constexpr (STAGED) {
-        static_assert(!STAGED || DEC_WAVES * staged_wave_bytes<HD>() >= decode_lds_floats(HD) * 4, "the join fits into the buffers");
+        static_assert(decode_staged_bytes(HD) >= decode_lds_floats(HD) * 4, "the join fits into the buffers");
         attend_range_staged<HD>(kv, first, DEC_WAVES * 32, lo_all, k_end, qf, row_pos, row_lo, scale * kLog2e, m, l, o,
-                                reinterpret_cast<unsigned char*>(sh) + __builtin_amdgcn_readfirstlane(wave) * staged_wave_bytes<HD>());
+                                reinterpret_cast<unsigned char*>(sh) + __builtin_amdgcn_readfirstlane(wave) * staged_wave_bytes(HD));
         __syncthreads();                                // (the join reuses the buffers)
     } else {
         attend_range<HD, 1, STREAM>(kv, first, DEC_WAVES * 32, lo_all, k_end, qf, row_pos, row_lo, tile_free, scale * kLog2e, m, l, o);
