@@ -18,6 +18,7 @@
 // request alone (the scheduler puts long and short together): it finishes on a chip that is draining,
 // faster per key than a place that shares the chip to the end (lone_ns; measured 8.3 against 9.5), and
 // cutting such a step lost 6 to 14 % where the estimate without this promised 10 to 19 %.
+// The caller gives another cost per split for heads of 128, whose decode kernel is another one (KernelChoices).
 #include <algorithm>
 #include <cstdint>
 #include <vector>

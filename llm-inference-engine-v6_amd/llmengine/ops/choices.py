@@ -71,6 +71,13 @@ class KernelChoices:
     decode_cut_rope_us: float = 4.8     # and the rotation kernel, where the single split would have rotated itself
     decode_cut_inside_us: float = 2.0   # what both cost at most where the decode kernel rotates: it then joins its splits itself
     decode_cut_each_us: float = 1.0     # and this per split
+    # The same for heads of 128, whose keys go through LDS: that kernel has one workgroup a compute unit, so that the pieces of a unit
+    # start one after the other. Measured at the 3B sizes over 17 to 80 requests at 400 to 6,000 tokens, of one length and of many,
+    # each with 1 to 8 splits (50 steps): with 1.0 the estimate's choice took 1.9 % longer than the best number of splits on average
+    # and 10 % at worst (ms a step: 20 requests of 2,000 tokens 0.95 in four, whole 0.92; 20 around 4,000 1.31 in eight, in two 1.19; 40 of
+    # 900 1.07 in five, whole 1.03), with this 0.8 % and 6 %, and in no step more than 0.3 % longer than before. (At the 1B sizes,
+    # heads of 64: 0.4 % and 5 % as it is.)
+    decode_cut_each_us_128: float = 3.5
     decode_cut_gain: float = 0.05       # and must promise this fraction of the whole keys' time
     # Portions of prompts: work items (a span of rows x a group of heads) the prefill kernel should
     # have at least (None: two per compute unit, three where the step has more than half a compute unit's

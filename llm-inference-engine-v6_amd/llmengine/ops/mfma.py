@@ -369,10 +369,11 @@ def decode_cut(lens, n_q: int, n_kv: int, head_dim: int, plan_len: int | None = 
         apart_us = (ch.decode_cut_join_us if S > GEMV_NORM_MAX_ROWS else 0.0) + (ch.decode_cut_rope_us if rotates else 0.0)
         if rotates:                                        # (the kernel that rotates joins its splits itself)
             apart_us = min(apart_us, ch.decode_cut_inside_us)
+    each_us = ch.decode_cut_each_us_128 if head_dim == 128 else ch.decode_cut_each_us
     from ..runtime import native
     n = native.library().llme_decode_cut((ctypes.c_int * S)(*lens), S, tiles, units, head_dim, longest, first, most,
                                          ch.decode_cut_tbs, ch.decode_cut_key_ns, ch.decode_cut_lone_ns,
-                                         ch.decode_cut_piece_us, apart_us, ch.decode_cut_each_us, ch.decode_cut_gain)
+                                         ch.decode_cut_piece_us, apart_us, each_us, ch.decode_cut_gain)
     if n < 1:
         raise kernels.KernelError(f"decode_cut: the host runtime refused its arguments (code {n})")
     return n
