@@ -180,8 +180,8 @@ static int launch_gemv_generic(const void* a, const void* w, void* out, int M, i
 }
 
 // 32-bit operands, more than 16 rows: v_mfma_f32_16x16x4_f32, whose products and sums are 32-bit like the vector unit's, at
-// twice its rate (64 multiply-adds a cycle and scheduler: 157 TFLOP/s). At that rate the operands need no LDS: a lane loads
-// 8 consecutive k of a row (two loads of 16 bytes; the four lanes of a row take 128 bytes together), and step s of eight
+// twice the rate of its single multiply-adds (32 against 16 a cycle and scheduler: 157 TFLOP/s). At that rate the operands
+// need no LDS: a lane loads 8 consecutive k of a row (two loads of 16 bytes; the four lanes of a row take 128 bytes together), and step s of eight
 // multiplies element s of every lane, which is k = 8 q + s for lane group q in both operands. A wavefront makes
 // 16 WMT x 16 WNT of the output; KW wavefronts share an output and take every KW-th 32 of k, their sums meeting in LDS in one
 // order (the same bits in every run). D blocks of 32 k are in flight per wavefront.

@@ -685,10 +685,10 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(const bf16* __restric
 // half turn for the first half of slab (h - 1) / 2 + 3 (into the buffer of the slab that ends here), the even
 // one behind it for the second. A half turn of 32 products a wavefront is 1,024 cycles of the matrix pipe: with all
 // of a half turn's loads asked for in one go, A's only in every second, it took 1,480 to 1,570 cycles; dealt out over
-// the rows and over both half turns it takes 1,300 to 1,360 (without loads 1,140; 8,191 x 28,672 x 4,096 went from 1,265 to
-// 1,311 TFLOP/s by this). The chip lowers its clock under this load (1.9 of 2.4 GHz), so fewer stalls win less than
-// their cycles. (Four wavefronts of 128 x 128 read a third less of LDS: 1,360 to 1,390 cycles at 2.05 GHz, and the
-// epilogue with half the wavefronts took more than that won.)
+// the rows and over both half turns it takes 1,300 to 1,360 (without loads 1,140; gate/up of 8,191 x 28,672 x 4,096 went
+// from 1,646 to 1,508 us, 1,276 TFLOP/s, by this and the epilogue below). The chip lowers its clock under this load (1.9 of
+// 2.4 GHz), so fewer stalls win less than their cycles. (Four wavefronts of 128 x 128 read a third less of LDS: 1,360 to 1,390
+// cycles at 2.05 GHz, and the epilogue with half the wavefronts took more than that won.)
 // Needs: W blocked (N a multiple of 16, K of 32). A slab that hangs over the end of k reads zeros
 // there (the loads of A's second half get an offset behind the descriptor's end).
 constexpr int DK = 64;
@@ -715,7 +715,8 @@ __device__ __forceinline__ void load_b128_to_lds(u32x4 rsrc, unsigned lds_base, 
 // (a gate and its up, a rotated entry and its partner are columns of one lane), so that the whole tile fits into LDS at once and
 // goes out in pieces of 16 bytes behind one barrier; 32-bit sums go through LDS in two passes, and what they are added to is asked
 // for before a pass is staged. (Measured on a tile of 256 x 256, from the last product to the last store issued: gated 8.6 us
-// when it went through LDS in 32 bits, adding 21 us when a thread asked for its addends piece by piece.)
+// when it went through LDS in 32 bits, adding 21 us when a thread asked for its addends piece by piece. What is left of a gated one
+// is its expf and division: half the instructions for them, in a form that was less exact, took 2 to 6 % off gate/up.)
 template <int WR, int WC, int WMT, int WNT, int MODE>
 __device__ __forceinline__ void direct_epilogue(f32x4 (&acc)[WMT][WNT], unsigned char* lds_raw, void* __restrict__ out, int M, int N,
                                                 int m0, int n0, int wm, int wn, int tid, int r, int q, const QkvTarget& qt,
@@ -1159,8 +1160,7 @@ static int launch_tile_direct(const bf16* A, const bf16* W, void* out, int M, in
 #undef LLME_DIRECT
 }
 
-// ----------------------------------------------------------------------------------------
-// skinny kernel: MT row tiles of 16 (M <= 16 MT), NW wavefronts per workgroup splitting k
+// The q/k/v product with rotation and cache write in its epilogue (kRopeCache): 256 x 256 tiles, then those through LDS.
 static int launch_direct_rope(const bf16* A, const bf16* W, int M, int N, int K, const QkvTarget& qt, hipStream_t stream) {
     return launch_tile_kernel<gemm_tile_direct_kernel<4, 2, 4, 8, kRopeCache>, 512>(160 * 1024, 256, 256, A, W, nullptr, M, N, K, 1,
                                                                                     stream, qt);
@@ -1178,6 +1178,8 @@ static int launch_tile_rope(const bf16* A, const bf16* W, int M, int N, int K, i
 #undef LLME_ROPE_TILE
 }
 
+// ----------------------------------------------------------------------------------------
+// skinny kernel: MT row tiles of 16 (M <= 16 MT), NW wavefronts per workgroup splitting k
 constexpr int SK_U = 4;                  // 32-element k steps per wavefront iteration
 constexpr int SK_CHUNK = 32 * SK_U;      // 128 elements
 
@@ -1438,10 +1440,10 @@ extern "C" int llme_gemm_bf16(const void* a, const void* w, void* out, int out_d
     if (auto_shape && blocked && direct != 0 && mode != kAtomicF32 && tiles_cost > 0.f) {
         // Large outputs: tiles of 256 x 256 by eight wavefronts, their slabs straight into LDS, load half the bytes per
         // product; one workgroup fills a compute unit. In the units of the estimate above a round of them costs 65,536 / 1.36:
-        // one round beats three of 128 x 128 tiles and two beat six, two do not beat five. (Measured, us, 128 x 128 / 256 x 256:
-        // gate/up of the 1B sizes at 700 rows 55 / 47, 1,300 rows 99 / 94, 500 rows 40 / 47; of the 8B sizes at 300 rows 98 / 90,
-        // 600 rows 158 / 166; down-proj, added: 8B sizes at 3,000 rows 341 / 287, 2,048 rows 234 / 283; 1B sizes at 6,000
-        // rows 197 / 170, 4,096 rows 135 / 167.)
+        // one round beats three of 128 x 128 tiles and two beat six, two do not beat five. (Measured, us, the best of the other
+        // tiles / 256 x 256: gate/up of the 1B sizes at 500 rows 42 / 52, 700 rows 56 / 52, 1,300 rows 104 / 104, 2,048 rows
+        // 150 / 121; of the 8B sizes at 300 rows 105 / 98, 600 rows 168 / 180, 5,000 rows 1,206 / 943; down-proj, added: 8B sizes
+        // at 3,000 rows 341 / 287, 2,048 rows 234 / 283; 1B sizes at 6,000 rows 197 / 170, 4,096 rows 135 / 167.)
         const long rounds = (static_cast<long>((M + 255) / 256) * ((N + 255) / 256) + cus - 1) / cus;
         if (static_cast<float>(rounds) * 65536.f / 1.36f < tiles_cost)
             return launch_tile_direct<4, 2, 4, 8>(A, W, out, M, N, K, mode, ksplit, stream);
@@ -1538,7 +1540,8 @@ extern "C" int llme_gemm_bf16_grouped_gated_extra(const void* a, const void* w, 
 // bfloat16; writes q_out [M, n_q hd] (rotated) and the rows' k (rotated) and v into the pages that
 // block_table[seq_idx[m]] names for positions[m]; cos/sin [max_pos, hd / 2] float32. Full rotation
 // only; hd 16, 32, 64 or 128 (a tile of 128 or 64 columns must hold whole heads). What the separate
-// kernels would store in between, the 32-bit q/k/v rows, never exists. tile_shape 0, 64, 96064, 128064, 96128 or 128.
+// kernels would store in between, the 32-bit q/k/v rows, never exists. tile_shape 0, 64, 96064, 128064, 96128, 128, or
+// 256256 (hd 64 or 128, blocked w).
 extern "C" int llme_gemm_bf16_qkv_rope(const void* a, const void* w, int M, int K, int blocked, const float* cos_t,
                                        const float* sin_t, const int* positions, const int* seq_idx,
                                        const int* block_table, int max_blocks, void* q_out, void* k_cache,
@@ -1580,7 +1583,10 @@ extern "C" int llme_gemm_bf16_qkv_rope(const void* a, const void* w, int M, int 
                 tile_shape = shapes[c];
             }
         }
-        // Long prompts: 256 x 256 tiles of the direct kernel (rotation in the registers), in the same units.
+        // Long prompts: 256 x 256 tiles of the direct kernel (rotation in the registers), in the same units. (Measured, us, the best
+        // of the others / these: 1B sizes at 2,048 rows 37 / 51, 4,096 rows 57 / 56, 5,400 rows 86 / 102, 8,192 rows 112 / 112; 3B sizes
+        // at 2,048 rows 75 / 73, 4,096 rows 133 / 152, 8,192 rows 258 / 237; 8B sizes at 1,024 rows 62 / 86, 2,048 rows 103 / 96, 2,700
+        // rows 160 / 187, 4,096 rows 207 / 200, 8,191 rows 400 / 325. Where the rule is wrong it costs 4 %: 3B sizes, 6,553 rows 223 / 233.)
         const long wgs = static_cast<long>((M + 255) / 256) * ((N + 255) / 256);
         if (blocked && (hd == 64 || hd == 128) && static_cast<double>((wgs + cus - 1) / cus) * (11.0 * K + 41000.0) < best) tile_shape = 256256;
     }
