@@ -10,7 +10,7 @@
 // operands to one on the matrix cores' 32-bit instruction (both further down). Tiling otherwise: a workgroup of 256
 // threads makes a 64 x 64 tile of the output, 4 x 4 per thread, stepping through K in slabs of 16 staged in LDS (stored
 // k-major so that the inner loop reads consecutive addresses).
-#include "common.h"
+#include "gemm_tiles.h"
 
 #include <type_traits>
 
@@ -188,7 +188,6 @@ static int launch_gemv_generic(const void* a, const void* w, void* out, int M, i
 // Measured at 149 rows, the 1B sizes (before: the 64 x 64 tile kernel above on 96 to 768 workgroups, one load at a time):
 // o-proj and down-proj 587 -> 69 us on average, q/k/v 236 -> 32, gate/up 398 -> 140 (71 TFLOP/s of its 10.0 GFLOP with
 // 64 x 64 tiles; 159 with 32 x 64). The error against 64 bits is half the former's (2.4e-6 of the logits, 4.7e-6): more and shorter sums.
-typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 template <int WMT, int WNT, int WR, int WC, int KW, int D, bool ACC>
 __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__ a, const float* __restrict__ w,
@@ -340,6 +339,12 @@ static int launch_generic(const void* a, const void* w, void* out, int M, int N,
     if constexpr (std::is_same_v<TA, float> && std::is_same_v<TW, float> && std::is_same_v<TO, float>) {
         if (!blocked && K % 4 == 0 && reinterpret_cast<uintptr_t>(a) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0) {
             const float *fa = static_cast<const float*>(a), *fw = static_cast<const float*>(w);
+            // Through LDS (gemm_panel.hip) wherever its pieces of four columns fit: operands straight from memory cost four times their
+            // bytes in the loads' path, since the lanes of a quarter lie in four rows.
+            if (N % 4 == 0 && K < (1 << 22) && reinterpret_cast<uintptr_t>(out) % 16 == 0) {
+                const PanelPlan plan = panel_plan(M, N, K, 1, 0, true);
+                return gemm_panel_f32(plan.mt, plan.bn, accumulate ? kAddF32 : kStoreF32, fa, fw, static_cast<float*>(out), M, N, K, 1, stream);
+            }
             return accumulate ? launch_gemm_f32<true>(fa, fw, static_cast<float*>(out), M, N, K, stream)
                               : launch_gemm_f32<false>(fa, fw, static_cast<float*>(out), M, N, K, stream);
         }

@@ -877,6 +877,33 @@ static void launch_skinny_nw(const bf16* x, const bf16* w, void* out, int M, int
     else launch_skinny<MT, 4>(x, w, out, M, N, K, mode, ksplit, blocked, stream);
 }
 
+// Codes of tile_shape from here on: the tiles of gemm_panel.hip, 1000 x rows + columns behind it (tests and measurements).
+constexpr int kPanelTile = 1000000;
+// The least k for which they are chosen: a sum of a few slabs never fills their ring, and neither way is much
+// faster (us, tiles through registers / these: 100 x 768 x 288 5.1 / 4.3, 270 x 4,096 x 384 5.7 / 6.3).
+constexpr int kPanelLeastK = 512;
+// The least columns of a stored 32-bit output for which they are: an output head's logits (150 rows x 32,768 x 4,096: 77 / 61 us). What
+// layers store keeps the one order of sums that all other tiles share: behind a matrix memory whose reads nearly cancel, another order
+// moved a prompt's bfloat16 logits by a tenth of their size, though its own error is no larger (2,995 rows x 2,048 x 12,288 would be 202 / 129 us).
+constexpr int kPanelLeastStored = 16384;
+
+// For a product of more than 64 rows that gemm_panel.hip takes: 1 where its tiles (plan) are the fastest, 2 where those of 256 x 256 are, 0 where the
+// kernels through staging registers are. Up to 64 rows every kernel waits for W, and these, a little faster alone (gate/up of the 1B sizes
+// at 64 rows 16.9 / 16.7 us, of 23 x 16,384 x 3,072 22.9 / 20.4), lost it again in the step (decode of 64 requests 1,656 / 1,679 us, of
+// 23 943 / 941). A sum of up to 288 rows that is better cut over k is, by the kernel below
+// (273 x 2,048 x 2,048 is not: 11.8 / 9.1). Larger ones by estimates: 256 x 256 tiles take 4 us + 0.0235 a k
+// in a round (700 rows x 16,384 x 2,048 51.7 against 55.5 here, 1,024 rows 59 / 79, 528 rows 52.7 / 48.4, 2,995 x 2,048 of k = 8,192 140 /
+// 92), tiles of 128 x 128 through registers, two a compute unit and added, 3 us + 0.0187 a k (4,096 x 2,048 x 2,048 41.7 / 50.0, but
+// alone on their compute units 2,048 x 2,048 of k = 8,192 79.4 / 67.2).
+static int choose_direct(int mode, int M, int N, int K, bool may_cut, const PanelPlan& plan, int cus) {
+    if (mode == kAddF32 && may_cut && M <= 288) return panel_plan(M, N, K, 0, 0).ksplit == 1 ? 1 : 0;
+    auto tiles = [&](int edge) { return static_cast<long>((M + edge - 1) / edge) * ((N + edge - 1) / edge); };
+    const float large = static_cast<float>((tiles(256) + cus - 1) / cus) * (4.f + 0.0235f * K);
+    const float staged = mode == kAddF32 && tiles(128) > cus ? static_cast<float>((tiles(128) + 2 * cus - 1) / (2 * cus)) * (3.f + 0.0187f * K) : large + 1.f;
+    if (plan.us <= large && plan.us <= staged) return 1;
+    return large <= staged ? 2 : 0;
+}
+
 }  // namespace llme
 
 using namespace llme;
@@ -952,6 +979,19 @@ extern "C" int llme_gemm_bf16(const void* a, const void* w, void* out, int out_d
     // workgroup per compute unit; a small output with a long k is cut over k instead (the
     // parts are added with atomics, so this needs an accumulating float32 output).
     if (gated) mode = gated == 2 ? kGatedReluBF16 : gated == 3 ? kGatedGeluBF16 : gated == 4 ? kGatedExtraBF16 : kGatedBF16;
+    const bool panel_takes = blocked && K < (1 << 22) && (mode == kStoreF32 || mode == kAddF32 || mode == kGatedBF16 ||
+                                                          (mode == kGatedExtraBF16 && t_gate_extra.pair_scale == nullptr));
+    if (tile_shape >= kPanelTile) {
+        const int bm = (tile_shape - kPanelTile) / 1000, bn = (tile_shape - kPanelTile) % 1000;
+        if (!panel_takes || bm % 16 != 0 || ksplit > 1) return kErrUnsupported;
+        return gemm_panel(bm / 16, bn, mode, A, W, out, M, N, K, 1, QkvTarget{}, t_gate_extra, stream);
+    }
+    if (tile_shape <= 0 && panel_takes && direct != 0 && ksplit <= 1 && M > 64 && K >= kPanelLeastK && (mode != kStoreF32 || N >= kPanelLeastStored)) {
+        const PanelPlan plan = panel_plan(M, N, K, 1, 0);
+        const int kind = choose_direct(mode, M, N, K, ksplit <= 0, plan, cus);
+        if (kind == 1) return gemm_panel(plan.mt, plan.bn, mode, A, W, out, M, N, K, 1, QkvTarget{}, t_gate_extra, stream);
+        if (kind == 2) return launch_tile_direct<4, 2, 4, 8>(A, W, out, M, N, K, mode, 1, stream);
+    }
     const bool auto_shape = tile_shape <= 0;
     float tiles_cost = -1.f;                           // of the chosen tile, in the units of the estimate below
     if (tile_shape <= 0) {
@@ -1155,6 +1195,18 @@ extern "C" int llme_gemm_bf16_qkv_rope(const void* a, const void* w, int M, int 
                        static_cast<bf16*>(k_cache), static_cast<bf16*>(v_cache), n_q, n_kv, hd, page};
     const bf16* A = static_cast<const bf16*>(a);
     const bf16* W = static_cast<const bf16*>(w);
+    if (tile_shape >= kPanelTile) {
+        const int bm = (tile_shape - kPanelTile) / 1000, bn = (tile_shape - kPanelTile) % 1000;
+        if (!blocked || bm % 16 != 0 || K >= (1 << 22)) return kErrUnsupported;
+        return gemm_panel(bm / 16, bn, kRopeCache, A, W, nullptr, M, N, K, 1, qt, GateExtra{}, stream);
+    }
+    if (tile_shape <= 0 && blocked && K >= kPanelLeastK && K < (1 << 22)) {
+        // The tiles of gemm_panel.hip while they are one round over the chip. (Measured, us, the best of the others / these: 1B sizes at 20 rows
+        // 13.7 / 8.0, 45: 14.6 / 8.7, 273: 14.7 / 9.9, 528: 15.9 / 15.9, 1,024: 23.6 / 19.9, 1,500: 30.5 / 24.8, in two rounds 2,048: 36.2 /
+        // 38.1; 3B sizes at 45 rows 24.1 / 16.8, 1,024: 45.6 / 36.3; 8B sizes at 150 rows 33.2 / 24.4, 528: 44.6 / 34.2, in two 1,024: 66.7 / 67.9.)
+        const PanelPlan plan = panel_plan(M, N, K, 1, hd);
+        if (plan.mt > 0 && plan.rounds == 1) return gemm_panel(plan.mt, plan.bn, kRopeCache, A, W, nullptr, M, N, K, 1, qt, GateExtra{}, stream);
+    }
     if (tile_shape <= 0) {
         // The tile with the least rounds of workgroups over the compute units x (a round's fixed cost,
         // which grows with k, + the tile's area): fitted to measurements at 80 to 1,024 rows. 1B sizes

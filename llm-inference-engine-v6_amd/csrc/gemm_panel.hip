@@ -1,0 +1,438 @@
+// out[m, n] (+)= sum_k a[m, k] * w[n, k] for a few dozen to a few hundred rows, bfloat16, blocked W.
+//
+// Between the kernels that stream W for up to 16 rows and the tiles of 256 x 256 for prompts lie products whose rows are one or two
+// tiles high, and outputs of few columns. Tiles through staging registers (gemm_tile_kernel) read 2.6 times the bytes there that
+// they must (273 rows x 16,384 columns in tiles of 96 x 64: 503 MB over the chip), and a compute unit gets 55 to 90 bytes a ns.
+// So the tile takes its height from the rows (BM = 16 MT, up to 192) x BN = 64 or 128 columns, one workgroup of eight wavefronts a
+// compute unit, with as many bytes on their way as LDS holds:
+//  * BN / 32 wavefronts share out the columns (32 each), KG = 256 / BN of them the k of a slab (32 each): a wavefront multiplies
+//    MT x 2 operand pairs a slab, and the KG parts of a sum join through LDS at the end.
+//  * a slab is A's BM rows x 32 KG and W's 16 blocks, two of which are a wavefront's own, all straight from memory into LDS.
+//  * NS slabs lie in LDS as a ring, all but the one that is read and the one that is multiplied on their way.
+// A slab's operands are in registers when its turn starts. The turn waits for the slab behind it, meets the barrier, and, row of
+// tiles by row of tiles, multiplies, reads the next slab's operand into the same registers and asks for a share of the slab NS - 1
+// ahead, into the buffer of the slab before, which everybody has multiplied. A wavefront passes the barrier with LDS reads on their
+// way: the buffer that they read is asked for again only behind the next one.
+// LDS holds A's chunks (8 rows x 64 k, lane 8 r + p: piece p ^ r of row r) and W's blocks as the kernel of 256 x 256 tiles does. In the
+// order of the operand, neighbouring lanes in neighbouring rows, a load of A took four times as long and a slab of 160 + 128 rows
+// 0.62 us instead of 0.38; half the wavefronts asking for A and half for W lost 15 % (a wavefront can only ask so fast).
+// Measured (us, tiles through registers / these): gate/up of the 1B sizes at 150 rows 22.9 / 22.6, 273: 35.9 / 27.3, 528:
+// 52.7 / 48.4; of the 8B sizes at 100 rows 52.3 / 46.9, 150: 70.8 / 54.4; sums: 1B down-proj at 2,048 rows 79.4 / 67.2, 2,995 rows of
+// k = 12,288 202 / 129; in parts (see below) at 96 rows 14.9 / 12.3, at 273 23.2 / 16.9.
+#include "gemm_tiles.h"
+
+namespace llme {
+
+template <int MT, int WNT, int CG, int KG>
+struct PanelSizes {
+    static constexpr int NW = CG * KG, BM = 16 * MT, BN = 16 * WNT * CG, SK = 32 * KG;
+    static constexpr int A_STAGE = BM * SK * 2, W_STAGE = WNT * NW * 1024, STAGE = A_STAGE + W_STAGE;
+    static constexpr int NS_MOST = 160 * 1024 / STAGE, NS = NS_MOST > 6 ? 6 : NS_MOST;
+    static constexpr int JOIN_MOST = 160 / (NW * WNT), JOIN_ROWS = MT < JOIN_MOST ? MT : JOIN_MOST;   // rows of tiles that join at a time
+    static constexpr int JOIN = NW * JOIN_ROWS * WNT * 1024, TURNED = BM * (BN + 4) * 4 + BM * 8;
+    static constexpr int LDS = NS * STAGE > JOIN ? NS * STAGE : JOIN;
+    static constexpr bool TURNS = TURNED <= LDS;                // the rotating epilogue's tile and its rows' places fit
+    static_assert(NS >= 3 && LDS <= 160 * 1024, "LDS");
+};
+
+// A lane's 16 bytes of an operand: 8 bfloat16 of k 8 q .., or 4 floats of k 4 q .., of which the s-th of every lane makes the k of
+// the s-th of four products (the same k in both operands).
+template <typename T> struct PanelOperand;
+template <> struct PanelOperand<bf16> {
+    using Type = bf16x8;
+    static __device__ __forceinline__ void multiply(const Type& w, const Type& a, f32x4& acc) {
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, a, acc, 0, 0, 0);
+    }
+};
+template <> struct PanelOperand<float> {
+    using Type = f32x4;
+    static __device__ __forceinline__ void multiply(const Type& w, const Type& a, f32x4& acc) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[s], a[s], acc, 0, 0, 0);
+    }
+};
+
+// T: bfloat16 or 32-bit. BLOCKED (bfloat16): W in blocks; otherwise (32-bit) row-major, its chunks loaded and read as A's.
+template <typename T, bool BLOCKED, int MT, int WNT, int CG, int KG, int MODE>
+__global__ __launch_bounds__(64 * CG * KG, 1) void gemm_panel_kernel(const T* __restrict__ a, const T* __restrict__ w,
+                                                            void* __restrict__ out, int M, int N, int K, int tiles_m, int tiles_n,
+                                                            int ksplit, QkvTarget qt, GateExtra gx) {
+    using S = PanelSizes<MT, WNT, CG, KG>;
+    constexpr int NW = S::NW, BM = S::BM, BN = S::BN, NS = S::NS;
+    static_assert(!BLOCKED || sizeof(T) == 2, "only bfloat16 matrices come in blocks");
+    constexpr int SLAB = 64 * KG;                               // bytes of a row in a slab
+    using Operand = typename PanelOperand<T>::Type;
+    constexpr int ROWS8 = BM / 8, CHUNKS = ROWS8 * (KG / 2);    // of A's slab: 8 rows x 64 k each
+    constexpr int LA = CHUNKS / NW, REST = CHUNKS % NW;         // a wavefront's: LA, the first REST wavefronts one more
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+
+    // A die gets consecutive tiles, rows fastest (up to 8 tiles of them), so that tiles which read the same W share its L2.
+    const int total = tiles_m * tiles_n * ksplit;
+    const int die = blockIdx.x % 8, per_die = total / 8, more = total % 8;
+    const int place_in = die * per_die + (die < more ? die : more) + blockIdx.x / 8;
+    const int split = place_in / (tiles_m * tiles_n), pid = place_in % (tiles_m * tiles_n);
+    constexpr int GROUP = 8;
+    const int g = pid / (GROUP * tiles_n), first_m = g * GROUP;
+    const int gsize = tiles_m - first_m < GROUP ? tiles_m - first_m : GROUP;
+    const int m0 = (first_m + pid % (GROUP * tiles_n) % gsize) * BM, n0 = pid % (GROUP * tiles_n) / gsize * BN;
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, q = lane >> 4;
+    const int cg = wave % CG, kg = wave / CG;
+
+    // this workgroup's share of k, in slabs
+    const unsigned row = static_cast<unsigned>(K) * sizeof(T);  // bytes
+    const int ns_all = static_cast<int>((row + SLAB - 1) / SLAB), ns_per = (ns_all + ksplit - 1) / ksplit;
+    const int s_begin = split * ns_per, s_end = s_begin + ns_per < ns_all ? s_begin + ns_per : ns_all;
+
+    const int a_rows = M - m0 < BM ? M - m0 : BM, w_rows = N - n0 < BN ? N - n0 : BN;
+    const u32x4 a_rsrc = raw_descriptor(a + static_cast<size_t>(m0) * K, a_rows * row);
+    const u32x4 w_rsrc = raw_descriptor(w + static_cast<size_t>(n0) * K, w_rows * row);
+    const unsigned lds_origin = static_cast<unsigned>(reinterpret_cast<size_t>(
+        (__attribute__((address_space(3))) unsigned char*)lds_raw));
+    constexpr unsigned kNowhere = 0xFFFFFF00u;                  // behind every descriptor's end: zeros, without a fetch
+    const unsigned last_at = (ns_all - 1) * SLAB;               // (k may end in the last slab: 16 bytes of a row are in or out whole)
+    // A's chunk j: rows 8 (j % ROWS8) .., bytes 128 (j / ROWS8) .. of the slab; lane 8 r' + p: row r', piece p ^ r' of its 128 bytes
+    unsigned a_off[LA + 1], a_last[LA + 1], w_off[WNT], w_last[WNT];
+    auto place_chunk = [&](int j, int rows8, unsigned& off, unsigned& last) {
+        const unsigned at = j / rows8 * 128 + ((lane & 7) ^ (lane >> 3)) * 16;
+        off = (j % rows8 * 8 + (lane >> 3)) * row + at;
+        last = last_at + at < row ? off : kNowhere;
+    };
+#pragma unroll
+    for (int i = 0; i <= LA; ++i) place_chunk(wave + NW * i, ROWS8, a_off[i], a_last[i]);
+#pragma unroll
+    for (int j = 0; j < WNT; ++j) {
+        if (BLOCKED) {
+            w_off[j] = (static_cast<unsigned>(cg * WNT + j) * (K / 32) + kg) * 1024u + lane * 16u;
+            w_last[j] = last_at + kg * 64 < row ? w_off[j] : kNowhere;
+        } else {
+            place_chunk(wave + NW * j, BN / 8, w_off[j], w_last[j]);
+        }
+    }
+    const bool one_more = wave < REST;
+    auto ask = [&](int s, int stage, int t) {                   // load t of slab s: W's blocks of this wavefront, then A's chunks
+        const bool past = s >= s_end, last = s == ns_all - 1;
+        const unsigned to = lds_origin + stage * S::STAGE;
+        if (t < WNT) {
+            load_b128_to_lds(w_rsrc, to + S::A_STAGE + (BLOCKED ? wave * WNT + t : wave + NW * t) * 1024,
+                             past ? kNowhere : last ? w_last[t] : w_off[t], s * (BLOCKED ? KG * 1024 : SLAB));
+        } else if (t < LA + WNT || one_more) {
+            const int i = t - WNT;
+            load_b128_to_lds(a_rsrc, to + (wave + NW * i) * 1024, past ? kNowhere : last ? a_last[i] : a_off[i], s * SLAB);
+        }
+    };
+    constexpr int LOADS = LA + WNT + (REST > 0 ? 1 : 0);
+    // at most `slabs` slabs of this wavefront's loads still on their way
+    auto wait_slabs = [&](auto slabs) {
+        constexpr int n = decltype(slabs)::value;
+        static_assert(n * (LA + WNT + 1) < 64, "the count of loads in flight has six bits");
+        if (REST > 0 && one_more) wait_vm<n * (LA + WNT + 1)>();
+        else wait_vm<n * (LA + WNT)>();
+    };
+    // The barrier of a turn: what a wavefront's LDS reads wait for is its own business (see below), the compiler keeps its order.
+    auto meet = [&] {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    f32x4 acc[MT][WNT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < WNT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    if (s_begin < s_end) {
+#pragma unroll
+        for (int d = 0; d < NS - 1; ++d)
+#pragma unroll
+            for (int t = 0; t < LOADS; ++t) ask(s_begin + d, d, t);
+        // this lane's place in an operand of A: chunk 2 g + r / 8 of column kg / 2, row r % 8 of it, piece 4 (kg % 2) + q
+        const unsigned in_chunk = (r & 7) * 128 + ((((kg & 1) * 4 + q) ^ (r & 7)) * 16);
+        const unsigned a_lane = ((kg >> 1) * ROWS8 + (r >> 3)) * 1024 + in_chunk;
+        const unsigned w_lane = S::A_STAGE + (BLOCKED ? wave * (WNT * 1024) + lane * 16
+                                                      : ((kg >> 1) * (BN / 8) + cg * (2 * WNT) + (r >> 3)) * 1024 + in_chunk);
+        auto read_a = [&](int stage, int i) { return *reinterpret_cast<const Operand*>(lds_raw + stage * S::STAGE + a_lane + i * 2048); };
+        auto read_w = [&](int stage, int j) { return *reinterpret_cast<const Operand*>(lds_raw + stage * S::STAGE + w_lane + j * (BLOCKED ? 1024 : 2048)); };
+        wait_slabs(std::integral_constant<int, NS - 2>{});
+        meet();
+        // (read in the order in which a turn reads: the compiler's waits for LDS then hold on both ways into the loop)
+        Operand fa[MT], fw0[WNT], fw1[WNT];
+        auto read_row = [&](int stage, int i, Operand (&into)[WNT]) {
+            fa[i] = read_a(stage, i);
+#pragma unroll
+            for (int j = 0; j < WNT; ++j)
+                if (j / 2 == i) into[j] = read_w(stage, j);
+        };
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+            read_row(0, i, fw0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        int st = 0, before = NS - 1;                            // the ring's places of slabs s and s - 1
+        auto turn = [&](int s, const Operand (&now)[WNT], Operand (&next)[WNT]) {
+            wait_slabs(std::integral_constant<int, NS - 3>{});  // slab s + 1 has landed ..
+            meet();                                             // .. everybody's share of it, and everybody has multiplied slab s - 1
+            const int behind = st + 1 == NS ? 0 : st + 1;
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+#pragma unroll
+                for (int j = 0; j < WNT; ++j) PanelOperand<T>::multiply(now[j], fa[i], acc[i][j]);
+                read_row(behind, i, next);
+#pragma unroll
+                for (int t = 0; t < LOADS; ++t)
+                    if (t * MT / LOADS == i) ask(s + NS - 1, before, t);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            before = st;
+            st = behind;
+        };
+        int s = s_begin;
+        for (; s + 1 < s_end; s += 2) {
+            turn(s, fw0, fw1);
+            turn(s + 1, fw1, fw0);
+        }
+        if (s < s_end) turn(s, fw0, fw1);
+    }
+    const int nw = n0 + cg * (16 * WNT) + q * 4;                // this lane's four columns of tile j: nw + 16 j ..; its row of tile i: m0 + 16 i + r
+    // what the sums are added to is asked for before they join (places past an edge ask for one that exists)
+    constexpr int OWN = (MT + KG - 1) / KG;                     // rows of tiles that a wavefront ends up with: i % KG == kg
+    f32x4 had[MODE == kAddF32 ? OWN : 1][WNT];
+    if constexpr (MODE == kAddF32) {
+#pragma unroll
+        for (int i = 0; i < OWN; ++i)
+#pragma unroll
+            for (int j = 0; j < WNT; ++j) {
+                const int m = m0 + (i * KG + kg) * 16 + r, n = nw + j * 16;
+                had[i][j] = *reinterpret_cast<const f32x4*>(static_cast<const float*>(out) + (i * KG + kg < MT && m < M && n < N ? static_cast<size_t>(m) * N + n : 0));
+            }
+    }
+    RowPlace place;
+    if constexpr (MODE == kRopeCache) {                         // where row m0 + tid goes
+        const int mrow = m0 + tid < M ? m0 + tid : M - 1;
+        place.pos = qt.positions[mrow];
+        place.page = qt.block_table[static_cast<size_t>(qt.seq_idx[mrow]) * qt.max_blocks + place.pos / qt.page];
+    }
+    wait_vm<0>();
+    // The KG wavefronts of a group of columns share its rows of tiles out and hand each other their parts where the ring was, 16 bytes a lane.
+    f32x4* parts = reinterpret_cast<f32x4*>(lds_raw);
+    auto part_at = [&](int of, int i, int j) { return ((of * CG + cg) * (S::JOIN_ROWS * WNT) + i % S::JOIN_ROWS * WNT + j) * 64 + lane; };
+#pragma unroll
+    for (int first = 0; first < MT; first += S::JOIN_ROWS) {
+        __syncthreads();                                        // (the ring, or the rows before, have been read)
+#pragma unroll
+        for (int i = first; i < MT && i < first + S::JOIN_ROWS; ++i)
+            if (i % KG != kg)
+#pragma unroll
+                for (int j = 0; j < WNT; ++j) parts[part_at(kg, i, j)] = acc[i][j];
+        __syncthreads();
+#pragma unroll
+        for (int i = first; i < MT && i < first + S::JOIN_ROWS; ++i) {
+            if (i % KG != kg) continue;
+#pragma unroll
+            for (int o = 1; o < KG; ++o) {
+                const int of = (kg + o) % KG;
+#pragma unroll
+                for (int j = 0; j < WNT; ++j) {
+                    const f32x4 p = parts[part_at(of, i, j)];
+                    acc[i][j][0] += p[0]; acc[i][j][1] += p[1]; acc[i][j][2] += p[2]; acc[i][j][3] += p[3];
+                }
+            }
+        }
+    }
+    if constexpr (MODE == kRopeCache) {
+        // the joined tile lies in LDS in 32 bits, with its rows' places, for the epilogue that all kernels share
+        constexpr int SS = BN + 4;
+        float* stage = reinterpret_cast<float*>(lds_raw);
+        int* row_pos = reinterpret_cast<int*>(lds_raw + static_cast<size_t>(BM) * SS * 4);
+        int* row_page = row_pos + BM;
+        __syncthreads();
+        if (tid < BM) {
+            row_pos[tid] = place.pos;
+            row_page[tid] = place.page;
+        }
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+            if (i % KG == kg)
+#pragma unroll
+                for (int j = 0; j < WNT; ++j) *reinterpret_cast<f32x4*>(stage + (i * 16 + r) * SS + cg * (16 * WNT) + j * 16 + q * 4) = acc[i][j];
+        __syncthreads();
+        store_staged<BM, BN, 64 * NW, MODE, false>(stage, row_pos, row_page, out, M, N, m0, n0, tid, qt, 0, gx, static_cast<size_t>(N));
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        const int m = m0 + i * 16 + r;
+        if (i % KG != kg || m >= M) continue;
+        if constexpr (is_gated(MODE)) {
+            typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
+#pragma unroll
+            for (int j = 0; j < WNT; j += 2) {
+                if (nw + j * 16 >= N) continue;
+                bf16x4 o, bg = {}, bu = {};
+                if (MODE == kGatedExtraBF16 && gx.bias != nullptr) {
+                    bg = *reinterpret_cast<const bf16x4*>(gx.bias + nw + j * 16);
+                    bu = *reinterpret_cast<const bf16x4*>(gx.bias + nw + j * 16 + 16);
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    o[e] = static_cast<__bf16>(gated_value<MODE>(acc[i][j][e], acc[i][j + 1][e], gx, static_cast<float>(bg[e]), static_cast<float>(bu[e])));
+                *reinterpret_cast<bf16x4*>(static_cast<bf16*>(out) + static_cast<size_t>(m) * (N / 2) + (n0 + cg * (16 * WNT) + j * 16) / 2 + q * 4) = o;
+            }
+        } else {
+            float* o = static_cast<float*>(out) + (static_cast<size_t>(MODE == kStoreF32 ? split : 0) * M + m) * N;   // (a part of its own)
+#pragma unroll
+            for (int j = 0; j < WNT; ++j) {
+                const int n = nw + j * 16;
+                if (n >= N) continue;
+                f32x4 v = acc[i][j];
+                if constexpr (MODE == kAddF32) {
+                    const f32x4 h = had[i / KG][j];
+                    v[0] += h[0]; v[1] += h[1]; v[2] += h[2]; v[3] += h[3];
+                }
+                *reinterpret_cast<f32x4*>(o + n) = v;
+            }
+        }
+    }
+}
+
+template <typename T, bool BLOCKED, int MT, int WNT, int CG, int KG, int MODE>
+static int launch_panel(const T* A, const T* W, void* out, int M, int N, int K, int ksplit, const QkvTarget& qt,
+                        const GateExtra& gx, hipStream_t stream) {
+    using S = PanelSizes<MT, WNT, CG, KG>;
+    if constexpr (MODE == kRopeCache && !S::TURNS) {
+        return kErrUnsupported;
+    } else {
+        static OncePerDevice told;
+        const int status = allow_lds(told, reinterpret_cast<const void*>(&gemm_panel_kernel<T, BLOCKED, MT, WNT, CG, KG, MODE>), S::LDS);
+        if (status != 0) return status;
+        const int tiles_m = (M + S::BM - 1) / S::BM, tiles_n = (N + S::BN - 1) / S::BN;
+        hipLaunchKernelGGL((gemm_panel_kernel<T, BLOCKED, MT, WNT, CG, KG, MODE>), dim3(tiles_m * tiles_n * ksplit), dim3(64 * S::NW), S::LDS, stream, A,
+                           W, out, M, N, K, tiles_m, tiles_n, ksplit, qt, gx);
+        return launch_status();
+    }
+}
+
+template <int MODE, bool BLOCKED, typename T>
+static int launch_panel_mode(int mt, int bn, const T* A, const T* W, void* out, int M, int N, int K, int ksplit, const QkvTarget& qt,
+                             const GateExtra& gx, hipStream_t stream) {
+#define LLME_PANEL(MT, BN) \
+    if (mt == MT && bn == BN) return launch_panel<T, BLOCKED, MT, 2, BN / 32, 256 / BN, MODE>(A, W, out, M, N, K, ksplit, qt, gx, stream);
+    LLME_PANEL(2, 64)
+    LLME_PANEL(3, 64)
+    LLME_PANEL(4, 64)
+    LLME_PANEL(5, 64)
+    LLME_PANEL(6, 64)
+    LLME_PANEL(3, 128)
+    LLME_PANEL(4, 128)
+    LLME_PANEL(5, 128)
+    LLME_PANEL(6, 128)
+    LLME_PANEL(7, 128)
+    LLME_PANEL(8, 128)
+    LLME_PANEL(9, 128)
+    LLME_PANEL(10, 128)
+    LLME_PANEL(11, 128)
+    LLME_PANEL(12, 128)
+#undef LLME_PANEL
+    return kErrUnsupported;
+}
+
+int gemm_panel(int mt, int bn, int mode, const bf16* A, const bf16* W, void* out, int M, int N, int K, int ksplit, const QkvTarget& qt,
+               const GateExtra& gx, hipStream_t stream) {
+    if (M <= 0 || N <= 0 || N % 16 != 0 || K <= 0 || K % 32 != 0 || K >= (1 << 22) || ksplit < 1) return kErrUnsupported;
+    if (is_gated(mode) && N % 32 != 0) return kErrUnsupported;
+    switch (mode) {
+        case kStoreF32: return launch_panel_mode<kStoreF32, true>(mt, bn, A, W, out, M, N, K, ksplit, qt, gx, stream);
+        case kAddF32: return launch_panel_mode<kAddF32, true>(mt, bn, A, W, out, M, N, K, 1, qt, gx, stream);
+        case kGatedBF16: return launch_panel_mode<kGatedBF16, true>(mt, bn, A, W, out, M, N, K, 1, qt, gx, stream);
+        case kGatedExtraBF16: return launch_panel_mode<kGatedExtraBF16, true>(mt, bn, A, W, out, M, N, K, 1, qt, gx, stream);
+        case kRopeCache: return bn % qt.hd ? kErrUnsupported : launch_panel_mode<kRopeCache, true>(mt, bn, A, W, out, M, N, K, 1, qt, gx, stream);
+        default: return kErrUnsupported;
+    }
+}
+
+// 32-bit operands, W row-major; K and N multiples of 4, all pointers 16-byte aligned.
+int gemm_panel_f32(int mt, int bn, int mode, const float* A, const float* W, float* out, int M, int N, int K, int ksplit, hipStream_t stream) {
+    if (M <= 0 || N <= 0 || N % 4 != 0 || K <= 0 || K % 4 != 0 || K >= (1 << 22) || ksplit < 1) return kErrUnsupported;
+    if (mode == kAddF32) return launch_panel_mode<kAddF32, false>(mt, bn, A, W, out, M, N, K, 1, QkvTarget{}, GateExtra{}, stream);
+    return launch_panel_mode<kStoreF32, false>(mt, bn, A, W, out, M, N, K, ksplit, QkvTarget{}, GateExtra{}, stream);
+}
+
+// The tile and the cut over k, by an estimate fitted to 700 timings of 20 to 4,096 rows at the 1B, 3B and 8B sizes (9 % off on
+// average; the chosen tile within 2 % of the best on average): rounds of workgroups over the chip x (3.2 us + 2.9 for the end of a tile
+// of 128 x 128, in proportion + the slabs' bytes at 98 a ns, less on a full chip and in large tiles, whose products take the time),
+// joined by their 2.5th powers with W's way from memory (1.2 us + 5.6 TB/s); parts cost their way out and back in the kernel that joins
+// them, 0.3 us a MB.
+// wide: 32-bit operands, whose products take the time (a compute unit makes 500 a ns).
+// ks_only: the number of parts (0: up to 8, of at least 256 k); heads: tiles hold whole heads of this many columns.
+PanelPlan panel_plan(int M, int N, int K, int ks_only, int heads, bool wide) {
+    // (the last plans made by this thread: a layer's products ask for the same few again and again, and steps with prompt rows wait for
+    // the host; an estimate of all tiles takes it 1.5 us)
+    struct Made {
+        int M = 0, N = 0, K = 0, other = 0;
+        PanelPlan plan{};
+    };
+    static thread_local Made memo[64];
+    const int other = ks_only * 2048 + heads * 2 + (wide ? 1 : 0);
+    Made& made = memo[(M * 7u + N / 16 * 13u + K / 16 * 5u + other) % 64u];
+    if (made.M == M && made.N == N && made.K == K && made.other == other) return made.plan;
+    static const int shapes[][2] = {{2, 64}, {3, 64}, {4, 64}, {5, 64}, {6, 64}, {3, 128}, {4, 128}, {5, 128}, {6, 128},
+                                    {7, 128}, {8, 128}, {9, 128}, {10, 128}, {11, 128}, {12, 128}};
+    const int cus = compute_units();
+    PanelPlan best{0, 0, 0, 0, 0.f};
+    for (const auto& s : shapes) {
+        const int bm = 16 * s[0], bn = s[1];
+        if (heads > 0 && bn % heads != 0) continue;
+        const long tiles = static_cast<long>((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+        for (int ks = ks_only > 0 ? ks_only : 1; ks <= (ks_only > 0 ? ks_only : 8); ++ks) {
+            if (ks > 1 && ks_only == 0 && K / ks < 256) break;
+            const long wgs = tiles * ks, rounds = (wgs + cus - 1) / cus;
+            const float full = wgs < cus ? static_cast<float>(wgs) / cus : 1.f, area = static_cast<float>(bm) * bn;
+            const float size = wide ? 4.f : 2.f, bytes = size * 1e-3f * K / ks * (bm + bn), rate = 98.f / (1.f + 0.54f * full * area / 24576.f);
+            const float multiplied = wide ? 2e-3f * K / ks * area / 500.f : 0.f;
+            const float chip = rounds * (3.2f + 2.9f * area / 16384.f + (multiplied > bytes / rate ? multiplied : bytes / rate));
+            const float memory = 1.2f + size * 1e-6f * N * K / 5.6f;
+            float us = powf(powf(chip, 2.5f) + powf(memory, 2.5f), 0.4f);
+            if (ks > 1) us += 0.3f * 4e-6f * ks * M * N;
+            if (best.mt == 0 || us < best.us) best = PanelPlan{s[0], bn, ks, static_cast<int>(rounds), us};
+        }
+    }
+    made = Made{M, N, K, other, best};
+    return best;
+}
+
+}  // namespace llme
+
+using namespace llme;
+
+// A sum over k that another kernel adds up (llme_parts_norm): how many parts of a [M, K] w [N, K] (bfloat16 and blocked, or wide: 32-bit and row-major) are worth it (0: none, the
+// product adds into its output itself). A product that adds its parts with atomics pays about 1 us a MB for them; up to 64 bfloat16
+// rows that is less than the longer norm costs, and both wait for W (down-proj of the 1B sizes with its weights from memory, us, atomics /
+// parts, and the norm 0.7 longer: 20 rows 10.1 / 10.2, 64 rows 12.1 / 11.3, 96 rows 14.9 / 12.3).
+extern "C" int llme_gemm_parts_plan(int M, int N, int K, int wide) {
+    if (M <= (wide ? 16 : 64) || M > 1024 || N % (wide ? 4 : 16) != 0 || K % (wide ? 4 : 32) != 0 || K >= (1 << 22)) return 0;
+    const PanelPlan p = panel_plan(M, N, K, 0, 0, wide != 0);
+    return p.ksplit > 1 ? p.ksplit : 0;
+}
+
+// parts [ksplit, M, N] float32: part i is the sum over the i-th share of k (whole slabs of the tile's; a share may be empty: zeros).
+// tile: 0 (chosen), or 1000 x rows + columns (tests and measurements).
+extern "C" int llme_gemm_parts(const void* a, const void* w, float* parts, int M, int N, int K, int ksplit, int tile, int wide,
+                               hipStream_t stream) {
+    if (ksplit < 1 || tile < 0 || tile / 1000 % 16 != 0) return kErrBadArgument;
+    if (M <= 0 || N <= 0) return 0;
+    int mt = tile / 16000, bn = tile % 1000;
+    if (tile == 0) {
+        const PanelPlan p = panel_plan(M, N, K, ksplit, 0, wide != 0);
+        mt = p.mt;
+        bn = p.bn;
+    }
+    if (wide) return gemm_panel_f32(mt, bn, kStoreF32, static_cast<const float*>(a), static_cast<const float*>(w), parts, M, N, K, ksplit, stream);
+    return gemm_panel(mt, bn, kStoreF32, static_cast<const bf16*>(a), static_cast<const bf16*>(w), parts, M, N, K, ksplit, QkvTarget{},
+                      GateExtra{}, stream);
+}
+
+LLME_LOAD_ENTRY(gemm_panel)

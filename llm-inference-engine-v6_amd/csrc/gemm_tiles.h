@@ -423,4 +423,15 @@ __device__ __forceinline__ void load_b128_to_lds(u32x4 rsrc, unsigned lds_base, 
                  : "memory", "m0");
 }
 
+// gemm_panel.hip: tiles of BM = 16 mt rows x bn columns, ksplit parts over k (kStoreF32 only, each a matrix of its own).
+struct PanelPlan {
+    int mt, bn, ksplit;
+    int rounds;                 // of workgroups over the chip
+    float us;                   // as estimated
+};
+PanelPlan panel_plan(int M, int N, int K, int ks_only, int heads, bool wide = false);
+int gemm_panel_f32(int mt, int bn, int mode, const float* A, const float* W, float* out, int M, int N, int K, int ksplit, hipStream_t stream);
+int gemm_panel(int mt, int bn, int mode, const bf16* A, const bf16* W, void* out, int M, int N, int K, int ksplit, const QkvTarget& qt,
+               const GateExtra& gx, hipStream_t stream);
+
 }  // namespace llme

@@ -155,7 +155,9 @@ class DecoderModel(Part):
                 self.pass_input.forward(h, h0, step)
             if hasattr(layer, "next_block"):
                 # (a block that can hand the streams' next read on is told which layer runs behind it in this pass)
-                layer.next_block = self.layers[self.schedule[i + 1].layer] if i + 1 < len(self.schedule) else None
+                # (none where the pass's input reads and writes the stream in between)
+                behind = self.schedule[i + 1] if i + 1 < len(self.schedule) else None
+                layer.next_block = self.layers[behind.layer] if behind is not None and not behind.enter else None
             layer.forward(h, step, caches[call.cache_id], call.write_cache)
         step.extra.pop("block.normed is for", None)
         step.extra.pop("block.stream_copy is for", None)

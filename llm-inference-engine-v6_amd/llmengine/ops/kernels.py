@@ -194,6 +194,17 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool =
     gemm_generic(a, w, out, accumulate)
 
 
+_product_in_parts = None            # (set by the matrix-core kernels)
+
+
+def add_product(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool, step) -> None:
+    """out (+)= a w^T, as `gemm` makes it; or, where the caller joins them (`mfma.may_leave_parts`) and it is faster, as parts of
+    the sum that are still to be added to `out`."""
+    if accumulate and _product_in_parts is not None and _product_in_parts(a, w, out, step):
+        return
+    gemm(a, w, out, accumulate, fixed_order=step.fixed_order, choices=step.choices)
+
+
 # --- attention -----------------------------------------------------------------------
 ATTENTION_MAX_HEAD_DIM = 256        # (a lane of attention_generic holds head_dim / 64 values of a row)
 
@@ -250,7 +261,7 @@ def attention_project(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
                                         w_o, out, accumulate)):
         return
     attention(q, k_cache, v_cache, o, step, block_table, n_q, n_kv, head_dim, scale, window)
-    gemm(o, w_o, out, accumulate, fixed_order=step.fixed_order, choices=choices)
+    add_product(o, w_o, out, accumulate, step)
 
 
 # --- sampling ------------------------------------------------------------------------

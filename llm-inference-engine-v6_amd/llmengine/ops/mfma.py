@@ -4,6 +4,7 @@ operand types and sizes fit; what they refuse goes to the plain-precision kernel
 from __future__ import annotations
 
 import ctypes
+import functools
 
 import torch
 
@@ -29,8 +30,8 @@ def gemm_bf16(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: b
               direct: int = -1, _supported: bool = False) -> None:
     """bfloat16 a [M, K] and w [N, K] -> out [M, N] (float32 or bfloat16), 32-bit accumulation.
     K must be a multiple of 8. gated: w holds gate and up rows interleaved in groups of 16 and
-    out is bfloat16 [M, N / 2] = silu(gate) * up (gated="relu": the rectifier instead of SiLU). waves / ksplit / tile (64, 128, 128096, 128064, 96128, 96064) /
-    force_tile override the launch choices (tests and measurements); direct: whether the product may
+    out is bfloat16 [M, N / 2] = silu(gate) * up (gated="relu": the rectifier instead of SiLU). waves / ksplit / tile (64, 128, 128096, 128064, 96128, 96064, or 1000000 + 1000 x rows +
+    columns of a tile of csrc/gemm_panel.hip) / force_tile override the launch choices (tests and measurements); direct: whether the product may
     use the 256 x 256 tile kernel whose slabs go from memory straight into LDS, which needs a blocked w
     (-1: where it pays, 0: never, 1: it must, with tile 256256)."""
     require(a, "a", torch.bfloat16, (None, None))
@@ -226,6 +227,118 @@ def _fast_gemm(a, w, out, accumulate, fixed_order=False, choices: KernelChoices 
 
 
 kernels._fast_gemm = _fast_gemm
+
+
+# --- sums into the residual stream that the next norm joins ------------------------------
+declare("llme_gemm_parts_plan", [_i, _i, _i, _i])
+declare("llme_gemm_parts", [_vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp])
+declare("llme_parts_norm", [_vp, _vp, _i, _vp, _i, _vp, _i, _i, _i, _f, _vp])
+
+
+@functools.lru_cache(maxsize=4096)
+def parts_plan(M: int, N: int, K: int, wide: bool = False) -> int:
+    """Parts over k that a product of these sizes should leave for the norm that reads its output next (0: none). wide: of
+    32-bit operands."""
+    return int(entry("llme_gemm_parts_plan")(M, N, K, 1 if wide else 0))
+
+
+def _parts_fit(a: torch.Tensor, w: torch.Tensor) -> bool:
+    if a.data_ptr() % 16 or w.data_ptr() % 16:
+        return False
+    if a.dtype == torch.float32:
+        return w.dtype == torch.float32 and w.dim() == 2
+    return a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and kernels.is_blocked(w)
+
+
+def gemm_parts(a: torch.Tensor, w: torch.Tensor, parts: torch.Tensor, tile: int = 0) -> None:
+    """parts[i] = the sum over the i-th share of k of a [M, K] w [N, K]^T (bfloat16 and w blocked, or both 32-bit and w row-major);
+    parts [n, M, N] float32. tile: 0 (chosen), or 1000 x rows + columns."""
+    require(a, "a", (torch.float32, torch.bfloat16), (None, None))
+    M, K = a.shape
+    N, _ = kernels._require_weight(w, "w", a.dtype, K)
+    require(parts, "parts", torch.float32, (None, M, N))
+    if not _parts_fit(a, w) or parts.data_ptr() % 16:
+        raise kernels.KernelError("gemm_parts: needs bfloat16 operands with a blocked weight or 32-bit ones with a row-major one, and "
+                                  "pointers 16-byte aligned")
+    _launch_parts(a, w, parts, M, N, K, tile)
+
+
+def _launch_parts(a, w, parts, M: int, N: int, K: int, tile: int = 0) -> None:
+    check(entry("llme_gemm_parts")(ptr(a), ptr(w), ptr(parts), M, N, K, parts.shape[0], tile, 1 if a.dtype == torch.float32 else 0,
+                                   stream()), "gemm_parts")
+
+
+def parts_norm(h: torch.Tensor, parts: torch.Tensor, weight: torch.Tensor, eps: float, out: torch.Tensor) -> None:
+    """h += the sum of parts [n, T, H]; out = weight * h / rms(h) of the updated rows (32-bit only with a 32-bit weight)."""
+    require(h, "h", torch.float32, (None, None))
+    T, H = h.shape
+    require(parts, "parts", torch.float32, (None, T, H))
+    require(weight, "weight", (torch.float32, torch.bfloat16), (H,))
+    require(out, "out", (torch.float32, torch.bfloat16), (T, H))
+    _launch_parts_norm(h, parts, weight, eps, out, T, H)
+
+
+def _launch_parts_norm(h, parts, weight, eps: float, out, T: int, H: int) -> None:
+    check(entry("llme_parts_norm")(ptr(h), ptr(parts), parts.shape[0], ptr(weight), 0 if weight.dtype == torch.float32 else 1, ptr(out),
+                                   0 if out.dtype == torch.float32 else 1, T, H, float(eps), stream()), "parts_norm")
+
+
+# Notes in a step's `extra`: the address of the stream that the next product may leave its sum for in parts; the parts; whether the
+# step's sums may be left in parts at all (asked once a step: steps with prompt rows are launched kernel by kernel).
+SUM_WANTED, SUM_PARTS, SUMS_MAY = "sum.may stay in parts", "sum.parts", "sum.parts allowed"
+
+
+PARTS_MIN_ROWS = {torch.bfloat16: 65, torch.float32: 17}        # (csrc/gemm_panel.hip, llme_gemm_parts_plan)
+
+
+def sums_may_stay_in_parts(step, h: torch.Tensor) -> bool:
+    """Whether products of the step that add into h may leave their sums in parts. Not where sums have a fixed order, which
+    products of one part keep."""
+    may = step.extra.get(SUMS_MAY)
+    if may is None:
+        T, H = h.shape
+        may = step.extra[SUMS_MAY] = (T >= PARTS_MIN_ROWS.get(step.act_dtype, T + 1) and not step.fixed_order
+                                      and choices_of(step).fast_gemm and H % 4 == 0 and H <= 8192 and h.is_contiguous()
+                                      and not tail_rows(T, choices_of(step)))
+    return may
+
+
+def may_leave_parts(step, h: torch.Tensor, norm) -> None:
+    """The next product that adds into h (`ops.add_product`) may leave its sum in parts, where the step's may: the caller hands them
+    to `norm` (`join_parts`) before anything reads h."""
+    if sums_may_stay_in_parts(step, h):
+        rms = norm.fused_rms()
+        if rms is not None and (rms[0].dtype == torch.float32 or step.act_dtype == torch.bfloat16):
+            step.extra[SUM_WANTED] = h.data_ptr()
+
+
+def product_in_parts(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, step) -> bool:
+    """Leaves a w^T in parts for `out` where the caller of the part joins them and it is faster; False: nothing is done."""
+    if step.extra.get(SUM_WANTED) != out.data_ptr() or not _parts_fit(a, w):
+        return False
+    M, K = a.shape
+    N = out.shape[1]
+    n = parts_plan(M, N, K, a.dtype == torch.float32)
+    if not n:
+        return False
+    del step.extra[SUM_WANTED]
+    parts = step.extra[SUM_PARTS] = step.buffer("sum.parts", (n, M, N), torch.float32)
+    _launch_parts(a, w, parts, M, N, K)
+    return True
+
+
+kernels._product_in_parts = product_in_parts
+
+
+def join_parts(h: torch.Tensor, norm, x: torch.Tensor, step) -> None:
+    """x = norm(h), with the parts that a product left for h added to it first."""
+    step.extra.pop(SUM_WANTED, None)
+    parts = step.extra.pop(SUM_PARTS, None)
+    if parts is None:
+        norm.forward(h, x)
+    else:
+        weight, eps = norm.fused_rms()
+        _launch_parts_norm(h, parts, weight, eps, x, h.shape[0], h.shape[1])
 
 
 # --- attention ---------------------------------------------------------------------------

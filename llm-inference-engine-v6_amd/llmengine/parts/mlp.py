@@ -86,7 +86,7 @@ class GatedMLP(FeedForward):
             ops.gemm_gated(x, self.w_gate_up, act, self.group,
                            lambda shape, dtype: step.buffer("mlp.gate_up", shape, dtype), choices=step.choices,
                            activation=self.activation)
-        ops.gemm(act, self.w_down, out, accumulate, fixed_order=step.fixed_order, choices=step.choices)
+        ops.add_product(act, self.w_down, out, accumulate, step)
         if self.bias:
             ops.window.add_row_bias(out, self.b_down)
 

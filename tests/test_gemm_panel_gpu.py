@@ -1,0 +1,151 @@
+"""Products whose rows are a tile or two high (csrc/gemm_panel.hip) and the norm that joins the parts of a sum."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+PANEL = 1000000
+TILES = [(16 * m, 64) for m in (2, 3, 6)] + [(16 * m, 128) for m in (3, 5, 8, 9, 12)]
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from llmengine import ops
+    return ops
+
+
+def _pair(M, N, K, seed):
+    g = torch.Generator().manual_seed(seed)
+    a = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    w = (torch.randn(N, K, generator=g) * 0.05).to(torch.bfloat16)
+    return a, w, a.double() @ w.double().T
+
+
+def _rel(got, want):
+    return float((got - want).norm() / want.norm())
+
+
+# rows around a tile's edges, columns that end inside a tile, k of less than a slab, of one, ending in a part of one and of many
+@pytest.mark.parametrize("M,N,K", [(1, 32, 32), (17, 64, 64), (33, 96, 160), (48, 160, 2048), (150, 288, 4128), (193, 2048, 288), (401, 320, 1056)])
+@pytest.mark.parametrize("rows,cols", TILES)
+def test_panel_tiles(ops, M, N, K, rows, cols):
+    """Every tile: stored, added and gated sums against 64 bits (32-bit sums of bfloat16 products: 2e-5 as for the other tiles,
+    5e-3 rounded, 8e-3 behind an activation)."""
+    a, w, ref = _pair(M, N, K, 5)
+    ad, wb, tile = a.to(DEV), ops.block_weight(w.to(DEV)), PANEL + 1000 * rows + cols
+    out = torch.full((M, N), float("nan"), device=DEV)
+    ops.gemm_bf16(ad, wb, out, tile=tile)
+    assert _rel(out.cpu().double(), ref) < 2e-5
+    base = torch.randn(M, N, generator=torch.Generator().manual_seed(6))
+    acc = base.clone().to(DEV)
+    ops.gemm_bf16(ad, wb, acc, accumulate=True, tile=tile)
+    assert _rel(acc.cpu().double(), ref + base.double()) < 2e-5
+    gated = torch.empty(M, N // 2, dtype=torch.bfloat16, device=DEV)
+    ops.gemm_bf16(ad, wb, gated, gated=True, tile=tile)
+    gu = ref.view(M, N // 32, 2, 16)
+    gate = gu[:, :, 0]
+    want = (gate * torch.sigmoid(gate) * gu[:, :, 1]).reshape(M, N // 2)
+    assert _rel(gated.cpu().double(), want) < 8e-3
+
+
+def test_panel_reads_zeros_behind_the_last_row_and_the_end_of_k(ops):
+    """What lies behind the operands' edges (the next rows' weights, here infinities and NaN) joins no sum."""
+    M, N, K = 20, 48, 96
+    a, w, ref = _pair(M + 30, N + 16, K, 7)
+    a[M:], w[N:] = float("nan"), float("inf")
+    ad, wb = a.to(DEV), ops.block_weight(w.to(DEV))
+    for rows, cols in TILES:
+        out = torch.zeros(M, N, device=DEV)
+        ops.gemm_bf16(ad[:M], wb[:N // 16], out, tile=PANEL + 1000 * rows + cols)
+        assert _rel(out.cpu().double(), ref[:M, :N]) < 2e-5, (rows, cols)
+
+
+@pytest.mark.parametrize("M,N,K,n", [(17, 64, 1024, 2), (45, 2048, 2048, 4), (150, 160, 4128, 8), (273, 272, 288, 5), (600, 96, 512, 3)])
+def test_parts_of_a_sum(ops, M, N, K, n):
+    """The parts add up to the product (also where the last share of k is empty), and run after run they are the same bits."""
+    a, w, ref = _pair(M, N, K, 8)
+    ad, wb = a.to(DEV), ops.block_weight(w.to(DEV))
+    parts = [torch.full((n, M, N), float("nan"), device=DEV) for _ in range(2)]
+    for p in parts:
+        ops.mfma.gemm_parts(ad, wb, p)
+    assert _rel(parts[0].cpu().double().sum(0), ref) < 2e-5 and torch.equal(parts[0], parts[1])
+
+
+@pytest.mark.parametrize("T,H,n", [(1, 4, 1), (17, 100, 2), (40, 2048, 3), (33, 3072, 8), (19, 4096, 5), (18, 8192, 9)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_parts_norm(ops, T, H, n, dtype):
+    g = torch.Generator().manual_seed(9)
+    h, parts = torch.randn(T, H, generator=g), torch.randn(n, T, H, generator=g)
+    weight = (1 + 0.1 * torch.randn(H, generator=g)).to(dtype)
+    hd, x = h.clone().to(DEV), torch.empty(T, H, dtype=torch.bfloat16, device=DEV)
+    ops.mfma.parts_norm(hd, parts.to(DEV), weight.to(DEV), 1e-5, x)
+    s = h.double() + parts.double().sum(0)
+    want = weight.double() * s / torch.sqrt((s * s).mean(-1, keepdim=True) + 1e-5)
+    assert _rel(hd.cpu().double(), s) < 1e-6 and _rel(x.cpu().double(), want) < 5e-3
+
+
+@pytest.mark.parametrize("hd,n_q,n_kv", [(16, 8, 4), (64, 8, 2), (128, 4, 2)])
+@pytest.mark.parametrize("T", [17, 100, 273])
+def test_panel_tiles_rotate_as_the_others(ops, hd, n_q, n_kv, T):
+    """The rotating epilogue behind every tile that holds whole heads: within bfloat16 rounding of the tile through registers (the
+    sums are joined in another order)."""
+    g, page, K = torch.Generator().manual_seed(10), 16, 544
+    x = torch.randn(T, K, generator=g).to(torch.bfloat16).to(DEV)
+    w = ops.block_weight((0.05 * torch.randn((n_q + 2 * n_kv) * hd, K, generator=g)).to(torch.bfloat16).to(DEV))
+    ang = torch.arange(T + 5, dtype=torch.float64)[:, None] / (10000.0 ** (torch.arange(hd // 2, dtype=torch.float64) * 2 / hd))[None, :]
+    cos, sin = torch.cos(ang).float().to(DEV), torch.sin(ang).float().to(DEV)
+    blocks = (T + 5 + page - 1) // page
+    positions, seq = torch.arange(5, T + 5, dtype=torch.int32, device=DEV), torch.zeros(T, dtype=torch.int32, device=DEV)
+    table = torch.randperm(blocks, generator=g).view(1, blocks).to(torch.int32).to(DEV)
+
+    def run(tile):
+        made = [torch.zeros(T, n_q * hd, dtype=torch.bfloat16, device=DEV), torch.zeros(blocks, n_kv, page, hd, dtype=torch.bfloat16, device=DEV),
+                torch.zeros(blocks, n_kv, hd, page, dtype=torch.bfloat16, device=DEV)]
+        ops.gemm_qkv_rope(x, w, cos, sin, positions, seq, table, *made, n_q, n_kv, hd, tile=tile)
+        return made
+    want = run(128)
+    for rows, cols in TILES:
+        if cols % hd:
+            continue
+        for a, b in zip(want, run(PANEL + 1000 * rows + cols)):
+            assert _rel(b.double(), a.double()) < 1e-3, (rows, cols)
+
+
+# pieces of 16 bytes past the end of k, columns that end inside a tile, one row of tiles and several
+@pytest.mark.parametrize("M,N,K", [(17, 64, 20), (33, 100, 2052), (81, 48, 64), (149, 272, 288), (300, 2048, 1024)])
+def test_panel_tiles_of_32_bit_operands(ops, M, N, K):
+    """32-bit operands with a row-major W: stored, added and in parts, against 64 bits (32-bit sums of up to 2,052 products, some
+    eight additions of which are of long partial sums: 1e-6)."""
+    g = torch.Generator().manual_seed(11)
+    a, w = torch.randn(M, K, generator=g), 0.05 * torch.randn(N, K, generator=g)
+    ref = a.double() @ w.double().T
+    ad, wd = a.to(DEV), w.to(DEV)
+    for accumulate in (False, True):
+        out = torch.full((M, N), 1.0 if accumulate else float("nan"), device=DEV)
+        ops.gemm_generic(ad, wd, out, accumulate)
+        assert _rel(out.cpu().double(), ref + (1.0 if accumulate else 0.0)) < 1e-6
+    for n in (2, 5):
+        for rows, cols in [(0, 0)] + TILES:
+            parts = torch.full((n, M, N), float("nan"), device=DEV)
+            ops.mfma.gemm_parts(ad, wd, parts, tile=1000 * rows + cols)
+            assert _rel(parts.cpu().double().sum(0), ref) < 1e-6, (n, rows, cols)
+
+
+@pytest.mark.parametrize("dtype,tol", [("fp32", 1e-5), ("bf16", 2e-2)])
+def test_a_step_whose_sums_stay_in_parts(ops, monkeypatch, dtype, tol):
+    """A prompt of rows enough that the sums into the stream are left in parts for the norms: the logits of the same model whose sums
+    have a fixed order, where no sum is (1e-5 and 2e-2 as the engine's other tests allow between orders of sums). The last
+    layer's down-proj, behind which no block's norm stands, adds into the stream itself."""
+    from llmengine import Engine
+    cfg = {"architectures": ["LlamaForCausalLM"], "model_type": "llama", "hidden_size": 1024, "intermediate_size": 2048, "num_hidden_layers": 3,
+           "num_attention_heads": 16, "num_key_value_heads": 4, "head_dim": 64, "vocab_size": 512, "max_position_embeddings": 1024,
+           "rms_norm_eps": 1e-5, "rope_theta": 10000.0, "tie_word_embeddings": True}
+    launched, wanted = ops.mfma._launch_parts, []
+    monkeypatch.setattr(ops.mfma, "_launch_parts", lambda *a, **k: wanted.append(a[2].shape) or launched(*a, **k))
+    prompt = [(7 * i * i + 3 * i) % 512 for i in range(150)]
+    logits = []
+    for fixed in (True, False):
+        engine = Engine.from_random(cfg, 3, dtype, std=0.05, norm_std=0.05, deterministic=fixed)
+        logits.append(torch.as_tensor(engine.forward_logits(prompt)).double())
+        assert len(wanted) == (0 if fixed else 5), wanted            # (o-proj three times, down-proj twice)
+    assert _rel(logits[1], logits[0]) < tol
