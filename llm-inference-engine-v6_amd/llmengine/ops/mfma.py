@@ -671,6 +671,7 @@ def attention_decode_rope(qkv, cos, sin, k_cache, v_cache, out, step, block_tabl
 
 
 # --- projections fused with the norm in front of them (decoding) ---------------------------
+declare("llme_gemv_norm_f32", [_vp, _vp, _vp, _i, _f, _vp, _vp, _i, _i, _i, _i, _vp])
 declare("llme_gemv_norm", [_vp, _vp, _vp, _i, _f, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp])
 
 GEMV_NORM_MAX_ROWS = 16
@@ -703,9 +704,9 @@ def qkv_sum_max_rows(decoded_only: bool, head_dim: int, choices: KernelChoices |
 
 
 def gemv_norm_supported(h: torch.Tensor, norm_weight: torch.Tensor, w: torch.Tensor, rows_out: int,
-                        gated: bool, choices: KernelChoices | None = None) -> bool:
-    """Whether a step may take gemv_norm: the kernel takes the operands, and the choices allow it."""
-    return (choices or DEFAULT).fast_gemm and _gemv_norm_fits(h, norm_weight, w, rows_out, gated)
+                        gated: bool, choices: KernelChoices | None = None, act: torch.dtype = torch.bfloat16) -> bool:
+    """Whether a step whose activations are `act` may take gemv_norm: the kernel takes the operands, and the choices allow it."""
+    return (choices or DEFAULT).fast_gemm and w.dtype == act and _gemv_norm_fits(h, norm_weight, w, rows_out, gated)
 
 
 def _gemv_norm_fits(h, norm_weight, w, rows_out: int, gated: bool) -> bool:
@@ -714,6 +715,10 @@ def _gemv_norm_fits(h, norm_weight, w, rows_out: int, gated: bool) -> bool:
         return False
     n_rows, k_w = kernels.weight_shape(w)
     n_out = n_rows // 2 if gated else n_rows
+    if w.dtype == torch.float32:
+        return (h.dtype == torch.float32 and w.dim() == 2 and norm_weight.dtype in (torch.float32, torch.bfloat16)
+                and 0 < rows_out <= GEMV_NORM_MAX_ROWS and K % 4 == 0 and k_w == K and (not gated or n_out % 16 == 0)
+                and w.data_ptr() % 16 == 0 and h.data_ptr() % 16 == 0 and norm_weight.data_ptr() % 16 == 0)
     return (h.dtype == torch.float32 and w.dtype == torch.bfloat16
             and norm_weight.dtype in (torch.float32, torch.bfloat16) and 0 < rows_out <= GEMV_NORM_MAX_ROWS
             and K % 8 == 0 and 16 * (K + 8) * 2 <= 132 * 1024 and k_w == K
@@ -725,19 +730,25 @@ def gemv_norm(h: torch.Tensor, norm_weight: torch.Tensor, eps: float, w: torch.T
               gated: bool = False, rows: torch.Tensor | None = None, tiles_per_round: int = 0,
               grid: int = 0) -> None:
     """out = (rmsnorm(h[rows]) with norm_weight) @ w^T for up to 16 rows of the 32-bit h; gated:
-    w holds gate and up rows interleaved in groups of 16 and out = silu(gate) * up in bfloat16."""
+    w holds gate and up rows interleaved in groups of 16 and out = silu(gate) * up, in bfloat16 as w is; a 32-bit w (row-major)
+    makes every output 32-bit."""
     require(h, "h", torch.float32, (None, None))
     K = h.shape[1]
     M = h.shape[0] if rows is None else rows.shape[0]
     if rows is not None:
         require(rows, "rows", torch.int32, (M,))
     require(norm_weight, "norm_weight", (torch.float32, torch.bfloat16), (K,))
-    n_rows, _ = kernels._require_weight(w, "w", torch.bfloat16, K)
+    n_rows, _ = kernels._require_weight(w, "w", (torch.float32, torch.bfloat16), K)
     N = n_rows // 2 if gated else n_rows
-    require(out, "out", torch.bfloat16 if gated else torch.float32, (M, N))
+    wide = w.dtype == torch.float32
+    require(out, "out", torch.bfloat16 if gated and not wide else torch.float32, (M, N))
     if not _gemv_norm_fits(h, norm_weight, w, M, gated):
         raise kernels.KernelError(f"gemv_norm: {M} rows (at most 16), K={K} (multiple of 8, 16 rows must fit "
                                   "into LDS) or the operand types are not supported")
+    if wide:
+        check(entry("llme_gemv_norm_f32")(ptr(h), ptr(rows), ptr(norm_weight), 0 if norm_weight.dtype == torch.float32 else 1, float(eps),
+                                          ptr(w), ptr(out), M, N, K, 1 if gated else 0, stream()), "gemv_norm")
+        return
     check(entry("llme_gemv_norm")(ptr(h), ptr(rows), ptr(norm_weight), 0 if norm_weight.dtype == torch.float32 else 1,
                                   float(eps), ptr(w), ptr(out), M, N, K, 1 if gated else 0, tiles_per_round, grid,
                                   1 if kernels.is_blocked(w) else 0, stream()),

@@ -101,8 +101,8 @@ class Attention(Mixer):
     def fuses_norm(self, h, norm, step):
         # A few rows (decoding): the q/k/v projection applies the norm itself.
         rms = norm.fused_rms()
-        return (rms is not None and step.act_dtype == torch.bfloat16
-                and ops.gemv_norm_supported(h, rms[0], self.w_qkv, h.shape[0], gated=False, choices=step.choices))
+        return rms is not None and ops.gemv_norm_supported(h, rms[0], self.w_qkv, h.shape[0], gated=False, choices=step.choices,
+                                                           act=step.act_dtype)
 
     def _bytes_read(self, step) -> int | None:
         """What a step of few rows reads in this layer: its weights, and the requests' keys and values, which count a third

@@ -73,8 +73,8 @@ class OutputHead(Head):
 
     def fuses_norm(self, h: torch.Tensor, norm, n_rows: int, step) -> bool:
         rms = norm.fused_rms()
-        return (rms is not None and step.act_dtype == torch.bfloat16
-                and ops.gemv_norm_supported(h, rms[0], self.weight, n_rows, gated=False, choices=step.choices))
+        return rms is not None and ops.gemv_norm_supported(h, rms[0], self.weight, n_rows, gated=False, choices=step.choices,
+                                                           act=step.act_dtype)
 
     def _finish(self, out: torch.Tensor) -> None:
         if self.scale != 1.0:

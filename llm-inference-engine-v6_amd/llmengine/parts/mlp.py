@@ -63,14 +63,14 @@ class GatedMLP(FeedForward):
     def fuses_norm(self, h, norm, step):
         # A few rows (decoding): one kernel applies the norm, both projections and the activation.
         rms = norm.fused_rms()
-        return (rms is not None and not self.bias and self.group == 16 and self.activation == "silu" and step.act_dtype == torch.bfloat16
-                and ops.gemv_norm_supported(h, rms[0], self.w_gate_up, h.shape[0], gated=True, choices=step.choices))
+        return (rms is not None and not self.bias and self.group == 16 and self.activation == "silu"
+                and ops.gemv_norm_supported(h, rms[0], self.w_gate_up, h.shape[0], gated=True, choices=step.choices, act=step.act_dtype))
 
     def forward(self, x, step, out, accumulate, pre_norm=None):
         T = x.shape[0]
         FF = self.intermediate_size
         if pre_norm is not None:
-            act = step.buffer("mlp.act", (T, FF), torch.bfloat16)
+            act = step.buffer("mlp.act", (T, FF), step.act_dtype)
             weight, eps = pre_norm.fused_rms()
             ops.gemv_norm(x, weight, eps, self.w_gate_up, act, gated=True)
         elif self.bias:

@@ -131,6 +131,30 @@ def test_panel_tiles_of_32_bit_operands(ops, M, N, K):
             assert _rel(parts.cpu().double().sum(0), ref) < 1e-6, (n, rows, cols)
 
 
+@pytest.mark.parametrize("M", [1, 2, 3, 8, 13, 16])
+@pytest.mark.parametrize("N,K", [(32, 60), (64, 1028), (9000, 64), (8224, 1024)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_32_bit_products_of_few_rows_with_the_norm_inside(ops, M, N, K, dtype):
+    """Whole columns and k in four, plain over chosen rows and gated, against 64 bits."""
+    g = torch.Generator().manual_seed(12)
+    h, w = torch.randn(M + 3, K, generator=g), 0.05 * torch.randn(N, K, generator=g)
+    weight = (1 + 0.1 * torch.randn(K, generator=g)).to(dtype)
+    rows = torch.randperm(M + 3, generator=g)[:M].to(torch.int32)
+
+    def normed(x):
+        x = x.double()
+        return weight.double() * x / torch.sqrt((x * x).mean(-1, keepdim=True) + 1e-5)
+    out = torch.full((M, N), float("nan"), device=DEV)
+    ops.gemv_norm(h.to(DEV), weight.to(DEV), 1e-5, w.to(DEV), out, rows=rows.to(DEV))
+    assert _rel(out.cpu().double(), normed(h[rows.long()]) @ w.double().T) < 1e-6
+    if N % 32 == 0:
+        gated = torch.full((M, N // 2), float("nan"), device=DEV)
+        ops.gemv_norm(h[:M].contiguous().to(DEV), weight.to(DEV), 1e-5, w.to(DEV), gated, gated=True)
+        gu = (normed(h[:M]) @ w.double().T).view(M, N // 32, 2, 16)
+        want = (gu[:, :, 0] * torch.sigmoid(gu[:, :, 0]) * gu[:, :, 1]).reshape(M, N // 2)
+        assert _rel(gated.cpu().double(), want) < 2e-6
+
+
 @pytest.mark.parametrize("dtype,tol", [("fp32", 1e-5), ("bf16", 2e-2)])
 def test_a_step_whose_sums_stay_in_parts(ops, monkeypatch, dtype, tol):
     """A prompt of rows enough that the sums into the stream are left in parts for the norms: the logits of the same model whose sums
