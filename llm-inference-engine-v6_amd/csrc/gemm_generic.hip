@@ -271,7 +271,8 @@ static int launch_gemv_generic(const void* a, const void* w, void* out, int M, i
     return launch_status();
 }
 
-// 32-bit operands, more than 16 rows: v_mfma_f32_16x16x4_f32, whose products and sums are 32-bit like the vector unit's, at
+// 32-bit operands, more than 16 rows, where the output's columns do not come in fours or it is not aligned (all others go through LDS, as
+// gemm_panel.hip does: gate/up at 149 rows 140 -> 95 us, o-proj and down-proj uncut 69 -> 47): v_mfma_f32_16x16x4_f32, whose products and sums are 32-bit like the vector unit's, at
 // twice the rate of its single multiply-adds (32 against 16 a cycle and scheduler: 157 TFLOP/s). At that rate the operands
 // need no LDS: a lane loads 8 consecutive k of a row (two loads of 16 bytes; the four lanes of a row take 128 bytes together), and step s of eight
 // multiplies element s of every lane, which is k = 8 q + s for lane group q in both operands. A wavefront makes

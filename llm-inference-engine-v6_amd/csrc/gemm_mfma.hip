@@ -297,8 +297,8 @@ __global__ __launch_bounds__(256, 2) void gemm_tile_kernel(const bf16* __restric
 // half turn for the first half of slab (h - 1) / 2 + 3 (into the buffer of the slab that ends here), the even
 // one behind it for the second. A half turn of 32 products a wavefront is 1,024 cycles of the matrix pipe: with all
 // of a half turn's loads asked for in one go, A's only in every second, it took 1,480 to 1,570 cycles; dealt out over
-// the rows and over both half turns it takes 1,300 to 1,360 (without loads 1,140; gate/up of 8,191 x 28,672 x 4,096 went
-// from 1,646 to 1,508 us, 1,276 TFLOP/s, by this and the epilogue below). The chip lowers its clock under this load (1.9 of
+// the rows and over both half turns it took 1,300 to 1,360 (without loads 1,140; gate/up of 8,191 x 28,672 x 4,096 went
+// from 1,646 to 1,508 us by this and the epilogue below), and with A's loads as they are now a tenth less (1,369 us, 1,405 TFLOP/s). The chip lowers its clock under this load (1.9 of
 // 2.4 GHz), so fewer stalls win less than their cycles. (Four wavefronts of 128 x 128 read a third less of LDS: 1,360 to 1,390
 // cycles at 2.05 GHz, and the epilogue with half the wavefronts took more than that won.)
 // Needs: W blocked (N a multiple of 16, K of 32). A slab that hangs over the end of k reads zeros

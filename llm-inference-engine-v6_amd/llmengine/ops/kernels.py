@@ -195,14 +195,16 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool =
 
 
 _product_in_parts = None            # (set by the matrix-core kernels)
+# A note in a step's `extra`: the address of the stream that the next product may leave its sum for in parts (`mfma.may_leave_parts`).
+SUM_WANTED = "sum.may stay in parts"
 
 
 def add_product(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool, step) -> None:
     """out (+)= a w^T, as `gemm` makes it; or, where the caller joins them (`mfma.may_leave_parts`) and it is faster, as parts of
     the sum that are still to be added to `out`."""
-    if accumulate and _product_in_parts is not None and _product_in_parts(a, w, out, step):
+    if accumulate and SUM_WANTED in step.extra and _product_in_parts(a, w, out, step):
         return
-    gemm(a, w, out, accumulate, fixed_order=step.fixed_order, choices=step.choices)
+    gemm(a, w, out, accumulate, step.fixed_order, step.choices)
 
 
 # --- attention -----------------------------------------------------------------------
@@ -261,7 +263,10 @@ def attention_project(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
                                         w_o, out, accumulate)):
         return
     attention(q, k_cache, v_cache, o, step, block_table, n_q, n_kv, head_dim, scale, window)
-    add_product(o, w_o, out, accumulate, step)
+    if accumulate and SUM_WANTED in step.extra:
+        add_product(o, w_o, out, accumulate, step)
+    else:
+        gemm(o, w_o, out, accumulate, fixed_order=step.fixed_order, choices=choices)
 
 
 # --- sampling ------------------------------------------------------------------------

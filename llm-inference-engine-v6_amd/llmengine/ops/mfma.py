@@ -285,7 +285,7 @@ def _launch_parts_norm(h, parts, weight, eps: float, out, T: int, H: int) -> Non
 
 # Notes in a step's `extra`: the address of the stream that the next product may leave its sum for in parts; the parts; whether the
 # step's sums may be left in parts at all (asked once a step: steps with prompt rows are launched kernel by kernel).
-SUM_WANTED, SUM_PARTS, SUMS_MAY = "sum.may stay in parts", "sum.parts", "sum.parts allowed"
+SUM_WANTED, SUM_PARTS, SUMS_MAY = kernels.SUM_WANTED, "sum.parts", "sum.parts allowed"
 
 
 PARTS_MIN_ROWS = {torch.bfloat16: 65, torch.float32: 17}        # (csrc/gemm_panel.hip, llme_gemm_parts_plan)
@@ -314,10 +314,13 @@ def may_leave_parts(step, h: torch.Tensor, norm) -> None:
 
 def product_in_parts(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, step) -> bool:
     """Leaves a w^T in parts for `out` where the caller of the part joins them and it is faster; False: nothing is done."""
-    if step.extra.get(SUM_WANTED) != out.data_ptr() or not _parts_fit(a, w):
+    if step.extra.get(SUM_WANTED) != out.data_ptr():
         return False
     M, K = a.shape
     N = out.shape[1]
+    # (what these operands would be refused for, `gemm` says)
+    if not _parts_fit(a, w) or not a.is_contiguous() or kernels.weight_shape(w) != (N, K) or tuple(out.shape) != (M, N):
+        return False
     n = parts_plan(M, N, K, a.dtype == torch.float32)
     if not n:
         return False

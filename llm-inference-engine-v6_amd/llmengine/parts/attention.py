@@ -184,7 +184,7 @@ class Attention(Mixer):
                 if ops.mfma.attention_decode_rope(qkv, cos, sin, k_cache, v_cache, o, step, block_table, n_q, n_kv, hd,
                                                   self.scale, self.window, done):
                     step.extra["attn.qkv_sum zero"] = (held.data_ptr(), held.numel())
-                    if not (accumulate and ops.mfma.product_in_parts(o, self.w_o, out, step)):
+                    if not (accumulate and ops.mfma.SUM_WANTED in step.extra and ops.mfma.product_in_parts(o, self.w_o, out, step)):
                         ops.gemm(o, self.w_o, out, accumulate, fixed_order=step.fixed_order, choices=step.choices)
                     return
             ops.rope_kv_write(qkv, cos, sin, step.positions, step.seq_idx, block_table, q, k_cache, v_cache,

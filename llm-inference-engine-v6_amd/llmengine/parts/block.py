@@ -39,7 +39,8 @@ class PreNormBlock(Block):
     def forward(self, h, step, cache, write_cache=True):
         T, H = h.shape
         x = step.buffer("block.normed", (T, H), step.act_dtype)
-        if ops.mfma.sums_may_stay_in_parts(step, h):
+        may = step.extra.get(ops.mfma.SUMS_MAY)
+        if ops.mfma.sums_may_stay_in_parts(step, h) if may is None else may:
             self._forward_in_parts(h, x, step, cache, write_cache)
             return
         if self.mixer.fuses_norm(h, self.mixer_norm, step):

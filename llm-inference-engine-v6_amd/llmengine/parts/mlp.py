@@ -86,7 +86,10 @@ class GatedMLP(FeedForward):
             ops.gemm_gated(x, self.w_gate_up, act, self.group,
                            lambda shape, dtype: step.buffer("mlp.gate_up", shape, dtype), choices=step.choices,
                            activation=self.activation)
-        ops.add_product(act, self.w_down, out, accumulate, step)
+        if ops.mfma.SUM_WANTED in step.extra:
+            ops.add_product(act, self.w_down, out, accumulate, step)
+        else:
+            ops.gemm(act, self.w_down, out, accumulate, fixed_order=step.fixed_order, choices=step.choices)
         if self.bias:
             ops.window.add_row_bias(out, self.b_down)
 
