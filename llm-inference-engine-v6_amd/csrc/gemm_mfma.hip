@@ -882,9 +882,7 @@ constexpr int kPanelTile = 1000000;
 // The least k for which they are chosen: a sum of a few slabs never fills their ring, and neither way is much
 // faster (us, tiles through registers / these: 100 x 768 x 288 5.1 / 4.3, 270 x 4,096 x 384 5.7 / 6.3).
 constexpr int kPanelLeastK = 512;
-// The least columns of a stored 32-bit output for which they are: an output head's logits (150 rows x 32,768 x 4,096: 77 / 61 us). What
-// layers store keeps the one order of sums that all other tiles share: behind a matrix memory whose reads nearly cancel, another order
-// moved a prompt's bfloat16 logits by a tenth of their size, though its own error is no larger (2,995 rows x 2,048 x 12,288 would be 202 / 129 us).
+// The least columns of a stored 32-bit output for which they are: an output head's logits (150 rows x 32,768 x 4,096: 69 / 57 us).
 constexpr int kPanelLeastStored = 16384;
 
 // For a product of more than 64 rows that gemm_panel.hip takes: 1 where its tiles (plan) are the fastest, 2 where those of 256 x 256 are, 0 where the

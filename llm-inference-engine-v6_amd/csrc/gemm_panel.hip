@@ -1,35 +1,44 @@
-// out[m, n] (+)= sum_k a[m, k] * w[n, k] for a few dozen to a few hundred rows, bfloat16, blocked W.
+// out[m, n] (+)= sum_k a[m, k] * w[n, k] for a few dozen to some thousand rows: bfloat16 with a blocked W, or 32-bit with a row-major W.
 //
 // Between the kernels that stream W for up to 16 rows and the tiles of 256 x 256 for prompts lie products whose rows are one or two
 // tiles high, and outputs of few columns. Tiles through staging registers (gemm_tile_kernel) read 2.6 times the bytes there that
 // they must (273 rows x 16,384 columns in tiles of 96 x 64: 503 MB over the chip), and a compute unit gets 55 to 90 bytes a ns.
 // So the tile takes its height from the rows (BM = 16 MT, up to 192) x BN = 64 or 128 columns, one workgroup of eight wavefronts a
 // compute unit, with as many bytes on their way as LDS holds:
-//  * BN / 32 wavefronts share out the columns (32 each), KG = 256 / BN of them the k of a slab (32 each): a wavefront multiplies
-//    MT x 2 operand pairs a slab, and the KG parts of a sum join through LDS at the end.
-//  * a slab is A's BM rows x 32 KG and W's 16 blocks, two of which are a wavefront's own, all straight from memory into LDS.
+//  * BN / 32 wavefronts share out the columns (32 each). bfloat16: the KS = 256 / BN wavefronts of a group of columns share out its rows of
+//    tiles, and each adds up all of k in turn, so that a sum has the one order that every other tile kernel gives it: whichever tile
+//    a product's rows are given, its results are the same bits. (Sharing out k instead, with the parts joined through LDS at
+//    the end, reads a fifth less of LDS and was no faster: parts of the 1B o-proj at 273 rows 8.2 / 8.0 us, of its down-proj 17.6 / 16.5,
+//    of the 8B down-proj at 528 rows 69.9 / 70.0, and with other orders of sums a prompt's bfloat16 logits moved by their rounding
+//    with the number of its rows. Wavefronts of 64 columns by a quarter of the rows: 0 to 2 % slower.) 32-bit: the wavefronts share out the
+//    steps of k, which is even for any number of rows; there the products take the time.
+//  * a slab is A's BM rows and W's BN columns of KS steps of k (64 bytes a row each), all straight from memory into LDS.
 //  * NS slabs lie in LDS as a ring, all but the one that is read and the one that is multiplied on their way.
-// A slab's operands are in registers when its turn starts. The turn waits for the slab behind it, meets the barrier, and, row of
-// tiles by row of tiles, multiplies, reads the next slab's operand into the same registers and asks for a share of the slab NS - 1
+// A slab's operands are in registers when its turn starts. The turn waits for the slab behind it, meets the barrier, and, step of k
+// by step of k and row of tiles by row of tiles, multiplies, reads the next slab's operand into the same registers and asks for a share of the slab NS - 1
 // ahead, into the buffer of the slab before, which everybody has multiplied. A wavefront passes the barrier with LDS reads on their
 // way: the buffer that they read is asked for again only behind the next one.
 // LDS holds A's chunks (8 rows x 64 k, lane 8 r + p: piece p ^ r of row r) and W's blocks as the kernel of 256 x 256 tiles does. In the
 // order of the operand, neighbouring lanes in neighbouring rows, a load of A took four times as long and a slab of 160 + 128 rows
 // 0.62 us instead of 0.38; half the wavefronts asking for A and half for W lost 15 % (a wavefront can only ask so fast).
-// Measured (us, tiles through registers / these): gate/up of the 1B sizes at 150 rows 22.9 / 22.6, 273: 35.9 / 27.3, 528:
-// 52.7 / 48.4; of the 8B sizes at 100 rows 52.3 / 46.9, 150: 70.8 / 54.4; sums: 1B down-proj at 2,048 rows 79.4 / 67.2, 2,995 rows of
-// k = 12,288 202 / 129; in parts (see below) at 96 rows 14.9 / 12.3, at 273 23.2 / 16.9.
+// Measured (us, weights from memory, tiles through registers / these): gate/up of the 1B sizes at 150 rows 22.1 / 20.2, 273:
+// 34.5 / 25.5, 528: 51.3 / 46.5; of the 8B sizes at 150 rows 63.9 / 49.3; sums: 1B down-proj at 2,048 rows 84.4 / 73.8, 2,995 rows of
+// k = 12,288 209 / 129; in parts (see below) against atomics at 96 rows 14.3 / 10.7, at 273 25.8 / 16.5.
 #include "gemm_tiles.h"
 
 namespace llme {
 
-template <int MT, int WNT, int CG, int KG>
+// CG x KS wavefronts; a slab is KS steps of 64 bytes of k. bfloat16: W in blocks, the wavefronts of a column group share out the rows (ROWS).
+// 32-bit: W row-major, its chunks loaded and read as A's, and they share out the steps of k.
+template <typename T, int MT, int CG, int KS>
 struct PanelSizes {
-    static constexpr int NW = CG * KG, BM = 16 * MT, BN = 16 * WNT * CG, SK = 32 * KG;
+    static constexpr bool BLOCKED = sizeof(T) == 2, ROWS = BLOCKED;
+    static constexpr int WNT = 2;                               // tiles of 16 columns a wavefront
+    static constexpr int NW = CG * KS, BM = 16 * MT, BN = 16 * WNT * CG, SK = 32 * KS;
     static constexpr int A_STAGE = BM * SK * 2, W_STAGE = WNT * NW * 1024, STAGE = A_STAGE + W_STAGE;
     static constexpr int NS_MOST = 160 * 1024 / STAGE, NS = NS_MOST > 6 ? 6 : NS_MOST;
     static constexpr int JOIN_MOST = 160 / (NW * WNT), JOIN_ROWS = MT < JOIN_MOST ? MT : JOIN_MOST;   // rows of tiles that join at a time
-    static constexpr int JOIN = NW * JOIN_ROWS * WNT * 1024, TURNED = BM * (BN + 4) * 4 + BM * 8;
+    static constexpr int JOIN = ROWS ? 0 : NW * JOIN_ROWS * WNT * 1024, TURNED = BM * (BN + 4) * 4 + BM * 8;
     static constexpr int LDS = NS * STAGE > JOIN ? NS * STAGE : JOIN;
     static constexpr bool TURNS = TURNED <= LDS;                // the rotating epilogue's tile and its rows' places fit
     static_assert(NS >= 3 && LDS <= 160 * 1024, "LDS");
@@ -52,17 +61,18 @@ template <> struct PanelOperand<float> {
     }
 };
 
-// T: bfloat16 or 32-bit. BLOCKED (bfloat16): W in blocks; otherwise (32-bit) row-major, its chunks loaded and read as A's.
-template <typename T, bool BLOCKED, int MT, int WNT, int CG, int KG, int MODE>
-__global__ __launch_bounds__(64 * CG * KG, 1) void gemm_panel_kernel(const T* __restrict__ a, const T* __restrict__ w,
+template <typename T, int MT, int CG, int KS, int MODE>
+__global__ __launch_bounds__(64 * CG * KS, 1) void gemm_panel_kernel(const T* __restrict__ a, const T* __restrict__ w,
                                                             void* __restrict__ out, int M, int N, int K, int tiles_m, int tiles_n,
                                                             int ksplit, QkvTarget qt, GateExtra gx) {
-    using S = PanelSizes<MT, WNT, CG, KG>;
-    constexpr int NW = S::NW, BM = S::BM, BN = S::BN, NS = S::NS;
-    static_assert(!BLOCKED || sizeof(T) == 2, "only bfloat16 matrices come in blocks");
-    constexpr int SLAB = 64 * KG;                               // bytes of a row in a slab
+    using S = PanelSizes<T, MT, CG, KS>;
+    constexpr int NW = S::NW, WNT = S::WNT, BM = S::BM, BN = S::BN, NS = S::NS;
+    constexpr bool BLOCKED = S::BLOCKED, ROWS = S::ROWS;
+    // a wavefront multiplies KW of a slab's steps of k with MTW rows of tiles, of which place i is row i RG + part (ROWS) or i
+    constexpr int KW = ROWS ? KS : 1, RG = ROWS ? KS : 1, MTW = (MT + RG - 1) / RG;
+    constexpr int SLAB = 64 * KS;                               // bytes of a row in a slab
     using Operand = typename PanelOperand<T>::Type;
-    constexpr int ROWS8 = BM / 8, CHUNKS = ROWS8 * (KG / 2);    // of A's slab: 8 rows x 64 k each
+    constexpr int ROWS8 = BM / 8, CHUNKS = ROWS8 * (KS / 2);    // of A's slab: 8 rows x 64 k each
     constexpr int LA = CHUNKS / NW, REST = CHUNKS % NW;         // a wavefront's: LA, the first REST wavefronts one more
     extern __shared__ __align__(16) unsigned char lds_raw[];
 
@@ -79,7 +89,7 @@ __global__ __launch_bounds__(64 * CG * KG, 1) void gemm_panel_kernel(const T* __
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, q = lane >> 4;
-    const int cg = wave % CG, kg = wave / CG;
+    const int cg = wave % CG, part = wave / CG;
 
     // this workgroup's share of k, in slabs
     const unsigned row = static_cast<unsigned>(K) * sizeof(T);  // bytes
@@ -105,8 +115,8 @@ __global__ __launch_bounds__(64 * CG * KG, 1) void gemm_panel_kernel(const T* __
 #pragma unroll
     for (int j = 0; j < WNT; ++j) {
         if (BLOCKED) {
-            w_off[j] = (static_cast<unsigned>(cg * WNT + j) * (K / 32) + kg) * 1024u + lane * 16u;
-            w_last[j] = last_at + kg * 64 < row ? w_off[j] : kNowhere;
+            w_off[j] = (static_cast<unsigned>(cg * WNT + j) * (K / 32) + part) * 1024u + lane * 16u;
+            w_last[j] = last_at + part * 64 < row ? w_off[j] : kNowhere;
         } else {
             place_chunk(wave + NW * j, BN / 8, w_off[j], w_last[j]);
         }
@@ -117,7 +127,7 @@ __global__ __launch_bounds__(64 * CG * KG, 1) void gemm_panel_kernel(const T* __
         const unsigned to = lds_origin + stage * S::STAGE;
         if (t < WNT) {
             load_b128_to_lds(w_rsrc, to + S::A_STAGE + (BLOCKED ? wave * WNT + t : wave + NW * t) * 1024,
-                             past ? kNowhere : last ? w_last[t] : w_off[t], s * (BLOCKED ? KG * 1024 : SLAB));
+                             past ? kNowhere : last ? w_last[t] : w_off[t], s * (BLOCKED ? KS * 1024 : SLAB));
         } else if (t < LA + WNT || one_more) {
             const int i = t - WNT;
             load_b128_to_lds(a_rsrc, to + (wave + NW * i) * 1024, past ? kNowhere : last ? a_last[i] : a_off[i], s * SLAB);
@@ -139,9 +149,10 @@ __global__ __launch_bounds__(64 * CG * KG, 1) void gemm_panel_kernel(const T* __
         __builtin_amdgcn_sched_barrier(0);
     };
 
-    f32x4 acc[MT][WNT];
+    auto mine = [&](int i) { return MT % RG == 0 || i < MTW - 1 || i * RG + part < MT; };   // (the same in a whole wavefront)
+    f32x4 acc[MTW][WNT];
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+    for (int i = 0; i < MTW; ++i)
 #pragma unroll
         for (int j = 0; j < WNT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
@@ -150,43 +161,52 @@ __global__ __launch_bounds__(64 * CG * KG, 1) void gemm_panel_kernel(const T* __
         for (int d = 0; d < NS - 1; ++d)
 #pragma unroll
             for (int t = 0; t < LOADS; ++t) ask(s_begin + d, d, t);
-        // this lane's place in an operand of A: chunk 2 g + r / 8 of column kg / 2, row r % 8 of it, piece 4 (kg % 2) + q
-        const unsigned in_chunk = (r & 7) * 128 + ((((kg & 1) * 4 + q) ^ (r & 7)) * 16);
-        const unsigned a_lane = ((kg >> 1) * ROWS8 + (r >> 3)) * 1024 + in_chunk;
-        const unsigned w_lane = S::A_STAGE + (BLOCKED ? wave * (WNT * 1024) + lane * 16
-                                                      : ((kg >> 1) * (BN / 8) + cg * (2 * WNT) + (r >> 3)) * 1024 + in_chunk);
-        auto read_a = [&](int stage, int i) { return *reinterpret_cast<const Operand*>(lds_raw + stage * S::STAGE + a_lane + i * 2048); };
-        auto read_w = [&](int stage, int j) { return *reinterpret_cast<const Operand*>(lds_raw + stage * S::STAGE + w_lane + j * (BLOCKED ? 1024 : 2048)); };
+        // this lane's place in an operand of A: chunk 2 g + r / 8 of column k / 64, row r % 8 of it, piece 4 (k / 32 % 2) + q
+        const unsigned in_chunk = (r >> 3) * 1024 + (r & 7) * 128 + ((((ROWS ? 0 : part & 1) * 4 + q) ^ (r & 7)) * 16);
+        const unsigned a_first = in_chunk + (ROWS ? part * 2048 : (part >> 1) * (ROWS8 * 1024)), a_lane[2] = {a_first, a_first ^ 64};
+        const unsigned w_lane = S::A_STAGE + (BLOCKED ? (ROWS ? cg : wave) * (WNT * 1024) + lane * 16
+                                                      : in_chunk + ((part >> 1) * (BN / 8) + cg * (2 * WNT)) * 1024);
+        auto read_a = [&](int stage, int k, int i) {
+            return *reinterpret_cast<const Operand*>(lds_raw + stage * S::STAGE + a_lane[k & 1] + (k >> 1) * (ROWS8 * 1024) + i * (RG * 2048));
+        };
+        auto read_w = [&](int stage, int k, int j) {
+            return *reinterpret_cast<const Operand*>(lds_raw + stage * S::STAGE + w_lane + k * (CG * WNT * 1024) + j * (BLOCKED ? 1024 : 2048));
+        };
         wait_slabs(std::integral_constant<int, NS - 2>{});
         meet();
         // (read in the order in which a turn reads: the compiler's waits for LDS then hold on both ways into the loop)
-        Operand fa[MT], fw0[WNT], fw1[WNT];
-        auto read_row = [&](int stage, int i, Operand (&into)[WNT]) {
-            fa[i] = read_a(stage, i);
+        Operand fa[KW][MTW], fw0[KW][WNT], fw1[KW][WNT];
+        auto read_row = [&](int stage, int k, int i, Operand (&into)[KW][WNT]) {
+            if (mine(i)) fa[k][i] = read_a(stage, k, i);
 #pragma unroll
             for (int j = 0; j < WNT; ++j)
-                if (j / 2 == i) into[j] = read_w(stage, j);
+                if (j / 2 == i) into[k][j] = read_w(stage, k, j);
         };
 #pragma unroll
-        for (int i = 0; i < MT; ++i) {
-            read_row(0, i, fw0);
-            __builtin_amdgcn_sched_barrier(0);
-        }
+        for (int k = 0; k < KW; ++k)
+#pragma unroll
+            for (int i = 0; i < MTW; ++i) {
+                read_row(0, k, i, fw0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
         int st = 0, before = NS - 1;                            // the ring's places of slabs s and s - 1
-        auto turn = [&](int s, const Operand (&now)[WNT], Operand (&next)[WNT]) {
+        auto turn = [&](int s, const Operand (&now)[KW][WNT], Operand (&next)[KW][WNT]) {
             wait_slabs(std::integral_constant<int, NS - 3>{});  // slab s + 1 has landed ..
             meet();                                             // .. everybody's share of it, and everybody has multiplied slab s - 1
             const int behind = st + 1 == NS ? 0 : st + 1;
 #pragma unroll
-            for (int i = 0; i < MT; ++i) {
+            for (int k = 0; k < KW; ++k)
 #pragma unroll
-                for (int j = 0; j < WNT; ++j) PanelOperand<T>::multiply(now[j], fa[i], acc[i][j]);
-                read_row(behind, i, next);
+                for (int i = 0; i < MTW; ++i) {
+                    if (mine(i))
 #pragma unroll
-                for (int t = 0; t < LOADS; ++t)
-                    if (t * MT / LOADS == i) ask(s + NS - 1, before, t);
-                __builtin_amdgcn_sched_barrier(0);
-            }
+                        for (int j = 0; j < WNT; ++j) PanelOperand<T>::multiply(now[k][j], fa[k][i], acc[i][j]);
+                    read_row(behind, k, i, next);
+#pragma unroll
+                    for (int t = 0; t < LOADS; ++t)
+                        if (t * (KW * MTW) / LOADS == k * MTW + i) ask(s + NS - 1, before, t);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             before = st;
             st = behind;
         };
@@ -199,15 +219,15 @@ __global__ __launch_bounds__(64 * CG * KG, 1) void gemm_panel_kernel(const T* __
     }
     const int nw = n0 + cg * (16 * WNT) + q * 4;                // this lane's four columns of tile j: nw + 16 j ..; its row of tile i: m0 + 16 i + r
     // what the sums are added to is asked for before they join (places past an edge ask for one that exists)
-    constexpr int OWN = (MT + KG - 1) / KG;                     // rows of tiles that a wavefront ends up with: i % KG == kg
+    constexpr int OWN = (MT + KS - 1) / KS;                     // rows of tiles that a wavefront ends up with: those of part, part + KS, ..
     f32x4 had[MODE == kAddF32 ? OWN : 1][WNT];
     if constexpr (MODE == kAddF32) {
 #pragma unroll
         for (int i = 0; i < OWN; ++i)
 #pragma unroll
             for (int j = 0; j < WNT; ++j) {
-                const int m = m0 + (i * KG + kg) * 16 + r, n = nw + j * 16;
-                had[i][j] = *reinterpret_cast<const f32x4*>(static_cast<const float*>(out) + (i * KG + kg < MT && m < M && n < N ? static_cast<size_t>(m) * N + n : 0));
+                const int m = m0 + (i * KS + part) * 16 + r, n = nw + j * 16;
+                had[i][j] = *reinterpret_cast<const f32x4*>(static_cast<const float*>(out) + (i * KS + part < MT && m < M && n < N ? static_cast<size_t>(m) * N + n : 0));
             }
     }
     RowPlace place;
@@ -217,34 +237,39 @@ __global__ __launch_bounds__(64 * CG * KG, 1) void gemm_panel_kernel(const T* __
         place.page = qt.block_table[static_cast<size_t>(qt.seq_idx[mrow]) * qt.max_blocks + place.pos / qt.page];
     }
     wait_vm<0>();
-    // The KG wavefronts of a group of columns share its rows of tiles out and hand each other their parts where the ring was, 16 bytes a lane.
-    f32x4* parts = reinterpret_cast<f32x4*>(lds_raw);
-    auto part_at = [&](int of, int i, int j) { return ((of * CG + cg) * (S::JOIN_ROWS * WNT) + i % S::JOIN_ROWS * WNT + j) * 64 + lane; };
+    if constexpr (!ROWS) {
+        // The KS wavefronts of a group of columns share its rows of tiles out and hand each other their parts where the ring was, 16 bytes a lane.
+        f32x4* parts = reinterpret_cast<f32x4*>(lds_raw);
+        auto part_at = [&](int of, int i, int j) { return ((of * CG + cg) * (S::JOIN_ROWS * WNT) + i % S::JOIN_ROWS * WNT + j) * 64 + lane; };
 #pragma unroll
-    for (int first = 0; first < MT; first += S::JOIN_ROWS) {
-        __syncthreads();                                        // (the ring, or the rows before, have been read)
+        for (int first = 0; first < MT; first += S::JOIN_ROWS) {
+            __syncthreads();                                    // (the ring, or the rows before, have been read)
 #pragma unroll
-        for (int i = first; i < MT && i < first + S::JOIN_ROWS; ++i)
-            if (i % KG != kg)
+            for (int i = first; i < MT && i < first + S::JOIN_ROWS; ++i)
+                if (i % KS != part)
 #pragma unroll
-                for (int j = 0; j < WNT; ++j) parts[part_at(kg, i, j)] = acc[i][j];
-        __syncthreads();
+                    for (int j = 0; j < WNT; ++j) parts[part_at(part, i, j)] = acc[i][j];
+            __syncthreads();
 #pragma unroll
-        for (int i = first; i < MT && i < first + S::JOIN_ROWS; ++i) {
-            if (i % KG != kg) continue;
+            for (int i = first; i < MT && i < first + S::JOIN_ROWS; ++i) {
+                if (i % KS != part) continue;
 #pragma unroll
-            for (int o = 1; o < KG; ++o) {
-                const int of = (kg + o) % KG;
+                for (int o = 1; o < KS; ++o) {
+                    const int of = (part + o) % KS;
 #pragma unroll
-                for (int j = 0; j < WNT; ++j) {
-                    const f32x4 p = parts[part_at(of, i, j)];
-                    acc[i][j][0] += p[0]; acc[i][j][1] += p[1]; acc[i][j][2] += p[2]; acc[i][j][3] += p[3];
+                    for (int j = 0; j < WNT; ++j) {
+                        const f32x4 p = parts[part_at(of, i, j)];
+                        acc[i][j][0] += p[0]; acc[i][j][1] += p[1]; acc[i][j][2] += p[2]; acc[i][j][3] += p[3];
+                    }
                 }
             }
         }
     }
+    // this wavefront's rows of tiles: place i of acc is row tile_of(i) of the tile, if it ends up here
+    auto tile_of = [&](int i) { return ROWS ? i * RG + part : i; };
+    auto ends_here = [&](int i) { return ROWS ? mine(i) : i % KS == part; };
     if constexpr (MODE == kRopeCache) {
-        // the joined tile lies in LDS in 32 bits, with its rows' places, for the epilogue that all kernels share
+        // the tile lies in LDS in 32 bits, with its rows' places, for the epilogue that all kernels share
         constexpr int SS = BN + 4;
         float* stage = reinterpret_cast<float*>(lds_raw);
         int* row_pos = reinterpret_cast<int*>(lds_raw + static_cast<size_t>(BM) * SS * 4);
@@ -255,18 +280,18 @@ __global__ __launch_bounds__(64 * CG * KG, 1) void gemm_panel_kernel(const T* __
             row_page[tid] = place.page;
         }
 #pragma unroll
-        for (int i = 0; i < MT; ++i)
-            if (i % KG == kg)
+        for (int i = 0; i < MTW; ++i)
+            if (ends_here(i))
 #pragma unroll
-                for (int j = 0; j < WNT; ++j) *reinterpret_cast<f32x4*>(stage + (i * 16 + r) * SS + cg * (16 * WNT) + j * 16 + q * 4) = acc[i][j];
+                for (int j = 0; j < WNT; ++j) *reinterpret_cast<f32x4*>(stage + (tile_of(i) * 16 + r) * SS + cg * (16 * WNT) + j * 16 + q * 4) = acc[i][j];
         __syncthreads();
         store_staged<BM, BN, 64 * NW, MODE, false>(stage, row_pos, row_page, out, M, N, m0, n0, tid, qt, 0, gx, static_cast<size_t>(N));
         return;
     }
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
-        const int m = m0 + i * 16 + r;
-        if (i % KG != kg || m >= M) continue;
+    for (int i = 0; i < MTW; ++i) {
+        const int m = m0 + tile_of(i) * 16 + r;
+        if (!ends_here(i) || m >= M) continue;
         if constexpr (is_gated(MODE)) {
             typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
 #pragma unroll
@@ -290,7 +315,7 @@ __global__ __launch_bounds__(64 * CG * KG, 1) void gemm_panel_kernel(const T* __
                 if (n >= N) continue;
                 f32x4 v = acc[i][j];
                 if constexpr (MODE == kAddF32) {
-                    const f32x4 h = had[i / KG][j];
+                    const f32x4 h = had[ROWS ? i : i / KS][j];
                     v[0] += h[0]; v[1] += h[1]; v[2] += h[2]; v[3] += h[3];
                 }
                 *reinterpret_cast<f32x4*>(o + n) = v;
@@ -299,28 +324,28 @@ __global__ __launch_bounds__(64 * CG * KG, 1) void gemm_panel_kernel(const T* __
     }
 }
 
-template <typename T, bool BLOCKED, int MT, int WNT, int CG, int KG, int MODE>
+template <typename T, int MT, int CG, int KS, int MODE>
 static int launch_panel(const T* A, const T* W, void* out, int M, int N, int K, int ksplit, const QkvTarget& qt,
                         const GateExtra& gx, hipStream_t stream) {
-    using S = PanelSizes<MT, WNT, CG, KG>;
+    using S = PanelSizes<T, MT, CG, KS>;
     if constexpr (MODE == kRopeCache && !S::TURNS) {
         return kErrUnsupported;
     } else {
         static OncePerDevice told;
-        const int status = allow_lds(told, reinterpret_cast<const void*>(&gemm_panel_kernel<T, BLOCKED, MT, WNT, CG, KG, MODE>), S::LDS);
+        const int status = allow_lds(told, reinterpret_cast<const void*>(&gemm_panel_kernel<T, MT, CG, KS, MODE>), S::LDS);
         if (status != 0) return status;
         const int tiles_m = (M + S::BM - 1) / S::BM, tiles_n = (N + S::BN - 1) / S::BN;
-        hipLaunchKernelGGL((gemm_panel_kernel<T, BLOCKED, MT, WNT, CG, KG, MODE>), dim3(tiles_m * tiles_n * ksplit), dim3(64 * S::NW), S::LDS, stream, A,
+        hipLaunchKernelGGL((gemm_panel_kernel<T, MT, CG, KS, MODE>), dim3(tiles_m * tiles_n * ksplit), dim3(64 * S::NW), S::LDS, stream, A,
                            W, out, M, N, K, tiles_m, tiles_n, ksplit, qt, gx);
         return launch_status();
     }
 }
 
-template <int MODE, bool BLOCKED, typename T>
+template <int MODE, typename T>
 static int launch_panel_mode(int mt, int bn, const T* A, const T* W, void* out, int M, int N, int K, int ksplit, const QkvTarget& qt,
                              const GateExtra& gx, hipStream_t stream) {
 #define LLME_PANEL(MT, BN) \
-    if (mt == MT && bn == BN) return launch_panel<T, BLOCKED, MT, 2, BN / 32, 256 / BN, MODE>(A, W, out, M, N, K, ksplit, qt, gx, stream);
+    if (mt == MT && bn == BN) return launch_panel<T, MT, BN / 32, 256 / BN, MODE>(A, W, out, M, N, K, ksplit, qt, gx, stream);
     LLME_PANEL(2, 64)
     LLME_PANEL(3, 64)
     LLME_PANEL(4, 64)
@@ -345,11 +370,11 @@ int gemm_panel(int mt, int bn, int mode, const bf16* A, const bf16* W, void* out
     if (M <= 0 || N <= 0 || N % 16 != 0 || K <= 0 || K % 32 != 0 || K >= (1 << 22) || ksplit < 1) return kErrUnsupported;
     if (is_gated(mode) && N % 32 != 0) return kErrUnsupported;
     switch (mode) {
-        case kStoreF32: return launch_panel_mode<kStoreF32, true>(mt, bn, A, W, out, M, N, K, ksplit, qt, gx, stream);
-        case kAddF32: return launch_panel_mode<kAddF32, true>(mt, bn, A, W, out, M, N, K, 1, qt, gx, stream);
-        case kGatedBF16: return launch_panel_mode<kGatedBF16, true>(mt, bn, A, W, out, M, N, K, 1, qt, gx, stream);
-        case kGatedExtraBF16: return launch_panel_mode<kGatedExtraBF16, true>(mt, bn, A, W, out, M, N, K, 1, qt, gx, stream);
-        case kRopeCache: return bn % qt.hd ? kErrUnsupported : launch_panel_mode<kRopeCache, true>(mt, bn, A, W, out, M, N, K, 1, qt, gx, stream);
+        case kStoreF32: return launch_panel_mode<kStoreF32>(mt, bn, A, W, out, M, N, K, ksplit, qt, gx, stream);
+        case kAddF32: return launch_panel_mode<kAddF32>(mt, bn, A, W, out, M, N, K, 1, qt, gx, stream);
+        case kGatedBF16: return launch_panel_mode<kGatedBF16>(mt, bn, A, W, out, M, N, K, 1, qt, gx, stream);
+        case kGatedExtraBF16: return launch_panel_mode<kGatedExtraBF16>(mt, bn, A, W, out, M, N, K, 1, qt, gx, stream);
+        case kRopeCache: return bn % qt.hd ? kErrUnsupported : launch_panel_mode<kRopeCache>(mt, bn, A, W, out, M, N, K, 1, qt, gx, stream);
         default: return kErrUnsupported;
     }
 }
@@ -357,8 +382,8 @@ int gemm_panel(int mt, int bn, int mode, const bf16* A, const bf16* W, void* out
 // 32-bit operands, W row-major; K and N multiples of 4, all pointers 16-byte aligned.
 int gemm_panel_f32(int mt, int bn, int mode, const float* A, const float* W, float* out, int M, int N, int K, int ksplit, hipStream_t stream) {
     if (M <= 0 || N <= 0 || N % 4 != 0 || K <= 0 || K % 4 != 0 || K >= (1 << 22) || ksplit < 1) return kErrUnsupported;
-    if (mode == kAddF32) return launch_panel_mode<kAddF32, false>(mt, bn, A, W, out, M, N, K, 1, QkvTarget{}, GateExtra{}, stream);
-    return launch_panel_mode<kStoreF32, false>(mt, bn, A, W, out, M, N, K, ksplit, QkvTarget{}, GateExtra{}, stream);
+    if (mode == kAddF32) return launch_panel_mode<kAddF32>(mt, bn, A, W, out, M, N, K, 1, QkvTarget{}, GateExtra{}, stream);
+    return launch_panel_mode<kStoreF32>(mt, bn, A, W, out, M, N, K, ksplit, QkvTarget{}, GateExtra{}, stream);
 }
 
 // The tile and the cut over k, by an estimate fitted to 700 timings of 20 to 4,096 rows at the 1B, 3B and 8B sizes (9 % off on

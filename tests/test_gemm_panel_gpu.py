@@ -5,7 +5,7 @@ import torch
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 PANEL = 1000000
-TILES = [(16 * m, 64) for m in (2, 3, 6)] + [(16 * m, 128) for m in (3, 5, 8, 9, 12)]
+TILES = [(16 * m, 64) for m in range(2, 7)] + [(16 * m, 128) for m in range(3, 13)]
 
 
 @pytest.fixture(scope="module")
@@ -30,22 +30,71 @@ def _rel(got, want):
 @pytest.mark.parametrize("rows,cols", TILES)
 def test_panel_tiles(ops, M, N, K, rows, cols):
     """Every tile: stored, added and gated sums against 64 bits (32-bit sums of bfloat16 products: 2e-5 as for the other tiles,
-    5e-3 rounded, 8e-3 behind an activation)."""
+    5e-3 rounded, 8e-3 behind an activation), and the same bits as the tile through registers makes of them."""
     a, w, ref = _pair(M, N, K, 5)
     ad, wb, tile = a.to(DEV), ops.block_weight(w.to(DEV)), PANEL + 1000 * rows + cols
     out = torch.full((M, N), float("nan"), device=DEV)
     ops.gemm_bf16(ad, wb, out, tile=tile)
     assert _rel(out.cpu().double(), ref) < 2e-5
+    other = torch.empty_like(out)
+    ops.gemm_bf16(ad, wb, other, tile=128)
+    assert torch.equal(out, other)
     base = torch.randn(M, N, generator=torch.Generator().manual_seed(6))
-    acc = base.clone().to(DEV)
+    acc, other = base.clone().to(DEV), base.clone().to(DEV)
     ops.gemm_bf16(ad, wb, acc, accumulate=True, tile=tile)
     assert _rel(acc.cpu().double(), ref + base.double()) < 2e-5
-    gated = torch.empty(M, N // 2, dtype=torch.bfloat16, device=DEV)
+    ops.gemm_bf16(ad, wb, other, accumulate=True, tile=128, ksplit=1)
+    assert torch.equal(acc, other)
+    gated, other = (torch.empty(M, N // 2, dtype=torch.bfloat16, device=DEV) for _ in range(2))
     ops.gemm_bf16(ad, wb, gated, gated=True, tile=tile)
+    ops.gemm_bf16(ad, wb, other, gated=True, tile=128)
+    assert torch.equal(gated, other)
     gu = ref.view(M, N // 32, 2, 16)
     gate = gu[:, :, 0]
     want = (gate * torch.sigmoid(gate) * gu[:, :, 1]).reshape(M, N // 2)
     assert _rel(gated.cpu().double(), want) < 8e-3
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 4096, 512), (70, 128, 2048), (150, 16384, 1024), (273, 3072, 2048), (528, 640, 544), (1040, 2048, 1024)])
+def test_the_chosen_tile_adds_in_the_order_of_the_others(ops, M, N, K):
+    """What a product of more than 64 rows stores, adds with a fixed order or gates does not depend on the tile that is chosen for its
+    sizes: the bits of the tile through registers, at sizes on both sides of every rule."""
+    a, w, _ = _pair(M, N, K, 12)
+    ad, wb = a.to(DEV), ops.block_weight(w.to(DEV))
+    for accumulate, gated in ((False, False), (True, False), (False, True)):
+        got, want = (torch.zeros(M, N // 2 if gated else N, dtype=torch.bfloat16 if gated else torch.float32, device=DEV) for _ in range(2))
+        ops.gemm_bf16(ad, wb, got, accumulate, gated=gated, ksplit=1 if accumulate else 0)
+        ops.gemm_bf16(ad, wb, want, accumulate, gated=gated, tile=128, ksplit=1 if accumulate else 0)
+        assert torch.equal(got, want), (accumulate, gated)
+
+
+# the chosen tile at sizes whose k ends inside a slab, with and without biases and a limit
+@pytest.mark.parametrize("T,FF,K,bias,limit", [(70, 256, 544, True, 0.0), (150, 208, 1056, False, 1.5), (273, 2048, 512, True, 2.0)])
+def test_panel_tiles_gate_with_biases_and_clamps(ops, T, FF, K, bias, limit):
+    """The gated epilogue that adds biases and clamps, behind every tile: against 64 bits (5e-3 as for the other tiles), and the bits
+    of the tile through registers."""
+    x, w, ref = _pair(T, 2 * FF, K, 13)
+    both = torch.randn(2 * FF, generator=torch.Generator().manual_seed(14)).to(torch.bfloat16)
+    ref = ref + (both.double() if bias else 0.0)
+    g, u = (ref.view(T, FF // 16, 2, 16)[:, :, i].reshape(T, FF) for i in (0, 1))
+    alpha = 1.702 if limit else 1.0
+    if limit:
+        g, u = g.clamp(max=limit), u.clamp(-limit, limit)
+        assert (g == limit).any() and (u == -limit).any()
+    want = g * torch.sigmoid(alpha * g) * (u + 1 if limit else u)
+    xd, wb, bd = x.to(DEV), ops.block_weight(w.to(DEV)), both.to(DEV) if bias else None
+    mfma = ops.mfma
+
+    def run(tile):
+        out = torch.zeros(T, FF, dtype=torch.bfloat16, device=DEV)
+        mfma.check(mfma.entry("llme_gemm_bf16_gated_extra")(mfma.ptr(xd), mfma.ptr(wb), mfma.ptr(out), T, 2 * FF, K, mfma.ptr(bd) if bias else None,
+                                                            limit, alpha, tile, 1, -1, mfma.stream()), "gemm_gated_extra")
+        return out
+    other, chosen = run(128), torch.zeros(T, FF, dtype=torch.bfloat16, device=DEV)
+    assert _rel(other.cpu().double(), want) < 5e-3
+    assert ops.gemm_gated_extra(xd, wb, chosen, 16, bd, limit, alpha) and torch.equal(chosen, other)
+    for rows, cols in TILES:
+        assert torch.equal(run(PANEL + 1000 * rows + cols), other), (rows, cols)
 
 
 def test_panel_reads_zeros_behind_the_last_row_and_the_end_of_k(ops):
@@ -87,8 +136,8 @@ def test_parts_norm(ops, T, H, n, dtype):
 @pytest.mark.parametrize("hd,n_q,n_kv", [(16, 8, 4), (64, 8, 2), (128, 4, 2)])
 @pytest.mark.parametrize("T", [17, 100, 273])
 def test_panel_tiles_rotate_as_the_others(ops, hd, n_q, n_kv, T):
-    """The rotating epilogue behind every tile that holds whole heads: within bfloat16 rounding of the tile through registers (the
-    sums are joined in another order)."""
+    """The rotating epilogue behind every tile that holds whole heads, and behind the chosen one: the bits of the tile through
+    registers."""
     g, page, K = torch.Generator().manual_seed(10), 16, 544
     x = torch.randn(T, K, generator=g).to(torch.bfloat16).to(DEV)
     w = ops.block_weight((0.05 * torch.randn((n_q + 2 * n_kv) * hd, K, generator=g)).to(torch.bfloat16).to(DEV))
@@ -104,11 +153,9 @@ def test_panel_tiles_rotate_as_the_others(ops, hd, n_q, n_kv, T):
         ops.gemm_qkv_rope(x, w, cos, sin, positions, seq, table, *made, n_q, n_kv, hd, tile=tile)
         return made
     want = run(128)
-    for rows, cols in TILES:
-        if cols % hd:
-            continue
-        for a, b in zip(want, run(PANEL + 1000 * rows + cols)):
-            assert _rel(b.double(), a.double()) < 1e-3, (rows, cols)
+    for tile in [0] + [PANEL + 1000 * rows + cols for rows, cols in TILES if cols % hd == 0]:
+        for a, b in zip(want, run(tile)):
+            assert torch.equal(b, a), tile
 
 
 # pieces of 16 bytes past the end of k, columns that end inside a tile, one row of tiles and several

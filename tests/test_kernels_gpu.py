@@ -1182,7 +1182,8 @@ def test_gemm_qkv_rope_gives_the_same_bits_in_every_tile(ops, hd, K):
     positions, seq_idx = torch.arange(T, dtype=torch.int32, device=DEV), torch.zeros(T, dtype=torch.int32, device=DEV)
     table = torch.randperm(blocks, generator=g).view(1, blocks).to(torch.int32).to(DEV)
     made = []
-    for tile in (128, 96128, 256256) + ((64, 96064, 128064) if hd == 64 else ()):
+    panel = [1000000 + 1000 * rows + cols for rows, cols in ((32, 64), (80, 64), (48, 128), (144, 128)) if cols >= hd]    # (csrc/gemm_panel.hip)
+    for tile in [128, 96128, 256256, 0] + panel + ([64, 96064, 128064] if hd == 64 else []):
         made.append((torch.zeros(T, n_q * hd, dtype=torch.bfloat16, device=DEV),
                      torch.zeros(blocks, n_kv, page, hd, dtype=torch.bfloat16, device=DEV),
                      torch.zeros(blocks, n_kv, hd, page, dtype=torch.bfloat16, device=DEV)))
