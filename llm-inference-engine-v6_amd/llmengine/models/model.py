@@ -149,15 +149,22 @@ class DecoderModel(Part):
             # the embedding's output is read again in front of every pass
             h0 = step.buffer("model.embedded", (T, self.hidden_size), torch.float32)
             self.embedding.forward(step.tokens, h0, step)
+        in_parts = not self.streams and ops.mfma.sums_may_stay_in_parts(step, h)
+        parts = None                    # of the stream, which the block in front left for the next one to add up
         for i, call in enumerate(self.schedule):
             layer = self.layers[call.layer]
             if call.enter:
                 self.pass_input.forward(h, h0, step)
-            if hasattr(layer, "next_block"):
+            hands_on = in_parts and hasattr(layer, "forward_in_parts")
+            if hands_on or hasattr(layer, "next_block"):
                 # (a block that can hand the streams' next read on is told which layer runs behind it in this pass)
                 # (none where the pass's input reads and writes the stream in between)
                 behind = self.schedule[i + 1] if i + 1 < len(self.schedule) else None
-                layer.next_block = self.layers[behind.layer] if behind is not None and not behind.enter else None
+                behind = self.layers[behind.layer] if behind is not None and not behind.enter else None
+                if hands_on:
+                    parts = layer.forward_in_parts(h, step, caches[call.cache_id], call.write_cache, parts, behind)
+                    continue
+                layer.next_block = behind
             layer.forward(h, step, caches[call.cache_id], call.write_cache)
         step.extra.pop("block.normed is for", None)
         step.extra.pop("block.stream_copy is for", None)

@@ -1,7 +1,7 @@
 """The HIP kernels of the engine, as Python functions over device tensors."""
 from .lib import KernelError, KernelLibraryError, library, load_kernels
 from .choices import KernelChoices
-from .kernels import (ATTENTION_MAX_HEAD_DIM, add_product, argmax, argmax_into, attention, attention_generic, attention_project, block_weight, can_block, clear, embed_gather, gemm,
+from .kernels import (ATTENTION_MAX_HEAD_DIM, argmax, argmax_into, attention, attention_generic, attention_project, block_weight, can_block, clear, embed_gather, gemm,
                       gemm_generic, is_blocked, policy, rmsnorm, rope_kv_write, rope_q_only, sample, sample_into, sampling_scratch, swiglu,
                       unblock_weight, weight_shape)
 
@@ -28,4 +28,4 @@ __all__ = ["window", "mlstm", "lightning", "token_input", "sigmoid_decay", "late
            "rotate_write", "short_conv", "sigmoid_attention", "sigmoid_attention_fits", "streams_read_norm", "streams_spread",
            "streams_write", "streams_write_read_norm", "unit_heads", "recurrent", "KernelChoices", "ATTENTION_MAX_HEAD_DIM", "gemm_bf16", "gemm_gated", "gemm_gated_extra", "gemm_squared_relu", "gemm_qkv_rope", "gemm_qkv_rope_supported", "gemv_norm_rope", "gemv_norm_rope_supported", "pair_rows_for_rotation", "gemv_norm", "gemv_norm_supported", "mfma", "KernelError", "KernelLibraryError", "library", "load_kernels", "argmax", "argmax_into", "attention", "attention_generic", "attention_project", "rope_q_only", "embed_gather", "block_weight", "can_block", "clear",
            "is_blocked", "unblock_weight", "weight_shape",
-           "add_product", "gemm", "gemm_generic", "policy", "rmsnorm", "rope_kv_write", "sample", "sample_into", "sampling_scratch", "swiglu"]
+           "gemm", "gemm_generic", "policy", "rmsnorm", "rope_kv_write", "sample", "sample_into", "sampling_scratch", "swiglu"]

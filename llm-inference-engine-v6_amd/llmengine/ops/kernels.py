@@ -194,17 +194,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool =
     gemm_generic(a, w, out, accumulate)
 
 
-_product_in_parts = None            # (set by the matrix-core kernels)
-# A note in a step's `extra`: the address of the stream that the next product may leave its sum for in parts (`mfma.may_leave_parts`).
-SUM_WANTED = "sum.may stay in parts"
-
-
-def add_product(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool, step) -> None:
-    """out (+)= a w^T, as `gemm` makes it; or, where the caller joins them (`mfma.may_leave_parts`) and it is faster, as parts of
-    the sum that are still to be added to `out`."""
-    if accumulate and SUM_WANTED in step.extra and _product_in_parts(a, w, out, step):
-        return
-    gemm(a, w, out, accumulate, step.fixed_order, step.choices)
+_product_in_parts = None            # set by ops/mfma.py
 
 
 # --- attention -----------------------------------------------------------------------
@@ -255,7 +245,7 @@ def attention_project(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
                       w_o: torch.Tensor, out: torch.Tensor, accumulate: bool) -> None:
     """attention (as above, into o) and the output projection behind it: out (+)= o w_o^T. Where a
     step of a few decoded tokens cuts its keys into splits, the splits' join and the projection are
-    one kernel, and o is not written."""
+    one kernel, and o is not written. accumulate may be a mfma.LeftSum."""
     # (only a step of up to 16 decoded tokens is asked about: steps launched kernel by kernel count their calls)
     choices = choices_of(step)
     if (q.shape[0] <= 16 and choices.fast_attention and choices.fast_gemm and _fast_attention_project is not None
@@ -263,9 +253,7 @@ def attention_project(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
                                         w_o, out, accumulate)):
         return
     attention(q, k_cache, v_cache, o, step, block_table, n_q, n_kv, head_dim, scale, window)
-    if accumulate and SUM_WANTED in step.extra:
-        add_product(o, w_o, out, accumulate, step)
-    else:
+    if accumulate is True or _product_in_parts is None or not _product_in_parts(accumulate, o, w_o, out, step):
         gemm(o, w_o, out, accumulate, fixed_order=step.fixed_order, choices=choices)
 
 

@@ -283,38 +283,40 @@ def _launch_parts_norm(h, parts, weight, eps: float, out, T: int, H: int) -> Non
                                    0 if out.dtype == torch.float32 else 1, T, H, float(eps), stream()), "parts_norm")
 
 
-# Notes in a step's `extra`: the address of the stream that the next product may leave its sum for in parts; the parts; whether the
-# step's sums may be left in parts at all (asked once a step: steps with prompt rows are launched kernel by kernel).
-SUM_WANTED, SUM_PARTS, SUMS_MAY = kernels.SUM_WANTED, "sum.parts", "sum.parts allowed"
-
-
 PARTS_MIN_ROWS = {torch.bfloat16: 65, torch.float32: 17}        # (csrc/gemm_panel.hip, llme_gemm_parts_plan)
 
 
 def sums_may_stay_in_parts(step, h: torch.Tensor) -> bool:
     """Whether products of the step that add into h may leave their sums in parts. Not where sums have a fixed order, which
     products of one part keep."""
-    may = step.extra.get(SUMS_MAY)
-    if may is None:
-        T, H = h.shape
-        may = step.extra[SUMS_MAY] = (T >= PARTS_MIN_ROWS.get(step.act_dtype, T + 1) and not step.fixed_order
-                                      and choices_of(step).fast_gemm and H % 4 == 0 and H <= 8192 and h.is_contiguous()
-                                      and not tail_rows(T, choices_of(step)))
-    return may
+    T, H = h.shape
+    return (T >= PARTS_MIN_ROWS.get(step.act_dtype, T + 1) and not step.fixed_order
+            and choices_of(step).fast_gemm and H % 4 == 0 and H <= 8192 and h.is_contiguous()
+            and not tail_rows(T, choices_of(step)))
 
 
-def may_leave_parts(step, h: torch.Tensor, norm) -> None:
-    """The next product that adds into h (`ops.add_product`) may leave its sum in parts, where the step's may: the caller hands them
-    to `norm` (`join_parts`) before anything reads h."""
-    if sums_may_stay_in_parts(step, h):
-        rms = norm.fused_rms()
-        if rms is not None and (rms[0].dtype == torch.float32 or step.act_dtype == torch.bfloat16):
-            step.extra[SUM_WANTED] = h.data_ptr()
+class LeftSum:
+    """What a part may be given as `accumulate`: its last product adds into the stream h, or (`product_in_parts`, where that is
+    faster) leaves its sum in `parts`, which the caller adds to h (`join_parts`). To everything else it means True."""
+    __slots__ = ("h", "parts")
+
+    def __init__(self, h: torch.Tensor):
+        self.h, self.parts = h, None
 
 
-def product_in_parts(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, step) -> bool:
-    """Leaves a w^T in parts for `out` where the caller of the part joins them and it is faster; False: nothing is done."""
-    if step.extra.get(SUM_WANTED) != out.data_ptr():
+def sum_for(norm, h: torch.Tensor, step) -> LeftSum | bool:
+    """The `accumulate` of the sublayer in front of `norm`, which reads h next, in a step whose sums may be left in parts."""
+    rms = norm.fused_rms()
+    return LeftSum(h) if rms is not None and (rms[0].dtype == torch.float32 or step.act_dtype == torch.bfloat16) else True
+
+
+def parts_left(adds: LeftSum | bool) -> torch.Tensor | None:
+    return None if adds is True else adds.parts
+
+
+def product_in_parts(adds: LeftSum | bool, a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, step) -> bool:
+    """Leaves a w^T in adds.parts, where that may be and is faster; False: nothing is done."""
+    if not isinstance(adds, LeftSum) or adds.parts is not None or out.data_ptr() != adds.h.data_ptr() or out.shape != adds.h.shape:
         return False
     M, K = a.shape
     N = out.shape[1]
@@ -324,19 +326,16 @@ def product_in_parts(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, step) 
     n = parts_plan(M, N, K, a.dtype == torch.float32)
     if not n:
         return False
-    del step.extra[SUM_WANTED]
-    parts = step.extra[SUM_PARTS] = step.buffer("sum.parts", (n, M, N), torch.float32)
-    _launch_parts(a, w, parts, M, N, K)
+    adds.parts = step.buffer("sum.parts", (n, M, N), torch.float32)
+    _launch_parts(a, w, adds.parts, M, N, K)
     return True
 
 
 kernels._product_in_parts = product_in_parts
 
 
-def join_parts(h: torch.Tensor, norm, x: torch.Tensor, step) -> None:
-    """x = norm(h), with the parts that a product left for h added to it first."""
-    step.extra.pop(SUM_WANTED, None)
-    parts = step.extra.pop(SUM_PARTS, None)
+def join_parts(h: torch.Tensor, parts: torch.Tensor | None, norm, x: torch.Tensor) -> None:
+    """x = norm(h), with the parts that a product left for h (None: there are none) added to it first."""
     if parts is None:
         norm.forward(h, x)
     else:

@@ -23,6 +23,7 @@ from .registry import register_part
 
 class Attention(Mixer):
     graph_safe = True
+    takes_left_sum = True
 
     def __init__(self, hidden_size: int, num_heads: int, num_kv_heads: int, head_dim: int,
                  position: PositionEncoding | None = None, scale: float | None = None, window: int = 0):
@@ -184,7 +185,7 @@ class Attention(Mixer):
                 if ops.mfma.attention_decode_rope(qkv, cos, sin, k_cache, v_cache, o, step, block_table, n_q, n_kv, hd,
                                                   self.scale, self.window, done):
                     step.extra["attn.qkv_sum zero"] = (held.data_ptr(), held.numel())
-                    if not (accumulate and ops.mfma.SUM_WANTED in step.extra and ops.mfma.product_in_parts(o, self.w_o, out, step)):
+                    if accumulate is True or not ops.mfma.product_in_parts(accumulate, o, self.w_o, out, step):
                         ops.gemm(o, self.w_o, out, accumulate, fixed_order=step.fixed_order, choices=step.choices)
                     return
             ops.rope_kv_write(qkv, cos, sin, step.positions, step.seq_idx, block_table, q, k_cache, v_cache,

@@ -249,6 +249,9 @@ class Mixer(Part):
     # the bytes of the weights of the layer that the mixer stands in, as the model computes with them (set when a model is
     # loaded; None: not known): how long a step of few rows keeps the chip busy with a layer
     layer_bytes: int | None = None
+    # whether `accumulate` may be an ops.mfma.LeftSum: the part then hands it to the product that ends in `out` and does nothing
+    # else with `out` than add to it. Others are given True.
+    takes_left_sum = False
 
     def cache_spec(self) -> CacheSpec | None:
         return None
@@ -279,6 +282,8 @@ class Mixer(Part):
 
 
 class FeedForward(Part):
+    takes_left_sum = False      # as a mixer's
+
     def fuses_norm(self, h: torch.Tensor, norm: "Norm", step) -> bool:
         return False
 

@@ -26,8 +26,6 @@ class PreNormBlock(Block):
                       "ffn_norm": "post_attention_layernorm", "feed_forward": "mlp"}
         if names:
             self.names.update(names)
-        # the block that runs behind this one and reads what it leaves (told by the model as it runs its schedule; None: unknown)
-        self.next_block = None
 
     def children(self):
         n = self.names
@@ -39,10 +37,6 @@ class PreNormBlock(Block):
     def forward(self, h, step, cache, write_cache=True):
         T, H = h.shape
         x = step.buffer("block.normed", (T, H), step.act_dtype)
-        may = step.extra.get(ops.mfma.SUMS_MAY)
-        if ops.mfma.sums_may_stay_in_parts(step, h) if may is None else may:
-            self._forward_in_parts(h, x, step, cache, write_cache)
-            return
         if self.mixer.fuses_norm(h, self.mixer_norm, step):
             self.mixer.forward(h, step, cache, h, True, write_cache, pre_norm=self.mixer_norm)
         else:
@@ -56,29 +50,36 @@ class PreNormBlock(Block):
             self.ffn_norm.forward(h, x)
             self.feed_forward.forward(x, step, h, True)
 
-    def _forward_in_parts(self, h, x, step, cache, write_cache):
-        """The same where a sublayer's last product may leave its sum into h in parts for the norm that reads h next: this block's
-        second, or the first of the block behind, if it is of the same kind and its mixer does not take the norm upon itself."""
+    def forward_in_parts(self, h, step, cache, write_cache, parts, behind):
+        """The same in a step whose sums may be left in parts (ops.mfma.sums_may_stay_in_parts): a sublayer's last product may leave
+        its sum into h in parts for the norm that reads h next, which is this block's second one, or the first one of the block
+        behind, if that is of the same kind and its mixer does not take the norm upon itself. parts: what the block in front left (None: h is
+        whole); returns what this one left for `behind` (None: h is whole)."""
+        x = step.buffer("block.normed", h.shape, step.act_dtype)
+
         def reads_by_norm(part, norm) -> bool:
             return part is not None and not part.fuses_norm(h, norm, step)
         if self.mixer.fuses_norm(h, self.mixer_norm, step):
             self.mixer.forward(h, step, cache, h, True, write_cache, pre_norm=self.mixer_norm)
+            parts = None
         else:
-            ops.mfma.join_parts(h, self.mixer_norm, x, step)
-            if reads_by_norm(self.feed_forward, self.ffn_norm):
-                ops.mfma.may_leave_parts(step, h, self.ffn_norm)
-            self.mixer.forward(x, step, cache, h, True, write_cache)
+            ops.mfma.join_parts(h, parts, self.mixer_norm, x)
+            adds = True
+            if self.mixer.takes_left_sum and reads_by_norm(self.feed_forward, self.ffn_norm):
+                adds = ops.mfma.sum_for(self.ffn_norm, h, step)
+            self.mixer.forward(x, step, cache, h, adds, write_cache)
+            parts = ops.mfma.parts_left(adds)
         if self.feed_forward is None:
-            return
+            return None
         if not reads_by_norm(self.feed_forward, self.ffn_norm):
             self.feed_forward.forward(h, step, h, True, pre_norm=self.ffn_norm)
-            return
-        ops.mfma.join_parts(h, self.ffn_norm, x, step)
-        behind = self.next_block
-        if isinstance(behind, PreNormBlock) and reads_by_norm(behind.mixer, behind.mixer_norm):
-            ops.mfma.may_leave_parts(step, h, behind.mixer_norm)
-        self.feed_forward.forward(x, step, h, True)
-        step.extra.pop(ops.mfma.SUM_WANTED, None)
+            return None
+        ops.mfma.join_parts(h, parts, self.ffn_norm, x)
+        adds = True
+        if self.feed_forward.takes_left_sum and isinstance(behind, PreNormBlock) and reads_by_norm(behind.mixer, behind.mixer_norm):
+            adds = ops.mfma.sum_for(behind.mixer_norm, h, step)
+        self.feed_forward.forward(x, step, h, adds)
+        return ops.mfma.parts_left(adds)
 
 
 class SandwichBlock(Block):

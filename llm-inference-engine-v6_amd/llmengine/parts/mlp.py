@@ -17,6 +17,7 @@ from .registry import register_part
 
 class GatedMLP(FeedForward):
     graph_safe = True
+    takes_left_sum = True
 
     def __init__(self, hidden_size: int, intermediate_size: int, activation: str = "silu", names: dict | None = None,
                  bias: bool = False):
@@ -86,9 +87,7 @@ class GatedMLP(FeedForward):
             ops.gemm_gated(x, self.w_gate_up, act, self.group,
                            lambda shape, dtype: step.buffer("mlp.gate_up", shape, dtype), choices=step.choices,
                            activation=self.activation)
-        if ops.mfma.SUM_WANTED in step.extra:
-            ops.add_product(act, self.w_down, out, accumulate, step)
-        else:
+        if accumulate is True or not ops.mfma.product_in_parts(accumulate, act, self.w_down, out, step):
             ops.gemm(act, self.w_down, out, accumulate, fixed_order=step.fixed_order, choices=step.choices)
         if self.bias:
             ops.window.add_row_bias(out, self.b_down)

@@ -220,3 +220,26 @@ def test_a_step_whose_sums_stay_in_parts(ops, monkeypatch, dtype, tol):
         logits.append(torch.as_tensor(engine.forward_logits(prompt)).double())
         assert len(wanted) == (0 if fixed else 5), wanted            # (o-proj three times, down-proj twice)
     assert _rel(logits[1], logits[0]) < tol
+
+
+def test_a_block_on_its_own_leaves_the_stream_whole(ops):
+    """A program that runs one block of a model itself, after passes of the whole model in which that block handed its last sum on in
+    parts: the stream behind it holds the whole sum, as before the first pass (the two differ by the order of 32-bit sums)."""
+    from llmengine import Engine
+    cfg = {"architectures": ["LlamaForCausalLM"], "model_type": "llama", "hidden_size": 1024, "intermediate_size": 2048, "num_hidden_layers": 2,
+           "num_attention_heads": 16, "num_key_value_heads": 4, "head_dim": 64, "vocab_size": 512, "max_position_embeddings": 1024,
+           "rms_norm_eps": 1e-5, "rope_theta": 10000.0, "tie_word_embeddings": True}
+    engine = Engine.from_random(cfg, 3, "fp32", std=0.05, norm_std=0.05)
+    model, left = engine.model, []
+    whole = model.forward
+
+    def forward(step, caches, rows):
+        h = step.buffer("test.hidden", (step.num_tokens, model.hidden_size), torch.float32)
+        model.embedding.forward(step.tokens, h, step)
+        model.layers[0].forward(h, step, caches[model.schedule[0].cache_id], True)
+        left.append(h.double())
+        return whole(step, caches, rows)
+    model.forward = forward
+    for _ in range(2):
+        engine.forward_logits([(7 * i * i + 3 * i) % 512 for i in range(150)])
+    assert _rel(left[1], left[0]) < 1e-5
