@@ -893,8 +893,12 @@ constexpr int kPanelLeastStored = 16384;
 // in a round (700 rows x 16,384 x 2,048 51.7 against 55.5 here, 1,024 rows 59 / 79, 528 rows 52.7 / 48.4, 2,995 x 2,048 of k = 8,192 140 /
 // 92), tiles of 128 x 128 through registers, two a compute unit and added, 3 us + 0.0187 a k (4,096 x 2,048 x 2,048 41.7 / 50.0, but
 // alone on their compute units 2,048 x 2,048 of k = 8,192 79.4 / 67.2).
-static int choose_direct(int mode, int M, int N, int K, bool may_cut, const PanelPlan& plan, int cus) {
-    if (mode == kAddF32 && may_cut && M <= 288) return panel_plan(M, N, K, 0, 0).ksplit == 1 ? 1 : 0;
+static int choose_direct(int mode, int M, int N, int K, bool may_cut, int cus, PanelPlan& plan) {
+    if (mode == kAddF32 && may_cut && M <= 288) {
+        plan = panel_plan(M, N, K, 0, 0);
+        return plan.ksplit == 1 ? 1 : 0;
+    }
+    plan = panel_plan(M, N, K, 1, 0);
     auto tiles = [&](int edge) { return static_cast<long>((M + edge - 1) / edge) * ((N + edge - 1) / edge); };
     const float large = static_cast<float>((tiles(256) + cus - 1) / cus) * (4.f + 0.0235f * K);
     const float staged = mode == kAddF32 && tiles(128) > cus ? static_cast<float>((tiles(128) + 2 * cus - 1) / (2 * cus)) * (3.f + 0.0187f * K) : large + 1.f;
@@ -985,8 +989,8 @@ extern "C" int llme_gemm_bf16(const void* a, const void* w, void* out, int out_d
         return gemm_panel(bm / 16, bn, mode, A, W, out, M, N, K, 1, QkvTarget{}, t_gate_extra, stream);
     }
     if (tile_shape <= 0 && panel_takes && direct != 0 && ksplit <= 1 && M > 64 && K >= kPanelLeastK && (mode != kStoreF32 || N >= kPanelLeastStored)) {
-        const PanelPlan plan = panel_plan(M, N, K, 1, 0);
-        const int kind = choose_direct(mode, M, N, K, ksplit <= 0, plan, cus);
+        PanelPlan plan;
+        const int kind = choose_direct(mode, M, N, K, ksplit <= 0, cus, plan);
         if (kind == 1) return gemm_panel(plan.mt, plan.bn, mode, A, W, out, M, N, K, 1, QkvTarget{}, t_gate_extra, stream);
         if (kind == 2) return launch_tile_direct<4, 2, 4, 8>(A, W, out, M, N, K, mode, 1, stream);
     }

@@ -394,16 +394,24 @@ int gemm_panel_f32(int mt, int bn, int mode, const float* A, const float* W, flo
 // wide: 32-bit operands, whose products take the time (a compute unit makes 500 a ns).
 // ks_only: the number of parts (0: up to 8, of at least 256 k); heads: tiles hold whole heads of this many columns.
 PanelPlan panel_plan(int M, int N, int K, int ks_only, int heads, bool wide) {
-    // (the last plans made by this thread: a layer's products ask for the same few again and again, and steps with prompt rows wait for
-    // the host; an estimate of all tiles takes it 1.5 us)
+    // The last plans made by this thread, in sets of four that replace their oldest: a layer's products ask for the same few again and
+    // again, and steps with prompt rows wait for the host, which an estimate of all tiles takes 1.5 us, of all cuts too 6. (Sizes of
+    // models are multiples of large powers of two: the set comes from the high bits of products with odd numbers.)
     struct Made {
         int M = 0, N = 0, K = 0, other = 0;
         PanelPlan plan{};
     };
-    static thread_local Made memo[64];
+    struct Set {
+        Made made[4];
+        unsigned oldest = 0;
+    };
+    static thread_local Set memo[16];
     const int other = ks_only * 2048 + heads * 2 + (wide ? 1 : 0);
-    Made& made = memo[(M * 7u + N / 16 * 13u + K / 16 * 5u + other) % 64u];
-    if (made.M == M && made.N == N && made.K == K && made.other == other) return made.plan;
+    unsigned mixed = 0;
+    for (const int v : {M, N, K, other}) mixed = (mixed ^ static_cast<unsigned>(v)) * 2654435761u, mixed ^= mixed >> 15;
+    Set& set = memo[mixed >> 28];
+    for (const Made& m : set.made)
+        if (m.M == M && m.N == N && m.K == K && m.other == other) return m.plan;
     static const int shapes[][2] = {{2, 64}, {3, 64}, {4, 64}, {5, 64}, {6, 64}, {3, 128}, {4, 128}, {5, 128}, {6, 128},
                                     {7, 128}, {8, 128}, {9, 128}, {10, 128}, {11, 128}, {12, 128}};
     const int cus = compute_units();
@@ -425,7 +433,7 @@ PanelPlan panel_plan(int M, int N, int K, int ks_only, int heads, bool wide) {
             if (best.mt == 0 || us < best.us) best = PanelPlan{s[0], bn, ks, static_cast<int>(rounds), us};
         }
     }
-    made = Made{M, N, K, other, best};
+    set.made[set.oldest++ % 4] = Made{M, N, K, other, best};
     return best;
 }
 
