@@ -882,17 +882,21 @@ constexpr int kPanelTile = 1000000;
 // The least k for which they are chosen: a sum of a few slabs never fills their ring, and neither way is much
 // faster (us, tiles through registers / these: 100 x 768 x 288 5.1 / 4.3, 270 x 4,096 x 384 5.7 / 6.3).
 constexpr int kPanelLeastK = 512;
-// The least columns of a stored 32-bit output for which they are: an output head's logits (150 rows x 32,768 x 4,096: 69 / 57 us).
-constexpr int kPanelLeastStored = 16384;
 
 // For a product of more than 64 rows that gemm_panel.hip takes: 1 where its tiles (plan) are the fastest, 2 where those of 256 x 256 are, 0 where the
 // kernels through staging registers are. Up to 64 rows every kernel waits for W, and these, a little faster alone (gate/up of the 1B sizes
 // at 64 rows 16.9 / 16.7 us, of 23 x 16,384 x 3,072 22.9 / 20.4), lost it again in the step (decode of 64 requests 1,656 / 1,679 us, of
 // 23 943 / 941). A sum of up to 288 rows that is better cut over k is, by the kernel below
-// (273 x 2,048 x 2,048 is not: 11.8 / 9.1). Larger ones by estimates: 256 x 256 tiles take 4 us + 0.0235 a k
-// in a round (700 rows x 16,384 x 2,048 51.7 against 55.5 here, 1,024 rows 59 / 79, 528 rows 52.7 / 48.4, 2,995 x 2,048 of k = 8,192 140 /
-// 92), tiles of 128 x 128 through registers, two a compute unit and added, 3 us + 0.0187 a k (4,096 x 2,048 x 2,048 41.7 / 50.0, but
-// alone on their compute units 2,048 x 2,048 of k = 8,192 79.4 / 67.2).
+// (273 x 2,048 x 2,048 is not: 11.5 / 9.0). Everything else by estimates (us, weights from memory; all but sums cut over k give the same bits):
+//  * 256 x 256 tiles take 4 us + 0.0235 a k in a round (gate/up: 700 rows x 16,384 x 2,048 53.3 against 54 to 67 here, 1,024 rows 59.6 / 75, 528 rows
+//    53 / 46.3).
+//  * these take 1.17 (added) or 1.06 (stored) times their plan, which was fitted to all kinds.
+//  * 128 x 128 tiles through registers, two a compute unit, take 3 us + 0.0070 to 0.0187 a k, by how many units have two (against these: added
+//    2,048 x 3,072 x 3,072 52.5 / 57.7, 2,048 x 4,096 x 4,096 78.7 / 85.1, but 1,500 rows 77.9 / 52.7; stored 4,096 x 1,536 x 2,048 33.3 /
+//    37.3, 1,024 x 6,144 x 4,096 62.3 / 66.8, but 1,024 x 5,136 x 2,048 35.5 / 27.5). Stored outputs of very many columns wait for W: 66 rows x
+//    128,256 x 2,048 110 here, 116 through registers, 120 in 256 x 256 tiles; 112 rows 124, 120, 126.
+//  * a sum of more than 288 rows that is cut over k meets in atomics, 1 us a MB (528 x 3,072 x 8,192 in two 48.8 / 51.9; 400 x 4,096 x 14,336 in two
+//    76.8 / 82.4, but 700 x 2,048 x 8,192 47.0 / 38.0).
 static int choose_direct(int mode, int M, int N, int K, bool may_cut, int cus, PanelPlan& plan) {
     if (mode == kAddF32 && may_cut && M <= 288) {
         plan = panel_plan(M, N, K, 0, 0);
@@ -900,9 +904,24 @@ static int choose_direct(int mode, int M, int N, int K, bool may_cut, int cus, P
     }
     plan = panel_plan(M, N, K, 1, 0);
     auto tiles = [&](int edge) { return static_cast<long>((M + edge - 1) / edge) * ((N + edge - 1) / edge); };
-    const float large = static_cast<float>((tiles(256) + cus - 1) / cus) * (4.f + 0.0235f * K);
-    const float staged = mode == kAddF32 && tiles(128) > cus ? static_cast<float>((tiles(128) + 2 * cus - 1) / (2 * cus)) * (3.f + 0.0187f * K) : large + 1.f;
-    if (plan.us <= large && plan.us <= staged) return 1;
+    float large = static_cast<float>((tiles(256) + cus - 1) / cus) * (4.f + 0.0235f * K);
+    if (is_gated(mode)) return plan.us <= large ? 1 : 2;
+    const float here = plan.us * (mode == kAddF32 ? 1.17f : 1.06f);
+    const long t128 = tiles(128), rounds = (t128 + 2 * cus - 1) / (2 * cus);
+    float staged = large + 1.f;
+    if (t128 > cus) staged = rounds * (3.f + (0.0070f + 0.0117f * t128 / (2 * cus * rounds)) * K);
+    if (M <= 128) {                                     // (W's way from memory, as the plan counts it)
+        const float memory = powf(1.2f + 2e-6f * N * K / 5.6f, 2.5f);
+        large = powf(powf(large, 2.5f) + memory, 0.4f);
+        staged = t128 > cus ? powf(powf(staged, 2.5f) + memory, 0.4f) : large + 1.f;
+    }
+    if (mode == kAddF32 && may_cut && K >= 4096 && t128 <= cus) {                       // (cut as the kernels below cut it)
+        long ks = t128 < cus && cus / t128 < 2 ? 2 : cus / t128;
+        ks = ks > 8 ? 8 : ks;
+        ks = ks > K / 512 ? K / 512 : ks;
+        staged = (t128 * ks + cus - 1) / cus * (0.0091f * K / ks) + 4e-6f * M * N * ks - 1.f;
+    }
+    if (here <= large && here <= staged) return 1;
     return large <= staged ? 2 : 0;
 }
 
@@ -988,7 +1007,7 @@ extern "C" int llme_gemm_bf16(const void* a, const void* w, void* out, int out_d
         if (!panel_takes || bm % 16 != 0 || ksplit > 1) return kErrUnsupported;
         return gemm_panel(bm / 16, bn, mode, A, W, out, M, N, K, 1, QkvTarget{}, t_gate_extra, stream);
     }
-    if (tile_shape <= 0 && panel_takes && direct != 0 && ksplit <= 1 && M > 64 && K >= kPanelLeastK && (mode != kStoreF32 || N >= kPanelLeastStored)) {
+    if (tile_shape <= 0 && panel_takes && direct != 0 && ksplit <= 1 && M > 64 && K >= kPanelLeastK) {
         PanelPlan plan;
         const int kind = choose_direct(mode, M, N, K, ksplit <= 0, cus, plan);
         if (kind == 1) return gemm_panel(plan.mt, plan.bn, mode, A, W, out, M, N, K, 1, QkvTarget{}, t_gate_extra, stream);
