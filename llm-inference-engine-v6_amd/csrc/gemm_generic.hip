@@ -271,9 +271,8 @@ static int launch_gemv_generic(const void* a, const void* w, void* out, int M, i
     return launch_status();
 }
 
-// 32-bit operands, more than 16 rows, where the output's columns do not come in fours or it is not aligned (all others go through LDS, as
-// gemm_panel.hip does: gate/up at 149 rows 140 -> 95 us, o-proj and down-proj uncut 69 -> 47): v_mfma_f32_16x16x4_f32, whose products and sums are 32-bit like the vector unit's, at
-// twice the rate of its single multiply-adds (32 against 16 a cycle and scheduler: 157 TFLOP/s). At that rate the operands
+// 32-bit operands, more than 16 rows, where launch_generic does not send them through LDS (gemm_panel.hip):
+// v_mfma_f32_16x16x4_f32, whose products and sums are 32-bit like the vector unit's, at twice the rate of its single multiply-adds (32 against 16 a cycle and scheduler: 157 TFLOP/s). At that rate the operands
 // need no LDS: a lane loads 8 consecutive k of a row (two loads of 16 bytes; the four lanes of a row take 128 bytes together), and step s of eight
 // multiplies element s of every lane, which is k = 8 q + s for lane group q in both operands. A wavefront makes
 // 16 WMT x 16 WNT of the output; KW wavefronts share an output and take every KW-th 32 of k, their sums meeting in LDS in one
@@ -432,9 +431,14 @@ static int launch_generic(const void* a, const void* w, void* out, int M, int N,
     if constexpr (std::is_same_v<TA, float> && std::is_same_v<TW, float> && std::is_same_v<TO, float>) {
         if (!blocked && K % 4 == 0 && reinterpret_cast<uintptr_t>(a) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0) {
             const float *fa = static_cast<const float*>(a), *fw = static_cast<const float*>(w);
-            // Through LDS (gemm_panel.hip) wherever its pieces of four columns fit: operands straight from memory cost four times their
-            // bytes in the loads' path, since the lanes of a quarter lie in four rows.
-            if (N % 4 == 0 && K < (1 << 22) && reinterpret_cast<uintptr_t>(out) % 16 == 0) {
+            // Through LDS (gemm_panel.hip) where its pieces of four columns fit: operands straight from memory cost four times their
+            // bytes in the loads' path, since the lanes of a quarter lie in four rows. Not where 32 x 32 tiles of few columns are one round
+            // over the chip and wait for memory alone: there a ring of slabs only fills and drains. (Measured, us, straight / through LDS:
+            // columns x k 64 x 2,048 at 17 rows 16.4 / 19.9, at 300 20.1 / 20.8; 2,048 x 2,048 at 17 rows 18.1 / 20.6, 97: 19.7 / 21.2,
+            // 200: 28.0 / 21.8; 2,048 x 8,192 at 65 rows 64.6 / 72.8; 2,560 x 2,048 at 97 rows, 320 tiles, 28.1 / 21.2; 3,072 x 2,048 at 32
+            // rows 21.9 / 21.2, 65: 29.7 / 21.8; 6,144 x 4,096 at 32 rows 42.1 / 38.6; 16,384 x 2,048 at 149 rows 137 / 87.)
+            const bool one_round = N < 3072 && static_cast<long>((M + 31) / 32) * ((N + 31) / 32) <= compute_units();
+            if (!one_round && N % 4 == 0 && K < (1 << 22) && reinterpret_cast<uintptr_t>(out) % 16 == 0) {
                 const PanelPlan plan = panel_plan(M, N, K, 1, 0, true);
                 return gemm_panel_f32(plan.mt, plan.bn, accumulate ? kAddF32 : kStoreF32, fa, fw, static_cast<float*>(out), M, N, K, 1, stream);
             }

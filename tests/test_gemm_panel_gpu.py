@@ -159,10 +159,11 @@ def test_panel_tiles_rotate_as_the_others(ops, hd, n_q, n_kv, T):
 
 
 # pieces of 16 bytes past the end of k, columns that end inside a tile, one row of tiles and several
-@pytest.mark.parametrize("M,N,K", [(17, 64, 20), (33, 100, 2052), (81, 48, 64), (149, 272, 288), (300, 2048, 1024)])
+@pytest.mark.parametrize("M,N,K", [(17, 64, 20), (33, 100, 2052), (81, 48, 64), (149, 272, 288), (300, 2048, 1024), (40, 3076, 68), (1100, 300, 100)])
 def test_panel_tiles_of_32_bit_operands(ops, M, N, K):
-    """32-bit operands with a row-major W: stored, added and in parts, against 64 bits (32-bit sums of up to 2,052 products, some
-    eight additions of which are of long partial sums: 1e-6)."""
+    """32-bit operands with a row-major W: stored and added (by the kernel that launch_generic takes for the sizes, of both) and in parts
+    (always the panel), against 64 bits (32-bit sums of up to 2,052 products, some eight additions of which are of long partial
+    sums: 1e-6)."""
     g = torch.Generator().manual_seed(11)
     a, w = torch.randn(M, K, generator=g), 0.05 * torch.randn(N, K, generator=g)
     ref = a.double() @ w.double().T

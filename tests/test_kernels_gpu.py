@@ -1053,10 +1053,11 @@ def test_gemm_qkv_rope_in_wide_tiles(ops, n_q, n_kv, hd, K, new):
 
 
 @pytest.mark.parametrize("M,N,K", [(17, 16, 4), (31, 33, 28), (33, 65, 32), (64, 64, 36), (149, 2048, 260), (149, 331, 1020),
-                                   (300, 1030, 132), (1025, 1500, 64), (249, 16211, 100), (2, 2048, 1028), (1, 70, 4096), (9, 515, 1024), (16, 8200, 96)])
+                                   (300, 1030, 132), (1025, 1500, 64), (1025, 1501, 64), (97, 2048, 260), (249, 16211, 100), (2, 2048, 1028), (1, 70, 4096), (9, 515, 1024), (16, 8200, 96)])
 def test_gemm_in_32_bits(ops, M, N, K):
-    """32-bit products on the matrix cores (more than 16 rows: each of the four tiles, rows, columns and k past the last tile,
-    k of less than a block) and of few rows with k in four, stored and added: against 64 bits within sqrt(K) roundings of the
+    """32-bit products on the matrix cores (more than 16 rows: each of the four tiles of csrc/gemm_generic.hip, and where they are more
+    than one round of aligned columns, tiles of csrc/gemm_panel.hip; rows, columns and k past the last tile, k of less than a
+    block) and of few rows with k in four, stored and added: against 64 bits within sqrt(K) roundings of the
     largest terms (each sum has K of them), and the same bits in every run."""
     a = torch.randn(M, K, generator=_gen(3))
     w = torch.randn(N, K, generator=_gen(4))
