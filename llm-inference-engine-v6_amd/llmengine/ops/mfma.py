@@ -712,18 +712,18 @@ def gemv_norm_supported(h: torch.Tensor, norm_weight: torch.Tensor, w: torch.Ten
 
 
 def _gemv_norm_fits(h, norm_weight, w, rows_out: int, gated: bool) -> bool:
-    K = h.shape[1]
-    if w.dim() not in (2, 5):
+    # (the rows first: steps of more rows, launched kernel by kernel, ask this twice a layer)
+    if not 0 < rows_out <= GEMV_NORM_MAX_ROWS or w.dim() not in (2, 5):
         return False
+    K = h.shape[1]
     n_rows, k_w = kernels.weight_shape(w)
     n_out = n_rows // 2 if gated else n_rows
     if w.dtype == torch.float32:
         return (h.dtype == torch.float32 and w.dim() == 2 and norm_weight.dtype in (torch.float32, torch.bfloat16)
-                and 0 < rows_out <= GEMV_NORM_MAX_ROWS and K % 4 == 0 and k_w == K and (not gated or n_out % 16 == 0)
+                and K % 4 == 0 and k_w == K and (not gated or n_out % 16 == 0)
                 and w.data_ptr() % 16 == 0 and h.data_ptr() % 16 == 0 and norm_weight.data_ptr() % 16 == 0)
     return (h.dtype == torch.float32 and w.dtype == torch.bfloat16
-            and norm_weight.dtype in (torch.float32, torch.bfloat16) and 0 < rows_out <= GEMV_NORM_MAX_ROWS
-            and K % 8 == 0 and 16 * (K + 8) * 2 <= 132 * 1024 and k_w == K
+            and norm_weight.dtype in (torch.float32, torch.bfloat16) and K % 8 == 0 and 16 * (K + 8) * 2 <= 132 * 1024 and k_w == K
             and (not gated or n_out % 16 == 0) and w.data_ptr() % 16 == 0 and h.data_ptr() % 16 == 0
             and norm_weight.data_ptr() % 16 == 0)
 
