@@ -283,16 +283,16 @@ def _launch_parts_norm(h, parts, weight, eps: float, out, T: int, H: int) -> Non
                                    0 if out.dtype == torch.float32 else 1, T, H, float(eps), stream()), "parts_norm")
 
 
-PARTS_MIN_ROWS = {torch.bfloat16: 65, torch.float32: 17}        # (csrc/gemm_panel.hip, llme_gemm_parts_plan)
+# The rows of the steps whose products llme_gemm_parts_plan (csrc/gemm_panel.hip) ever cuts.
+PARTS_MIN_ROWS, PARTS_MAX_ROWS = {torch.bfloat16: 65, torch.float32: 17}, 1024
 
 
 def sums_may_stay_in_parts(step, h: torch.Tensor) -> bool:
     """Whether products of the step that add into h may leave their sums in parts. Not where sums have a fixed order, which
     products of one part keep."""
     T, H = h.shape
-    return (T >= PARTS_MIN_ROWS.get(step.act_dtype, T + 1) and not step.fixed_order
-            and choices_of(step).fast_gemm and H % 4 == 0 and H <= 8192 and h.is_contiguous()
-            and not tail_rows(T, choices_of(step)))
+    return (PARTS_MIN_ROWS.get(step.act_dtype, T + 1) <= T <= PARTS_MAX_ROWS and not step.fixed_order
+            and choices_of(step).fast_gemm and H % 4 == 0 and H <= 8192 and h.is_contiguous())
 
 
 class LeftSum:

@@ -1,6 +1,10 @@
 """The plans of products whose rows are a tile or two high (csrc/gemm_panel.hip), which the host makes: no device."""
 import time
+import types
 
+import torch
+
+from llmengine import ops
 from llmengine.ops import mfma
 
 
@@ -23,3 +27,13 @@ def test_a_models_plans_are_kept_side_by_side():
     for rows in (273, 150):
         step = [(rows, n, k, wide) for n, k in ((3072, 2048), (2048, 2048), (16384, 2048), (2048, 8192)) for wide in (0, 1)]
         assert _seconds(plan, step) < 1.6 * one
+
+
+def test_only_steps_whose_products_are_ever_cut_hand_parts_on():
+    """The rows from which and up to which a step's blocks ask for parts are those for which the plan names any."""
+    sizes = [(2048, 8192), (2048, 2048), (4096, 14336), (256, 8192), (8192, 8192)]
+    for dtype, rows in ((torch.bfloat16, (1, 16, 64, 65, 700, 1024, 1025, 2000, 2048)), (torch.float32, (1, 16, 17, 700, 1024, 1025, 2000))):
+        step = types.SimpleNamespace(act_dtype=dtype, fixed_order=False, choices=ops.KernelChoices())
+        for T in rows:
+            cut = any(mfma.parts_plan(T, N, K, dtype == torch.float32) for N, K in sizes)
+            assert mfma.sums_may_stay_in_parts(step, torch.empty(T, 2048)) == cut, (dtype, T)
