@@ -123,14 +123,16 @@ __global__ __launch_bounds__(64 * CG * KS, 1) void gemm_panel_kernel(const T* __
     }
     const bool one_more = wave < REST;
     auto ask = [&](int s, int stage, int t) {                   // load t of slab s: W's blocks of this wavefront, then A's chunks
+        // (past the share's end nothing is fetched: the offset of no lane is inside, and the scalar one is 0, since a descriptor's end less
+        // a scalar offset that lies behind it, which is what a lane's offset is held against, would wrap around)
         const bool past = s >= s_end, last = s == ns_all - 1;
-        const unsigned to = lds_origin + stage * S::STAGE;
+        const unsigned to = lds_origin + stage * S::STAGE, slab = past ? 0 : s;
         if (t < WNT) {
             load_b128_to_lds(w_rsrc, to + S::A_STAGE + (BLOCKED ? wave * WNT + t : wave + NW * t) * 1024,
-                             past ? kNowhere : last ? w_last[t] : w_off[t], s * (BLOCKED ? KS * 1024 : SLAB));
+                             past ? kNowhere : last ? w_last[t] : w_off[t], slab * (BLOCKED ? KS * 1024 : SLAB));
         } else if (t < LA + WNT || one_more) {
             const int i = t - WNT;
-            load_b128_to_lds(a_rsrc, to + (wave + NW * i) * 1024, past ? kNowhere : last ? a_last[i] : a_off[i], s * SLAB);
+            load_b128_to_lds(a_rsrc, to + (wave + NW * i) * 1024, past ? kNowhere : last ? a_last[i] : a_off[i], slab * SLAB);
         }
     };
     constexpr int LOADS = LA + WNT + (REST > 0 ? 1 : 0);
