@@ -884,9 +884,9 @@ constexpr int kPanelTile = 1000000;
 constexpr int kPanelLeastK = 512;
 
 // For a product of more than 64 rows that gemm_panel.hip takes: 1 where its tiles (plan) are the fastest, 2 where those of 256 x 256 are, 0 where the
-// kernels through staging registers are. Up to 64 rows every kernel waits for W, and these, a little faster alone (gate/up of the 1B sizes
-// at 64 rows 16.9 / 16.7 us, of 23 x 16,384 x 3,072 22.9 / 20.4), lost it again in the step (decode of 64 requests 1,656 / 1,679 us, of
-// 23 943 / 941). A sum of up to 288 rows that is better cut over k is, by the kernel below
+// kernels through staging registers are. Up to 64 rows every kernel waits for W, and these (then with k shared out among their
+// wavefronts), a little faster alone (gate/up of the 1B sizes at 64 rows 16.9 / 16.7 us, of 23 x 16,384 x 3,072 22.9 / 20.4), lost it
+// again in the step (decode of 64 requests 1,656 / 1,679 us, of 23 943 / 941). A sum of up to 288 rows that is better cut over k is, by the kernel below
 // (273 x 2,048 x 2,048 is not: 11.5 / 9.0). Everything else by estimates (us, weights from memory; all but sums cut over k give the same bits):
 //  * 256 x 256 tiles take 4 us + 0.0235 a k in a round (gate/up: 700 rows x 16,384 x 2,048 53.3 against 54 to 67 here, 1,024 rows 59.6 / 75, 528 rows
 //    53 / 46.3).
@@ -1000,6 +1000,8 @@ extern "C" int llme_gemm_bf16(const void* a, const void* w, void* out, int out_d
     // workgroup per compute unit; a small output with a long k is cut over k instead (the
     // parts are added with atomics, so this needs an accumulating float32 output).
     if (gated) mode = gated == 2 ? kGatedReluBF16 : gated == 3 ? kGatedGeluBF16 : gated == 4 ? kGatedExtraBF16 : kGatedBF16;
+    // (gemm_panel.hip has the epilogues of what dense layers and heads make of a blocked weight: the rectified and GELU gates, the squared
+    // rectifier and sums stored in bfloat16 are the kernels' below, as are experts' rows with a scale of their own)
     const bool panel_takes = blocked && K < (1 << 22) && (mode == kStoreF32 || mode == kAddF32 || mode == kGatedBF16 ||
                                                           (mode == kGatedExtraBF16 && t_gate_extra.pair_scale == nullptr));
     if (tile_shape >= kPanelTile) {
@@ -1013,6 +1015,8 @@ extern "C" int llme_gemm_bf16(const void* a, const void* w, void* out, int out_d
         if (kind == 1) return gemm_panel(plan.mt, plan.bn, mode, A, W, out, M, N, K, 1, QkvTarget{}, t_gate_extra, stream);
         if (kind == 2) return launch_tile_direct<4, 2, 4, 8>(A, W, out, M, N, K, mode, 1, stream);
     }
+    // From here on, of more than 64 rows: row-major weights, k of less than kPanelLeastK, what gemm_panel.hip does not take, and what
+    // choose_direct leaves to these tiles. (The figures below that name gated outputs or sums of larger sizes were taken before it did.)
     const bool auto_shape = tile_shape <= 0;
     float tiles_cost = -1.f;                           // of the chosen tile, in the units of the estimate below
     if (tile_shape <= 0) {
@@ -1195,8 +1199,8 @@ extern "C" int llme_gemm_bf16_grouped_gated_extra(const void* a, const void* w, 
 // bfloat16; writes q_out [M, n_q hd] (rotated) and the rows' k (rotated) and v into the pages that
 // block_table[seq_idx[m]] names for positions[m]; cos/sin [max_pos, hd / 2] float32. Full rotation
 // only; hd 16, 32, 64 or 128 (a tile of 128 or 64 columns must hold whole heads). What the separate
-// kernels would store in between, the 32-bit q/k/v rows, never exists. tile_shape 0, 64, 96064, 128064, 96128, 128, or
-// 256256 (hd 64 or 128, blocked w).
+// kernels would store in between, the 32-bit q/k/v rows, never exists. tile_shape 0, 64, 96064, 128064, 96128, 128,
+// 256256 (hd 64 or 128, blocked w), or kPanelTile + 1000 x rows + columns (blocked w). The same bits in every tile.
 extern "C" int llme_gemm_bf16_qkv_rope(const void* a, const void* w, int M, int K, int blocked, const float* cos_t,
                                        const float* sin_t, const int* positions, const int* seq_idx,
                                        const int* block_table, int max_blocks, void* q_out, void* k_cache,
@@ -1222,9 +1226,10 @@ extern "C" int llme_gemm_bf16_qkv_rope(const void* a, const void* w, int M, int 
         return gemm_panel(bm / 16, bn, kRopeCache, A, W, nullptr, M, N, K, 1, qt, GateExtra{}, stream);
     }
     if (tile_shape <= 0 && blocked && K >= kPanelLeastK && K < (1 << 22)) {
-        // The tiles of gemm_panel.hip while they are one round over the chip. (Measured, us, the best of the others / these: 1B sizes at 20 rows
-        // 13.7 / 8.0, 45: 14.6 / 8.7, 273: 14.7 / 9.9, 528: 15.9 / 15.9, 1,024: 23.6 / 19.9, 1,500: 30.5 / 24.8, in two rounds 2,048: 36.2 /
-        // 38.1; 3B sizes at 45 rows 24.1 / 16.8, 1,024: 45.6 / 36.3; 8B sizes at 150 rows 33.2 / 24.4, 528: 44.6 / 34.2, in two 1,024: 66.7 / 67.9.)
+        // The tiles of gemm_panel.hip while they are one round over the chip. (Measured, us, weights from memory, the best of the others /
+        // these: 1B sizes at 20 rows 12.6 / 11.3, 45: 15.1 / 10.7, 273: 14.5 / 11.2, 528: 17.3 / 16.1, 1,024: 25.2 / 21.4, 1,500: 34.0 / 25.4,
+        // in two rounds 2,048: 39.4 / 40.1; 3B sizes at 45 rows 25.7 / 22.3, 1,024: 48.7 / 37.5; 8B sizes at 150 rows 33.2 / 25.0, 528: 44.3 /
+        // 36.4, in two 1,024: 69.9 / 70.1.)
         const PanelPlan plan = panel_plan(M, N, K, 1, hd);
         if (plan.mt > 0 && plan.rounds == 1) return gemm_panel(plan.mt, plan.bn, kRopeCache, A, W, nullptr, M, N, K, 1, qt, GateExtra{}, stream);
     }

@@ -388,8 +388,9 @@ int gemm_panel_f32(int mt, int bn, int mode, const float* A, const float* W, flo
     return launch_panel_mode<kStoreF32>(mt, bn, A, W, out, M, N, K, ksplit, QkvTarget{}, GateExtra{}, stream);
 }
 
-// The tile and the cut over k, by an estimate fitted to 700 timings of 20 to 4,096 rows at the 1B, 3B and 8B sizes (9 % off on
-// average; the chosen tile within 2 % of the best on average): rounds of workgroups over the chip x (3.2 us + 2.9 for the end of a tile
+// The tile and the cut over k, by an estimate fitted to 700 timings of 20 to 4,096 rows at the 1B, 3B and 8B sizes, when these tiles
+// shared out k (9 % off on average). With rows shared out, weights from memory and added sums among them, it is 4 to 13 % short, and the
+// tile that it chooses takes 0.8 % longer than the best on average over 200 sizes, 9 % at worst: rounds of workgroups over the chip x (3.2 us + 2.9 for the end of a tile
 // of 128 x 128, in proportion + the slabs' bytes at 98 a ns, less on a full chip and in large tiles, whose products take the time),
 // joined by their 2.5th powers with W's way from memory (1.2 us + 5.6 TB/s); parts cost their way out and back in the kernel that joins
 // them, 0.3 us a MB.
@@ -446,7 +447,8 @@ using namespace llme;
 // A sum over k that another kernel adds up (llme_parts_norm): how many parts of a [M, K] w [N, K] (bfloat16 and blocked, or wide: 32-bit and row-major) are worth it (0: none, the
 // product adds into its output itself). A product that adds its parts with atomics pays about 1 us a MB for them; up to 64 bfloat16
 // rows that is less than the longer norm costs, and both wait for W (down-proj of the 1B sizes with its weights from memory, us, atomics /
-// parts, and the norm 0.7 longer: 20 rows 10.1 / 10.2, 64 rows 12.1 / 11.3, 96 rows 14.9 / 12.3).
+// parts, and the norm 0.7 to 1.7 longer: 20 rows 10.1 / 10.2, 64 rows 12.1 / 11.3, with rows shared out 70 rows 13.0 / 10.0, 96 rows
+// 14.3 / 10.7).
 extern "C" int llme_gemm_parts_plan(int M, int N, int K, int wide) {
     if (M <= (wide ? 16 : 64) || M > 1024 || N % (wide ? 4 : 16) != 0 || K % (wide ? 4 : 32) != 0 || K >= (1 << 22)) return 0;
     const PanelPlan p = panel_plan(M, N, K, 0, 0, wide != 0);

@@ -131,11 +131,11 @@ __global__ __launch_bounds__(256) void norm_add_vec_kernel(float* __restrict__ y
     }
 }
 
-// A product whose sum over k was left in parts (llme_gemm_bf16_parts) joins the stream in the norm that reads the stream next:
+// A product whose sum over k was left in parts (llme_gemm_parts) joins the stream in the norm that reads the stream next:
 //   h[t] += sum_p parts[p][t];   x[t] = w * h[t] / sqrt(mean(h[t]^2) + eps)
 // The parts are added up in their order, then to h. Bound by the trip to memory: the row of h, the weight and four parts at a time are
-// asked for before anything waits. (273 rows of 2,048 in three parts: 5.0 us, the norm alone 4.1; the atomic sums that this
-// replaces made down-proj 23 us where storing parts makes it 17.)
+// asked for before anything waits. (In a step of 273 rows of 2,048, five parts: 5.5 us, the norm alone 3.8; the atomic sums that
+// this replaces make down-proj 25.7 us where storing parts makes it 18.3.)
 template <typename TW, typename TO, int NV>
 __global__ __launch_bounds__(256) void parts_norm_kernel(float* __restrict__ h, const float* __restrict__ parts, int n, size_t stride,
                                                          const TW* __restrict__ w, TO* __restrict__ x, int H, float eps) {

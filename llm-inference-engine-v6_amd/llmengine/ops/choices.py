@@ -24,6 +24,8 @@ class KernelChoices:
     join_project: bool = True
     # decoding, 17 to 64 tokens with the keys in one split: rotation and cache write inside the attention kernel
     decode_rope: bool = True
+    # (The lines of the next three were drawn with the rotating product in tiles through registers, whose figures they name. Steps
+    # that take it now have those of csrc/gemm_panel.hip, 4 to 9 us a layer less; where the lines would lie with them is not measured.)
     # decoding with heads of 64, the most tokens whose q/k/v product is still cut over k and added into a cleared
     # buffer, so that the attention kernel rotates and writes the cache (without decode_rope: 64, as for every
     # other step). Measured at the 1B sizes and a context of 2,048, ms a step with 64 / 128 here: 65 tokens

@@ -170,8 +170,9 @@ def gemm_qkv_rope(x: torch.Tensor, w_qkv: torch.Tensor, cos: torch.Tensor, sin: 
     x [T, K] bfloat16 (normed), w_qkv [(n_q + 2 n_kv) hd, K] bfloat16 (row-major or blocked); q heads
     and k heads are rotated at the rows' positions, q goes to q_out [T, n_q hd], k and v into the
     rows' pages. The 32-bit q/k/v rows that the separate kernels pass between them never exist.
-    Full rotation, head size 16, 32, 64 or 128. tile: 0 (chosen), 64, 96064, 128064, 96128, 128, or 256256 (heads of 64
-    or 128, w_qkv blocked)."""
+    Full rotation, head size 16, 32, 64 or 128. tile: 0 (chosen), 64, 96064, 128064, 96128, 128, 256256 (heads of 64
+    or 128, w_qkv blocked), or 1000000 + 1000 x rows + columns of a tile of csrc/gemm_panel.hip (w_qkv blocked): the same
+    bits in every one."""
     require(x, "x", torch.bfloat16, (None, None))
     T, K = x.shape
     n_rows, _ = kernels._require_weight(w_qkv, "w_qkv", torch.bfloat16, K)
@@ -230,6 +231,9 @@ kernels._fast_gemm = _fast_gemm
 
 
 # --- sums into the residual stream that the next norm joins ------------------------------
+# Between the two products of a pre-norm block and the norms behind them, where a part says that it takes a LeftSum: attention and
+# the gated feed-forward. Other mixers and feed-forwards add into the stream (with atomics where they are cut over k), and so does the last
+# layer's down-projection, behind which the final norm reads only the wanted rows.
 declare("llme_gemm_parts_plan", [_i, _i, _i, _i])
 declare("llme_gemm_parts", [_vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp])
 declare("llme_parts_norm", [_vp, _vp, _i, _vp, _i, _vp, _i, _i, _i, _f, _vp])
@@ -689,7 +693,7 @@ def qkv_sum_max_rows(decoded_only: bool, head_dim: int, choices: KernelChoices |
     single decoded tokens keeps that way further: with heads of 64 (choices.qkv_sum_rows_decoding) the
     attention kernel then rotates and writes the cache itself (attention_decode_rope); with heads of 128
     (choices.qkv_sum_rows_decoding_128) the rotation kernel does, and the product's tiles of 96 or 128 rows
-    with the rotation in their epilogue are the slower way until then.
+    with the rotation in their epilogue, as they were when the line was drawn, are the slower way until then.
     rotating_layer_bytes: of a step that holds prompt rows and whose product can rotate and write the cache in
     its epilogue, the bytes that the layer reads (None: any other step). Such steps are launched kernel by kernel,
     and with heads of up to 64 and up to choices.launch_bound_layer_bytes the chip is through with a layer before
