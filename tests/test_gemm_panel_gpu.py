@@ -55,13 +55,15 @@ def test_panel_tiles(ops, M, N, K, rows, cols):
     assert _rel(gated.cpu().double(), want) < 8e-3
 
 
-@pytest.mark.parametrize("M,N,K", [(65, 4096, 512), (70, 128, 2048), (150, 16384, 1024), (273, 3072, 2048), (528, 640, 544), (1040, 2048, 1024)])
+@pytest.mark.parametrize("M,N,K", [(65, 4096, 512), (65, 16, 512), (70, 128, 2048), (150, 16384, 1024), (273, 3072, 2048), (528, 640, 544), (1040, 2048, 1024)])
 def test_the_chosen_tile_adds_in_the_order_of_the_others(ops, M, N, K):
     """What a product of more than 64 rows stores, adds with a fixed order or gates does not depend on the tile that is chosen for its
     sizes: the bits of the tile through registers, at sizes on both sides of every rule."""
     a, w, _ = _pair(M, N, K, 12)
     ad, wb = a.to(DEV), ops.block_weight(w.to(DEV))
     for accumulate, gated in ((False, False), (True, False), (False, True)):
+        if gated and N % 32:
+            continue
         got, want = (torch.zeros(M, N // 2 if gated else N, dtype=torch.bfloat16 if gated else torch.float32, device=DEV) for _ in range(2))
         ops.gemm_bf16(ad, wb, got, accumulate, gated=gated, ksplit=1 if accumulate else 0)
         ops.gemm_bf16(ad, wb, want, accumulate, gated=gated, tile=128, ksplit=1 if accumulate else 0)
