@@ -15,7 +15,7 @@ from dataclasses import dataclass
 import torch
 
 from .. import ops
-from ..parts.base import Block, CacheSpec, Head, Norm, Part, TokenEmbedding
+from ..parts.base import Block, CacheSpec, Head, Norm, Part, TokenEmbedding, forward_declares
 
 
 @dataclass(frozen=True)
@@ -155,13 +155,15 @@ class DecoderModel(Part):
             layer = self.layers[call.layer]
             if call.enter:
                 self.pass_input.forward(h, h0, step)
-            hands_on = in_parts and hasattr(layer, "forward_in_parts")
+            hands_on = in_parts and forward_declares(layer, "hands_parts_on")
             if hands_on or hasattr(layer, "next_block"):
                 # (a block that can hand the streams' next read on is told which layer runs behind it in this pass)
                 # (none where the pass's input reads and writes the stream in between)
                 behind = self.schedule[i + 1] if i + 1 < len(self.schedule) else None
                 behind = self.layers[behind.layer] if behind is not None and not behind.enter else None
                 if hands_on:
+                    if behind is not None and not forward_declares(behind, "hands_parts_on"):
+                        behind = None
                     parts = layer.forward_in_parts(h, step, caches[call.cache_id], call.write_cache, parts, behind)
                     continue
                 layer.next_block = behind

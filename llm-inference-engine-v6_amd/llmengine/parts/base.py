@@ -26,6 +26,7 @@ manager made from the mixer's `cache_spec`.
 """
 from __future__ import annotations
 
+import functools
 from dataclasses import dataclass, field
 from typing import Callable, Mapping
 
@@ -48,6 +49,20 @@ def join_name(prefix: str, local: str) -> str:
     """The full name of a part's tensor: the part's prefix (which ends in a dot) and the local
     name; a part whose only tensor carries the part's own name calls it ""."""
     return prefix + local if local else prefix.rstrip(".")
+
+
+@functools.lru_cache(maxsize=256)
+def _forward_declares(cls: type, flag: str) -> bool:
+    for c in cls.__mro__:
+        if "forward" in vars(c):
+            return bool(vars(c).get(flag, False))
+    return False
+
+
+def forward_declares(part, flag: str) -> bool:
+    """Whether the class whose `forward` the part runs says `flag` of it. A class that overrides `forward` speaks for its own, and
+    nobody does for a part whose `forward` was replaced."""
+    return "forward" not in getattr(part, "__dict__", ()) and _forward_declares(type(part), flag)
 
 
 @dataclass(frozen=True)
@@ -249,8 +264,8 @@ class Mixer(Part):
     # the bytes of the weights of the layer that the mixer stands in, as the model computes with them (set when a model is
     # loaded; None: not known): how long a step of few rows keeps the chip busy with a layer
     layer_bytes: int | None = None
-    # whether `accumulate` may be an ops.mfma.LeftSum: the part then hands it to the product that ends in `out` and does nothing
-    # else with `out` than add to it. Others are given True.
+    # whether `accumulate` of this class's `forward` may be an ops.mfma.LeftSum: it then hands it to the product that ends in `out`
+    # and does nothing else with `out` than add to it (asked by forward_declares). Others are given True.
     takes_left_sum = False
 
     def cache_spec(self) -> CacheSpec | None:
@@ -299,6 +314,8 @@ class FeedForward(Part):
 
 class Block(Part):
     mixer: Mixer
+    # whether a pass of the model may run `forward_in_parts` in the place of this class's `forward` (asked by forward_declares)
+    hands_parts_on = False
 
     def forward(self, h: torch.Tensor, step, cache: LayerCache | None, write_cache: bool = True) -> None:
         raise NotImplementedError

@@ -9,13 +9,14 @@ from __future__ import annotations
 import torch
 
 from .. import ops
-from .base import Block, FeedForward, Mixer, Norm, ParamSpec
+from .base import Block, FeedForward, Mixer, Norm, ParamSpec, forward_declares
 from .registry import register_part
 from .token_input import TokenInput
 
 
 class PreNormBlock(Block):
     graph_safe = True
+    hands_parts_on = True
 
     def __init__(self, mixer: Mixer, feed_forward: FeedForward | None, mixer_norm: Norm, ffn_norm: Norm | None,
                  names: dict | None = None):
@@ -53,8 +54,8 @@ class PreNormBlock(Block):
     def forward_in_parts(self, h, step, cache, write_cache, parts, behind):
         """The same in a step whose sums may be left in parts (ops.mfma.sums_may_stay_in_parts): a sublayer's last product may leave
         its sum into h in parts for the norm that reads h next, which is this block's second one, or the first one of the block
-        behind, if that is of the same kind and its mixer does not take the norm upon itself. parts: what the block in front left (None: h is
-        whole); returns what this one left for `behind` (None: h is whole)."""
+        behind, if its mixer does not take the norm upon itself. parts: what the block in front left (None: h is whole); behind: the
+        block that runs next, if it can be handed parts (None: it cannot); returns what is left for it (None: h is whole)."""
         x = step.buffer("block.normed", h.shape, step.act_dtype)
 
         def reads_by_norm(part, norm) -> bool:
@@ -65,7 +66,7 @@ class PreNormBlock(Block):
         else:
             ops.mfma.join_parts(h, parts, self.mixer_norm, x)
             adds = True
-            if self.mixer.takes_left_sum and reads_by_norm(self.feed_forward, self.ffn_norm):
+            if forward_declares(self.mixer, "takes_left_sum") and reads_by_norm(self.feed_forward, self.ffn_norm):
                 adds = ops.mfma.sum_for(self.ffn_norm, h, step)
             self.mixer.forward(x, step, cache, h, adds, write_cache)
             parts = ops.mfma.parts_left(adds)
@@ -76,7 +77,7 @@ class PreNormBlock(Block):
             return None
         ops.mfma.join_parts(h, parts, self.ffn_norm, x)
         adds = True
-        if self.feed_forward.takes_left_sum and isinstance(behind, PreNormBlock) and reads_by_norm(behind.mixer, behind.mixer_norm):
+        if behind is not None and forward_declares(self.feed_forward, "takes_left_sum") and reads_by_norm(behind.mixer, behind.mixer_norm):
             adds = ops.mfma.sum_for(behind.mixer_norm, h, step)
         self.feed_forward.forward(x, step, h, adds)
         return ops.mfma.parts_left(adds)

@@ -246,3 +246,33 @@ def test_a_block_on_its_own_leaves_the_stream_whole(ops):
     for _ in range(2):
         engine.forward_logits([(7 * i * i + 3 * i) % 512 for i in range(150)])
     assert _rel(left[1], left[0]) < 1e-5
+
+
+def test_parts_and_blocks_whose_forward_was_replaced_see_the_whole_stream(ops):
+    """A block and a mixer whose `forward` a program has replaced (to look at what they make) run as they were given, with a whole stream
+    in front of and behind them, in a step whose other sums stay in parts."""
+    from llmengine import Engine
+    cfg = {"architectures": ["LlamaForCausalLM"], "model_type": "llama", "hidden_size": 1024, "intermediate_size": 2048, "num_hidden_layers": 4,
+           "num_attention_heads": 16, "num_key_value_heads": 4, "head_dim": 64, "vocab_size": 512, "max_position_embeddings": 1024,
+           "rms_norm_eps": 1e-5, "rope_theta": 10000.0, "tie_word_embeddings": True}
+    prompt, seen, logits = [(7 * i * i + 3 * i) % 512 for i in range(150)], [], []
+    for fixed in (True, False):
+        engine = Engine.from_random(cfg, 3, "fp32", std=0.05, norm_std=0.05, deterministic=fixed)
+        block, mixer = engine.model.layers[1], engine.model.layers[2].mixer
+        block_forward, mixer_forward, states = block.forward, mixer.forward, []
+
+        def watched_block(h, *args):
+            states.append(h.double())
+            block_forward(h, *args)
+            states.append(h.double())
+
+        def watched_mixer(x, step, cache, out, accumulate, *args):
+            mixer_forward(x, step, cache, out, accumulate, *args)
+            states.append(out.double())
+        block.forward, mixer.forward = watched_block, watched_mixer
+        logits.append(torch.as_tensor(engine.forward_logits(prompt)).double())
+        seen.append(states)
+    assert len(seen[0]) == len(seen[1]) == 3
+    for whole, got in zip(*seen):
+        assert _rel(got, whole) < 1e-5
+    assert _rel(logits[1], logits[0]) < 1e-5
