@@ -296,7 +296,8 @@ def sums_may_stay_in_parts(step, h: torch.Tensor) -> bool:
     products of one part keep."""
     T, H = h.shape
     return (PARTS_MIN_ROWS.get(step.act_dtype, T + 1) <= T <= PARTS_MAX_ROWS and not step.fixed_order
-            and choices_of(step).fast_gemm and H % 4 == 0 and H <= 8192 and h.is_contiguous())
+            and choices_of(step).fast_gemm and H % 4 == 0 and H <= 8192 and h.is_contiguous() and h.dtype == torch.float32
+            and h.data_ptr() % 16 == 0)
 
 
 class LeftSum:
@@ -311,7 +312,13 @@ class LeftSum:
 def sum_for(norm, h: torch.Tensor, step) -> LeftSum | bool:
     """The `accumulate` of the sublayer in front of `norm`, which reads h next, in a step whose sums may be left in parts."""
     rms = norm.fused_rms()
-    return LeftSum(h) if rms is not None and (rms[0].dtype == torch.float32 or step.act_dtype == torch.bfloat16) else True
+    if rms is None:
+        return True
+    w = rms[0]
+    if ((w.dtype == torch.float32 or w.dtype == torch.bfloat16 == step.act_dtype) and w.dim() == 1 and w.numel() == h.shape[1]
+            and w.is_contiguous() and w.data_ptr() % 16 == 0 and w.is_cuda == h.is_cuda):
+        return LeftSum(h)
+    return True             # (what the norm alone would take unaligned, or refuse, it is given alone)
 
 
 def parts_left(adds: LeftSum | bool) -> torch.Tensor | None:
@@ -320,12 +327,14 @@ def parts_left(adds: LeftSum | bool) -> torch.Tensor | None:
 
 def product_in_parts(adds: LeftSum | bool, a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, step) -> bool:
     """Leaves a w^T in adds.parts, where that may be and is faster; False: nothing is done."""
-    if not isinstance(adds, LeftSum) or adds.parts is not None or out.data_ptr() != adds.h.data_ptr() or out.shape != adds.h.shape:
+    # (into the very tensor whose sum it is, which sums_may_stay_in_parts has looked at: no view of it, none of its rows)
+    if not isinstance(adds, LeftSum) or adds.parts is not None or out is not adds.h:
         return False
-    M, K = a.shape
-    N = out.shape[1]
+    M, N = out.shape
+    K = a.shape[1]
     # (what these operands would be refused for, `gemm` says)
-    if not _parts_fit(a, w) or not a.is_contiguous() or kernels.weight_shape(w) != (N, K) or tuple(out.shape) != (M, N):
+    if (not _parts_fit(a, w) or not a.is_contiguous() or not w.is_contiguous() or kernels.weight_shape(w) != (N, K)
+            or a.shape[0] != M or not a.is_cuda == w.is_cuda == out.is_cuda):
         return False
     n = parts_plan(M, N, K, a.dtype == torch.float32)
     if not n:

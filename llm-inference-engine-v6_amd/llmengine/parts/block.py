@@ -57,27 +57,25 @@ class PreNormBlock(Block):
         behind, if its mixer does not take the norm upon itself. parts: what the block in front left (None: h is whole); behind: the
         block that runs next, if it can be handed parts (None: it cannot); returns what is left for it (None: h is whole)."""
         x = step.buffer("block.normed", h.shape, step.act_dtype)
-
-        def reads_by_norm(part, norm) -> bool:
-            return part is not None and not part.fuses_norm(h, norm, step)
-        if self.mixer.fuses_norm(h, self.mixer_norm, step):
+        ffn_reads = self.feed_forward is not None and not self.feed_forward.fuses_norm(h, self.ffn_norm, step)
+        if parts is None and self.mixer.fuses_norm(h, self.mixer_norm, step):
             self.mixer.forward(h, step, cache, h, True, write_cache, pre_norm=self.mixer_norm)
-            parts = None
         else:
             ops.mfma.join_parts(h, parts, self.mixer_norm, x)
             adds = True
-            if forward_declares(self.mixer, "takes_left_sum") and reads_by_norm(self.feed_forward, self.ffn_norm):
+            if ffn_reads and forward_declares(self.mixer, "takes_left_sum"):
                 adds = ops.mfma.sum_for(self.ffn_norm, h, step)
             self.mixer.forward(x, step, cache, h, adds, write_cache)
             parts = ops.mfma.parts_left(adds)
         if self.feed_forward is None:
             return None
-        if not reads_by_norm(self.feed_forward, self.ffn_norm):
+        if not ffn_reads:
             self.feed_forward.forward(h, step, h, True, pre_norm=self.ffn_norm)
             return None
         ops.mfma.join_parts(h, parts, self.ffn_norm, x)
         adds = True
-        if behind is not None and forward_declares(self.feed_forward, "takes_left_sum") and reads_by_norm(behind.mixer, behind.mixer_norm):
+        if (behind is not None and forward_declares(self.feed_forward, "takes_left_sum")
+                and not behind.mixer.fuses_norm(h, behind.mixer_norm, step)):
             adds = ops.mfma.sum_for(behind.mixer_norm, h, step)
         self.feed_forward.forward(x, step, h, adds)
         return ops.mfma.parts_left(adds)

@@ -2,6 +2,7 @@
 import time
 import types
 
+import pytest
 import torch
 
 from llmengine import ops
@@ -37,3 +38,27 @@ def test_only_steps_whose_products_are_ever_cut_hand_parts_on():
         for T in rows:
             cut = any(mfma.parts_plan(T, N, K, dtype == torch.float32) for N, K in sizes)
             assert mfma.sums_may_stay_in_parts(step, torch.empty(T, 2048)) == cut, (dtype, T)
+
+
+def test_what_a_norm_cannot_join_is_not_left_in_parts():
+    """A norm's weight that the joining kernel does not take (unaligned, strided, of another type) and operands that a product refuses:
+    the sublayer adds into the stream itself, and says what it refuses itself."""
+    h = torch.zeros(100, 256)
+    step = types.SimpleNamespace(act_dtype=torch.bfloat16, fixed_order=False, choices=ops.KernelChoices(),
+                                 buffer=lambda *a: pytest.fail("parts were asked for"))
+
+    def adds(weight):
+        return mfma.sum_for(types.SimpleNamespace(fused_rms=lambda: weight if weight is None else (weight, 1e-5)), h, step)
+    whole = torch.ones(257)
+    assert isinstance(adds(torch.ones(256)), mfma.LeftSum) and isinstance(adds(torch.ones(256, dtype=torch.bfloat16)), mfma.LeftSum)
+    for weight in (None, whole[1:], torch.ones(512)[::2], whole, torch.ones(256, dtype=torch.float16), torch.ones(1, 256)):
+        assert adds(weight) is True
+    step.act_dtype = torch.float32
+    assert adds(torch.ones(256, dtype=torch.bfloat16)) is True
+    a, w = torch.zeros(100, 8192), torch.zeros(256, 8192)
+    assert mfma.parts_plan(100, 256, 8192, True) > 1
+    left = adds(torch.ones(256))
+    for bad_a, bad_w, out in ((a, torch.zeros(8192, 256).T, h), (torch.zeros(8192, 100).T, w, h), (a, w.to(torch.bfloat16), h), (a[:, :4096], w, h),
+                              (a, w, torch.zeros(100, 256)), (a[:50], w, h[:50]), (a, w, h[:])):
+        assert not mfma.product_in_parts(left, bad_a, bad_w, out, step) and left.parts is None
+    assert not mfma.product_in_parts(True, a, w, h, step) and not mfma.product_in_parts(False, a, w, h, step)
