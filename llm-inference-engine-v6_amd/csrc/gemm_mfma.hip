@@ -902,7 +902,7 @@ static int choose_direct(int mode, int M, int N, int K, bool may_cut, int cus, P
         plan = panel_plan(M, N, K, 0, 0);
         return plan.ksplit == 1 ? 1 : 0;
     }
-    plan = panel_plan(M, N, K, 1, 0);
+    plan = panel_plan(M, N, K, 1, 0, false, is_gated(mode));
     auto tiles = [&](int edge) { return static_cast<long>((M + edge - 1) / edge) * ((N + edge - 1) / edge); };
     float large = static_cast<float>((tiles(256) + cus - 1) / cus) * (4.f + 0.0235f * K);
     if (is_gated(mode)) return plan.us <= large ? 1 : 2;
@@ -1228,7 +1228,7 @@ extern "C" int llme_gemm_bf16_qkv_rope(const void* a, const void* w, int M, int 
     if (tile_shape <= 0 && blocked && K >= kPanelLeastK && K < (1 << 22)) {
         // The tiles of gemm_panel.hip while they are one round over the chip. (Measured, us, weights from memory, the best of the others /
         // these: 1B sizes at 20 rows 12.6 / 11.3, 45: 15.1 / 10.7, 273: 14.5 / 11.2, 528: 17.3 / 16.1, 1,024: 25.2 / 21.4, 1,500: 34.0 / 25.4,
-        // in two rounds 2,048: 39.4 / 40.1; 3B sizes at 45 rows 25.7 / 22.3, 1,024: 48.7 / 37.5; 8B sizes at 150 rows 33.2 / 25.0, 528: 44.3 /
+        // 2,048 in tiles of 128 x 192: 37.6 / 28.6; 3B sizes at 45 rows 25.7 / 22.3, 1,024: 48.7 / 37.5; 8B sizes at 150 rows 33.2 / 25.0, 528: 44.3 /
         // 36.4, in two 1,024: 69.9 / 70.1.)
         const PanelPlan plan = panel_plan(M, N, K, 1, hd);
         if (plan.mt > 0 && plan.rounds == 1) return gemm_panel(plan.mt, plan.bn, kRopeCache, A, W, nullptr, M, N, K, 1, qt, GateExtra{}, stream);

@@ -3,9 +3,9 @@
 // Between the kernels that stream W for up to 16 rows and the tiles of 256 x 256 for prompts lie products whose rows are one or two
 // tiles high, and outputs of few columns. Tiles through staging registers (gemm_tile_kernel) read 2.6 times the bytes there that
 // they must (273 rows x 16,384 columns in tiles of 96 x 64: 503 MB over the chip), and a compute unit gets 55 to 90 bytes a ns.
-// So the tile takes its height from the rows (BM = 16 MT, up to 192) x BN = 64 or 128 columns, one workgroup of eight wavefronts a
-// compute unit, with as many bytes on their way as LDS holds:
-//  * BN / 32 wavefronts share out the columns (32 each). bfloat16: the KS = 256 / BN wavefronts of a group of columns share out its rows of
+// So the tile takes its height from the rows (BM = 16 MT, up to 192) x BN = 64 or 128 columns (bfloat16: 192 and 256 too), one workgroup of
+// eight wavefronts a compute unit, with as many bytes on their way as LDS holds:
+//  * BN / 32 wavefronts share out the columns (32 each; of a tile of 192 or 256 four wavefronts 48 or 64 each). bfloat16: the KS = 256 / BN wavefronts of a group of columns share out its rows of
 //    tiles, and each adds up all of k in turn, so that a sum has the one order that every other tile kernel gives it: whichever tile
 //    a product's rows are given, its results are the same bits. (Sharing out k instead, with the parts joined through LDS at
 //    the end, reads a fifth less of LDS and was no faster: parts of the 1B o-proj at 273 rows 8.2 / 8.0 us, of its down-proj 17.6 / 16.5,
@@ -30,17 +30,17 @@ namespace llme {
 
 // CG x KS wavefronts; a slab is KS steps of 64 bytes of k. bfloat16: W in blocks, the wavefronts of a column group share out the rows (ROWS).
 // 32-bit: W row-major, its chunks loaded and read as A's, and they share out the steps of k.
-template <typename T, int MT, int CG, int KS>
+template <typename T, int MT, int CG, int KS, int WT = 2, bool HALF = false>
 struct PanelSizes {
     static constexpr bool BLOCKED = sizeof(T) == 2, ROWS = BLOCKED;
-    static constexpr int WNT = 2;                               // tiles of 16 columns a wavefront
-    static constexpr int NW = CG * KS, BM = 16 * MT, BN = 16 * WNT * CG, SK = 32 * KS;
-    static constexpr int A_STAGE = BM * SK * 2, W_STAGE = WNT * NW * 1024, STAGE = A_STAGE + W_STAGE;
+    static constexpr int WNT = WT;                              // tiles of 16 columns a wavefront (HALF: slabs of 32 k)
+    static constexpr int NW = CG * KS, BM = 16 * MT, BN = 16 * WNT * CG, SK = HALF ? 32 : 32 * KS;
+    static constexpr int A_STAGE = BM * SK * 2, W_STAGE = BN * SK * 2, STAGE = A_STAGE + W_STAGE;
     static constexpr int NS_MOST = 160 * 1024 / STAGE, NS = NS_MOST > 6 ? 6 : NS_MOST;
     static constexpr int JOIN_MOST = 160 / (NW * WNT), JOIN_ROWS = MT < JOIN_MOST ? MT : JOIN_MOST;   // rows of tiles that join at a time
     static constexpr int JOIN = ROWS ? 0 : NW * JOIN_ROWS * WNT * 1024, TURNED = BM * (BN + 4) * 4 + BM * 8;
     static constexpr int LDS = NS * STAGE > JOIN ? NS * STAGE : JOIN;
-    static constexpr bool TURNS = TURNED <= LDS;                // the rotating epilogue's tile and its rows' places fit
+    static constexpr bool TURNS = TURNED <= 160 * 1024;         // the rotating epilogue's tile and its rows' places fit
     static_assert(NS >= 3 && LDS <= 160 * 1024, "LDS");
 };
 
@@ -61,19 +61,20 @@ template <> struct PanelOperand<float> {
     }
 };
 
-template <typename T, int MT, int CG, int KS, int MODE>
+template <typename T, int MT, int CG, int KS, int WT, bool HALF, int MODE>
 __global__ __launch_bounds__(64 * CG * KS, 1) void gemm_panel_kernel(const T* __restrict__ a, const T* __restrict__ w,
                                                             void* __restrict__ out, int M, int N, int K, int tiles_m, int tiles_n,
                                                             int ksplit, QkvTarget qt, GateExtra gx) {
-    using S = PanelSizes<T, MT, CG, KS>;
+    using S = PanelSizes<T, MT, CG, KS, WT, HALF>;
     constexpr int NW = S::NW, WNT = S::WNT, BM = S::BM, BN = S::BN, NS = S::NS;
     constexpr bool BLOCKED = S::BLOCKED, ROWS = S::ROWS;
     // a wavefront multiplies KW of a slab's steps of k with MTW rows of tiles, of which place i is row i RG + part (ROWS) or i
-    constexpr int KW = ROWS ? KS : 1, RG = ROWS ? KS : 1, MTW = (MT + RG - 1) / RG;
-    constexpr int SLAB = 64 * KS;                               // bytes of a row in a slab
+    constexpr int KW = ROWS && !HALF ? KS : 1, RG = ROWS ? KS : 1, MTW = (MT + RG - 1) / RG;
+    constexpr int SLAB = HALF ? 64 : 64 * KS;                   // bytes of a row in a slab
     using Operand = typename PanelOperand<T>::Type;
     constexpr int ROWS8 = BM / 8, CHUNKS = ROWS8 * (KS / 2);    // of A's slab: 8 rows x 64 k each
-    constexpr int LA = CHUNKS / NW, REST = CHUNKS % NW;         // a wavefront's: LA, the first REST wavefronts one more
+    constexpr int JOBS = HALF ? MT + BN / 16 : CHUNKS;          // (a slab of 32 k: all its loads in one row, A's chunks of 16 rows x 32 k first)
+    constexpr int LA = JOBS / NW, REST = JOBS % NW, LW = HALF ? 0 : WNT;  // a wavefront's: LA, the first REST wavefronts one more
     extern __shared__ __align__(16) unsigned char lds_raw[];
 
     // A die gets consecutive tiles, rows fastest (up to 8 tiles of them), so that tiles which read the same W share its L2.
@@ -121,13 +122,29 @@ __global__ __launch_bounds__(64 * CG * KS, 1) void gemm_panel_kernel(const T* __
             place_chunk(wave + NW * j, BN / 8, w_off[j], w_last[j]);
         }
     }
+    u32x4 job_rsrc[LA + 1];                                     // HALF: where job wave + NW t reads, and how far a slab is
+    unsigned job_step[LA + 1];
+    if constexpr (HALF) {
+#pragma unroll
+        for (int t = 0; t <= LA; ++t) {
+            const int j = wave + NW * t;
+            const bool of_a = j < MT;
+            job_rsrc[t] = of_a ? a_rsrc : w_rsrc;
+            job_step[t] = of_a ? SLAB : 1024;
+            // A's chunk j: rows 16 j .., lane 4 r + p: row r, piece p ^ (r / 4's place in 0 2 3 1) of its 64 bytes
+            a_off[t] = of_a ? (j * 16 + (lane >> 2)) * row + (((lane & 3) ^ ((0x78 >> (lane >> 4) * 2) & 3)) * 16)
+                            : static_cast<unsigned>(j - MT) * (K / 32) * 1024u + lane * 16u;
+        }
+    }
     const bool one_more = wave < REST;
     auto ask = [&](int s, int stage, int t) {                   // load t of slab s: W's blocks of this wavefront, then A's chunks
         // (past the share's end nothing is fetched: the offset of no lane is inside, and the scalar one is 0, since a descriptor's end less
         // a scalar offset that lies behind it, which is what a lane's offset is held against, would wrap around)
         const bool past = s >= s_end, last = s == ns_all - 1;
         const unsigned to = lds_origin + stage * S::STAGE, slab = past ? 0 : s;
-        if (t < WNT) {
+        if constexpr (HALF) {
+            if (t < LA || one_more) load_b128_to_lds(job_rsrc[t], to + (wave + NW * t) * 1024, past ? kNowhere : a_off[t], slab * job_step[t]);
+        } else if (t < WNT) {
             load_b128_to_lds(w_rsrc, to + S::A_STAGE + (BLOCKED ? wave * WNT + t : wave + NW * t) * 1024,
                              past ? kNowhere : last ? w_last[t] : w_off[t], slab * (BLOCKED ? KS * 1024 : SLAB));
         } else if (t < LA + WNT || one_more) {
@@ -135,13 +152,13 @@ __global__ __launch_bounds__(64 * CG * KS, 1) void gemm_panel_kernel(const T* __
             load_b128_to_lds(a_rsrc, to + (wave + NW * i) * 1024, past ? kNowhere : last ? a_last[i] : a_off[i], slab * SLAB);
         }
     };
-    constexpr int LOADS = LA + WNT + (REST > 0 ? 1 : 0);
+    constexpr int LOADS = LA + LW + (REST > 0 ? 1 : 0);
     // at most `slabs` slabs of this wavefront's loads still on their way
     auto wait_slabs = [&](auto slabs) {
         constexpr int n = decltype(slabs)::value;
-        static_assert(n * (LA + WNT + 1) < 64, "the count of loads in flight has six bits");
-        if (REST > 0 && one_more) wait_vm<n * (LA + WNT + 1)>();
-        else wait_vm<n * (LA + WNT)>();
+        static_assert(n * (LA + LW + 1) < 64, "the count of loads in flight has six bits");
+        if (REST > 0 && one_more) wait_vm<n * (LA + LW + 1)>();
+        else wait_vm<n * (LA + LW)>();
     };
     // The barrier of a turn: what a wavefront's LDS reads wait for is its own business (see below), the compiler keeps its order.
     auto meet = [&] {
@@ -166,9 +183,12 @@ __global__ __launch_bounds__(64 * CG * KS, 1) void gemm_panel_kernel(const T* __
         // this lane's place in an operand of A: chunk 2 g + r / 8 of column k / 64, row r % 8 of it, piece 4 (k / 32 % 2) + q
         const unsigned in_chunk = (r >> 3) * 1024 + (r & 7) * 128 + ((((ROWS ? 0 : part & 1) * 4 + q) ^ (r & 7)) * 16);
         const unsigned a_first = in_chunk + (ROWS ? part * 2048 : (part >> 1) * (ROWS8 * 1024)), a_lane[2] = {a_first, a_first ^ 64};
+        const unsigned half_lane = part * 1024 + r * 64 + (q ^ ((0x78 >> (r >> 2) * 2) & 3)) * 16;
         const unsigned w_lane = S::A_STAGE + (BLOCKED ? (ROWS ? cg : wave) * (WNT * 1024) + lane * 16
                                                       : in_chunk + ((part >> 1) * (BN / 8) + cg * (2 * WNT)) * 1024);
         auto read_a = [&](int stage, int k, int i) {
+            if constexpr (HALF) return *reinterpret_cast<const Operand*>(lds_raw + stage * S::STAGE + half_lane + i * (RG * 1024));
+            else
             return *reinterpret_cast<const Operand*>(lds_raw + stage * S::STAGE + a_lane[k & 1] + (k >> 1) * (ROWS8 * 1024) + i * (RG * 2048));
         };
         auto read_w = [&](int stage, int k, int j) {
@@ -326,18 +346,19 @@ __global__ __launch_bounds__(64 * CG * KS, 1) void gemm_panel_kernel(const T* __
     }
 }
 
-template <typename T, int MT, int CG, int KS, int MODE>
+template <typename T, int MT, int CG, int KS, int WT, bool HALF, int MODE>
 static int launch_panel(const T* A, const T* W, void* out, int M, int N, int K, int ksplit, const QkvTarget& qt,
                         const GateExtra& gx, hipStream_t stream) {
-    using S = PanelSizes<T, MT, CG, KS>;
-    if constexpr (MODE == kRopeCache && !S::TURNS) {
+    using S = PanelSizes<T, MT, CG, KS, WT, HALF>;
+    if constexpr ((MODE == kRopeCache && !S::TURNS) || (is_gated(MODE) && WT % 2 != 0)) {
         return kErrUnsupported;
     } else {
         static OncePerDevice told;
-        const int status = allow_lds(told, reinterpret_cast<const void*>(&gemm_panel_kernel<T, MT, CG, KS, MODE>), S::LDS);
+        constexpr int LDS = MODE == kRopeCache && S::TURNED > S::LDS ? S::TURNED : S::LDS;
+        const int status = allow_lds(told, reinterpret_cast<const void*>(&gemm_panel_kernel<T, MT, CG, KS, WT, HALF, MODE>), LDS);
         if (status != 0) return status;
         const int tiles_m = (M + S::BM - 1) / S::BM, tiles_n = (N + S::BN - 1) / S::BN;
-        hipLaunchKernelGGL((gemm_panel_kernel<T, MT, CG, KS, MODE>), dim3(tiles_m * tiles_n * ksplit), dim3(64 * S::NW), S::LDS, stream, A,
+        hipLaunchKernelGGL((gemm_panel_kernel<T, MT, CG, KS, WT, HALF, MODE>), dim3(tiles_m * tiles_n * ksplit), dim3(64 * S::NW), LDS, stream, A,
                            W, out, M, N, K, tiles_m, tiles_n, ksplit, qt, gx);
         return launch_status();
     }
@@ -347,7 +368,7 @@ template <int MODE, typename T>
 static int launch_panel_mode(int mt, int bn, const T* A, const T* W, void* out, int M, int N, int K, int ksplit, const QkvTarget& qt,
                              const GateExtra& gx, hipStream_t stream) {
 #define LLME_PANEL(MT, BN) \
-    if (mt == MT && bn == BN) return launch_panel<T, MT, BN / 32, 256 / BN, MODE>(A, W, out, M, N, K, ksplit, qt, gx, stream);
+    if (mt == MT && bn == BN) return launch_panel<T, MT, BN / 32, 256 / BN, 2, false, MODE>(A, W, out, M, N, K, ksplit, qt, gx, stream);
     LLME_PANEL(2, 64)
     LLME_PANEL(3, 64)
     LLME_PANEL(4, 64)
@@ -364,6 +385,18 @@ static int launch_panel_mode(int mt, int bn, const T* A, const T* W, void* out, 
     LLME_PANEL(11, 128)
     LLME_PANEL(12, 128)
 #undef LLME_PANEL
+    // bfloat16 only: three or four tiles of columns a wavefront (48 columns are no pairs of gate and up), from 160 rows on in slabs of 32 k
+    if constexpr (sizeof(T) == 2) {
+#define LLME_PANEL(MT, BN, HALF) \
+    if (mt == MT && bn == BN) return launch_panel<T, MT, 4, 2, BN / 64, HALF, MODE>(A, W, out, M, N, K, ksplit, qt, gx, stream);
+        LLME_PANEL(6, 192, false)
+        LLME_PANEL(8, 192, false)
+        LLME_PANEL(10, 192, true)
+        LLME_PANEL(12, 192, true)
+        LLME_PANEL(8, 256, true)
+        LLME_PANEL(12, 256, true)
+#undef LLME_PANEL
+    }
     return kErrUnsupported;
 }
 
@@ -388,15 +421,29 @@ int gemm_panel_f32(int mt, int bn, int mode, const float* A, const float* W, flo
     return launch_panel_mode<kStoreF32>(mt, bn, A, W, out, M, N, K, ksplit, QkvTarget{}, GateExtra{}, stream);
 }
 
+// Tiles of 192 and 256 columns are there for the rounds that they save: a product takes whole rounds of one tile a compute unit, and
+// what fills one and a half rounds of 128 x 128 is one round of 128 x 192 (16 x 16 of them cover 2,048 x 3,072). A turn of 128 x 192 x 64 takes
+// 0.63 us, of 128 x 128 0.46 (0.26 of it the matrix pipes at the 2.0 GHz that the chip holds under them, 0.31 the loads alone). From 160 x 192 on three
+// slabs of 64 k are all that LDS holds, too few: 192 x 192 x 64 took 1.15 us. HALF slabs of 32 k make the ring six places (192 x 256: five) for a
+// barrier every 32 k: 0.95 us. A's chunks are then 16 rows x 32 k: four lanes a row are 64 bytes side by side, which is what the loads'
+// path wants, and a row's four pieces are permuted by 0 2 3 1 of its number's bits 2 and 3, so that the 16 lanes that LDS serves at a time
+// (0-3, 12-15, 20-23, 24-27 and so on) meet no bank twice. Measured (us, weights from memory, the best before / with these; one round unless said):
+// rotating q/k/v of the 1B sizes (3,072 x 2,048) at 2,048 rows 37.6 / 28.6, 2,600: 39.3 / 34.5, 2,995: 46.8 / 38.4; stored 6,160 x 2,048 at 1,200 rows
+// 44.1 / 33.9; added 3,072 x 3,072 at 2,048 rows 49.4 / 41.4, 2,995: 70.3 / 58.1; added 3,072 x 8,192 at 2,048 rows 114 / 96; in parts at 1,000 rows 67 / 50;
+// gated 16,384 x 2,048 at 430 rows 39.0 / 34.0, in three rounds at 2,300 rows 150 / 136. Against two wavefronts a compute unit's pipe with 256 x 256 of
+// these (HALF): 99 us where gemm_mfma.hip's loop of that tile takes 83.
+
 // The tile and the cut over k, by an estimate fitted to 700 timings of 20 to 4,096 rows at the 1B, 3B and 8B sizes, when these tiles
 // shared out k (9 % off on average). With rows shared out, weights from memory and added sums among them, it is 4 to 13 % short, and the
 // tile that it chooses takes 0.8 % longer than the best on average over 200 sizes, 9 % at worst: rounds of workgroups over the chip x (3.2 us + 2.9 for the end of a tile
 // of 128 x 128, in proportion + the slabs' bytes at 98 a ns, less on a full chip and in large tiles, whose products take the time),
 // joined by their 2.5th powers with W's way from memory (1.2 us + 5.6 TB/s); parts cost their way out and back in the kernel that joins
 // them, 0.3 us a MB.
+// HALF slabs: 0.93 (k = 2,048) to 1.09 (14,336) of it, 1.03 times that in more rounds than one (the chip's clock falls in long products).
 // wide: 32-bit operands, whose products take the time (a compute unit makes 500 a ns).
-// ks_only: the number of parts (0: up to 8, of at least 256 k); heads: tiles hold whole heads of this many columns.
-PanelPlan panel_plan(int M, int N, int K, int ks_only, int heads, bool wide) {
+// ks_only: the number of parts (0: up to 8, of at least 256 k); heads: tiles hold whole heads of this many columns; pairs: a wavefront holds
+// whole pairs of gate and up (32 columns each, which the 48 of a tile of 192 are not).
+PanelPlan panel_plan(int M, int N, int K, int ks_only, int heads, bool wide, bool pairs) {
     // The last plans made by this thread, in sets of four that replace their oldest: a layer's products ask for the same few again and
     // again, and steps with prompt rows wait for the host, which an estimate of all tiles takes 1.5 us, of all cuts too 6. (Sizes of
     // models are multiples of large powers of two: the set comes from the high bits of products with odd numbers.)
@@ -409,19 +456,21 @@ PanelPlan panel_plan(int M, int N, int K, int ks_only, int heads, bool wide) {
         unsigned oldest = 0;
     };
     static thread_local Set memo[16];
-    const int other = ks_only * 2048 + heads * 2 + (wide ? 1 : 0);
+    const int other = ks_only * 4096 + heads * 4 + (pairs ? 2 : 0) + (wide ? 1 : 0);
     unsigned mixed = 0;
     for (const int v : {M, N, K, other}) mixed = (mixed ^ static_cast<unsigned>(v)) * 2654435761u, mixed ^= mixed >> 15;
     Set& set = memo[mixed >> 28];
     for (const Made& m : set.made)
         if (m.M == M && m.N == N && m.K == K && m.other == other) return m.plan;
     static const int shapes[][2] = {{2, 64}, {3, 64}, {4, 64}, {5, 64}, {6, 64}, {3, 128}, {4, 128}, {5, 128}, {6, 128},
-                                    {7, 128}, {8, 128}, {9, 128}, {10, 128}, {11, 128}, {12, 128}};
+                                    {7, 128}, {8, 128}, {9, 128}, {10, 128}, {11, 128}, {12, 128},
+                                    {6, 192}, {8, 192}, {10, 192}, {12, 192}, {8, 256}, {12, 256}};
     const int cus = compute_units();
     PanelPlan best{0, 0, 0, 0, 0.f};
     for (const auto& s : shapes) {
         const int bm = 16 * s[0], bn = s[1];
-        if (heads > 0 && bn % heads != 0) continue;
+        const bool half = bn == 256 || (bn == 192 && s[0] >= 10);
+        if ((heads > 0 && bn % heads != 0) || (bn > 128 && wide) || (bn == 192 && pairs) || (heads > 0 && s[0] == 12 && bn == 256)) continue;
         const long tiles = static_cast<long>((M + bm - 1) / bm) * ((N + bn - 1) / bn);
         for (int ks = ks_only > 0 ? ks_only : 1; ks <= (ks_only > 0 ? ks_only : 8); ++ks) {
             if (ks > 1 && ks_only == 0 && K / ks < 256) break;
@@ -429,7 +478,8 @@ PanelPlan panel_plan(int M, int N, int K, int ks_only, int heads, bool wide) {
             const float full = wgs < cus ? static_cast<float>(wgs) / cus : 1.f, area = static_cast<float>(bm) * bn;
             const float size = wide ? 4.f : 2.f, bytes = size * 1e-3f * K / ks * (bm + bn), rate = 98.f / (1.f + 0.54f * full * area / 24576.f);
             const float multiplied = wide ? 2e-3f * K / ks * area / 500.f : 0.f;
-            const float chip = rounds * (3.2f + 2.9f * area / 16384.f + (multiplied > bytes / rate ? multiplied : bytes / rate));
+            const float of_half = half ? (0.903f + 1.3e-5f * K / ks) * (rounds > 1 ? 1.03f : 1.f) : 1.f;
+            const float chip = of_half * rounds * (3.2f + 2.9f * area / 16384.f + (multiplied > bytes / rate ? multiplied : bytes / rate));
             const float memory = 1.2f + size * 1e-6f * N * K / 5.6f;
             float us = powf(powf(chip, 2.5f) + powf(memory, 2.5f), 0.4f);
             if (ks > 1) us += 0.3f * 4e-6f * ks * M * N;

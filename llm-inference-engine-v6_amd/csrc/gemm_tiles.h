@@ -429,7 +429,7 @@ struct PanelPlan {
     int rounds;                 // of workgroups over the chip
     float us;                   // as estimated
 };
-PanelPlan panel_plan(int M, int N, int K, int ks_only, int heads, bool wide = false);
+PanelPlan panel_plan(int M, int N, int K, int ks_only, int heads, bool wide = false, bool pairs = false);
 int gemm_panel_f32(int mt, int bn, int mode, const float* A, const float* W, float* out, int M, int N, int K, int ksplit, hipStream_t stream);
 int gemm_panel(int mt, int bn, int mode, const bf16* A, const bf16* W, void* out, int M, int N, int K, int ksplit, const QkvTarget& qt,
                const GateExtra& gx, hipStream_t stream);

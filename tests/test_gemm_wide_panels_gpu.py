@@ -1,0 +1,86 @@
+"""Tiles of 192 and 256 columns (csrc/gemm_panel.hip), from 160 rows on in slabs of 32 k."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+PANEL = 1000000
+TILES = [(96, 192), (128, 192), (160, 192), (192, 192), (128, 256), (192, 256)]
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from llmengine import ops
+    return ops
+
+
+def _pair(M, N, K, seed):
+    g = torch.Generator().manual_seed(seed)
+    return torch.randn(M, K, generator=g).to(torch.bfloat16), (torch.randn(N, K, generator=g) * 0.05).to(torch.bfloat16)
+
+
+# one row, a tile's edges in rows and columns, k of one to seven slabs of 32 (fewer than the ring holds) and of many; what lies behind
+# the last row and column joins no sum
+@pytest.mark.parametrize("M,N,K", [(1, 16, 32), (97, 208, 64), (161, 320, 160), (193, 448, 224), (385, 528, 2080)])
+@pytest.mark.parametrize("rows,cols", TILES)
+def test_wide_panels(ops, M, N, K, rows, cols):
+    """Stored and added sums against 64 bits (32-bit sums of bfloat16 products: 2e-5), and the bits of the tile through registers, which
+    adds k in the same order; gated ones in whole pairs of columns only."""
+    a, w = _pair(M + 9, N + 16, K, 21)
+    ref = a[:M].double() @ w[:N].double().T
+    a[M:], w[N:] = float("nan"), float("inf")
+    ad, wb, tile = a.to(DEV)[:M], ops.block_weight(w.to(DEV))[:N // 16], PANEL + 1000 * rows + cols
+    base = torch.randn(M, N, generator=torch.Generator().manual_seed(22))
+    for accumulate in (False, True):
+        got, other = base.clone().to(DEV), base.clone().to(DEV)
+        ops.gemm_bf16(ad, wb, got, accumulate, tile=tile)
+        ops.gemm_bf16(ad, wb, other, accumulate, tile=128, ksplit=1)
+        want = ref + base.double() if accumulate else ref
+        assert float((got.cpu().double() - want).norm() / want.norm()) < 2e-5 and torch.equal(got, other)
+    if N % 32:
+        return
+    got, other = (torch.zeros(M, N // 2, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    ops.gemm_bf16(ad, wb, other, gated=True, tile=128)
+    if cols == 256:
+        ops.gemm_bf16(ad, wb, got, gated=True, tile=tile)
+        assert torch.equal(got, other)
+    else:
+        with pytest.raises(ops.KernelError):
+            ops.gemm_bf16(ad, wb, got, gated=True, tile=tile)
+
+
+@pytest.mark.parametrize("T,n_q,n_kv,hd,tiles", [(2050, 8, 2, 64, TILES[:5]), (200, 10, 1, 64, TILES[:5]), (300, 3, 1, 128, TILES[4:5])])
+def test_wide_panels_rotate_as_the_others(ops, T, n_q, n_kv, hd, tiles):
+    g, page, K = torch.Generator().manual_seed(23), 16, 544
+    x, w = _pair(T, (n_q + 2 * n_kv) * hd, K, 24)
+    x, w = x.to(DEV), ops.block_weight(w.to(DEV))
+    cos, sin = (torch.rand(T + 5, hd // 2, generator=g).to(DEV) for _ in range(2))
+    blocks = (T + 5 + page - 1) // page
+    positions, seq = torch.arange(5, T + 5, dtype=torch.int32, device=DEV), torch.zeros(T, dtype=torch.int32, device=DEV)
+    table = torch.randperm(blocks, generator=g).view(1, blocks).to(torch.int32).to(DEV)
+
+    def run(tile):
+        q = torch.zeros(T, n_q * hd, dtype=torch.bfloat16, device=DEV)
+        k = torch.zeros(blocks, n_kv, page, hd, dtype=torch.bfloat16, device=DEV)
+        v = torch.zeros(blocks, n_kv, hd, page, dtype=torch.bfloat16, device=DEV)
+        ops.mfma.gemm_qkv_rope(x, w, cos, sin, positions, seq, table, q, k, v, n_q, n_kv, hd, tile=tile)
+        return q, k, v
+    want = run(128)
+    for rows, cols in [(0, 0)] + tiles:
+        got = run(PANEL + 1000 * rows + cols if rows else 0)
+        assert all(torch.equal(a, b) for a, b in zip(got, want)), (rows, cols)
+
+
+# rows and columns at which each of these tiles is the chosen one on 256 compute units, k at the least that they are chosen for and above
+@pytest.mark.parametrize("M,N,K,gated", [(2048, 3072, 544, False), (2300, 3072, 2048, False), (2995, 3072, 512, False), (1400, 16384, 512, True),
+                                         (1800, 4608, 2048, False), (1000, 3072, 8192, False)])
+def test_the_chosen_wide_panel_adds_in_the_order_of_the_others(ops, M, N, K, gated):
+    a, w = _pair(M, N, K, 25)
+    ad, wb = a.to(DEV), ops.block_weight(w.to(DEV))
+    for accumulate in (False, True):
+        if gated and accumulate:
+            continue
+        got, want = (torch.zeros(M, N // 2 if gated else N, dtype=torch.bfloat16 if gated else torch.float32, device=DEV) for _ in range(2))
+        ops.gemm_bf16(ad, wb, got, accumulate, gated=gated, ksplit=1 if accumulate else 0)
+        ops.gemm_bf16(ad, wb, want, accumulate, gated=gated, tile=128, ksplit=1 if accumulate else 0)
+        assert torch.equal(got, want), accumulate
