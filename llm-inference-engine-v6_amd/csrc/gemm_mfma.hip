@@ -889,7 +889,7 @@ constexpr int kPanelLeastK = 512;
 // again in the step (decode of 64 requests 1,656 / 1,679 us, of 23 943 / 941). A sum of up to 288 rows that is better cut over k is, by the kernel below
 // (273 x 2,048 x 2,048 is not: 11.5 / 9.0). Everything else by estimates (us, weights from memory; all but sums cut over k give the same bits):
 //  * 256 x 256 tiles take 4 us + 0.0235 a k in a round (gate/up: 700 rows x 16,384 x 2,048 53.3 against 54 to 67 here, 1,024 rows 59.6 / 75, 528 rows
-//    53 / 46.3).
+//    53 / 46.3), less where the end is short (the squared rectifier: 1,800 rows x 12,288 x 2,048 94 against 98 here; 273 rows 31.3 / 23.8).
 //  * these take 1.17 (added) or 1.06 (stored) times their plan, which was fitted to all kinds.
 //  * 128 x 128 tiles through registers, two a compute unit, take 3 us + 0.0070 to 0.0187 a k, by how many units have two (against these: added
 //    2,048 x 3,072 x 3,072 52.5 / 57.7, 2,048 x 4,096 x 4,096 78.7 / 85.1, but 1,500 rows 77.9 / 52.7; stored 4,096 x 1,536 x 2,048 33.3 /
@@ -904,7 +904,7 @@ static int choose_direct(int mode, int M, int N, int K, bool may_cut, int cus, P
     }
     plan = panel_plan(M, N, K, 1, 0, false, is_gated(mode));
     auto tiles = [&](int edge) { return static_cast<long>((M + edge - 1) / edge) * ((N + edge - 1) / edge); };
-    float large = static_cast<float>((tiles(256) + cus - 1) / cus) * (4.f + 0.0235f * K);
+    float large = static_cast<float>((tiles(256) + cus - 1) / cus) * (4.f + (mode == kSquaredReluBF16 ? 0.0220f : 0.0235f) * K);
     if (is_gated(mode)) return plan.us <= large ? 1 : 2;
     const float here = plan.us * (mode == kAddF32 ? 1.17f : 1.06f);
     const long t128 = tiles(128), rounds = (t128 + 2 * cus - 1) / (2 * cus);
@@ -1000,9 +1000,9 @@ extern "C" int llme_gemm_bf16(const void* a, const void* w, void* out, int out_d
     // workgroup per compute unit; a small output with a long k is cut over k instead (the
     // parts are added with atomics, so this needs an accumulating float32 output).
     if (gated) mode = gated == 2 ? kGatedReluBF16 : gated == 3 ? kGatedGeluBF16 : gated == 4 ? kGatedExtraBF16 : kGatedBF16;
-    // (gemm_panel.hip has the epilogues of what dense layers and heads make of a blocked weight: the rectified and GELU gates, the squared
-    // rectifier and sums stored in bfloat16 are the kernels' below, as are experts' rows with a scale of their own)
-    const bool panel_takes = blocked && K < (1 << 22) && (mode == kStoreF32 || mode == kAddF32 || mode == kGatedBF16 ||
+    // (gemm_panel.hip has the epilogues of what dense layers and heads make of a blocked weight: the rectified and GELU gates and
+    // sums stored in bfloat16 are the kernels' below, as are experts' rows with a scale of their own)
+    const bool panel_takes = blocked && K < (1 << 22) && (mode == kStoreF32 || mode == kAddF32 || mode == kGatedBF16 || mode == kSquaredReluBF16 ||
                                                           (mode == kGatedExtraBF16 && t_gate_extra.pair_scale == nullptr));
     if (tile_shape >= kPanelTile) {
         const int bm = (tile_shape - kPanelTile) / 1000, bn = (tile_shape - kPanelTile) % 1000;

@@ -329,6 +329,16 @@ __global__ __launch_bounds__(64 * CG * KS, 1) void gemm_panel_kernel(const T* __
                     o[e] = static_cast<__bf16>(gated_value<MODE>(acc[i][j][e], acc[i][j + 1][e], gx, static_cast<float>(bg[e]), static_cast<float>(bu[e])));
                 *reinterpret_cast<bf16x4*>(static_cast<bf16*>(out) + static_cast<size_t>(m) * (N / 2) + (n0 + cg * (16 * WNT) + j * 16) / 2 + q * 4) = o;
             }
+        } else if constexpr (is_stored_bf16(MODE)) {
+            typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
+#pragma unroll
+            for (int j = 0; j < WNT; ++j) {
+                if (nw + j * 16 >= N) continue;
+                bf16x4 o;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = static_cast<__bf16>(stored_value<MODE>(acc[i][j][e]));
+                *reinterpret_cast<bf16x4*>(static_cast<bf16*>(out) + static_cast<size_t>(m) * N + nw + j * 16) = o;
+            }
         } else {
             float* o = static_cast<float*>(out) + (static_cast<size_t>(MODE == kStoreF32 ? split : 0) * M + m) * N;   // (a part of its own)
 #pragma unroll
@@ -409,6 +419,7 @@ int gemm_panel(int mt, int bn, int mode, const bf16* A, const bf16* W, void* out
         case kAddF32: return launch_panel_mode<kAddF32>(mt, bn, A, W, out, M, N, K, 1, qt, gx, stream);
         case kGatedBF16: return launch_panel_mode<kGatedBF16>(mt, bn, A, W, out, M, N, K, 1, qt, gx, stream);
         case kGatedExtraBF16: return launch_panel_mode<kGatedExtraBF16>(mt, bn, A, W, out, M, N, K, 1, qt, gx, stream);
+        case kSquaredReluBF16: return launch_panel_mode<kSquaredReluBF16>(mt, bn, A, W, out, M, N, K, 1, qt, gx, stream);
         case kRopeCache: return bn % qt.hd ? kErrUnsupported : launch_panel_mode<kRopeCache>(mt, bn, A, W, out, M, N, K, 1, qt, gx, stream);
         default: return kErrUnsupported;
     }

@@ -84,3 +84,22 @@ def test_the_chosen_wide_panel_adds_in_the_order_of_the_others(ops, M, N, K, gat
         ops.gemm_bf16(ad, wb, got, accumulate, gated=gated, ksplit=1 if accumulate else 0)
         ops.gemm_bf16(ad, wb, want, accumulate, gated=gated, tile=128, ksplit=1 if accumulate else 0)
         assert torch.equal(got, want), accumulate
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 48, 512), (200, 528, 2080), (273, 12288, 512), (1500, 3072, 544)])
+def test_squared_rectifier_behind_the_panels(ops, M, N, K):
+    """The squared positive part, stored in bfloat16: every tile and the chosen one give the bits of the square of the stored sum."""
+    a, w = _pair(M, N, K, 26)
+    ad, wb = a.to(DEV), ops.block_weight(w.to(DEV))
+    p = torch.empty(M, N, device=DEV)
+    ops.gemm_bf16(ad, wb, p, tile=128)
+    want = torch.clamp(p, min=0.0).square().to(torch.bfloat16)
+    got = torch.zeros_like(want)
+    ops.gemm_squared_relu(ad, wb, got, None)
+    assert torch.equal(got, want)
+    m = ops.mfma
+    for rows, cols in TILES + [(32, 64), (96, 64), (48, 128), (144, 128)]:
+        got.zero_()
+        m.check(m.entry("llme_gemm_bf16")(m.ptr(ad), m.ptr(wb), m.ptr(got), 1, M, N, K, 0, 5, 0, 0, PANEL + 1000 * rows + cols, 1, -1,
+                                          m.stream()), "squared")
+        assert torch.equal(got, want), (rows, cols)
