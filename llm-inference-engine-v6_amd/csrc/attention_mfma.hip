@@ -294,8 +294,7 @@ static int launch_staged(int hd, dim3 grid, hipStream_t stream, ARGS... args) {
 // the entry points' `tuning` argument (0: every choice is the entry point's):
 //   bits 0-7   rows per work item of the prefill kernel without LDS: 16, 32 or 64 (0: by head size)
 //   bits 8-11  1 + shared: -1 the kernel that shares K and V through LDS where it takes the sizes
-//              (the default), 0 never, 1 wherever it can, 2 / 3 the same with one / two wavefronts
-//              per tile whatever the number of work items
+//              (the default), 0 never, 1, 2 or 3 wherever it can
 //   bits 12-13 1 + read_once: whether the decode kernel loads keys and values with the read-once
 //              hint: -1 the entry point chooses, 0 never, 1 always
 //   bit 14     the decode kernel's splits are left unjoined in part_o / part_ml: the caller joins them
@@ -303,13 +302,13 @@ static int launch_staged(int hd, dim3 grid, hipStream_t stream, ARGS... args) {
 //   bit 15     the prefill kernel that shares K and V through LDS takes work items of half the rows (16
 //              per row group instead of 32): for steps with few items (see attention_prefill.hip)
 struct Tuning {
-    int rows, shared, key_waves, read_once, no_join, half_rows;
+    int rows, shared, read_once, no_join, half_rows;
 };
 static bool parse_tuning(int packed, Tuning* t) {
     if (packed < 0 || packed >= (1 << 16)) return false;
     const int rows = packed & 0xFF, shared = ((packed >> 8) & 0xF) - 1, read_once = ((packed >> 12) & 0x3) - 1;
     if (rows % 16 != 0 || rows > 64 || shared > 3 || read_once > 1) return false;
-    *t = Tuning{rows, shared > 1 ? 1 : shared, shared > 1 ? shared - 1 : 0, read_once, (packed >> 14) & 1,
+    *t = Tuning{rows, shared > 1 ? 1 : shared, read_once, (packed >> 14) & 1,
                 (packed >> 15) & 1};
     return true;
 }
@@ -356,8 +355,7 @@ static int launch_for_head(const bf16* q, const bf16* kc, const bf16* vc, bf16* 
             }
             const int status = launch_prefill_shared(q, kc, vc, out, q_start, ctx_len, table, max_blocks, n_seq, n_q,
                                                      n_kv, HD, page, scale, window, prefill_groups, shared_rows, queue,
-                                                     prefill_splits, prefill_run, pre_part_o, pre_part_ml,
-                                                     tuning.key_waves, beside, stream);
+                                                     prefill_splits, prefill_run, pre_part_o, pre_part_ml, beside, stream);
             if (status != 0) return status;
             if (together && nsplit > 1 && prefill_splits > 1) {
                 hipLaunchKernelGGL(attention_join_both_kernel, dim3(n_seq + n_rows, n_q), dim3(64), 0, stream, part_o,

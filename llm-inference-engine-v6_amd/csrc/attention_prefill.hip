@@ -3,22 +3,24 @@
 // attention_tiles.h. What differs from the kernel that loads straight into registers is where
 // the operands come from: a workgroup's four wavefronts need the same keys (heads of one kv
 // head over the same rows, or neighbouring rows of one head), so the workgroup fetches every
-// 64-key stretch of K and V once, 16 bytes per thread and load, into LDS, and each wavefront
-// reads its operands from there. Global loads per key drop fourfold, and a thread holds only
-// a few registers of data in flight, so the next stretch travels while this one is computed.
+// 64-key stretch of K and V once, straight into LDS, and each wavefront reads its operands from there.
 //
 // Work item = (request, span of rows, group of HPW query heads of one kv head): wavefront w
 // takes head w % HPW of the group and the row group w / HPW of the span, each row group being
 // QT tiles of 16 rows. HPW is the largest of 4, 2, 1 that divides the heads per kv head.
-// Stretches run from the first key the span's first row sees to the last row's own key; a
-// wavefront skips the 32-key blocks that none of its rows sees and masks the rest by position.
+// Stretches run from the first key the span's first row sees to the last row's own key.
 //
-// LDS: two stages of K [64 keys][hd + 16] and V [hd][64 + 8]. The paddings are measured: LDS
-// has 64 banks of 4 bytes; the 16-byte operand reads (lane = key l % 16, dims 8 (l / 16) ..) run
-// at full rate with rows of 2 hd + 32 bytes and at half rate with 2 hd + 16, the 8-byte reads
-// of V (lane = dim l % 16, keys 4 (l / 16) ..) at full rate with rows of 144 bytes.
-// Per stretch one barrier: after it the stage written during the last stretch is read, and
-// the other, which everybody has finished reading, is written from the registers.
+// What bounds it: a wavefront's 32 rows x 64 keys are 32 exponentials a lane (16 cycles each), as many multiply-adds and maxima, half as many
+// conversions (about 800 cycles), 36 matrix instructions of 16 cycles with heads of 64 and 68 with heads of 128 (576, 1,088), and 16 or
+// 32 KB read from LDS (128 bytes a cycle for the whole unit: 128, 256). One after the other, with a wait of LDS's latency at every
+// operand, that was 1,900 and 4,100 cycles. So a turn multiplies the NEXT stretch's scores while it makes this stretch's weights, reads
+// every operand a step before it is multiplied, loads straight into LDS a stretch ahead (K two: its scores are a turn ahead), meets once, and has
+// the matrix cores add up the weights (a column of ones: 4 instructions for 64 of the vector units'). Two wavefronts for a
+// tile, each with half the keys, which steps of few items used to take, are no faster now (45 to 1,024 tokens: 1 to 4 % slower, 256 rows behind
+// 8,192: 50 / 40; 256 rows behind 1,024 beside 17 decoded requests took 20.7 with them, 21.0 without).
+// Measured on whole prompts, us, before / now, 32 query and 8 kv heads: heads of 64, 512 tokens 9.8 / 9.2, 1,024 17.7 / 15.4, 2,048 43.5 / 33.0, 4,096
+// 120 / 99, 8,192 387 / 318 (862 TFLOP/s); heads of 128, 1,024 30.5 / 21.6, 2,048 64 / 53.6, prompts of 2,000, 3,691 and 2,500 together
+// 291 / 220 (890 TFLOP/s); 256 rows behind 8,192, heads of 64, in 8 runs of keys 54 / 40.
 //
 // Takes head sizes 64 and 128 and pages that are multiples of 16; other sizes go to the kernel
 // without LDS.
@@ -31,149 +33,41 @@
 // the decode kernel. Items with few keys have one run and write their output themselves.
 #include "attention_tiles.h"
 
+#include <type_traits>
+
 namespace llme {
 
 constexpr int KB = 64;                     // keys per stretch
 
+// Two buffers of K and two of V, a stretch each: in K a half is [16 keys][HD], in V [HD][16 keys]. Behind them zeros, 16 bytes every 512, which
+// are read in the place of the values of a block that none of a wavefront's rows sees (a weight of zero alone would let an infinity through).
 template <int HD>
 struct StageLayout {
-    static constexpr int KS = HD + 16;     // K row stride (elements)
-    static constexpr int VS = KB + 8;      // V row stride (elements)
-    static constexpr int K_ELEMS = KB * KS;
-    static constexpr int V_ELEMS = HD * VS;
-    static constexpr int STAGE = K_ELEMS + V_ELEMS;
-    static constexpr int BYTES = 2 * STAGE * 2;
+    static constexpr int HALF = 16 * HD * 2;           // bytes
+    static constexpr int OPERAND = KB / 16 * HALF;
+    static constexpr int ZEROS = 4 * OPERAND;
+    static constexpr int BYTES = ZEROS + HD / 16 * 512;
 };
 
-// What one thread fetches of a stretch: NC chunks of 16 bytes of K and as many of V. Chunk i
-// of thread tid has the running number tid + threads i; of K it is key idx / (hd / 8), dims
-// 8 (idx % (hd / 8)) ..; of V the 16-key half idx / (2 hd), dim (idx % (2 hd)) / 2, keys
-// 8 (idx % 2) .. of the half. For head sizes 64 and 128 the 64 chunks of a wavefront then lie
-// in one 16-key half, the same for K and V: (64 wave + threads i) / (2 hd). A half has one page,
-// so the page's id, whether the half is to be read at all and the page's address are the
-// same for the whole wavefront: scalar work, and the loads take a scalar base and a 32-bit
-// offset per lane that never changes.
-template <int HD, int THREADS>
-struct Fetched {
-    static constexpr int NC = HD * 8 / THREADS;    // 64 keys x hd / 8 chunks over the workgroup's threads
-    bf16x8 k[NC];
-    bf16x8 v[NC];
-};
-
-template <int HD, int THREADS>
-__device__ __forceinline__ int chunk_half(int wave, int i) { return (64 * wave + THREADS * i) / (2 * HD); }
-
-// Per lane and chunk, fixed for the kernel: offsets (elements) from the start of the half's
-// keys in its page (K) or of the kv head's part of the page (V), and the places in a stage.
-template <int HD, int THREADS>
-struct ChunkPlaces {
-    static constexpr int NC = HD * 8 / THREADS;
-    unsigned k_off[NC], v_off[NC];         // global, in elements
-    unsigned k_lds[NC], v_lds[NC];         // in a stage, in elements
-};
-
-template <int HD, int THREADS>
-__device__ __forceinline__ ChunkPlaces<HD, THREADS> chunk_places(int tid, int page) {
-    using L = StageLayout<HD>;
-    constexpr int CK = HD / 8;
-    ChunkPlaces<HD, THREADS> c;
-#pragma unroll
-    for (int i = 0; i < HD * 8 / THREADS; ++i) {
-        const int idx = tid + THREADS * i;
-        const int key = idx / CK, dim = (idx % CK) * 8;
-        c.k_off[i] = (key & 15) * HD + dim;
-        c.k_lds[i] = key * L::KS + dim;
-        const int half = idx / (2 * HD), rem = idx % (2 * HD);
-        const int vdim = rem / 2, c2 = rem % 2;
-        c.v_off[i] = vdim * page + 8 * c2;
-        c.v_lds[i] = L::K_ELEMS + vdim * L::VS + 16 * half + 8 * c2;
-    }
-    return c;
-}
-
-// The pages of the NC halves that this wavefront fetches of the stretch at t0: page id (or -1:
-// the half has no key in [key_lo, key_end), nothing is read for it) and the first key's place
-// in the page. All scalar.
-template <int HD, int THREADS>
-struct StretchPages {
-    int pg[HD * 8 / THREADS];
-    int off[HD * 8 / THREADS];
-};
-
-template <int HD, int THREADS>
-__device__ __forceinline__ StretchPages<HD, THREADS> lookup_stretch(const PagedKV& kv, int t0, int key_lo, int key_end,
-                                                                    int wave) {
-    StretchPages<HD, THREADS> p;
-#pragma unroll
-    for (int i = 0; i < HD * 8 / THREADS; ++i) {
-        const int h0 = t0 + 16 * chunk_half<HD, THREADS>(wave, i);
-        const PagePlace pl = page_of(kv, h0);
-        p.off[i] = pl.offset;
-        p.pg[i] = (h0 < key_end && h0 + 15 >= key_lo) ? __builtin_amdgcn_readfirstlane(kv.table[pl.block]) : -1;
-    }
-    return p;
-}
-
-// Every turn issues the same loads: a half that is not to be read reads the pool's first page
-// instead and counts as zeros.
-template <int HD, int THREADS>
-__device__ __forceinline__ void fetch_stretch(const PagedKV& kv, const StretchPages<HD, THREADS>& p,
-                                              const ChunkPlaces<HD, THREADS>& c, Fetched<HD, THREADS>& f) {
-#pragma unroll
-    for (int i = 0; i < HD * 8 / THREADS; ++i) {
-        const bool ok = p.pg[i] >= 0;                                                     // scalar
-        const size_t base = static_cast<size_t>(ok ? p.pg[i] : 0) * kv.page_stride + kv.head_off;   // scalar
-        const bf16* ksrc = kv.k + base + static_cast<size_t>(ok ? p.off[i] : 0) * HD;
-        const bf16* vsrc = kv.v + base + (ok ? p.off[i] : 0);
-        const bf16x8 xk = *reinterpret_cast<const bf16x8*>(ksrc + c.k_off[i]);
-        const bf16x8 xv = *reinterpret_cast<const bf16x8*>(vsrc + c.v_off[i]);
-        f.k[i] = ok ? xk : zero_frag();
-        f.v[i] = ok ? xv : zero_frag();
-    }
-}
-
-template <int HD, int THREADS>
-__device__ __forceinline__ void store_stretch(bf16* stage, const ChunkPlaces<HD, THREADS>& c,
-                                              const Fetched<HD, THREADS>& f) {
-#pragma unroll
-    for (int i = 0; i < HD * 8 / THREADS; ++i) {
-        *reinterpret_cast<bf16x8*>(stage + c.k_lds[i]) = f.k[i];
-        *reinterpret_cast<bf16x8*>(stage + c.v_lds[i]) = f.v[i];
-    }
-}
-
-// The operands of the 32-key block `sb` (0 or 1) of a stage, as attention_tiles.h lays them out.
+// The place of a 16-byte piece in row `key` of K's buffer (key within its 32-key block): pieces are permuted by bits of the
+// row's number such that the 16 lanes that LDS serves at a time (0-3, 12-15, 20-23, 24-27 and so on), which read rows 8 (r / 4) + r % 4 at
+// neighbouring pieces (see block_scores), meet no bank twice.
 template <int HD>
-__device__ __forceinline__ void read_block(const bf16* stage, int sb, KFrag<HD>& kf, VFrag<HD>& vf) {
-    using L = StageLayout<HD>;
-    const int lane = threadIdx.x & 63, r = lane & 15, g4 = lane >> 4;
-#pragma unroll
-    for (int hf = 0; hf < 2; ++hf)
-#pragma unroll
-        for (int c = 0; c < HD / 32; ++c)
-            kf.kf[hf][c] = *reinterpret_cast<const bf16x8*>(stage + (32 * sb + 16 * hf + r) * L::KS + c * 32 + g4 * 8);
-    const bf16* vs = stage + L::K_ELEMS;
-#pragma unroll
-    for (int dt = 0; dt < HD / 16; ++dt) {
-        const bf16* p = vs + (dt * 16 + r) * L::VS + 32 * sb + 4 * g4;
-        const bf16x4 lo4 = *reinterpret_cast<const bf16x4*>(p);
-        const bf16x4 hi4 = *reinterpret_cast<const bf16x4*>(p + 16);
-        vf.vf[dt] = __builtin_shufflevector(lo4, hi4, 0, 1, 2, 3, 4, 5, 6, 7);
-    }
+__device__ __forceinline__ unsigned k_turn(int key) {
+    return HD == 128 ? ((key >> 3) & 3) << 2 | (key & 3) : ((key >> 3) & 3) << 1 | ((key >> 1) & 1);
 }
 
 // One work item: span `bx` (counted over the requests with two or more tokens, the last spans of
 // a request first) for head group `by`, run `z` of its keys (SPLIT; else all keys).
-template <int HD, int QT, int HPW, int KW, bool SPLIT>
+template <int HD, int QT, int HPW, bool SPLIT>
 __device__ __forceinline__ void prefill_item(int bx, int by, int z, int nsplit, int run, float* __restrict__ part_o,
-                                             float* __restrict__ part_ml, bf16* lds, const bf16* __restrict__ q,
+                                             float* __restrict__ part_ml, unsigned char* lds, const bf16* __restrict__ q,
                                              const bf16* __restrict__ k_cache, const bf16* __restrict__ v_cache,
                                              bf16* __restrict__ out, const int* __restrict__ q_start,
                                              const int* __restrict__ ctx_len, const int* __restrict__ block_table,
                                              int max_blocks, int n_seq, int n_q, int n_kv, int page, float scale,
                                              int window) {
     constexpr int DC = HD / 32, DT = HD / 16, ROWS = 16 * QT, RG = 4 / HPW, SPAN = RG * ROWS;
-    constexpr int THREADS = 256 * KW;
     using L = StageLayout<HD>;
 
     // which request and which of its spans this workgroup has
@@ -196,11 +90,9 @@ __device__ __forceinline__ void prefill_item(int bx, int by, int z, int nsplit, 
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63, r = lane & 15, g4 = lane >> 4;
     const int G = n_q / n_kv;
-    const int tile = wave % 4;                             // which rows and head; KW wavefronts share a tile
-    const int ks = wave / 4;                               // and take the 32-key blocks sb with sb % KW == ks
-    const int head = by * HPW + tile % HPW;                // HPW divides G: one kv head per workgroup
+    const int head = by * HPW + wave % HPW;                // HPW divides G: one kv head per workgroup
     const int kvh = (by * HPW) / G;
-    const int rg = tile / HPW;
+    const int rg = wave / HPW;
     const int pos_span = ctx_len[s] + (first - q_start[s]); // position of the span's first row
 
     // this wavefront's rows
@@ -209,24 +101,23 @@ __device__ __forceinline__ void prefill_item(int bx, int by, int z, int nsplit, 
     n_rows = n_rows < 0 ? 0 : (n_rows > ROWS ? ROWS : n_rows);
     const int pos0 = pos_span + rg * ROWS;
     bf16x8 qf[QT][DC];
-    int row_pos[QT], row_lo[QT], tile_free[QT];
-    float m[QT], l[QT];
-    f32x4 o[QT][DT];
+    float m[QT];                                           // of row r
+    f32x4 l[QT], o[QT][DT];                                // of rows 4 g4 + e
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
         const int rr = qt * 16 + r;
         const bool ok = rr < n_rows;
         load_q<HD>(q + (static_cast<size_t>(ok ? first_w + rr : first) * n_q + head) * HD, ok, qf[qt]);
-        row_pos[qt] = ok ? pos0 + rr : -1;
-        row_lo[qt] = (window > 0 && pos0 + rr - window + 1 > 0) ? pos0 + rr - window + 1 : 0;
-        tile_free[qt] = (window == 0 && qt * 16 + 16 <= n_rows) ? pos0 + qt * 16 : -1;
         m[qt] = kNoMax;
-        l[qt] = 0.f;
+        l[qt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) o[qt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    const int my_end = n_rows > 0 ? pos0 + n_rows : 0;      // this wavefront's rows see keys < my_end
+    int my_end = n_rows > 0 ? pos0 + n_rows : 0;            // this wavefront's rows see keys < my_end
     const int my_lo = (window > 0 && pos0 - window + 1 > 0) ? pos0 - window + 1 : 0;
+    // stretches that begin at free_lo or behind and end before free_hi are seen whole by every row
+    const int free_lo = (window > 0 && pos0 + ROWS - window > 0) ? pos0 + ROWS - window : 0;
+    const int free_hi = n_rows > 0 ? pos0 + 1 : 0;
 
     // the workgroup's keys
     int key_end = pos_span + n_span;
@@ -239,109 +130,239 @@ __device__ __forceinline__ void prefill_item(int bx, int by, int z, int nsplit, 
         k_begin += z * run * KB;
         if (z < runs - 1) key_end = k_begin + run * KB;    // (the last run takes the rest)
     }
-    PagedKV kv{k_cache, v_cache, block_table + static_cast<size_t>(s) * max_blocks, page, n_kv, kvh, HD,
-               page_magic_of(page), static_cast<unsigned>(n_kv) * page * HD, static_cast<unsigned>(kvh) * page * HD};
+    my_end = my_end < key_end ? my_end : key_end;
+    const PagedKV kv{k_cache, v_cache, block_table + static_cast<size_t>(s) * max_blocks, page, n_kv, kvh, HD,
+                     page_magic_of(page), static_cast<unsigned>(n_kv) * page * HD, static_cast<unsigned>(kvh) * page * HD};
     const float scale_log2 = scale * kLog2e;
+    const int n_stretch = (key_end - k_begin + KB - 1) / KB;
 
-    const ChunkPlaces<HD, THREADS> places = chunk_places<HD, THREADS>(tid, page);
-    Fetched<HD, THREADS> fetched;
-    StretchPages<HD, THREADS> pages = lookup_stretch<HD, THREADS>(kv, k_begin, key_lo, key_end, wave);
-    fetch_stretch<HD, THREADS>(kv, pages, places, fetched);
-    pages = lookup_stretch<HD, THREADS>(kv, k_begin + KB, key_lo, key_end, wave);
-    store_stretch<HD, THREADS>(lds, places, fetched);
-    fetch_stretch<HD, THREADS>(kv, pages, places, fetched);           // past key_end: no page ids, zeros
-    pages = lookup_stretch<HD, THREADS>(kv, k_begin + 2 * KB, key_lo, key_end, wave);
-    lds_barrier();
-    int st = 0;
-    for (int t0 = k_begin; t0 < key_end; t0 += KB, st ^= 1) {
-        const bf16* stage = lds + st * L::STAGE;
+    // ---- loads: half `wave` of every stretch is this wavefront's, its K and its V in NL pieces of 1 KB each ----
+    constexpr int NL = HD / 32, K_ROWS = 1024 / (2 * HD);               // keys in 1 KB of K
+    // a half without a key in [key_lo, key_end) is not to be read (its page may not be there): of K the nearest one that has is, whose
+    // scores are replaced, and V's places become zeros (an offset that is nowhere within the descriptor)
+    const int first_half = key_lo & ~15, last_half = (key_end - 1) & ~15;
+    constexpr unsigned kOutside = 0x40000000u;
+    auto half_at = [&](int j) {
+        const int h0 = k_begin + j * KB + 16 * wave;
+        return h0 > last_half ? last_half : h0 < first_half ? first_half : h0;
+    };
+    // the page ids of this wavefront's half in 64 stretches, one a lane
+    auto look_up = [&](int j) { return kv.table[page_of(kv, half_at(j + lane)).block]; };
+    unsigned k_off[2];                                      // of a lane in 1 KB of K: one of two, by its place in the half
 #pragma unroll
-        for (int sb = 0; sb < 2; ++sb) {
-            const int tb = t0 + 32 * sb;
-            if (sb % KW == ks && tb < my_end && tb + 32 > my_lo) {         // the same for the whole wavefront
-                KFrag<HD> kf;
-                VFrag<HD> vf;
-                read_block<HD>(stage, sb, kf, vf);
-                f32x4 sc[QT][2];
-                block_scores<HD, QT>(kf, qf, sc);
-                bf16x8 pf[QT];
-                block_weights<HD, QT>(sc, tb, row_pos, row_lo, tile_free, scale_log2, m, l, o, pf);
-#pragma unroll
-                for (int qt = 0; qt < QT; ++qt)
-#pragma unroll
-                    for (int dt = 0; dt < DT; ++dt)
-                        o[qt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf[qt], vf.vf[dt], o[qt][dt], 0, 0, 0);
-            }
-        }
-        if (t0 + KB < key_end) {                            // the same for the whole workgroup
-            store_stretch<HD, THREADS>(lds + (st ^ 1) * L::STAGE, places, fetched);
-            fetch_stretch<HD, THREADS>(kv, pages, places, fetched);
-            pages = lookup_stretch<HD, THREADS>(kv, t0 + 3 * KB, key_lo, key_end, wave);
-            lds_barrier();
-        }
+    for (int u = 0; u < 2; ++u) {
+        const int key = 16 * (wave & 1) + (HD == 128 ? 8 * u : K_ROWS * u) + lane / (64 / K_ROWS), slot = lane % (64 / K_ROWS);
+        k_off[u] = static_cast<unsigned>(lane / (64 / K_ROWS)) * (HD * 2) + (slot ^ k_turn<HD>(key)) * 16;
     }
+    const unsigned v_off = static_cast<unsigned>(lane >> 1) * (kv.page * 2) + (lane & 1) * 16;
+    const unsigned lds_base = static_cast<unsigned>(reinterpret_cast<size_t>((__attribute__((address_space(3))) unsigned char*)lds));
+    auto descriptor = [](const bf16* p, unsigned bytes) {
+        const unsigned long long at = reinterpret_cast<unsigned long long>(p);
+        return u32x4{static_cast<unsigned>(at), static_cast<unsigned>(at >> 32) & 0xFFFFu, bytes, 0x00020000u};
+    };
+    struct Half {
+        int page, offset;
+        bool inside;
+    };
+    auto ask_k = [&](const Half& h, int buffer) {
+        const u32x4 rsrc = descriptor(kv.k + static_cast<size_t>(h.page) * kv.page_stride + kv.head_off + static_cast<size_t>(h.offset) * HD, L::HALF);
+#pragma unroll
+        for (int i = 0; i < NL; ++i)
+            load_1kb_to_lds(rsrc, lds_base + buffer * L::OPERAND + wave * L::HALF + i * 1024, k_off[HD == 128 ? i >> 1 : i], i * 1024);
+    };
+    auto ask_v = [&](const Half& h, int buffer) {
+        const u32x4 rsrc = descriptor(kv.v + static_cast<size_t>(h.page) * kv.page_stride + kv.head_off + h.offset, static_cast<unsigned>(HD - 1) * kv.page * 2 + 32);
+#pragma unroll
+        for (int i = 0; i < NL; ++i)
+            load_1kb_to_lds(rsrc, lds_base + (2 + buffer) * L::OPERAND + wave * L::HALF + i * 1024, h.inside ? v_off : kOutside,
+                            h.inside ? i * 32 * kv.page * 2 : 0);
+    };
+    int ids = look_up(0);
+    auto half_of = [&](int j) {
+        return Half{__builtin_amdgcn_readlane(ids, j & 63), __builtin_amdgcn_readfirstlane(page_of(kv, half_at(j)).offset),
+                    half_at(j) == k_begin + j * KB + 16 * wave};
+    };
+    // what everybody asked for is there, and everybody is done with what it read
+    auto meet = [&] { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
 
-    if (KW == 2) {
-        // The two wavefronts of a tile have seen every other 32-key block each: the second hands
-        // its maxima, sums and accumulators over through LDS (the stages are done with), the
-        // first brings both to the common maximum and adds them.
-        constexpr int PER_QT = 2 + DT * 4;                 // floats per lane and row tile
-        float* hand = reinterpret_cast<float*>(lds) + tile * (QT * PER_QT * 64);
-        static_assert(4 * QT * PER_QT * 64 * 4 <= L::BYTES, "the hand-over must fit into the stages");
-        __syncthreads();                                   // everybody has read its last stage
-        if (ks == 1) {
+    // ---- products ----
+    // (what only the rare branches of a turn make of the lane's number is made there and not kept in registers throughout)
+    auto rarely = [](int x) {
+        asm volatile("" : "+v"(x));
+        return x;
+    };
+    constexpr int NB = KB / 32;                             // 32-key blocks of a stretch
+    bf16x8 ones;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ones[i] = static_cast<__bf16>(1.f);
+    const unsigned char* k_lane = lds + (8 * (r >> 2) + (r & 3)) * (2 * HD);
+    const unsigned k_piece = (g4 ^ k_turn<HD>(8 * (r >> 2) + (r & 3))) * 16;
+    const unsigned char* v_lane = lds + 2 * L::OPERAND + (g4 >> 1) * L::HALF + r * 32 + (g4 & 1) * 16;
+    // Scores of row i of K's operand of half hf: key 8 (i / 4) + 4 hf + i % 4, so that a lane, whose results are rows 4 g4 + e, gets the
+    // eight keys 8 g4 .. of the block, which are 16 bytes of V's rows.
+    auto read_k = [&](int buffer, int b, int hf, bf16x8 (&kf)[DC]) {
+#pragma unroll
+        for (int c = 0; c < DC; ++c)
+            kf[c] = *reinterpret_cast<const bf16x8*>(k_lane + buffer * L::OPERAND + b * 2 * L::HALF + hf * (4 * 2 * HD) + (k_piece ^ (c * 64)));
+    };
+    auto scores_of = [&](const bf16x8 (&kf)[DC], f32x4 (&to)[QT]) {
+#pragma unroll
+        for (int c = 0; c < DC; ++c)
+#pragma unroll
+            for (int qt = 0; qt < QT; ++qt)
+                to[qt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[c], qf[qt][c], c == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : to[qt], 0, 0, 0);
+    };
+    auto all_scores = [&](int buffer, f32x4 (&to)[NB][2][QT]) {
+#pragma unroll
+        for (int g = 0; g < 2 * NB; ++g) {
+            bf16x8 kf[DC];
+            read_k(buffer, g >> 1, g & 1, kf);
+            scores_of(kf, to[g >> 1][g & 1]);
+        }
+    };
+    auto weights_of = [&](const f32x4& sc, int qt, int hf, bf16x8& pf) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) pf[hf * 4 + e] = static_cast<__bf16>(fast_exp2(fmaf(sc[e], scale_log2, -m[qt])));
+    };
+    Half h_v = half_of(0), h_k = half_of(1);                // of the V and the K that are asked for next
+    ask_k(h_v, 0);
+    ask_v(h_v, 0);
+    if (n_stretch > 1) ask_k(h_k, 1);
+    h_v = h_k;
+    f32x4 sa[NB][2][QT], sb[NB][2][QT];
+    meet();
+    all_scores(0, sa);
+
+    // One stretch: its weights and values, and the next one's scores. cur: its scores; buffer: of its V (the next K lies in the other).
+    auto turn = [&](int j, auto which, f32x4 (&cur)[NB][2][QT], f32x4 (&next)[NB][2][QT]) {
+        constexpr int BUFFER = decltype(which)::value;
+        meet();
+        bf16x8 kf[2][DC];
+        read_k(BUFFER ^ 1, 0, 0, kf[0]);                    // (on its way while the loads are asked for and the maxima made)
+        __builtin_amdgcn_sched_barrier(0);
+        const int t0 = k_begin + j * KB;
+        if (j + 2 < n_stretch) {
+            if (((j + 2) & 63) == 0) {
+                ids = look_up(j + 2);
+                asm volatile("" ::"v"(ids));               // (waited for here, and not wherever it is read)
+            }
+            h_k = half_of(j + 2);
+            ask_k(h_k, BUFFER);
+        }
+        if (j + 1 < n_stretch) ask_v(h_v, BUFFER ^ 1);
+        h_v = h_k;
+        if (t0 >= my_end) return;                           // (no row sees any of it, nor of what follows)
+        if (t0 + KB <= my_lo) {                        // (no row sees any of it yet)
+            all_scores(BUFFER ^ 1, next);
+            return;
+        }
+        if (t0 < free_lo || t0 + KB > free_hi) {
+            const int l_ = rarely(lane), r_ = l_ & 15, g_ = l_ >> 4;
 #pragma unroll
             for (int qt = 0; qt < QT; ++qt) {
-                float* p = hand + qt * PER_QT * 64 + lane;
-                p[0] = m[qt];
-                p[64] = l[qt];
+                const int row = qt * 16 + r_;
+                const int last = (row < n_rows ? pos0 + row : -1) - t0 - g_ * 8, first_seen = window > 0 ? pos0 + row - window + 1 - t0 - g_ * 8 : -KB;
 #pragma unroll
-                for (int dt = 0; dt < DT; ++dt)
+                for (int b = 0; b < NB; ++b)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) p[(2 + dt * 4 + e) * 64] = o[qt][dt][e];
+                    for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const int t = 32 * b + hf * 4 + e;
+                            cur[b][hf][qt][e] = (t <= last && t >= first_seen) ? cur[b][hf][qt][e] : -INFINITY;
+                        }
             }
         }
-        __syncthreads();
-        if (ks == 1) return;
+        float mx[QT];
+        bool moves = false;
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt) {
-            const float* p = hand + qt * PER_QT * 64 + lane;
-            const float m1 = p[0], l1 = p[64];
-            const float mx = fmaxf(m[qt], m1);
-            const float a0 = fast_exp2(m[qt] - mx), a1 = fast_exp2(m1 - mx);
-            m[qt] = mx;
-            l[qt] = l[qt] * a0 + l1 * a1;
-            float ar0[4], ar1[4];
+            mx[qt] = cur[0][0][qt][0];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {                   // factors of O's row 4 g4 + e
-                ar0[e] = __shfl(a0, g4 * 4 + e, 64);
-                ar1[e] = __shfl(a1, g4 * 4 + e, 64);
-            }
+            for (int b = 0; b < NB; ++b)
 #pragma unroll
-            for (int dt = 0; dt < DT; ++dt)
+                for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) o[qt][dt][e] = o[qt][dt][e] * ar0[e] + p[(2 + dt * 4 + e) * 64] * ar1[e];
+                    for (int e = 0; e < 4; ++e) mx[qt] = fmaxf(mx[qt], cur[b][hf][qt][e]);
+            moves |= fmaf(mx[qt], scale_log2, -m[qt]) > kLazy;
         }
+        if (__any(moves)) {                                 // some row's maximum moves (see block_weights): rescale what is summed
+            const int l_ = rarely(lane);
+            auto from = [](float x, int at) { return __int_as_float(__builtin_amdgcn_ds_bpermute(at * 4, __float_as_int(x))); };
+#pragma unroll
+            for (int qt = 0; qt < QT; ++qt) {
+                float mr = fmaxf(mx[qt], from(mx[qt], l_ ^ 16));
+                mr = fmaxf(mr, from(mr, l_ ^ 32));
+                const float ms = mr * scale_log2;
+                const float m_new = (ms > m[qt] + kLazy) ? ms : m[qt];
+                const float alpha = fast_exp2(m[qt] - m_new);
+                m[qt] = m_new;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {               // factor of row 4 g4 + e
+                    const float ar = from(alpha, (l_ >> 4) * 4 + e);
+                    l[qt][e] *= ar;
+#pragma unroll
+                    for (int dt = 0; dt < DT; ++dt) o[qt][dt][e] *= ar;
+                }
+            }
+        }
+        const unsigned char* v_at[2] = {v_lane + BUFFER * L::OPERAND, v_lane + BUFFER * L::OPERAND + 2 * L::HALF};
+        if (t0 + 32 <= my_lo) v_at[0] = lds + L::ZEROS;
+        if (t0 + 32 >= my_end) v_at[1] = lds + L::ZEROS;
+        bf16x8 pf[NB][QT];
+        // No branch from here on: the next scores' products and these weights' exponentials go side by side. The compiler puts a read of
+        // LDS where it is used and waits for it there, so the order is given: every step reads what the next one multiplies. (Behind
+        // the last stretch the products are of whatever LDS holds, and nobody's.)
+        constexpr int NV = 4, STEPS = NB * DT / NV;     // values: NV tiles of columns a step
+        bf16x8 vf[2][NV];
+        auto read_values = [&](int step, bf16x8 (&to)[NV]) {
+#pragma unroll
+            for (int i = 0; i < NV; ++i) to[i] = *reinterpret_cast<const bf16x8*>(v_at[step * NV / DT] + (step * NV + i) % DT * 512);
+        };
+#pragma unroll
+        for (int g = 0; g < 2 * NB; ++g) {
+            if (g + 1 < 2 * NB) read_k(BUFFER ^ 1, (g + 1) >> 1, (g + 1) & 1, kf[(g + 1) & 1]);
+            else read_values(0, vf[0]);
+            scores_of(kf[g & 1], next[g >> 1][g & 1]);
+#pragma unroll
+            for (int qt = 0; qt < QT; ++qt) weights_of(cur[g >> 1][g & 1][qt], qt, g & 1, pf[g >> 1][qt]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int u = 0; u < STEPS; ++u) {
+            if (u + 1 < STEPS) read_values(u + 1, vf[(u + 1) & 1]);
+            const int b = u * NV / DT;
+#pragma unroll
+            for (int i = 0; i < NV; ++i)
+#pragma unroll
+                for (int qt = 0; qt < QT; ++qt) {
+                    f32x4& to = o[qt][(u * NV + i) % DT];
+                    to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf[b][qt], vf[u & 1][i], to, 0, 0, 0);
+                }
+            if (u * NV % DT == 0)
+#pragma unroll
+                for (int qt = 0; qt < QT; ++qt) l[qt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf[b][qt], ones, l[qt], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    for (int j = 0; j < n_stretch; j += 2) {                // (one behind the last only meets the others)
+        turn(j, std::integral_constant<int, 0>{}, sa, sb);
+        turn(j + 1, std::integral_constant<int, 1>{}, sb, sa);
     }
 
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
-        float lt = l[qt];
-        lt += __shfl_xor(lt, 16, 64);
-        lt += __shfl_xor(lt, 32, 64);
         if (SPLIT && runs > 1) {
-            // this run's part of row `row`, head `head`: statistics from the lanes of the row's
-            // first quarter, outputs unscaled (the join divides)
-            if (g4 == 0 && qt * 16 + r < n_rows) {
-                const size_t pidx = (static_cast<size_t>(first_w + qt * 16 + r) * n_q + head) * nsplit + z;
-                part_ml[pidx * 2] = m[qt];
-                part_ml[pidx * 2 + 1] = lt;
-            }
+            // this run's part of row `row`, head `head`: the maximum from the lanes of the row's first quarter, the sum from a lane that
+            // has it, outputs unscaled (the join divides)
+            if (g4 == 0 && qt * 16 + r < n_rows)
+                part_ml[((static_cast<size_t>(first_w + qt * 16 + r) * n_q + head) * nsplit + z) * 2] = m[qt];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int row = qt * 16 + g4 * 4 + e;
                 if (row >= n_rows) continue;
                 const size_t pidx = (static_cast<size_t>(first_w + row) * n_q + head) * nsplit + z;
+                if (r == 0) part_ml[pidx * 2 + 1] = l[qt][e];
 #pragma unroll
                 for (int dt = 0; dt < DT; ++dt) part_o[pidx * HD + dt * 16 + r] = o[qt][dt][e];
             }
@@ -349,11 +370,9 @@ __device__ __forceinline__ void prefill_item(int bx, int by, int z, int nsplit, 
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const int rr = g4 * 4 + e;
-            const float l_row = __shfl(lt, rr, 64);
-            const int row = qt * 16 + rr;
+            const int row = qt * 16 + g4 * 4 + e;
             if (row >= n_rows) continue;
-            const float inv = 1.0f / l_row;
+            const float inv = 1.0f / l[qt][e];
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt)
                 out[(static_cast<size_t>(first_w + row) * n_q + head) * HD + dt * 16 + r] =
@@ -367,10 +386,12 @@ __device__ __forceinline__ void prefill_item(int bx, int by, int z, int nsplit, 
 // leaves most of the chip idle while the few longest finish. queue[0] counts the items taken,
 // queue[1] the workgroups that have left; both are zero before and after the kernel (the last
 // workgroup to leave clears them), so the same two integers serve every launch on a stream.
-// KW = 2: eight wavefronts, two per tile, each taking every other 32-key block: half the time
-// for a work item, for batches with too few items to fill the chip.
-template <int HD, int QT, int HPW, int KW, bool SPLIT>
-__global__ __launch_bounds__(256 * KW) void attention_prefill_shared_kernel(
+// (Registers: 128 with heads of 64 and one tile of rows a wavefront, for four workgroups a unit: 2,048 tokens 34.2 us with three, 32.7 with four.
+// Otherwise up to 256, for the two that LDS holds of heads of 128.)
+template <int HD, int QT>
+constexpr int kWavesASimd = HD == 64 && QT == 1 ? 4 : 2;
+template <int HD, int QT, int HPW, bool SPLIT>
+__global__ __launch_bounds__(256, (kWavesASimd<HD, QT>)) void attention_prefill_shared_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k_cache, const bf16* __restrict__ v_cache,
     bf16* __restrict__ out, const int* __restrict__ q_start, const int* __restrict__ ctx_len,
     const int* __restrict__ block_table, int max_blocks, int n_seq, int n_q, int n_kv, int page, float scale,
@@ -378,7 +399,7 @@ __global__ __launch_bounds__(256 * KW) void attention_prefill_shared_kernel(
     float* __restrict__ part_ml, DecodeBeside beside) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
     __shared__ int next_item;
-    bf16* lds = reinterpret_cast<bf16*>(lds_raw);
+    unsigned char* lds = lds_raw;
     if (static_cast<int>(blockIdx.x) < beside.blocks) {
         // one of the step's decode work items: the workgroup's first four wavefronts, the stages' LDS
         static_assert(decode_lds_floats(HD) * 4 <= StageLayout<HD>::BYTES, "the decode item's sums must fit into the stages");
@@ -389,6 +410,8 @@ __global__ __launch_bounds__(256 * KW) void attention_prefill_shared_kernel(
                               (b % per_seq) / beside.nsplit, b % beside.nsplit, reinterpret_cast<float*>(lds_raw));
         return;
     }
+    if (threadIdx.x < HD / 16 * 4)                          // (an item meets before it reads them)
+        *reinterpret_cast<unsigned*>(lds + StageLayout<HD>::ZEROS + threadIdx.x / 4 * 512 + threadIdx.x % 4 * 4) = 0;
     const int head_groups = n_q / HPW;
     const int n_items = spans * head_groups * (SPLIT ? nsplit : 1);
     if (queue == nullptr) {
@@ -403,7 +426,7 @@ __global__ __launch_bounds__(256 * KW) void attention_prefill_shared_kernel(
             if (item >= n_items) continue;                 // (only in the last round)
             if (round > 0) __syncthreads();                // everybody is done with the last item's LDS
             const int whole = SPLIT ? item / nsplit : item;
-            prefill_item<HD, QT, HPW, KW, SPLIT>(whole / head_groups, whole % head_groups, SPLIT ? item % nsplit : 0, nsplit,
+            prefill_item<HD, QT, HPW, SPLIT>(whole / head_groups, whole % head_groups, SPLIT ? item % nsplit : 0, nsplit,
                                                  run, part_o, part_ml, lds, q, k_cache, v_cache, out, q_start, ctx_len,
                                                  block_table, max_blocks, n_seq, n_q, n_kv, page, scale, window);
         }
@@ -416,7 +439,7 @@ __global__ __launch_bounds__(256 * KW) void attention_prefill_shared_kernel(
         const int item = __builtin_amdgcn_readfirstlane(next_item);
         if (item >= n_items) break;                        // the counter only grows: every workgroup gets here
         const int whole = SPLIT ? item / nsplit : item;     // (an item's runs are neighbours in the queue)
-        prefill_item<HD, QT, HPW, KW, SPLIT>(whole / head_groups, whole % head_groups, SPLIT ? item % nsplit : 0, nsplit,
+        prefill_item<HD, QT, HPW, SPLIT>(whole / head_groups, whole % head_groups, SPLIT ? item % nsplit : 0, nsplit,
                                              run, part_o, part_ml, lds, q, k_cache, v_cache, out, q_start, ctx_len,
                                              block_table, max_blocks, n_seq, n_q, n_kv, page, scale, window);
     }
@@ -430,8 +453,6 @@ __global__ __launch_bounds__(256 * KW) void attention_prefill_shared_kernel(
     }
 }
 
-constexpr long kSplitBelowItems = 768;
-
 static int heads_per_workgroup(int n_q, int n_kv) {
     const int G = n_q / n_kv;
     return G % 4 == 0 ? 4 : (G % 2 == 0 ? 2 : 1);
@@ -441,22 +462,23 @@ static int heads_per_workgroup(int n_q, int n_kv) {
 // fewer items to spread over the chip), times the row groups of a workgroup. The caller may halve
 // them (16 per row group) where a step has few items: an item's time is set by its walk over the
 // keys, a stretch after the other, and a stretch of 16 rows is shorter than one of 32. Measured on
-// whole prompts (us, 32 / 16 rows; 32 query and 8 kv heads): heads of 64, 256 tokens 9.6 / 7.2, 1,024
-// 20.7 / 17.1, 2,048 40.0 / 39.1, 3,072 80.8 / 73.6, 4,096 96.8 / 121; heads of 128, 512 tokens 19.0 /
-// 15.4, 1,024 30.0 / 29.0, 2,048 57.8 / 71.7: half the rows win until the items of 32 rows number
-// one workgroup less per compute unit than LDS lets it hold (four with heads of 64, two with 128).
+// whole prompts (us, 32 / 16 rows; 32 query and 8 kv heads): heads of 64, 256 tokens 8.2 / 6.5, 1,024
+// 19.4 / 15.4, 2,048 36.9 / 32.7, 2,500 45.8 / 44.5, 2,700 49.5 / 53.1, 3,072 59.0 / 63.3; heads of 128, 512 tokens 15.9 /
+// 12.0, 1,000 26.2 / 21.1, 1,600 41.4 / 36.5, 1,800 46.2 / 45.6, 2,048 53.7 / 54.8; 24 query heads, 2,000 tokens 48.5 / 44.1, 2,400
+// 59.5 / 59.2, 3,000 75 / 86: half the rows win until the items of 32 rows number two and a half a compute unit with heads
+// of 64 and seven quarters with heads of 128.
 int prefill_shared_rows(int hd, int n_q, int n_kv) {
     if ((hd != 64 && hd != 128) || n_kv <= 0 || n_q % n_kv != 0) return 0;
     return 32 * (4 / heads_per_workgroup(n_q, n_kv));
 }
 
-template <int HD, int QT, int HPW, int KW, bool SPLIT>
+template <int HD, int QT, int HPW, bool SPLIT>
 static int launch_shared(const bf16* q, const bf16* kc, const bf16* vc, bf16* out, const int* q_start,
                          const int* ctx_len, const int* table, int max_blocks, int n_seq, int n_q, int n_kv, int page,
                          float scale, int window, int items, int* queue, int nsplit, int run, float* part_o,
                          float* part_ml, const DecodeBeside& beside, hipStream_t stream) {
     constexpr int LDS = StageLayout<HD>::BYTES;
-    auto kernel = attention_prefill_shared_kernel<HD, QT, HPW, KW, SPLIT>;
+    auto kernel = attention_prefill_shared_kernel<HD, QT, HPW, SPLIT>;
     static OncePerDevice told;                         // per instantiation
     const int status = allow_lds(told, reinterpret_cast<const void*>(kernel), LDS);
     if (status != 0) return status;
@@ -466,7 +488,7 @@ static int launch_shared(const bf16* q, const bf16* kc, const bf16* vc, bf16* ou
         hipError_t e = hipGetDevice(&dev);
         if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
         if (e == hipSuccess)
-            e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kernel), 256 * KW,
+            e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kernel), 256,
                                                              LDS);
         if (e != hipSuccess) return static_cast<int>(e);
         resident = cus * (per_cu > 0 ? per_cu : 1);
@@ -476,7 +498,7 @@ static int launch_shared(const bf16* q, const bf16* kc, const bf16* vc, bf16* ou
     // against 47.5 with the counter; 4,096 tokens, 1,024 items on 768, 101.8 against 115.6; 8,192 tokens,
     // 2,048 items on 768, 359 against 340)
     int* counter = n_items <= 2 * resident ? nullptr : queue;
-    hipLaunchKernelGGL(kernel, dim3(beside.blocks + (n_items < resident ? n_items : resident)), dim3(256 * KW), LDS, stream,
+    hipLaunchKernelGGL(kernel, dim3(beside.blocks + (n_items < resident ? n_items : resident)), dim3(256), LDS, stream,
                        q, kc, vc, out, q_start, ctx_len, table, max_blocks, n_seq, n_q, n_kv, page, scale, window, items,
                        counter, nsplit, run, part_o, part_ml, beside);
     return launch_status();
@@ -485,25 +507,19 @@ static int launch_shared(const bf16* q, const bf16* kc, const bf16* vc, bf16* ou
 int launch_prefill_shared(const bf16* q, const bf16* kc, const bf16* vc, bf16* out, const int* q_start,
                           const int* ctx_len, const int* table, int max_blocks, int n_seq, int n_q, int n_kv, int hd,
                           int page, float scale, int window, int items, int rows_per_item, int* queue, int nsplit,
-                          int run, float* part_o, float* part_ml, int key_waves, const DecodeBeside& beside,
+                          int run, float* part_o, float* part_ml, const DecodeBeside& beside,
                           hipStream_t stream) {
     if (queue == nullptr) return kErrBadArgument;
     if (nsplit < 1 || (nsplit > 1 && (run < 1 || part_o == nullptr || part_ml == nullptr))) return kErrBadArgument;
     const int hpw = heads_per_workgroup(n_q, n_kv);
     const int rows = rows_per_item / (4 / hpw);            // per row group
-    // Two wavefronts per tile while the items are too few to keep three workgroups of four
-    // wavefronts on every compute unit: then an item's length, not the chip, sets the time.
-    int kw = static_cast<long>(items) * (n_q / hpw) <= kSplitBelowItems ? 2 : 1;
-    if (key_waves == 1 || key_waves == 2) kw = key_waves;  // (forced by the caller: tests, measurements)
 #define LLME_SHARED_ARGS q, kc, vc, out, q_start, ctx_len, table, max_blocks, n_seq, n_q, n_kv, page, scale, window, \
                          items, queue, nsplit, run, part_o, part_ml, beside, stream
 #define LLME_SHARED(HD, QT, HPW)                                                       \
     if (hd == HD && rows == 16 * QT && hpw == HPW) {                                   \
         if (nsplit > 1)                                                                \
-            return kw == 2 ? launch_shared<HD, QT, HPW, 2, true>(LLME_SHARED_ARGS)     \
-                           : launch_shared<HD, QT, HPW, 1, true>(LLME_SHARED_ARGS);    \
-        return kw == 2 ? launch_shared<HD, QT, HPW, 2, false>(LLME_SHARED_ARGS)        \
-                       : launch_shared<HD, QT, HPW, 1, false>(LLME_SHARED_ARGS);       \
+            return launch_shared<HD, QT, HPW, true>(LLME_SHARED_ARGS);                 \
+        return launch_shared<HD, QT, HPW, false>(LLME_SHARED_ARGS);                    \
     }
     LLME_SHARED(64, 2, 4) LLME_SHARED(64, 2, 2) LLME_SHARED(64, 2, 1)
     LLME_SHARED(128, 2, 4) LLME_SHARED(128, 2, 2) LLME_SHARED(128, 2, 1)

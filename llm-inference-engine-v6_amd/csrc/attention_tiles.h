@@ -361,6 +361,12 @@ __device__ __forceinline__ void load_1kb_to_lds_once(const void* base, unsigned 
                  : "s"(lds_base), "v"(voffset), "s"(rsrc), "s"(soffset)
                  : "memory", "m0");
 }
+__device__ __forceinline__ void load_1kb_to_lds(u32x4 rsrc, unsigned lds_base, unsigned voffset, unsigned soffset) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :
+                 : "s"(lds_base), "v"(voffset), "s"(rsrc), "s"(soffset)
+                 : "memory", "m0");
+}
 // Waits until at most N of the wavefront's vector memory operations are on their way, for the compiler's loads from LDS too.
 template <int N> __device__ __forceinline__ void wait_loads() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
@@ -751,7 +757,7 @@ struct DecodeBeside {
 int launch_prefill_shared(const bf16* q, const bf16* k_cache, const bf16* v_cache, bf16* out, const int* q_start,
                           const int* ctx_len, const int* block_table, int max_blocks, int n_seq, int n_q, int n_kv,
                           int hd, int page, float scale, int window, int items, int rows_per_item, int* queue,
-                          int nsplit, int run, float* part_o, float* part_ml, int key_waves, const DecodeBeside& beside,
+                          int nsplit, int run, float* part_o, float* part_ml, const DecodeBeside& beside,
                           hipStream_t stream);
 
 // Runs that the keys [k_begin, key_end) of a prefill work item are cut into: `run` stretches of 64

@@ -367,8 +367,8 @@ def attention_tuning(rows: int = 0, shared: int = -1, read_once: int = -1, half_
     """Overrides of the attention kernels' launch choices for one call (tests, measurements), as
     the entry points take them; 0 leaves every choice to the entry point. rows: rows per work item
     of the prefill kernel without LDS (16, 32, 64; 0: by head size). shared: the prefill kernel that
-    shares K and V through LDS: -1 where it takes the sizes, 0 never, 1 wherever it can, 2 / 3 with
-    one / two wavefronts per tile whatever the number of items. read_once: the decode kernel's
+    shares K and V through LDS: -1 where it takes the sizes, 0 never, 1, 2 or 3 wherever it
+    can. read_once: the decode kernel's
     cache hint on keys and values: -1 the entry point chooses, 0 off, 1 on. half_rows: work items of
     half the rows in the kernel that shares K and V (plan_attention sets it by itself for steps with
     few items; the choice prefill_half_rows False keeps it from that)."""
@@ -447,10 +447,10 @@ def plan_attention(new_lens, ctx_lens, n_q: int, n_kv: int, head_dim: int, plan_
         if splits > 1:
             plan["prefill_splits"], plan["prefill_run"] = splits, run
         elif (ch.prefill_half_rows and not tuning & TUNING_HALF_ROWS
-              and items <= (3 if head_dim == 64 else 1) * compute_units()):
+              and 4 * items <= (10 if head_dim == 64 else 7) * compute_units()):
             # few items whose keys are not cut (short prompts, portions early in a prompt): work items of
-            # half the rows, until the items of whole rows number one workgroup less per compute unit than
-            # LDS lets it hold (measurements in attention_prefill.hip). Where the keys are cut the items are
+            # half the rows, until the items of whole rows number two and a half a compute unit with heads of 64,
+            # seven quarters with heads of 128 (measurements in attention_prefill.hip). Where the keys are cut the items are
             # many already, and half rows were no faster (256 tokens behind 16,128: 2.75 against 2.66 ms a step).
             tuning |= TUNING_HALF_ROWS
         if tuning & TUNING_HALF_ROWS:
