@@ -86,7 +86,8 @@ __device__ __forceinline__ void prefill_item(int bx, int by, int z, int nsplit, 
         acc += nt;
     }
     if (!found) return;                                    // the whole workgroup
-    const int tid = threadIdx.x;
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));                          // (what is made of it is made per item, and not kept in registers from one to the next)
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63, r = lane & 15, g4 = lane >> 4;
     const int G = n_q / n_kv;
@@ -386,12 +387,14 @@ __device__ __forceinline__ void prefill_item(int bx, int by, int z, int nsplit, 
 // leaves most of the chip idle while the few longest finish. queue[0] counts the items taken,
 // queue[1] the workgroups that have left; both are zero before and after the kernel (the last
 // workgroup to leave clears them), so the same two integers serve every launch on a stream.
-// (Registers: 128 with heads of 64 and one tile of rows a wavefront, for four workgroups a unit: 2,048 tokens 34.2 us with three, 32.7 with four.
-// Otherwise up to 256, for the two that LDS holds of heads of 128.)
-template <int HD, int QT>
-constexpr int kWavesASimd = HD == 64 && QT == 1 ? 4 : 2;
+// (Registers: 128 with heads of 64, whole keys and one tile of rows a wavefront, for four workgroups a unit: 2,048 tokens 34.2 us with three,
+// 32.7 with four. Otherwise up to 256, for the two that LDS holds of heads of 128. None of it may lie in scratch memory: with prefill_item inlined
+// twice, once for the fixed order and once for the counter, and with what it makes of the thread's number hoisted in front of the loop, 12 registers did,
+// and short items fetched them in front of their keys: 256 rows behind 1,024 beside 18 decoded requests 20.5 us a launch, 19.8 without.)
+template <int HD, int QT, bool SPLIT>
+constexpr int kWavesASimd = HD == 64 && QT == 1 && !SPLIT ? 4 : 2;
 template <int HD, int QT, int HPW, bool SPLIT>
-__global__ __launch_bounds__(256, (kWavesASimd<HD, QT>)) void attention_prefill_shared_kernel(
+__global__ __launch_bounds__(256, (kWavesASimd<HD, QT, SPLIT>)) void attention_prefill_shared_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k_cache, const bf16* __restrict__ v_cache,
     bf16* __restrict__ out, const int* __restrict__ q_start, const int* __restrict__ ctx_len,
     const int* __restrict__ block_table, int max_blocks, int n_seq, int n_q, int n_kv, int page, float scale,
@@ -414,35 +417,27 @@ __global__ __launch_bounds__(256, (kWavesASimd<HD, QT>)) void attention_prefill_
         *reinterpret_cast<unsigned*>(lds + StageLayout<HD>::ZEROS + threadIdx.x / 4 * 512 + threadIdx.x % 4 * 4) = 0;
     const int head_groups = n_q / HPW;
     const int n_items = spans * head_groups * (SPLIT ? nsplit : 1);
-    if (queue == nullptr) {
-        // Few items per workgroup: a fixed order, to and fro over the workgroups (the items are
-        // sorted, heaviest first: workgroup w of G takes w, 2 G - 1 - w, 2 G + w, ..), so that every
-        // workgroup's items add up to about the same number of keys. The counter's answer is a trip
-        // to memory per item, with two barriers around it, and costs more than its evening-out
-        // wins until a workgroup has several items to take.
-        const int G = static_cast<int>(gridDim.x) - beside.blocks, w = static_cast<int>(blockIdx.x) - beside.blocks;
-        for (int round = 0; round * G < n_items; ++round) {
-            const int item = round * G + ((round & 1) ? G - 1 - w : w);
-            if (item >= n_items) continue;                 // (only in the last round)
-            if (round > 0) __syncthreads();                // everybody is done with the last item's LDS
-            const int whole = SPLIT ? item / nsplit : item;
-            prefill_item<HD, QT, HPW, SPLIT>(whole / head_groups, whole % head_groups, SPLIT ? item % nsplit : 0, nsplit,
-                                                 run, part_o, part_ml, lds, q, k_cache, v_cache, out, q_start, ctx_len,
-                                                 block_table, max_blocks, n_seq, n_q, n_kv, page, scale, window);
+    // Few items per workgroup (no queue): a fixed order, to and fro over the workgroups (the items are
+    // sorted, heaviest first: workgroup w of G takes w, 2 G - 1 - w, 2 G + w, ..), so that every
+    // workgroup's items add up to about the same number of keys. The counter's answer is a trip
+    // to memory per item, with two barriers around it, and costs more than its evening-out
+    // wins until a workgroup has several items to take.
+    const int G = static_cast<int>(gridDim.x) - beside.blocks, w = static_cast<int>(blockIdx.x) - beside.blocks;
+    for (int round = 0;; ++round) {
+        if (queue != nullptr || round > 0) __syncthreads();    // everybody is done with the last item's LDS
+        int item = round * G + ((round & 1) ? G - 1 - w : w);
+        if (queue != nullptr) {
+            if (threadIdx.x == 0) next_item = atomicAdd(queue, 1);
+            __syncthreads();
+            item = __builtin_amdgcn_readfirstlane(next_item);
         }
-        return;
-    }
-    for (;;) {
-        __syncthreads();                                   // everybody is done with the last item's LDS
-        if (threadIdx.x == 0) next_item = atomicAdd(queue, 1);
-        __syncthreads();
-        const int item = __builtin_amdgcn_readfirstlane(next_item);
-        if (item >= n_items) break;                        // the counter only grows: every workgroup gets here
-        const int whole = SPLIT ? item / nsplit : item;     // (an item's runs are neighbours in the queue)
+        if (item >= n_items) break;                        // the counter, and the first item of a round, only grow: every workgroup gets here
+        const int whole = SPLIT ? item / nsplit : item;     // (an item's runs are neighbours in either order)
         prefill_item<HD, QT, HPW, SPLIT>(whole / head_groups, whole % head_groups, SPLIT ? item % nsplit : 0, nsplit,
                                              run, part_o, part_ml, lds, q, k_cache, v_cache, out, q_start, ctx_len,
                                              block_table, max_blocks, n_seq, n_q, n_kv, page, scale, window);
     }
+    if (queue == nullptr) return;
     if (threadIdx.x == 0) {
         // whoever leaves last has seen every other workgroup take its final number: nobody touches
         // the counter any more
