@@ -294,7 +294,8 @@ static int launch_staged(int hd, dim3 grid, hipStream_t stream, ARGS... args) {
 // the entry points' `tuning` argument (0: every choice is the entry point's):
 //   bits 0-7   rows per work item of the prefill kernel without LDS: 16, 32 or 64 (0: by head size)
 //   bits 8-11  1 + shared: -1 the kernel that shares K and V through LDS where it takes the sizes
-//              (the default), 0 never, 1, 2 or 3 wherever it can
+//              (the default), 0 never, 1 wherever it can, 2 / 3 the same with work items of whole / half the rows
+//              whatever their number (2: who plans the step does not set bit 15; 3: as with bit 15)
 //   bits 12-13 1 + read_once: whether the decode kernel loads keys and values with the read-once
 //              hint: -1 the entry point chooses, 0 never, 1 always
 //   bit 14     the decode kernel's splits are left unjoined in part_o / part_ml: the caller joins them
@@ -308,8 +309,7 @@ static bool parse_tuning(int packed, Tuning* t) {
     if (packed < 0 || packed >= (1 << 16)) return false;
     const int rows = packed & 0xFF, shared = ((packed >> 8) & 0xF) - 1, read_once = ((packed >> 12) & 0x3) - 1;
     if (rows % 16 != 0 || rows > 64 || shared > 3 || read_once > 1) return false;
-    *t = Tuning{rows, shared > 1 ? 1 : shared, read_once, (packed >> 14) & 1,
-                (packed >> 15) & 1};
+    *t = Tuning{rows, shared > 1 ? 1 : shared, read_once, (packed >> 14) & 1, shared == 3 ? 1 : (packed >> 15) & 1};
     return true;
 }
 static bool decode_reads_once(const Tuning& t) { return t.read_once != 0; }

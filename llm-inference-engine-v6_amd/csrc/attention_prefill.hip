@@ -390,7 +390,7 @@ __device__ __forceinline__ void prefill_item(int bx, int by, int z, int nsplit, 
 // (Registers: 128 with heads of 64, whole keys and one tile of rows a wavefront, for four workgroups a unit: 2,048 tokens 34.2 us with three,
 // 32.7 with four. Otherwise up to 256, for the two that LDS holds of heads of 128. None of it may lie in scratch memory: with prefill_item inlined
 // twice, once for the fixed order and once for the counter, and with what it makes of the thread's number hoisted in front of the loop, 12 registers did,
-// and short items fetched them in front of their keys: 256 rows behind 1,024 beside 18 decoded requests 20.5 us a launch, 19.8 without.)
+// and short items fetched them in front of their keys: 256 rows behind 1,024 beside 17 decoded requests 20.5 us a launch, 19.8 without.)
 template <int HD, int QT, bool SPLIT>
 constexpr int kWavesASimd = HD == 64 && QT == 1 && !SPLIT ? 4 : 2;
 template <int HD, int QT, int HPW, bool SPLIT>
@@ -404,9 +404,8 @@ __global__ __launch_bounds__(256, (kWavesASimd<HD, QT, SPLIT>)) void attention_p
     __shared__ int next_item;
     unsigned char* lds = lds_raw;
     if (static_cast<int>(blockIdx.x) < beside.blocks) {
-        // one of the step's decode work items: the workgroup's first four wavefronts, the stages' LDS
-        static_assert(decode_lds_floats(HD) * 4 <= StageLayout<HD>::BYTES, "the decode item's sums must fit into the stages");
-        if (threadIdx.x >= DEC_WAVES * 64) return;
+        // one of the step's decode work items: the workgroup's four wavefronts, the stages' LDS
+        static_assert(DEC_WAVES * 64 == 256 && decode_lds_floats(HD) * 4 <= StageLayout<HD>::BYTES, "the decode item's sums must fit into the stages");
         const int b = blockIdx.x, per_seq = beside.head_tiles * beside.nsplit;
         decode_item<HD, true>(q, k_cache, v_cache, out, beside.part_o, beside.part_ml, q_start, ctx_len, block_table,
                               max_blocks, n_q, n_kv, page, scale, window, beside.split_len, beside.nsplit, b / per_seq,

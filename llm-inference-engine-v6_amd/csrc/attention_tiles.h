@@ -500,7 +500,7 @@ __device__ __forceinline__ void load_q(const bf16* qrow, bool ok, bf16x8 (&qf)[(
 
 
 // ------------------------------------------------------------------------------------------
-// decode: one token per request. A workgroup's four wavefronts (the first DEC_WAVES of it) take
+// decode: one token per request. A workgroup's DEC_WAVES wavefronts take
 // one split of the keys of one (request s, kv head and tile of 16 query heads `head_tile`, split);
 // they take every fourth 32-key block each and add up through LDS (sh: decode_lds_floats(HD)
 // floats). A device function so that two kernels can hold it: the decode kernel, and the kernel

@@ -367,17 +367,22 @@ def attention_tuning(rows: int = 0, shared: int = -1, read_once: int = -1, half_
     """Overrides of the attention kernels' launch choices for one call (tests, measurements), as
     the entry points take them; 0 leaves every choice to the entry point. rows: rows per work item
     of the prefill kernel without LDS (16, 32, 64; 0: by head size). shared: the prefill kernel that
-    shares K and V through LDS: -1 where it takes the sizes, 0 never, 1, 2 or 3 wherever it
-    can. read_once: the decode kernel's
+    shares K and V through LDS: -1 where it takes the sizes, 0 never, 1 wherever it can, 2 / 3 the same
+    with work items of whole / half the rows whatever their number. read_once: the decode kernel's
     cache hint on keys and values: -1 the entry point chooses, 0 off, 1 on. half_rows: work items of
-    half the rows in the kernel that shares K and V (plan_attention sets it by itself for steps with
+    half the rows in the kernel that shares K and V, as shared=3 (plan_attention sets it by itself for steps with
     few items; the choice prefill_half_rows False keeps it from that)."""
     if rows not in (0, 16, 32, 64) or not -1 <= shared <= 3 or not -1 <= read_once <= 1:
         raise kernels.KernelError(f"attention_tuning: rows {rows}, shared {shared}, read_once {read_once}")
-    return rows | (shared + 1) << 8 | (read_once + 1) << 12 | (TUNING_HALF_ROWS if half_rows else 0)
+    return rows | (shared + 1) << 8 | (read_once + 1) << 12 | (TUNING_HALF_ROWS if half_rows or shared == 3 else 0)
 
 
 TUNING_HALF_ROWS = 1 << 15
+
+
+def _keeps_whole_rows(tuning: int) -> bool:
+    return tuning >> 8 & 0xF == 1 + 2                      # (shared=2)
+
 
 _work_queues: dict = {}
 
@@ -446,7 +451,7 @@ def plan_attention(new_lens, ctx_lens, n_q: int, n_kv: int, head_dim: int, plan_
             run = (stretches + splits - 1) // splits       # stretches of 64 keys per run
         if splits > 1:
             plan["prefill_splits"], plan["prefill_run"] = splits, run
-        elif (ch.prefill_half_rows and not tuning & TUNING_HALF_ROWS
+        elif (ch.prefill_half_rows and not tuning & TUNING_HALF_ROWS and not _keeps_whole_rows(tuning)
               and 4 * items <= (10 if head_dim == 64 else 7) * compute_units()):
             # few items whose keys are not cut (short prompts, portions early in a prompt): work items of
             # half the rows, until the items of whole rows number two and a half a compute unit with heads of 64,

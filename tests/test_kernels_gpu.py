@@ -624,14 +624,16 @@ def test_attention_mfma_prefill_and_mixed(ops, n_q, n_kv, hd, page):
                                               (8, 2, 128, 16), (2, 1, 128, 32), (5, 5, 128, 16)])
 @pytest.mark.parametrize("rows,shared", [(0, -1), (0, 2), (0, 3), (32, 0), (0, 0)])
 def test_attention_prefill_shared_and_direct(ops, n_q, n_kv, hd, page, rows, shared):
-    """The prefill kernel that shares K and V through LDS, for 4, 2 and 1 heads of a kv head per
-    workgroup, spans that end inside a 64-key stretch, portions that start deep in a context,
+    """The prefill kernel that shares K and V through LDS (items of the planned, of whole and of half the rows), for 4, 2
+    and 1 heads of a kv head per workgroup, spans that end inside a 64-key stretch, portions that start deep in a context,
     and the kernel without LDS at the same sizes."""
     lens = [330, 2, 131, 64, 517, 65, 9]
     news = [330, 2, 67, 64, 130, 3, 1]
     out, ref, plan = _attn_case(ops, lens, news, n_q, n_kv, hd, page, seed=61,
                                 tuning=ops.mfma.attention_tuning(rows=rows, shared=shared))
     assert plan["n_decode"] == 1 and plan["groups"] >= 6
+    if shared >= 2:
+        assert bool(plan["tuning"] & ops.mfma.TUNING_HALF_ROWS) == (shared == 3) and plan["prefill_splits"] == 1
     assert _rel(out, ref) < 8e-3
 
 
@@ -650,13 +652,15 @@ def test_attention_prefill_shared_window(ops, window, n_q, n_kv):
 def test_attention_prefill_cut_keys(ops, n_q, n_kv, hd, page, splits, key_waves, run):
     """Prompt portions whose keys are cut into runs that a second kernel joins: runs that end
     inside a span's own rows, a last run that takes the rest, items with a single run beside items
-    with several (and all of them single), whole prompts and decoded tokens beside them, with one
-    and two wavefronts per tile."""
+    with several (and all of them single), whole prompts and decoded tokens beside them, with items of
+    whole and of half the rows (2, 3)."""
     lens = [700, 2, 131, 64, 517, 65, 9]
     news = [40, 2, 67, 64, 130, 3, 1]
     out, ref, plan = _attn_case(ops, lens, news, n_q, n_kv, hd, page, seed=63, prefill_splits=splits, prefill_run=run,
                                 tuning=ops.mfma.attention_tuning(shared=key_waves))
     assert plan["n_decode"] == 1 and plan["prefill_splits"] == splits
+    if key_waves >= 2:
+        assert bool(plan["tuning"] & ops.mfma.TUNING_HALF_ROWS) == (key_waves == 3)
     assert not out.isnan().any()
     assert _rel(out, ref) < 8e-3
 
@@ -666,8 +670,8 @@ def test_attention_prefill_cut_keys(ops, n_q, n_kv, hd, page, splits, key_waves,
 def test_attention_decoded_tokens_beside_prompt_portions(ops, n_q, n_kv, hd, page, splits, key_waves):
     """A step with decoded tokens far into their requests (their keys cut into several splits) and
     prompt portions (their keys whole or cut into runs): where the prompt kernel shares K and V
-    through LDS, one launch holds both kinds of work and one launch both joins; head size 48 takes
-    the separate kernels."""
+    through LDS, one launch holds both kinds of work and one launch both joins (items of the planned rows, of half
+    and of whole ones: 3, 2); head size 48 takes the separate kernels."""
     lens = [900, 700, 1300, 2, 640, 33, 257]
     news = [1, 40, 1, 2, 1, 1, 130]
     out, ref, plan = _attn_case(ops, lens, news, n_q, n_kv, hd, page, seed=66, prefill_splits=splits if hd != 48 else None,

@@ -24,8 +24,9 @@ def ops():
 def test_turns(ops, hd, n_q, n_kv, page, window, half):
     lens, news = [2, 63, 64, 65, 129, 4230, 4129], [2, 63, 64, 33, 129, 70, 3]
     out, ref, plan = kernel_tests._attn_case(ops, lens, news, n_q, n_kv, hd, page, window=window, seed=71, prefill_splits=1,
-                                             tuning=ops.mfma.attention_tuning(half_rows=half))
-    assert plan["prefill_splits"] == 1 and not out.isnan().any()
+                                             tuning=ops.mfma.attention_tuning(shared=3 if half else 2))
+    assert plan["prefill_splits"] == 1 and bool(plan["tuning"] & ops.mfma.TUNING_HALF_ROWS) == half
+    assert not out.isnan().any()
     assert kernel_tests._rel(out, ref) < 8e-3              # bfloat16 in and out, 32-bit sums
 
 
@@ -40,8 +41,8 @@ def test_values_of_unseen_blocks_reach_no_row(ops, hd, n_q, n_kv, half):
     q = torch.randn(T, n_q * hd, generator=g).to(torch.bfloat16).to(DEV)
     blocks = (T + page - 1) // page
     i32 = dict(dtype=torch.int32, device=DEV)
-    plan = ops.mfma.plan_attention([T], [0], n_q, n_kv, hd, tuning=ops.mfma.attention_tuning(half_rows=half))
-    plan["prefill_splits"] = 1
+    plan = ops.mfma.plan_attention([T], [0], n_q, n_kv, hd, tuning=ops.mfma.attention_tuning(shared=3 if half else 2))
+    assert plan["prefill_splits"] == 1 and bool(plan["tuning"] & ops.mfma.TUNING_HALF_ROWS) == half
 
     def run(values):
         kc = torch.zeros(blocks * page, n_kv, hd)
@@ -63,3 +64,15 @@ def test_values_of_unseen_blocks_reach_no_row(ops, hd, n_q, n_kv, half):
     assert untouched[0] == 0 and untouched[-1] == T - 1
     assert torch.equal(got[untouched], want[untouched]) and not got[untouched].isnan().any()
     assert got[at].isinf().all() and got[at + window - 1].isinf().all()
+
+
+@pytest.mark.parametrize("hd,n_q,n_kv", [(64, 8, 2), (64, 3, 3), (128, 8, 2), (128, 3, 3)])
+@pytest.mark.parametrize("window", [0, 1, 7, 64, 65, 200])
+@pytest.mark.parametrize("half", [False, True])
+def test_turns_behind_a_window_and_beside_decoded_tokens(ops, hd, n_q, n_kv, window, half):
+    """Items of whole and of half the rows whose keys are not cut: first stretches that no row of a wavefront sees yet, decoded tokens in
+    the same launch."""
+    out, ref, plan = kernel_tests._attn_case(ops, [300, 70, 1, 190, 333], [140, 70, 1, 2, 1], n_q, n_kv, hd, 16, window=window, seed=73,
+                                             tuning=ops.mfma.attention_tuning(shared=3 if half else 2))
+    assert plan["prefill_splits"] == 1 and plan["n_decode"] == 2 and bool(plan["tuning"] & ops.mfma.TUNING_HALF_ROWS) == half
+    assert not out.isnan().any() and kernel_tests._rel(out, ref) < 8e-3      # bfloat16 in and out, 32-bit sums
