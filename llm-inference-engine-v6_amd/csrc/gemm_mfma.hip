@@ -925,6 +925,18 @@ static int choose_direct(int mode, int M, int N, int K, bool may_cut, int cus, P
     return large <= staged ? 2 : 0;
 }
 
+// choose_direct's answer where it is asked (panel_takes, of the entry point below, holds), or 0.
+static int direct_choice(int mode, int M, int N, int K, int ksplit, int cus, PanelPlan& plan) {
+    return ksplit <= 1 && M > 64 && K >= kPanelLeastK ? choose_direct(mode, M, N, K, ksplit <= 0, cus, plan) : 0;
+}
+
+// Whether the rotating product takes the plan's tiles of gemm_panel.hip: while they are one round over the chip.
+static bool rotates_in_panels(int M, int N, int K, int hd, PanelPlan& plan) {
+    if (K < kPanelLeastK || K >= (1 << 22)) return false;
+    plan = panel_plan(M, N, K, 1, hd);
+    return plan.mt > 0 && plan.rounds == 1;
+}
+
 }  // namespace llme
 
 using namespace llme;
@@ -1009,9 +1021,9 @@ extern "C" int llme_gemm_bf16(const void* a, const void* w, void* out, int out_d
         if (!panel_takes || bm % 16 != 0 || ksplit > 1) return kErrUnsupported;
         return gemm_panel(bm / 16, bn, mode, A, W, out, M, N, K, 1, QkvTarget{}, t_gate_extra, stream);
     }
-    if (tile_shape <= 0 && panel_takes && direct != 0 && ksplit <= 1 && M > 64 && K >= kPanelLeastK) {
+    if (tile_shape <= 0 && panel_takes && direct != 0) {
         PanelPlan plan;
-        const int kind = choose_direct(mode, M, N, K, ksplit <= 0, cus, plan);
+        const int kind = direct_choice(mode, M, N, K, ksplit, cus, plan);
         if (kind == 1) return gemm_panel(plan.mt, plan.bn, mode, A, W, out, M, N, K, 1, QkvTarget{}, t_gate_extra, stream);
         if (kind == 2) return launch_tile_direct<4, 2, 4, 8>(A, W, out, M, N, K, mode, 1, stream);
     }
@@ -1225,13 +1237,13 @@ extern "C" int llme_gemm_bf16_qkv_rope(const void* a, const void* w, int M, int 
         if (!blocked || bm % 16 != 0 || K >= (1 << 22)) return kErrUnsupported;
         return gemm_panel(bm / 16, bn, kRopeCache, A, W, nullptr, M, N, K, 1, qt, GateExtra{}, stream);
     }
-    if (tile_shape <= 0 && blocked && K >= kPanelLeastK && K < (1 << 22)) {
-        // The tiles of gemm_panel.hip while they are one round over the chip. (Measured, us, weights from memory, the best of the others /
+    if (tile_shape <= 0 && blocked) {
+        // (Measured, us, weights from memory, the best of the others /
         // these: 1B sizes at 20 rows 12.6 / 11.3, 45: 15.1 / 10.7, 273: 14.5 / 11.2, 528: 17.3 / 16.1, 1,024: 25.2 / 21.4, 1,500: 34.0 / 25.4,
         // 2,048 in tiles of 128 x 192: 37.6 / 28.6; 3B sizes at 45 rows 25.7 / 22.3, 1,024: 48.7 / 37.5; 8B sizes at 150 rows 33.2 / 25.0, 528: 44.3 /
         // 36.4, in two 1,024: 69.9 / 70.1.)
-        const PanelPlan plan = panel_plan(M, N, K, 1, hd);
-        if (plan.mt > 0 && plan.rounds == 1) return gemm_panel(plan.mt, plan.bn, kRopeCache, A, W, nullptr, M, N, K, 1, qt, GateExtra{}, stream);
+        PanelPlan plan;
+        if (rotates_in_panels(M, N, K, hd, plan)) return gemm_panel(plan.mt, plan.bn, kRopeCache, A, W, nullptr, M, N, K, 1, qt, GateExtra{}, stream);
     }
     if (tile_shape <= 0) {
         // The tile with the least rounds of workgroups over the compute units x (a round's fixed cost,
@@ -1269,6 +1281,22 @@ extern "C" int llme_gemm_bf16_qkv_rope(const void* a, const void* w, int M, int 
     if (tile_shape == 96064 && hd <= 64) return launch_tile_rope<3, 2>(A, W, M, N, K, blocked, qt, stream);
     if (tile_shape == 96128) return launch_tile_rope<3, 4>(A, W, M, N, K, blocked, qt, stream);
     return kErrBadArgument;
+}
+
+// The tiles that a product with a blocked bfloat16 weight is given on this device (tests, measurements): 1000000 + 1000 x rows + columns of
+// those of gemm_panel.hip, 256256, or 0 for the kernels through staging registers. kind: 0 stored, 1 added, 2 gated, 3 squared rectifier,
+// 4 rotating with heads of `hd` columns (0: not in one round of panel tiles), 5 left in `ksplit` parts. -1: no such product.
+extern "C" int llme_gemm_bf16_chosen(int kind, int M, int N, int K, int ksplit, int hd) {
+    if (kind < 0 || kind > 5 || M <= 0 || N <= 0 || N % 16 != 0 || K <= 0 || K % 32 != 0 || K >= (1 << 22) || (kind == 5 && ksplit < 1) ||
+        (kind == 4 && hd <= 0))
+        return -1;
+    static const int modes[4] = {kStoreF32, kAddF32, kGatedBF16, kSquaredReluBF16};
+    PanelPlan plan{0, 0, 0, 0, 0.f};
+    int way = 1;
+    if (kind == 5) plan = panel_plan(M, N, K, ksplit, 0);
+    else if (kind == 4) way = rotates_in_panels(M, N, K, hd, plan) ? 1 : 0;
+    else way = direct_choice(modes[kind], M, N, K, ksplit, compute_units(), plan);
+    return way == 1 ? kPanelTile + 16000 * plan.mt + plan.bn : way == 2 ? 256256 : 0;
 }
 
 LLME_LOAD_ENTRY(gemm_mfma)

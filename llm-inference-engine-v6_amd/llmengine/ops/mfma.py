@@ -54,6 +54,20 @@ def gemm_bf16(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: b
           "gemm_bf16")
 
 
+declare("llme_gemm_bf16_chosen", [_i, _i, _i, _i, _i, _i])
+_CHOSEN_KINDS = ("stored", "added", "gated", "squared", "rotating", "parts")
+
+
+def gemm_bf16_chosen(kind: str, M: int, N: int, K: int, ksplit: int = 0, head_dim: int = 0) -> int:
+    """The tile that a product [M, K] x blocked [N, K] is given (tests, measurements), as gemm_bf16's `tile` names it: of csrc/gemm_panel.hip,
+    256256, or 0 for the kernels through staging registers. kind: "stored", "added", "gated", "squared", "rotating" (head_dim) or
+    "parts" (ksplit of them)."""
+    got = entry("llme_gemm_bf16_chosen")(_CHOSEN_KINDS.index(kind), M, N, K, ksplit, head_dim)
+    if got < 0:
+        raise kernels.KernelError(f"gemm_bf16_chosen: {kind} [{M}, {K}] x [{N}, {K}], {ksplit} parts, heads of {head_dim}")
+    return got
+
+
 FEW_ROWS = 16                       # rows up to which gated products stream their weights (csrc/gemm_few_rows.hip)
 
 

@@ -95,7 +95,7 @@ def test_panel_tiles_gate_with_biases_and_clamps(ops, T, FF, K, bias, limit):
     other, chosen = run(128), torch.zeros(T, FF, dtype=torch.bfloat16, device=DEV)
     assert _rel(other.cpu().double(), want) < 5e-3
     assert ops.gemm_gated_extra(xd, wb, chosen, 16, bd, limit, alpha) and torch.equal(chosen, other)
-    for rows, cols in TILES:
+    for rows, cols in TILES + [(128, 256), (192, 256)]:
         assert torch.equal(run(PANEL + 1000 * rows + cols), other), (rows, cols)
 
 

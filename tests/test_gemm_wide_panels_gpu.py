@@ -71,12 +71,24 @@ def test_wide_panels_rotate_as_the_others(ops, T, n_q, n_kv, hd, tiles):
         assert all(torch.equal(a, b) for a, b in zip(got, want)), (rows, cols)
 
 
-# rows and columns at which each of these tiles is the chosen one on 256 compute units, k at the least that they are chosen for and above
-@pytest.mark.parametrize("M,N,K,gated", [(2048, 3072, 544, False), (2300, 3072, 2048, False), (2995, 3072, 512, False), (1400, 16384, 512, True),
-                                         (1800, 4608, 2048, False), (1000, 3072, 8192, False)])
-def test_the_chosen_wide_panel_adds_in_the_order_of_the_others(ops, M, N, K, gated):
+def _chosen_on_256_units(ops, want, *args):
+    """That the sizes still mean what the test takes them for (the plans are drawn for 256 compute units)."""
+    got = ops.mfma.gemm_bf16_chosen(*args)
+    assert got == want or ops.mfma.compute_units() != 256, (args, got)
+
+
+# sizes at which each of these tiles is the chosen one, stored and added, or gated (two of them hold pairs), at the least k that they are chosen for
+# and above; and sizes just outside, where the tiles through registers (0), 256 x 256 or narrower panels are
+@pytest.mark.parametrize("M,N,K,gated,tile", [
+    (329, 12288, 2048, False, PANEL + 96192), (1924, 3072, 1024, False, PANEL + 128192), (403, 12288, 2048, False, PANEL + 128192),
+    (2300, 3072, 2048, False, PANEL + 160192), (1800, 4608, 2048, False, PANEL + 192192), (390, 16384, 2048, False, PANEL + 128256),
+    (2119, 4096, 1024, False, PANEL + 192256), (218, 28672, 512, True, PANEL + 128256), (390, 12288, 512, True, PANEL + 128256),
+    (292, 28672, 2048, True, PANEL + 192256), (1287, 6144, 1024, True, PANEL + 192256),
+    (2048, 3072, 544, False, 0), (2995, 3072, 512, False, 256256), (1400, 16384, 512, True, 256256), (1000, 3072, 8192, False, PANEL + 112128)])
+def test_the_chosen_wide_panel_adds_in_the_order_of_the_others(ops, M, N, K, gated, tile):
     a, w = _pair(M, N, K, 25)
     ad, wb = a.to(DEV), ops.block_weight(w.to(DEV))
+    _chosen_on_256_units(ops, tile, "gated" if gated else "stored", M, N, K)
     for accumulate in (False, True):
         if gated and accumulate:
             continue
@@ -86,9 +98,38 @@ def test_the_chosen_wide_panel_adds_in_the_order_of_the_others(ops, M, N, K, gat
         assert torch.equal(got, want), accumulate
 
 
-@pytest.mark.parametrize("M,N,K", [(65, 48, 512), (200, 528, 2080), (273, 12288, 512), (1500, 3072, 544)])
-def test_squared_rectifier_behind_the_panels(ops, M, N, K):
+# shares of k that end inside the others' slabs, a short last one, and empty ones (eight of five slabs of 64 k)
+@pytest.mark.parametrize("M,N,K,n", [(200, 400, 288, 8), (193, 208, 1056, 3), (97, 272, 2080, 2), (385, 528, 544, 3), (129, 256, 4128, 8)])
+@pytest.mark.parametrize("rows,cols", TILES)
+def test_parts_of_a_sum_in_wide_panels(ops, M, N, K, n, rows, cols):
+    """The parts add up to the product (32-bit sums of bfloat16 products: 2e-5), each is there, and run after run they are the same bits."""
+    a, w = _pair(M, N, K, 27)
+    ref = a.double() @ w.double().T
+    ad, wb = a.to(DEV), ops.block_weight(w.to(DEV))
+    parts = [torch.full((n, M, N), float("nan"), device=DEV) for _ in range(2)]
+    for p in parts:
+        ops.mfma.gemm_parts(ad, wb, p, tile=1000 * rows + cols)
+    assert torch.equal(parts[0], parts[1])
+    assert float((parts[0].cpu().double().sum(0) - ref).norm() / ref.norm()) < 2e-5
+
+
+@pytest.mark.parametrize("M,N,K,n,tile", [(1000, 3072, 8192, 2, PANEL + 128192), (800, 4096, 14336, 2, PANEL + 160192)])
+def test_the_chosen_wide_panel_of_a_sum_in_parts(ops, M, N, K, n, tile):
+    _chosen_on_256_units(ops, tile, "parts", M, N, K, n)
+    assert ops.mfma.compute_units() != 256 or ops.mfma.entry("llme_gemm_parts_plan")(M, N, K, 0) == n
+    a, w = _pair(M, N, K, 28)
+    ref = a.double() @ w.double().T
+    ad, wb, parts = a.to(DEV), ops.block_weight(w.to(DEV)), torch.full((n, M, N), float("nan"), device=DEV)
+    ops.mfma.gemm_parts(ad, wb, parts)
+    assert float((parts.cpu().double().sum(0) - ref).norm() / ref.norm()) < 2e-5
+
+
+# (the third and the fourth: the chosen tile is no panel)
+@pytest.mark.parametrize("M,N,K,tile", [(65, 48, 512, PANEL + 32064), (200, 528, 2080, PANEL + 32064), (273, 12288, 512, 0), (1500, 3072, 544, 0),
+                                        (325, 12288, 1024, PANEL + 96192), (1287, 6144, 1024, PANEL + 192192)])
+def test_squared_rectifier_behind_the_panels(ops, M, N, K, tile):
     """The squared positive part, stored in bfloat16: every tile and the chosen one give the bits of the square of the stored sum."""
+    _chosen_on_256_units(ops, tile, "squared", M, N, K)
     a, w = _pair(M, N, K, 26)
     ad, wb = a.to(DEV), ops.block_weight(w.to(DEV))
     p = torch.empty(M, N, device=DEV)
