@@ -883,13 +883,26 @@ constexpr int kPanelTile = 1000000;
 // faster (us, tiles through registers / these: 100 x 768 x 288 5.1 / 4.3, 270 x 4,096 x 384 5.7 / 6.3).
 constexpr int kPanelLeastK = 512;
 
-// For a product of more than 64 rows that gemm_panel.hip takes: 1 where its tiles (plan) are the fastest, 2 where those of 256 x 256 are, 0 where the
+// The squared rectifier's products that the tiles through registers keep: one round of 128 x 96 and narrower ones fills the chip where the panels of the
+// same rows leave a quarter of it idle or read W twice (us, weights from memory, through registers / panels: 112 rows x 12,288 x 2,048 19.1 / 20.3,
+// x 16,384 x 2,048 20.1 / 21.4, x 16,384 x 4,096 34.4 / 38.4, 192 x 12,288 x 2,048 20.4 / 21.8, 249: 21.8 / 24.0, 256 x 12,288 x 4,096 39.1 / 42.1; on the other
+// side of each line 80 x 12,288 x 2,048 17.7 / 17.4, 112 x 11,264 x 2,048 19.4 / 18.7, 160 x 11,264 x 2,048 21.1 / 20.5, 257 x 12,288 x 2,048 30.3 / 24.6, 224 x
+// 9,216 x 2,048 20.6 / 19.4, 192 x 14,336 x 2,048 24.7 / 22.4). Of more than 64 columns a compute unit neither side is better throughout (96 x 20,480 x 2,048
+// 12 % for registers, 256 x 24,576 x 2,048 11 % for panels), and no model here has so many.
+static bool squares_through_registers(int M, int N, int cus) {
+    const long t = static_cast<long>((M + 127) / 128) * ((N + 95) / 96);
+    return N > 64 * cus || (M > 96 && M <= 128 && 2 * t >= cus) || (M > 128 && M <= 256 && t <= cus && (M > 192 ? 10 * t >= 9 * cus : 20 * t >= 19 * cus));
+}
+
+// For a product of more than 64 rows that gemm_panel.hip takes: 1 where its tiles (plan) are the fastest, 2 where those of 256 x 256 are (not said of squares), 0 where the
 // kernels through staging registers are. Up to 64 rows every kernel waits for W, and these (then with k shared out among their
 // wavefronts), a little faster alone (gate/up of the 1B sizes at 64 rows 16.9 / 16.7 us, of 23 x 16,384 x 3,072 22.9 / 20.4), lost it
 // again in the step (decode of 64 requests 1,656 / 1,679 us, of 23 943 / 941). A sum of up to 288 rows that is better cut over k is, by the kernel below
 // (273 x 2,048 x 2,048 is not: 11.5 / 9.0). Everything else by estimates (us, weights from memory; all but sums cut over k give the same bits):
 //  * 256 x 256 tiles take 4 us + 0.0235 a k in a round (gate/up: 700 rows x 16,384 x 2,048 53.3 against 54 to 67 here, 1,024 rows 59.6 / 75, 528 rows
-//    53 / 46.3), less where the end is short (the squared rectifier: 1,800 rows x 12,288 x 2,048 94 against 98 here; 273 rows 31.3 / 23.8).
+//    53 / 46.3). The squared rectifier's 5.5 + 0.0207 a k, whose end is short (1,800 rows x 12,288 x 2,048 94 against 98 here, x 4,096 178 / 190; 273 rows
+//    31.3 / 23.8); what these do not take is left to the code below, which knows the 256 x 256 tiles of squares too (1,800 x 5,120 x 1,024 27.2,
+//    29.4 where this one chose).
 //  * these take 1.17 (added) or 1.06 (stored) times their plan, which was fitted to all kinds.
 //  * 128 x 128 tiles through registers, two a compute unit, take 3 us + 0.0070 to 0.0187 a k, by how many units have two (against these: added
 //    2,048 x 3,072 x 3,072 52.5 / 57.7, 2,048 x 4,096 x 4,096 78.7 / 85.1, but 1,500 rows 77.9 / 52.7; stored 4,096 x 1,536 x 2,048 33.3 /
@@ -902,9 +915,10 @@ static int choose_direct(int mode, int M, int N, int K, bool may_cut, int cus, P
         plan = panel_plan(M, N, K, 0, 0);
         return plan.ksplit == 1 ? 1 : 0;
     }
+    if (mode == kSquaredReluBF16 && squares_through_registers(M, N, cus)) return 0;
     plan = panel_plan(M, N, K, 1, 0, false, is_gated(mode));
     auto tiles = [&](int edge) { return static_cast<long>((M + edge - 1) / edge) * ((N + edge - 1) / edge); };
-    float large = static_cast<float>((tiles(256) + cus - 1) / cus) * (4.f + (mode == kSquaredReluBF16 ? 0.0220f : 0.0235f) * K);
+    float large = static_cast<float>((tiles(256) + cus - 1) / cus) * (mode == kSquaredReluBF16 ? 5.5f + 0.0207f * K : 4.f + 0.0235f * K);
     if (is_gated(mode)) return plan.us <= large ? 1 : 2;
     const float here = plan.us * (mode == kAddF32 ? 1.17f : 1.06f);
     const long t128 = tiles(128), rounds = (t128 + 2 * cus - 1) / (2 * cus);
@@ -922,6 +936,7 @@ static int choose_direct(int mode, int M, int N, int K, bool may_cut, int cus, P
         staged = (t128 * ks + cus - 1) / cus * (0.0091f * K / ks) + 4e-6f * M * N * ks - 1.f;
     }
     if (here <= large && here <= staged) return 1;
+    if (mode == kSquaredReluBF16) return 0;
     return large <= staged ? 2 : 0;
 }
 
@@ -1284,7 +1299,7 @@ extern "C" int llme_gemm_bf16_qkv_rope(const void* a, const void* w, int M, int 
 }
 
 // The tiles that a product with a blocked bfloat16 weight is given on this device (tests, measurements): 1000000 + 1000 x rows + columns of
-// those of gemm_panel.hip, 256256, or 0 for the kernels through staging registers. kind: 0 stored, 1 added, 2 gated, 3 squared rectifier,
+// those of gemm_panel.hip, 256256, or 0 for the rest (through staging registers; squares in 256 x 256 tiles too). kind: 0 stored, 1 added, 2 gated, 3 squared rectifier,
 // 4 rotating with heads of `hd` columns (0: not in one round of panel tiles), 5 left in `ksplit` parts. -1: no such product.
 extern "C" int llme_gemm_bf16_chosen(int kind, int M, int N, int K, int ksplit, int hd) {
     if (kind < 0 || kind > 5 || M <= 0 || N <= 0 || N % 16 != 0 || K <= 0 || K % 32 != 0 || K >= (1 << 22) || (kind == 5 && ksplit < 1) ||

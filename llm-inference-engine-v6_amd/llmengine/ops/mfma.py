@@ -60,7 +60,7 @@ _CHOSEN_KINDS = ("stored", "added", "gated", "squared", "rotating", "parts")
 
 def gemm_bf16_chosen(kind: str, M: int, N: int, K: int, ksplit: int = 0, head_dim: int = 0) -> int:
     """The tile that a product [M, K] x blocked [N, K] is given (tests, measurements), as gemm_bf16's `tile` names it: of csrc/gemm_panel.hip,
-    256256, or 0 for the kernels through staging registers. kind: "stored", "added", "gated", "squared", "rotating" (head_dim) or
+    256256, or 0 for the rest (the kernels through staging registers; squares in 256 x 256 tiles too). kind: "stored", "added", "gated", "squared", "rotating" (head_dim) or
     "parts" (ksplit of them)."""
     got = entry("llme_gemm_bf16_chosen")(_CHOSEN_KINDS.index(kind), M, N, K, ksplit, head_dim)
     if got < 0:

@@ -124,8 +124,9 @@ def test_the_chosen_wide_panel_of_a_sum_in_parts(ops, M, N, K, n, tile):
     assert float((parts.cpu().double().sum(0) - ref).norm() / ref.norm()) < 2e-5
 
 
-# (the third and the fourth: the chosen tile is no panel)
+# (0: the chosen tile is no panel)
 @pytest.mark.parametrize("M,N,K,tile", [(65, 48, 512, PANEL + 32064), (200, 528, 2080, PANEL + 32064), (273, 12288, 512, 0), (1500, 3072, 544, 0),
+                                        (249, 12288, 1024, 0),
                                         (325, 12288, 1024, PANEL + 96192), (1287, 6144, 1024, PANEL + 192192)])
 def test_squared_rectifier_behind_the_panels(ops, M, N, K, tile):
     """The squared positive part, stored in bfloat16: every tile and the chosen one give the bits of the square of the stored sum."""
