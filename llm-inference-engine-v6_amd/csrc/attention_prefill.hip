@@ -17,10 +17,11 @@
 // every operand a step before it is multiplied, loads straight into LDS a stretch ahead (K two: its scores are a turn ahead), meets once, and has
 // the matrix cores add up the weights (a column of ones: 4 instructions for 64 of the vector units'). Two wavefronts for a
 // tile, each with half the keys, which steps of few items used to take, are no faster now (45 to 1,024 tokens: 1 to 4 % slower, 256 rows behind
-// 8,192: 50 / 40; 256 rows behind 1,024 beside 17 decoded requests took 20.7 with them, 21.0 without).
-// Measured on whole prompts, us, before / now, 32 query and 8 kv heads: heads of 64, 512 tokens 9.8 / 9.2, 1,024 17.7 / 15.4, 2,048 43.5 / 33.0, 4,096
-// 120 / 99, 8,192 387 / 318 (862 TFLOP/s); heads of 128, 1,024 30.5 / 21.6, 2,048 64 / 53.6, prompts of 2,000, 3,691 and 2,500 together
-// 291 / 220 (890 TFLOP/s); 256 rows behind 8,192, heads of 64, in 8 runs of keys 54 / 40.
+// 8,192: 50 / 40).
+// Measured on one card, us, one thing after the other / so, 32 query and 8 kv heads: heads of 64, 45 tokens 4.74 / 4.85, 512 9.6 / 9.4, 1,024 17.0 / 15.0,
+// 2,048 39.3 / 30.8, 4,096 109 / 88, 8,192 390 / 321 (857 TFLOP/s); heads of 128, 1,024 29.0 / 20.6, 2,048 58.9 / 49.2, prompts of 2,000, 3,691 and 2,500
+// together 282 / 208 (940 TFLOP/s); 256 rows behind 8,192, heads of 64, in 8 runs of keys 51 / 40, behind 1,024 beside 17 decoded requests 20.1 / 19.9.
+// (Cards differ: 2,048 tokens with heads of 64 took 30.2 to 36.7, 8,192 305 to 337.)
 //
 // Takes head sizes 64 and 128 and pages that are multiples of 16; other sizes go to the kernel
 // without LDS.
@@ -387,8 +388,8 @@ __device__ __forceinline__ void prefill_item(int bx, int by, int z, int nsplit, 
 // leaves most of the chip idle while the few longest finish. queue[0] counts the items taken,
 // queue[1] the workgroups that have left; both are zero before and after the kernel (the last
 // workgroup to leave clears them), so the same two integers serve every launch on a stream.
-// (Registers: 128 with heads of 64, whole keys and one tile of rows a wavefront, for four workgroups a unit: 2,048 tokens 34.2 us with three,
-// 32.7 with four. Otherwise up to 256, for the two that LDS holds of heads of 128. None of it may lie in scratch memory: with prefill_item inlined
+// (Registers: 128 with heads of 64, whole keys and one tile of rows a wavefront, for the four workgroups a unit that LDS holds (three are as
+// fast: 2,048 tokens 30.6 us, 30.4 with four). Otherwise up to 256, for the two that LDS holds of heads of 128. None of it may lie in scratch memory: with prefill_item inlined
 // twice, once for the fixed order and once for the counter, and with what it makes of the thread's number hoisted in front of the loop, 12 registers did,
 // and short items fetched them in front of their keys: 256 rows behind 1,024 beside 17 decoded requests 20.5 us a launch, 19.8 without.)
 template <int HD, int QT, bool SPLIT>
@@ -456,11 +457,11 @@ static int heads_per_workgroup(int n_q, int n_kv) {
 // fewer items to spread over the chip), times the row groups of a workgroup. The caller may halve
 // them (16 per row group) where a step has few items: an item's time is set by its walk over the
 // keys, a stretch after the other, and a stretch of 16 rows is shorter than one of 32. Measured on
-// whole prompts (us, 32 / 16 rows; 32 query and 8 kv heads): heads of 64, 256 tokens 8.2 / 6.5, 1,024
-// 19.4 / 15.4, 2,048 36.9 / 32.7, 2,500 45.8 / 44.5, 2,700 49.5 / 53.1, 3,072 59.0 / 63.3; heads of 128, 512 tokens 15.9 /
-// 12.0, 1,000 26.2 / 21.1, 1,600 41.4 / 36.5, 1,800 46.2 / 45.6, 2,048 53.7 / 54.8; 24 query heads, 2,000 tokens 48.5 / 44.1, 2,400
-// 59.5 / 59.2, 3,000 75 / 86: half the rows win until the items of 32 rows number two and a half a compute unit with heads
-// of 64 and seven quarters with heads of 128.
+// whole prompts (us, 32 / 16 rows; 32 query and 8 kv heads): heads of 64, 256 tokens 8.5 / 6.7, 1,024
+// 19.5 / 15.3, 2,048 35.8 / 31.1, 2,500 42.4 / 41.4, 2,700 45.1 / 46.6, 3,072 52.4 / 58.2; heads of 128, 512 tokens 15.4 /
+// 11.5, 1,000 25.1 / 19.7, 1,600 38.2 / 33.2, 1,800 43.0 / 40.8, 2,048 48.9 / 49.0; 24 query heads, 2,000 tokens 44.9 / 38.4, 2,400
+// 54.4 / 51.1, 3,000 69 / 80: half the rows win until the items of 32 rows number two and a half a compute unit with heads
+// of 64 and, at least, seven quarters with heads of 128.
 int prefill_shared_rows(int hd, int n_q, int n_kv) {
     if ((hd != 64 && hd != 128) || n_kv <= 0 || n_q % n_kv != 0) return 0;
     return 32 * (4 / heads_per_workgroup(n_q, n_kv));
@@ -488,9 +489,12 @@ static int launch_shared(const bf16* q, const bf16* kc, const bf16* vc, bf16* ou
         resident = cus * (per_cu > 0 ? per_cu : 1);
     }
     const int n_items = items * (n_q / HPW) * (SPLIT ? nsplit : 1);
-    // (measured, 32/8 heads of 64: 2,048 tokens, 512 items on 256 workgroups, 40.8 us in the fixed order
-    // against 47.5 with the counter; 4,096 tokens, 1,024 items on 768, 101.8 against 115.6; 8,192 tokens,
-    // 2,048 items on 768, 359 against 340)
+    // (measured with 32 query and 8 kv heads, us, fixed order / counter; 512 workgroups are resident with items of 32 rows. Up to two rounds the
+    // fixed order wins by up to 17 % and loses 5 % at most: heads of 64, 4,096 tokens, 1,024 items, 87.4 / 93.2, three prompts of 1,000 28.8 / 34.9, four of
+    // 700 behind 2,048 88.3 / 84.1; heads of 128, 2,048 tokens 48.2 / 54.1, 4,096 134 / 139. Between two and three it is 4 to 11 % faster where requests
+    // are equal (5,000 tokens 121 / 126, three prompts of 1,500 49.0 / 55.1), but 7 to 31 % slower where a long one is not the first or long ones meet
+    // (900, 1,300, 3,000 and 700 tokens 84.0 / 78.4, 3,000 and 3,100 122.7 / 103.6, 2,000, 3,691 and 2,500 195 / 134, with heads of 128 278 / 203): the heaviest
+    // items of every request are first in that request alone. From three rounds on the counter is no slower (8,192 tokens 312 / 310))
     int* counter = n_items <= 2 * resident ? nullptr : queue;
     hipLaunchKernelGGL(kernel, dim3(beside.blocks + (n_items < resident ? n_items : resident)), dim3(256), LDS, stream,
                        q, kc, vc, out, q_start, ctx_len, table, max_blocks, n_seq, n_q, n_kv, page, scale, window, items,

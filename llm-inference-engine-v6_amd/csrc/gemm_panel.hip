@@ -5,8 +5,8 @@
 // they must (273 rows x 16,384 columns in tiles of 96 x 64: 503 MB over the chip), and a compute unit gets 55 to 90 bytes a ns.
 // So the tile takes its height from the rows (BM = 16 MT, up to 192) x BN = 64 or 128 columns (bfloat16: 192 and 256 too), one workgroup of
 // eight wavefronts a compute unit, with as many bytes on their way as LDS holds:
-//  * BN / 32 wavefronts share out the columns (32 each; of a tile of 192 or 256 four wavefronts 48 or 64 each). bfloat16: the KS = 256 / BN wavefronts of a group of columns share out its rows of
-//    tiles, and each adds up all of k in turn, so that a sum has the one order that every other tile kernel gives it: whichever tile
+//  * BN / 32 wavefronts share out the columns (32 each; of a tile of 192 or 256 four wavefronts 48 or 64 each). bfloat16: the KS wavefronts of a group of columns (256 / BN;
+//    two with 192 and 256) share out its rows of tiles, and each adds up all of k in turn, so that a sum has the one order that every other tile kernel gives it: whichever tile
 //    a product's rows are given, its results are the same bits. (Sharing out k instead, with the parts joined through LDS at
 //    the end, reads a fifth less of LDS and was no faster: parts of the 1B o-proj at 273 rows 8.2 / 8.0 us, of its down-proj 17.6 / 16.5,
 //    of the 8B down-proj at 528 rows 69.9 / 70.0, and with other orders of sums a prompt's bfloat16 logits moved by their rounding
@@ -395,7 +395,7 @@ static int launch_panel_mode(int mt, int bn, const T* A, const T* W, void* out, 
     LLME_PANEL(11, 128)
     LLME_PANEL(12, 128)
 #undef LLME_PANEL
-    // bfloat16 only: three or four tiles of columns a wavefront (48 columns are no pairs of gate and up), from 160 rows on in slabs of 32 k
+    // bfloat16 only: three or four tiles of columns a wavefront (48 columns are no pairs of gate and up); those that HALF is for in slabs of 32 k
     if constexpr (sizeof(T) == 2) {
 #define LLME_PANEL(MT, BN, HALF) \
     if (mt == MT && bn == BN) return launch_panel<T, MT, 4, 2, BN / 64, HALF, MODE>(A, W, out, M, N, K, ksplit, qt, gx, stream);
@@ -434,8 +434,8 @@ int gemm_panel_f32(int mt, int bn, int mode, const float* A, const float* W, flo
 
 // Tiles of 192 and 256 columns are there for the rounds that they save: a product takes whole rounds of one tile a compute unit, and
 // what fills one and a half rounds of 128 x 128 is one round of 128 x 192 (16 x 16 of them cover 2,048 x 3,072). A turn of 128 x 192 x 64 takes
-// 0.63 us, of 128 x 128 0.46 (0.26 of it the matrix pipes at the 2.0 GHz that the chip holds under them, 0.31 the loads alone). From 160 x 192 on three
-// slabs of 64 k are all that LDS holds, too few: 192 x 192 x 64 took 1.15 us. HALF slabs of 32 k make the ring six places (192 x 256: five) for a
+// 0.63 us, of 128 x 128 0.46 (0.26 of it the matrix pipes at the 2.0 GHz that the chip holds under them, 0.31 the loads alone). Of 160 x 192, 192 x 192 and
+// both tiles of 256 columns LDS holds three slabs of 64 k at most, too few: 192 x 192 x 64 took 1.15 us. HALF slabs of 32 k make their ring six places (192 x 256: five) for a
 // barrier every 32 k: 0.95 us. A's chunks are then 16 rows x 32 k: four lanes a row are 64 bytes side by side, which is what the loads'
 // path wants, and a row's four pieces are permuted by 0 2 3 1 of its number's bits 2 and 3, so that the 16 lanes that LDS serves at a time
 // (0-3, 12-15, 20-23, 24-27 and so on) meet no bank twice. Measured (us, weights from memory, the best before / with these; one round unless said):

@@ -92,24 +92,23 @@ class KernelChoices:
     prefill_min_run: int = 512
     prefill_max_splits: int = 16
     # Two runs are not worth their join: a 256-token portion beside 17 decoded tokens at the 1B sizes takes
-    # 2.18 ms in two runs against 2.07 whole behind 1,024 tokens, 2.28 against 2.27 behind 2,048 (four
-    # runs: 2.20), and behind 3,000 tokens 2.32 in three or six runs against 2.49 whole.
-    # (A whole prompt of 2,048 tokens, whose last rows' items walk twice the average, was also tried with
+    # 1.788 ms in two runs (1.797 in four) against 1.666 whole behind 1,024 tokens, and behind 2,048 four runs win: 1.817
+    # against 1.840 whole; behind 3,072 1.912 against 2.032, behind 4,096 1.963 against 2.214. (At the 8B sizes, heads of 128,
+    # 4 layers, four runs behind 2,048 tokens are 3 % slower than whole keys: 1.050 / 1.017.)
+    # (With the kernel before this one, a whole prompt of 2,048 tokens, whose last rows' items walk twice the average, was also tried with
     # the items behind 1,024 keys cut in two: 6.5 to 6.6 ms against 5.95 whole; the partial outputs and
     # the join cost more than the evener load wins.)
     prefill_min_splits: int = 3
     # More than a quarter of a workgroup per compute unit (65 to 128 items on 256 units: portions of 257
     # to 512 tokens of 32 heads): the keys are cut only where an item has at least this many keys for
-    # every item of the step, since whole keys in items of half the rows are faster until then and the
-    # join costs 13 us a layer whatever the length. Measured at the 1B sizes beside 17 decoded tokens (ms a
-    # step, cut / whole): 320 tokens behind 2,048: 2.55 / 2.32, behind 4,096: 2.61 / 2.63, behind 8,192:
-    # 2.91 / 3.29; 512 tokens behind 1,024: 2.83 / 2.49, behind 4,096: 3.10 / 2.95, behind 8,192: 3.55 / 3.62,
-    # behind 16,384: 4.44 / 4.97; 768 tokens (192 items, cut in four) behind 8,192: 4.85 / 4.85, behind 16,384:
-    # 6.31 / 6.85, behind 32,768: 9.12 / 10.91. (Up to 64 items the cut never lost: 256 tokens behind 8,192:
-    # 2.53 / 3.09.)
-    # For heads of 64; a key of a head of 128 is twice the work, and half as many keys are long: at the 8B
-    # sizes (8 layers) 768 tokens behind 8,192: 5.46 / 6.32, at the 3B sizes 3.53 / 4.68, behind 1,024 whole
-    # keys win at both (4.33 / 4.42 and 2.64 / 2.73 whole / cut).
+    # every item of the step (of heads of 128 half as many), since whole keys in items of half the rows are faster until then and the
+    # join costs a launch a layer whatever the length. The line was drawn with the kernel before this one, whose walks were longer. Measured
+    # with this one beside 17 decoded tokens, ms a step, cut / whole, 1B sizes: 320 tokens behind 2,048: 1.933 / 1.947, behind 4,096 (whole by the
+    # line): 2.110 / 2.311, behind 8,192: 2.311 / 3.031; 512 tokens behind 1,024: 2.505 / 2.297, behind 4,096: 2.811 / 2.843, behind 8,192: 3.093 /
+    # 3.600, behind 16,384: 3.678 / 5.114; 768 tokens (192 items, cut in four) behind 4,096: 3.551 / 3.217, behind 8,192: 4.051 / 3.972, behind 16,384:
+    # 5.062 / 5.485: with heads of 64 some 48 would do. With heads of 128 whole keys hold on longer than the line says: 768 tokens behind 8,192
+    # at the 3B sizes (8 layers) 2.882 / 2.744, at the 8B sizes (4 layers) 2.241 / 2.211; 512 behind 4,096 1.555 / 1.553; behind 1,024 whole keys
+    # win at both (768 tokens 2.188 / 2.055 and 1.918 / 1.793).
     prefill_cut_keys_per_item: int = 64
 
     def key(self) -> tuple:
