@@ -903,7 +903,8 @@ static bool squares_through_registers(int M, int N, int cus) {
 //    53 / 46.3). The squared rectifier's 5.5 + 0.0207 a k, whose end is short (1,800 rows x 12,288 x 2,048 94 against 98 here, x 4,096 178 / 190; 273 rows
 //    31.3 / 23.8); what these do not take is left to the code below, which knows the 256 x 256 tiles of squares too (1,800 x 5,120 x 1,024 27.2,
 //    29.4 where this one chose).
-//  * these take 1.17 (added) or 1.06 (stored) times their plan, which was fitted to all kinds.
+//  * these take 1.17 (added; in tiles of 192 and 256 columns with a short k 1.25: 3,213 x 3,072 x 3,072 72.4 us against 67.1 in 256 x 256, 2,059 rows 56.5
+//    against 53.0 through registers) or 1.06 (stored) times their plan, which was fitted to all kinds.
 //  * 128 x 128 tiles through registers, two a compute unit, take 3 us + 0.0070 to 0.0187 a k, by how many units have two (against these: added
 //    2,048 x 3,072 x 3,072 52.5 / 57.7, 2,048 x 4,096 x 4,096 78.7 / 85.1, but 1,500 rows 77.9 / 52.7; stored 4,096 x 1,536 x 2,048 33.3 /
 //    37.3, 1,024 x 6,144 x 4,096 62.3 / 66.8, but 1,024 x 5,136 x 2,048 35.5 / 27.5). Stored outputs of very many columns wait for W: 66 rows x
@@ -920,7 +921,7 @@ static int choose_direct(int mode, int M, int N, int K, bool may_cut, int cus, P
     auto tiles = [&](int edge) { return static_cast<long>((M + edge - 1) / edge) * ((N + edge - 1) / edge); };
     float large = static_cast<float>((tiles(256) + cus - 1) / cus) * (mode == kSquaredReluBF16 ? 5.5f + 0.0207f * K : 4.f + 0.0235f * K);
     if (is_gated(mode)) return plan.us <= large ? 1 : 2;
-    const float here = plan.us * (mode == kAddF32 ? 1.17f : 1.06f);
+    const float here = plan.us * (mode != kAddF32 ? 1.06f : plan.bn > 128 && K < 4096 ? 1.25f : 1.17f);
     const long t128 = tiles(128), rounds = (t128 + 2 * cus - 1) / (2 * cus);
     float staged = large + 1.f;
     if (t128 > cus) staged = rounds * (3.f + (0.0070f + 0.0117f * t128 / (2 * cus * rounds)) * K);

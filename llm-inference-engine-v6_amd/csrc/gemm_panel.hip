@@ -451,6 +451,11 @@ int gemm_panel_f32(int mt, int bn, int mode, const float* A, const float* W, flo
 // joined by their 2.5th powers with W's way from memory (1.2 us + 5.6 TB/s); parts cost their way out and back in the kernel that joins
 // them, 0.3 us a MB.
 // HALF slabs: 0.93 (k = 2,048) to 1.09 (14,336) of it, 1.03 times that in more rounds than one (the chip's clock falls in long products).
+// Products that are not cut: tiles of 192 and 256 columns take 3 to 6 % longer than that against the narrower ones, 160 and 192 x 192 in more rounds
+// than one up to 20 % (a fit to 650 pairs of 130 to 4,096 rows at the same sizes). Without it sizes that two tiles of one area cover in as many rounds,
+// or a wide one in a round less, went to the slower: added 1,779 x 3,072 x 8,192 in 128 x 192 93.0 us, in 192 x 128 85.2; stored 2,641 x 6,160 x 3,072 in
+// two rounds of 192 x 192 117, in three of 192 x 128 108, 3,397 rows in three of 160 x 192 153, in four of 176 x 128 135; gated 540 x 16,384 x 3,072 in one
+// of 192 x 256 67.8, in two of 144 x 128 62.7.
 // wide: 32-bit operands, whose products take the time (a compute unit makes 500 a ns).
 // ks_only: the number of parts (0: up to 8, of at least 256 k); heads: tiles hold whole heads of this many columns; pairs: a wavefront holds
 // whole pairs of gate and up (32 columns each, which the 48 of a tile of 192 are not).
@@ -473,9 +478,10 @@ PanelPlan panel_plan(int M, int N, int K, int ks_only, int heads, bool wide, boo
     Set& set = memo[mixed >> 28];
     for (const Made& m : set.made)
         if (m.M == M && m.N == N && m.K == K && m.other == other) return m.plan;
-    static const int shapes[][2] = {{2, 64}, {3, 64}, {4, 64}, {5, 64}, {6, 64}, {3, 128}, {4, 128}, {5, 128}, {6, 128},
-                                    {7, 128}, {8, 128}, {9, 128}, {10, 128}, {11, 128}, {12, 128},
-                                    {6, 192}, {8, 192}, {10, 192}, {12, 192}, {8, 256}, {12, 256}};
+    // rows / 16, columns, and how much longer than estimated a tile takes, against those of 64 and 128 columns, in hundredths
+    static const int shapes[][3] = {{2, 64, 0}, {3, 64, 0}, {4, 64, 0}, {5, 64, 0}, {6, 64, 0}, {3, 128, 0}, {4, 128, 0}, {5, 128, 0}, {6, 128, 0},
+                                    {7, 128, 0}, {8, 128, 0}, {9, 128, 0}, {10, 128, 0}, {11, 128, 0}, {12, 128, 0},
+                                    {6, 192, 4}, {8, 192, 3}, {10, 192, 6}, {12, 192, 6}, {8, 256, 3}, {12, 256, 4}};
     const int cus = compute_units();
     PanelPlan best{0, 0, 0, 0, 0.f};
     for (const auto& s : shapes) {
@@ -493,6 +499,7 @@ PanelPlan panel_plan(int M, int N, int K, int ks_only, int heads, bool wide, boo
             const float chip = of_half * rounds * (3.2f + 2.9f * area / 16384.f + (multiplied > bytes / rate ? multiplied : bytes / rate));
             const float memory = 1.2f + size * 1e-6f * N * K / 5.6f;
             float us = powf(powf(chip, 2.5f) + powf(memory, 2.5f), 0.4f);
+            if (ks_only == 1) us *= half && bn == 192 && rounds > 1 ? 1.2f : 1.f + 0.01f * s[2];
             if (ks > 1) us += 0.3f * 4e-6f * ks * M * N;
             if (best.mt == 0 || us < best.us) best = PanelPlan{s[0], bn, ks, static_cast<int>(rounds), us};
         }

@@ -80,11 +80,11 @@ def _chosen_on_256_units(ops, want, *args):
 # sizes at which each of these tiles is the chosen one, stored and added, or gated (two of them hold pairs), at the least k that they are chosen for
 # and above; and sizes just outside, where the tiles through registers (0), 256 x 256 or narrower panels are
 @pytest.mark.parametrize("M,N,K,gated,tile", [
-    (329, 12288, 2048, False, PANEL + 96192), (1924, 3072, 1024, False, PANEL + 128192), (403, 12288, 2048, False, PANEL + 128192),
+    (329, 12288, 2048, False, PANEL + 96192), (403, 12288, 2048, False, PANEL + 128192),
     (2300, 3072, 2048, False, PANEL + 160192), (1800, 4608, 2048, False, PANEL + 192192), (390, 16384, 2048, False, PANEL + 128256),
-    (2119, 4096, 1024, False, PANEL + 192256), (218, 28672, 512, True, PANEL + 128256), (390, 12288, 512, True, PANEL + 128256),
+    (514, 16384, 2048, False, PANEL + 192256), (218, 28672, 512, True, PANEL + 128256), (390, 12288, 512, True, PANEL + 128256),
     (292, 28672, 2048, True, PANEL + 192256), (1287, 6144, 1024, True, PANEL + 192256),
-    (2048, 3072, 544, False, 0), (2995, 3072, 512, False, 256256), (1400, 16384, 512, True, 256256), (1000, 3072, 8192, False, PANEL + 112128)])
+    (1924, 3072, 1024, False, 0), (2119, 4096, 1024, False, 256256), (2048, 3072, 544, False, 0), (2995, 3072, 512, False, 256256), (1400, 16384, 512, True, 256256), (1000, 3072, 8192, False, PANEL + 112128)])
 def test_the_chosen_wide_panel_adds_in_the_order_of_the_others(ops, M, N, K, gated, tile):
     a, w = _pair(M, N, K, 25)
     ad, wb = a.to(DEV), ops.block_weight(w.to(DEV))
@@ -127,7 +127,7 @@ def test_the_chosen_wide_panel_of_a_sum_in_parts(ops, M, N, K, n, tile):
 # (0: the chosen tile is no panel)
 @pytest.mark.parametrize("M,N,K,tile", [(65, 48, 512, PANEL + 32064), (200, 528, 2080, PANEL + 32064), (273, 12288, 512, 0), (1500, 3072, 544, 0),
                                         (249, 12288, 1024, 0),
-                                        (325, 12288, 1024, PANEL + 96192), (1287, 6144, 1024, PANEL + 192192)])
+                                        (325, 12288, 1024, 0), (329, 12288, 2048, PANEL + 96192), (1287, 6144, 1024, PANEL + 192192)])
 def test_squared_rectifier_behind_the_panels(ops, M, N, K, tile):
     """The squared positive part, stored in bfloat16: every tile and the chosen one give the bits of the square of the stored sum."""
     _chosen_on_256_units(ops, tile, "squared", M, N, K)
